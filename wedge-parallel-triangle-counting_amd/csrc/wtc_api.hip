@@ -154,10 +154,11 @@ namespace {
 // Byte offsets of the pieces of a split count's workspace in one buffer
 // (each on a 256-byte boundary), and the buffer's size.
 struct SplitLayout {
-    size_t wsfull, hist1, part_base, c2base, hist2, sub_base, c3base, hist3, sub_tot, list_bid, slab_row, key_tot;
+    size_t wsfull, tile_v, part_base, part_cnt, c2base, hist2, sub_base, c3base, hist3, sub_tot, list_bid, slab_row, key_tot;
     size_t part_tot, key_part;
     size_t recid, rec, recaux, recid2, rec2, recaux2, rpin, rp32, total;
-    uint32_t chunks, slabs, keys, parts, subs, c2cap, c3cap;
+    uint32_t slabs, subs, chunk;
+    SplitGrids g;
     uint64_t cap;
     int ob;  // offset width of the split kernels (4 for a narrowed 8-byte CSR)
 };
@@ -180,14 +181,26 @@ SplitLayout split_plan(uint32_t n, uint64_t m, uint32_t rows, int ob_in) {
     const bool narrow = split_narrow(ob_in, m);
     const int ob = narrow ? 4 : ob_in;
     L.ob = ob;
-    L.chunks = std::min<uint32_t>(kSplitChunksMax, std::max<uint32_t>(1, n / kSplitChunkVerts));
     L.slabs = (uint32_t)split_slabs(m);
-    L.keys = rows + L.slabs;
-    L.parts = (L.keys + kSplitPart - 1) / kSplitPart;
-    L.subs = L.parts * kSplitFan2;
+    L.g.keys = rows + L.slabs;
     L.cap = std::max<uint64_t>(m, 1);  // an in-edge is an edge
-    L.c2cap = (uint32_t)((L.cap + kSplitChunk2 - 1) / kSplitChunk2) + L.parts;
-    L.c3cap = (uint32_t)((L.cap + kSplitChunk3 - 1) / kSplitChunk3) + L.subs;
+    // the smallest parts that kSplitPartsMax of them cover the keys with;
+    // while a part's keys are few enough, the second level is the last
+    uint32_t shift = kSplitFinalMin;
+    while (((uint64_t)L.g.keys + (1ull << shift) - 1) >> shift > kSplitPartsMax) shift++;
+    const bool three = shift > kSplitFinalMax;
+    L.g.part_shift = shift;
+    L.g.final_shift = three ? kSplitSubShift : shift;
+    L.g.parts = (uint32_t)(((uint64_t)L.g.keys + (1ull << shift) - 1) >> shift);
+    L.subs = three ? L.g.parts << (shift - kSplitSubShift) : 0;
+    // about a thousand blocks a level, within the limits of a block
+    uint64_t chunk = kSplitChunkMin;
+    while (chunk < kSplitChunkMax && L.cap / chunk > 1024) chunk *= 2;
+    L.chunk = (uint32_t)chunk;
+    L.g.chunks = (uint32_t)std::min<uint64_t>(kSplitChunksMax, std::max<uint64_t>(1, L.cap / kSplitChunkEdges));
+    const uint32_t blocks = (uint32_t)((L.cap + chunk - 1) / chunk);
+    L.g.c2cap = three ? blocks + L.g.parts : 0;
+    L.g.c3cap = blocks + (three ? L.subs : L.g.parts);
     size_t off = 0;
     auto take = [&](size_t bytes) {
         const size_t at = off;
@@ -196,26 +209,27 @@ SplitLayout split_plan(uint32_t n, uint64_t m, uint32_t rows, int ob_in) {
     };
     const size_t pair = 2 * (size_t)ob;
     L.wsfull = take(2 * ((size_t)n + 1) * sizeof(uint64_t));  // ws_full, then ie_pre
-    L.hist1 = take((size_t)L.chunks * L.parts * sizeof(uint64_t));
-    L.part_base = take(((size_t)L.parts + 1) * sizeof(uint64_t));
-    L.c2base = take(((size_t)L.parts + 1) * sizeof(uint32_t));
-    L.hist2 = take((size_t)L.c2cap * kSplitFan2 * sizeof(uint32_t));
-    L.sub_base = take(((size_t)L.subs + 1) * sizeof(uint64_t));
-    L.c3base = take(((size_t)L.subs + 1) * sizeof(uint32_t));
-    L.hist3 = take((size_t)L.c3cap * kSplitSub * sizeof(uint32_t));
+    L.tile_v = take((size_t)(L.cap / kSplitTileMin + 1) * sizeof(uint32_t));
+    L.part_base = take((size_t)L.g.parts * sizeof(uint64_t));
+    L.part_cnt = take((size_t)L.g.parts * sizeof(uint64_t));
+    L.c2base = take(((size_t)L.g.parts + 1) * sizeof(uint32_t));
+    L.hist2 = take((size_t)L.g.c2cap * kSplitFan2 * sizeof(uint32_t));
+    L.sub_base = take((size_t)L.subs * sizeof(uint64_t));
+    L.c3base = take(((size_t)std::max(L.subs, L.g.parts) + 1) * sizeof(uint32_t));
+    L.hist3 = take(((size_t)L.g.c3cap << L.g.final_shift) * sizeof(uint32_t));
     L.sub_tot = take((size_t)L.subs * sizeof(uint32_t));
-    L.list_bid = take((size_t)L.parts * sizeof(uint32_t));
+    L.list_bid = take((size_t)L.g.parts * sizeof(uint32_t));
     L.slab_row = take(((size_t)L.slabs + 1) * sizeof(uint32_t));
-    L.part_tot = take((size_t)L.parts * sizeof(uint64_t));
-    L.key_part = take(((size_t)L.keys / kKeyChunk + 2) * sizeof(uint64_t));
-    L.key_tot = take((size_t)L.keys * sizeof(uint32_t));
+    L.part_tot = take((size_t)L.g.parts * sizeof(uint64_t));
+    L.key_part = take(((size_t)L.g.keys / kKeyChunk + 2) * sizeof(uint64_t));
+    L.key_tot = take((size_t)L.g.keys * sizeof(uint32_t));
     L.recid = take((size_t)L.cap * sizeof(uint16_t));
     L.rec = take((size_t)L.cap * pair);
     L.recaux = take((size_t)L.cap * sizeof(uint32_t));
-    L.recid2 = take((size_t)L.cap * sizeof(uint8_t));
+    L.recid2 = take(three ? (size_t)L.cap * sizeof(uint8_t) : 0);
     L.rec2 = take((size_t)L.cap * pair);
     L.recaux2 = take((size_t)L.cap * sizeof(uint32_t));
-    L.rpin = take(((size_t)L.keys + 1) * (size_t)ob);
+    L.rpin = take(((size_t)L.g.keys + 1) * (size_t)ob);
     L.rp32 = narrow ? take(((size_t)n + 1) * sizeof(uint32_t)) : 0;
     L.total = off;
     return L;
@@ -225,22 +239,25 @@ SplitLayout split_plan(uint32_t n, uint64_t m, uint32_t rows, int ob_in) {
 
 size_t split_workspace_bytes(uint32_t n, uint64_t m, uint32_t rows, int ob) { return split_plan(n, m, rows, ob).total; }
 
-int split_layout(SplitDesc *sd, char *base, uint32_t n, uint64_t m, uint32_t rows, int ob, uint32_t **rp32) {
+int split_layout(SplitDesc *sd, SplitGrids *grids, char *base, uint32_t n, uint64_t m, uint32_t rows, int ob,
+                 uint32_t **rp32) {
     const SplitLayout L = split_plan(n, m, rows, ob);
+    *grids = L.g;
     if (rp32) *rp32 = L.rp32 ? reinterpret_cast<uint32_t *>(base + L.rp32) : nullptr;
     sd->rows = rows;
-    sd->keys = L.keys;
+    sd->keys = L.g.keys;
     sd->slabs = L.slabs;
-    sd->chunks = L.chunks;
-    sd->parts = L.parts;
+    sd->parts = L.g.parts;
+    sd->part_shift = L.g.part_shift;
+    sd->final_shift = L.g.final_shift;
     sd->subs = L.subs;
+    sd->chunk = L.chunk;
     sd->cap = L.cap;
-    sd->c2cap = L.c2cap;
-    sd->c3cap = L.c3cap;
     sd->ws_full = reinterpret_cast<uint64_t *>(base + L.wsfull);
     sd->ie_pre = sd->ws_full + (size_t)n + 1;
-    sd->hist1 = reinterpret_cast<uint64_t *>(base + L.hist1);
+    sd->tile_v = reinterpret_cast<uint32_t *>(base + L.tile_v);
     sd->part_base = reinterpret_cast<uint64_t *>(base + L.part_base);
+    sd->part_cnt = reinterpret_cast<uint64_t *>(base + L.part_cnt);
     sd->c2base = reinterpret_cast<uint32_t *>(base + L.c2base);
     sd->hist2 = reinterpret_cast<uint32_t *>(base + L.hist2);
     sd->sub_base = reinterpret_cast<uint64_t *>(base + L.sub_base);
@@ -259,8 +276,11 @@ int split_layout(SplitDesc *sd, char *base, uint32_t n, uint64_t m, uint32_t row
     sd->rec2 = base + L.rec2;
     sd->rec_aux2 = reinterpret_cast<uint32_t *>(base + L.recaux2);
     sd->rp_in = base + L.rpin;
-    sd->ie = sd->rec;  // the third level writes the pairs over A's
-    sd->ie_aux = sd->rec_aux;
+    // the final level reads B and writes over A, or reads A and writes where B would be
+    const bool three = L.subs != 0;
+    sd->ie = three ? sd->rec : sd->rec2;
+    sd->ie_aux = three ? sd->rec_aux : sd->rec_aux2;
+    sd->packed = three ? sd->rec2 : sd->rec;
     return L.ob;
 }
 
@@ -269,7 +289,7 @@ int split_layout(SplitDesc *sd, char *base, uint32_t n, uint64_t m, uint32_t row
 // against the bitmap in HBM, as the reference does.
 bool split_eligible(const Tuning &t, const GraphDesc &d, uint64_t m) {
     return t.kernel == kKernelSplit && d.mode == kModeTiles && d.a > 0 && d.bm_rows > 0 &&
-           (uint64_t)d.bm_rows + split_slabs(m) <= (uint64_t)kSplitPartsMax * kSplitPart &&
+           (uint64_t)d.bm_rows + split_slabs(m) <= (uint64_t)kSplitPartsMax << kSplitPartMax &&
            split_rows_lds(d.bm_rows) <= t.lds_bytes && (reinterpret_cast<uintptr_t>(d.colInd) & 15u) == 0;
 }
 
@@ -366,7 +386,7 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
             base = s.sp.as<char>();
         }
         uint32_t *rp32 = nullptr;
-        split_ob = split_layout(&sd, base, hd[0].n, m[0], split_rows, ob, &rp32);
+        split_ob = split_layout(&sd, &plan->split_grids, base, hd[0].n, m[0], split_rows, ob, &rp32);
         if (rp32) {  // the split kernels read the 4-byte copy the count starts by making
             split_rp_src = static_cast<const uint64_t *>(hd[0].rowPtr);
             split_rp_dst = rp32;
@@ -413,11 +433,6 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
     plan->split = split;
     plan->split_off = split_off;
     plan->split_rows = split_rows;
-    plan->split_chunks = sd.chunks;
-    plan->split_keys = sd.keys;
-    plan->split_c2cap = sd.c2cap;
-    plan->split_c3cap = sd.c3cap;
-    plan->split_parts = sd.parts;
     plan->split_key_part = sd.key_part;
     plan->split_wpb = t.split_wpb;
     plan->split_ob = split_ob;
@@ -440,8 +455,7 @@ int launch_set(Slot &s, const SetPlan &p, bool timed) {
         WTC_HIPC(launch_split_prefix(ddesc, sd, ob, p.blocks, s.partials.as<uint64_t>(), s.stream));
         WTC_HIPC(launch_split_range(ddesc, sd, ob, s.stream));
         if (timed) WTC_HIPC(hipEventRecord(s.ev[1], s.stream));
-        WTC_HIPC(launch_split_transpose(ddesc, sd, ob, p.split_chunks, p.split_c2cap, p.split_c3cap, p.split_parts,
-                                        p.split_keys, p.split_key_part, meta, dcounts, s.stream));
+        WTC_HIPC(launch_split_transpose(ddesc, sd, ob, p.split_grids, p.split_key_part, meta, dcounts, s.stream));
         if (timed) WTC_HIPC(hipEventRecord(s.ev[2], s.stream));
         WTC_HIPC(launch_split_rows(ddesc, sd, ob, p.split_rows, p.split_wpb, meta, dcounts, s.rows_grid,
                                    s.stream));

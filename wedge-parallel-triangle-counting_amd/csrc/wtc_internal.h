@@ -173,7 +173,8 @@ struct SetPlan {
     // split count: SplitDesc at byte split_off of the descriptor buffer
     bool split = false;
     size_t split_off = 0;
-    uint32_t split_rows = 0, split_keys = 0, split_chunks = 0, split_c2cap = 0, split_c3cap = 0, split_parts = 0;
+    uint32_t split_rows = 0;
+    SplitGrids split_grids;
     uint32_t split_wpb = 8;
     uint64_t *split_key_part = nullptr;  // device: the key-block prefix of the transposition
     // offset width of the split kernels, and for a narrowed 8-byte CSR the
@@ -210,7 +211,8 @@ size_t split_workspace_bytes(uint32_t n, uint64_t m, uint32_t rows, int ob);
 // whose positions fit 32 bits, split_narrow) and, through rp32, where the
 // count copies its row offsets to 4 bytes (null when not narrowed).
 bool split_narrow(int ob, uint64_t m);
-int split_layout(SplitDesc *sd, char *base, uint32_t n, uint64_t m, uint32_t rows, int ob, uint32_t **rp32 = nullptr);
+int split_layout(SplitDesc *sd, SplitGrids *grids, char *base, uint32_t n, uint64_t m, uint32_t rows, int ob,
+                 uint32_t **rp32 = nullptr);
 // Waits for the slot (or, if it is done, does not wait) and reads results.
 int finish_set(Slot &s, uint64_t *counts, uint64_t *wedges, RunTimes *rt);
 // True when the slot's last enqueue has completed.

@@ -95,22 +95,23 @@ enum : int {
 };
 
 // Split count of one graph (wtc_split.hip).  The in-edges are grouped by key
-// in three counting-sort levels: by part of kSplitPart keys, by sub-part of
-// kSplitSub keys (kSplitFan2 per part), by key.  Each level's scatter keeps
-// at most kSplitFan2 or kSplitSub output runs open per block, so that the
-// lines of a run fill in the L2 cache before they are written back.
-// kSplitChunk2/3: records per block of the second and third levels;
-// kSplitBlock: threads per transposition block; kSplitTile: in-edges per
-// tile of the row kernel.
-constexpr uint32_t kSplitPart = 32768;
+// in counting-sort levels: by part of 1 << part_shift keys, at most
+// kSplitPartsMax parts, then by key.  With up to kSplitPartsMax <<
+// kSplitFinalMax keys (R-MAT-24: 389,000) a part is at most 1 <<
+// kSplitFinalMax keys and the second level groups by key; beyond that (up to
+// kSplitPartsMax << kSplitPartMax keys), parts are first grouped by sub-part
+// of kSplitSub keys (at most kSplitFan2 a part).  kSplitBlock: threads per
+// transposition block; kSplitTile: in-edges per tile of the row kernel.
+constexpr uint32_t kSplitPartMax = 15;
 constexpr uint32_t kSplitPartsMax = 256;
-constexpr uint32_t kSplitSub = 256;
+constexpr uint32_t kSplitFinalMin = 8, kSplitFinalMax = 11;
 constexpr uint32_t kSplitSubShift = 8;
-constexpr uint32_t kSplitFan2 = kSplitPart / kSplitSub;
-static_assert(kSplitSub == 1u << kSplitSubShift && kSplitFan2 * kSplitSub == kSplitPart, "key levels");
-static_assert(kSplitPart <= 65536 && kSplitSub <= 256, "A keys fit 16 bits, B keys 8");
-constexpr uint32_t kSplitChunk2 = 65536;
-constexpr uint32_t kSplitChunk3 = 65536;
+constexpr uint32_t kSplitSub = 1u << kSplitSubShift;
+constexpr uint32_t kSplitFan2 = 1u << (kSplitPartMax - kSplitSubShift);
+static_assert(kSplitPartMax <= 16 && kSplitSubShift <= 8, "A keys fit 16 bits, B keys 8");
+// Records per block of the second and final levels: kSplitChunkMax, or as
+// few as kSplitChunkMin for small graphs, so that the levels fill the GPU.
+constexpr uint32_t kSplitChunkMax = 65536, kSplitChunkMin = 8192;
 constexpr int kSplitBlock = 1024;
 constexpr uint32_t kSplitTile = 1024;
 // Keys per block of the key-offset scan (four per thread).
@@ -131,45 +132,49 @@ constexpr uint32_t kSlabTile = 1024;
 // width.  Every in-edge (v, j) (j a position of adj+(v) other than its last)
 // is grouped by a key: w - thr for w = colInd[j] >= thr (a top row), else
 // rows + the slab of w.  Records (key, pair, slab_aux) go through the
-// levels A -> B -> ie: A bucketed by part, B by sub-part, ie by key (the
-// pairs only, in A's pair array; a list record's slab_aux in A's aux
-// array).  A record's position names its part (in A) or sub-part (in B), so
-// A keeps the key's low 15 bits and B its low 8.  A top record's pair is the tail [lo, hi) of colInd; a list
+// levels A -> ie or A -> B -> ie: A bucketed by part, B by sub-part, ie by
+// key (the pairs, and a list record's slab_aux), in the arrays of the level
+// before the last: B's when there is no B.  A record's position names its
+// part (in A) or sub-part (in B), so A keeps the key's low part_shift bits
+// and B its low 8.  A top record's pair is the tail [lo, hi) of colInd; a list
 // record's is (j, hi), its tail [j + 1, hi) (the one in-edge whose tail the
 // range cuts at the front: [clip_lo, hi)).
 struct SplitDesc {
     uint64_t *ws_full;    // n+1: the full wedge prefix
     uint64_t *ie_pre;     // n+1: prefix of the in-edges (positions of adj+(v) but the last) of each row
-    uint64_t *hist1;      // chunks x parts: first-level counts, then record offsets
-    uint64_t *part_base;  // parts+1: first record of each part; part_base[parts] = the in-edges
+    uint32_t *tile_v;     // first-level tiles: the vertex each starts in
+    uint64_t *part_base;  // parts: first record slot of each part
+    uint64_t *part_cnt;   // parts: records of each part so far
     uint32_t *c2base;     // parts+1: first second-level block of each part
     uint32_t *hist2;      // c2cap x kSplitFan2: second-level counts, then column prefixes
-    uint64_t *sub_base;   // subs+1: first record of each sub-part
-    uint32_t *c3base;     // subs+1: first third-level block of each sub-part
-    uint32_t *hist3;      // c3cap x kSplitSub: third-level counts, then column prefixes
+    uint64_t *sub_base;   // subs: first record of each sub-part
+    uint32_t *c3base;     // final buckets+1: first final-level block of each part or sub-part
+    uint32_t *hist3;      // c3cap << final_shift: final-level counts, then column prefixes
     uint32_t *sub_tot;    // subs: records of each sub-part
     uint32_t *list_bid;   // parts: the first list vertex w whose key lies in each part (0 up to the first list part)
     uint32_t *slab_row;   // slabs+1: the first vertex w with rowPtr[w] >= s*kSlabSpan (set for s*kSlabSpan <= rowPtr[thr])
-    uint64_t *part_tot;   // parts: records of each part
+    uint64_t *part_tot;   // parts: record slots of each part (>= its records)
     uint64_t *key_part;   // key blocks: in-edges of each block of kKeyChunk keys, then their prefix
     uint32_t *key_tot;    // keys: in-edges of each key
-    uint16_t *rec_id;     // cap: A keys within their part (key mod kSplitPart)
-    void *rec;            // cap pairs of OffT: A pairs, then ie
-    uint32_t *rec_aux;    // cap: A slab_aux words (list records), then ie_aux
-    uint8_t *rec_id2;     // cap: B keys within their sub-part (key mod kSplitSub)
-    void *rec2;           // cap pairs of OffT: B pairs, then the packed top ids (three 21-bit ids per word)
+    uint16_t *rec_id;     // cap: A keys within their part
+    void *rec;            // cap pairs of OffT: A pairs
+    uint32_t *rec_aux;    // cap: A slab_aux words (list records)
+    uint8_t *rec_id2;     // cap: B keys within their sub-part
+    void *rec2;           // cap pairs of OffT: B pairs
     uint32_t *rec_aux2;   // cap: B slab_aux words
     void *rp_in;          // keys+1 OffT: first in-edge of each key
-    void *ie;             // = rec: the records' pairs grouped by key
-    uint32_t *ie_aux;     // = rec_aux: the list records' slab_aux words, beside ie
+    void *ie;             // the records' pairs grouped by key: rec2 (two levels) or rec (three)
+    uint32_t *ie_aux;     // the list records' slab_aux words, beside ie
+    void *packed;         // the packed top ids: over the pairs that ie is not in
     uint64_t cap;         // records each array holds (>= the in-edges)
     uint32_t rows;        // top rows: n - thr
     uint32_t keys;        // rows + slabs
-    uint32_t chunks;      // vertex chunks of the first level (about equal shares of the in-edges)
-    uint32_t parts;       // parts of kSplitPart keys (<= kSplitPartsMax)
-    uint32_t subs;        // sub-parts: parts * kSplitFan2
+    uint32_t parts;       // parts of 1 << part_shift keys (<= kSplitPartsMax)
+    uint32_t part_shift;  // log2 of a part's keys
+    uint32_t final_shift;  // log2 of the keys of a final-level bucket: part_shift, or kSplitSubShift with three levels
+    uint32_t subs;        // sub-parts (three levels)
     uint32_t slabs;       // slabs of the list rows: ceil(m / kSlabSpan)
-    uint32_t c2cap, c3cap;  // second- and third-level blocks the hists hold (>= those the records need)
+    uint32_t chunk;       // records per block of the second and final levels
     // device-filled by the range kernel
     uint64_t w_lo, w_hi;  // the counted wedges of the full order, clamped to [0, W]
     uint64_t clip_j;      // the in-edge whose tail the range cuts at the front (~0: none)
@@ -178,7 +183,6 @@ struct SplitDesc {
     uint32_t clip;        // 1 unless [w_lo, w_hi) is the whole order
     uint32_t pad_;
 };
-static_assert(sizeof(SplitDesc) == 280, "SplitDesc layout");
 
 // Where adj+(w) of a list row lies in its slab's window: bits 0-12 its start
 // rowPtr[w] - slab*kSlabSpan, bits 13-25 its length (kSlabAuxLong: longer

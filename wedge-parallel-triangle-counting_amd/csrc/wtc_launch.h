@@ -61,13 +61,17 @@ hipError_t launch_split_prefix(const GraphDesc *desc, const SplitDesc *sd, int o
 hipError_t launch_split_range(const GraphDesc *desc, SplitDesc *sd, int ob, hipStream_t st);
 // dst[i] = src[i] for i < count (8-byte row offsets below 2^32 to 4 bytes).
 hipError_t launch_split_narrow_offsets(const uint64_t *src, uint32_t *dst, uint64_t count, hipStream_t st);
-// The three-level counting sort of the in-edges by key (chunks first-level
-// blocks; c2cap and c3cap bound the second- and third-level blocks; parts
-// parts, keys keys; key_part = the SplitDesc's key_part, on the device);
-// zeroes the tile counters, the wedge tallies and counts[0].
-hipError_t launch_split_transpose(const GraphDesc *desc, const SplitDesc *sd, int ob, uint32_t chunks,
-                                  uint32_t c2cap, uint32_t c3cap, uint32_t parts, uint32_t keys, uint64_t *key_part,
-                                  uint64_t *meta, unsigned long long *counts, hipStream_t st);
+// The counting sort of the in-edges by key (key_part = the SplitDesc's
+// key_part, on the device); zeroes the tile counters, the wedge tallies and
+// counts[0].
+struct SplitGrids {
+    uint32_t chunks = 0;          // blocks of the first level
+    uint32_t c2cap = 0, c3cap = 0;  // bounds of the second and final levels' blocks
+    uint32_t parts = 0, keys = 0;
+    uint32_t part_shift = 0, final_shift = 0;  // equal: two levels, else three
+};
+hipError_t launch_split_transpose(const GraphDesc *desc, const SplitDesc *sd, int ob, const SplitGrids &g,
+                                  uint64_t *key_part, uint64_t *meta, unsigned long long *counts, hipStream_t st);
 // Waves per block of the row kernel: 4, 8 or 16.
 bool valid_split_waves(int wpb);
 // LDS bytes of the row kernel's bitmap for `rows` top rows.
@@ -80,11 +84,12 @@ hipError_t launch_split_rows(const GraphDesc *desc, const SplitDesc *sd, int ob,
 hipError_t split_slabs_grid(int ob, int num_cus, uint32_t *grid);
 hipError_t launch_split_slabs(const GraphDesc *desc, const SplitDesc *sd, int ob, uint64_t *meta,
                               unsigned long long *counts, uint32_t grid, hipStream_t st);
-// Vertex chunks of the transposition (equal shares of the in-edges): one
-// per kSplitChunkVerts vertices, at least 1 and at most kSplitChunksMax.
-constexpr uint32_t kSplitChunksMax = 1024;
-static_assert(kSplitChunksMax <= (uint32_t)kSplitBlock, "one first-level chunk per thread of the part scan");
-constexpr uint32_t kSplitChunkVerts = 2048;
+// Blocks of the transposition's first level: two per CU (its LDS), and no
+// more than a block per 8192 edges.
+constexpr uint32_t kSplitChunksMax = 512;
+constexpr uint32_t kSplitChunkEdges = 8192;
+// In-edges of the first level's smallest tile.
+constexpr uint32_t kSplitTileMin = 2048;
 
 // Fewest wedges a grab of the counting kernels covers: every grab is one
 // atomic on a shared counter, so a grab of a few 64-wedge tiles (spread 1)

@@ -25,15 +25,13 @@
 //
 // Pipeline on one stream: k_split_partials, k_scan_partials (twice) and
 // k_split_scan (the full wedge prefix and the in-edge prefix);
-// k_split_range; the transposition in three counting-sort levels,
-// k_split_l1count, k_split_l1cols, k_split_l1bases, k_split_l1
-// (records bucketed by part of kSplitPart keys), k_split_level_count<2>,
-// k_split_levelcols<2>, k_split_subscan, k_split_level_scatter<2> (each
-// part's records bucketed by sub-part of kSplitSub keys),
-// k_split_level_count<3>, k_split_levelcols<3>, k_split_keysum,
-// k_scan_partials, k_split_keyscan, k_split_level_scatter<3> (each
-// sub-part's records grouped by key), k_split_pack (colInd as 21-bit ids
-// above thr, over the second level's records);
+// k_split_range; the transposition, a counting sort by key: k_split_parthist
+// and k_split_partbase (part sizes), k_split_l1 (records bucketed by part),
+// k_split_bases; with many keys k_split_level_count, k_split_levelcols2,
+// k_split_bases and k_split_level_scatter to sub-parts; then
+// k_split_level_count, k_split_levelcols3, k_split_keysum, k_scan_partials,
+// k_split_keyscan and k_split_level_scatter by key; k_split_pack (colInd as
+// ids above thr of 16 to 21 bits, over the last level's input);
 // k_split_rows (top rows); k_split_slabs (list rows).
 #include <type_traits>
 #include <utility>
@@ -148,7 +146,8 @@ __global__ __launch_bounds__(kBlock) void k_split_scan(const GraphDesc *__restri
 // one in-edge whose tail the range cuts at the front (row i0 of v_lo holding
 // wedge w_lo: its tail starts w_lo - base(i0) ids in).  Thread q < parts:
 // list_bid[q], the first list vertex w (below thr) whose key rows +
-// rowPtr[w] / kSlabSpan lies in part q or later (keys grow with w).
+// rowPtr[w] / kSlabSpan lies in part q or later (keys grow with w), and the
+// part's counters zeroed.
 template <typename OffT>
 __global__ __launch_bounds__(kSplitPartsMax) void k_split_range(const GraphDesc *__restrict__ desc,
                                                                 SplitDesc *__restrict__ sd) {
@@ -157,10 +156,10 @@ __global__ __launch_bounds__(kSplitPartsMax) void k_split_range(const GraphDesc 
     const OffT *__restrict__ rowPtr = static_cast<const OffT *>(D.rowPtr);
     const uint32_t q = threadIdx.x;
     if (q < S.parts) {
-        const uint64_t first = S.rows / kSplitPart;  // the part of the first list key
+        const uint64_t first = S.rows >> S.part_shift;  // the part of the first list key
         uint32_t bid = 0;
         if (q > first) {
-            const uint64_t at = ((uint64_t)q * kSplitPart - S.rows) * kSlabSpan;  // colInd position
+            const uint64_t at = (((uint64_t)q << S.part_shift) - S.rows) * kSlabSpan;  // colInd position
             uint32_t lo = 0, hi = D.thr;  // the first w in [0, thr] with rowPtr[w] >= at (thr: none below)
             while (lo < hi) {
                 const uint32_t mid = lo + ((hi - lo) >> 1);
@@ -170,6 +169,8 @@ __global__ __launch_bounds__(kSplitPartsMax) void k_split_range(const GraphDesc 
             bid = lo;
         }
         S.list_bid[q] = bid;
+        S.part_tot[q] = 0;
+        S.part_cnt[q] = 0;
     }
     if (threadIdx.x != 0) return;
     const uint32_t n = D.n;
@@ -208,16 +209,6 @@ __global__ __launch_bounds__(kSplitPartsMax) void k_split_range(const GraphDesc 
 
 // ------------------------------------------------------------ transposition
 
-// First vertex of chunk c of `chunks`: the vertex holding in-edge
-// floor(c*K/chunks) (K = all in-edges), so that chunks hold about equal
-// shares of the in-edges; chunk `chunks` starts at n.  Wave-uniform.
-__device__ __forceinline__ uint32_t chunk_start(cptr<uint64_t> ie_pre, uint32_t n, uint32_t c, uint32_t chunks) {
-    if (c >= chunks) return n;
-    const uint64_t K = ie_pre[n];
-    const uint64_t t = (uint64_t)(((unsigned __int128)K * c) / chunks);
-    return rightmost_le(ie_pre, 0u, n - 1, t);
-}
-
 // Clips the tail [j+1, e) of in-edge j of an end vertex of the counted
 // range (row start rb, full-order base ws) to its wedges in [w_lo, w_hi):
 // the tail ids of row i = j - rb are the wedges [base, base + L) of the full
@@ -238,32 +229,40 @@ __device__ __forceinline__ void clip_tail(OffT j, OffT e, OffT rb, uint64_t ws, 
     }
 }
 
-// First-level count, by positions: block b counts the in-edges of vertex
-// chunk b (clipped to the counted vertices) per part into hist1[b][part],
-// the same in-edges the scatter pass of k_split_l1 takes.  An in-edge is a
-// position of adj+(v) other than the row's last, so the block counts every
-// position of its chunk's rows (colInd read once, coalesced), takes back
-// each row's last position, and, when the counted range clips its end
-// vertices, takes back their in-edges whose clipped tail is empty.  A list
-// vertex's part comes from list_bid (no rowPtr read).
+// Records staged in LDS per tile of a scatter: 4096 with 4-byte offsets,
+// 2048 with 8-byte ones (32 KB of pairs either way).
 template <typename OffT>
-__global__ __launch_bounds__(kSplitBlock) void k_split_l1count(const GraphDesc *__restrict__ desc,
-                                                               const SplitDesc *__restrict__ sd) {
+struct LevelTile {
+    static constexpr uint32_t kT = sizeof(OffT) == 4 ? 4096 : 2048;
+    static_assert(kT >= kSplitTileMin, "tile_v holds a vertex per tile");
+};
+
+// First-level part sizes, as an upper bound: every position of the counted
+// vertices' rows in its id's part (the in-edges are all of them but each
+// row's last, and fewer where the range clips a row).  Positions in order
+// run through a row's ascending ids, so neighbouring lanes mostly share a
+// part: one LDS atomic per run of equal parts instead of one per id, which
+// with few parts all fell on the same counters (R-MAT-20: 112 us).  A list
+// vertex's part comes from list_bid (no rowPtr read).  Also finds the vertex
+// that each tile of k_split_l1 starts in.
+template <typename OffT>
+__global__ __launch_bounds__(kSplitBlock) void k_split_parthist(const GraphDesc *__restrict__ desc,
+                                                                const SplitDesc *__restrict__ sd) {
     __shared__ uint32_t s_cnt[kSplitPartsMax];
     __shared__ uint32_t s_bid[kSplitPartsMax];
     const GraphDesc &D = desc[0];
     const SplitDesc &S = sd[0];
     const OffT *__restrict__ rowPtr = static_cast<const OffT *>(D.rowPtr);
     const gptr<uint32_t> colInd = to_global(D.colInd);
-    const uint32_t n = D.n, thr = D.thr, parts = S.parts;
-    const uint32_t b = blockIdx.x;
+    const uint32_t thr = D.thr, parts = S.parts, shift = S.part_shift;
+    if (S.v_lo > S.v_hi) return;  // nothing counted
     for (uint32_t i = threadIdx.x; i < parts; i += kSplitBlock) {
         s_cnt[i] = 0u;
         s_bid[i] = S.list_bid[i];
     }
     __syncthreads();
     auto part_of = [&](uint32_t id) -> uint32_t {
-        if (id >= thr) return (id - thr) / kSplitPart;
+        if (id >= thr) return (id - thr) >> shift;
         uint32_t lo = 0, hi = parts;  // s_bid[lo] <= id < s_bid[hi]
         while (hi - lo > 1) {
             const uint32_t mid = (lo + hi) >> 1;
@@ -272,245 +271,43 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_l1count(const GraphDesc *
         }
         return lo;
     };
-    const bool clip = S.clip != 0;
-    const uint32_t v_lo = S.v_lo, v_hi = S.v_hi;
-    const cptr<uint64_t> ie_pre = to_const(static_cast<const uint64_t *>(S.ie_pre));
-    uint64_t c0 = uni32(chunk_start(ie_pre, n, b, S.chunks)), c1 = uni32(chunk_start(ie_pre, n, b + 1, S.chunks));
-    if (clip) {
-        c0 = c0 > v_lo ? c0 : v_lo;
-        c1 = c1 < (uint64_t)v_hi + 1 ? c1 : (uint64_t)v_hi + 1;
+    // the vertex that each first-level tile starts in
+    {
+        const cptr<uint64_t> iep = to_const(static_cast<const uint64_t *>(S.ie_pre));
+        const uint64_t K0 = iep[S.v_lo], K1 = iep[(uint64_t)S.v_hi + 1];
+        const uint64_t tiles = (K1 - K0 + LevelTile<OffT>::kT - 1) / LevelTile<OffT>::kT;
+        for (uint64_t t = blockIdx.x * (uint64_t)kSplitBlock + threadIdx.x; t < tiles; t += gridDim.x * (uint64_t)kSplitBlock)
+            S.tile_v[t] = rightmost_le(to_global(static_cast<const uint64_t *>(S.ie_pre)), S.v_lo, S.v_hi,
+                                       K0 + t * LevelTile<OffT>::kT);
     }
-    if (c0 < c1) {  // block-uniform
-        const OffT p0 = rowPtr[c0], p1 = rowPtr[c1];
-        constexpr uint32_t kIn = 8;  // loads in flight per thread
-        for (OffT q0 = p0 + threadIdx.x; q0 < p1; q0 += kIn * kSplitBlock) {
-            uint32_t id[kIn];
+    const uint64_t p0 = rowPtr[S.v_lo], p1 = rowPtr[(uint64_t)S.v_hi + 1];
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    constexpr uint32_t kIn = 8;  // loads in flight per thread
+    constexpr uint64_t kStep = (uint64_t)kIn * kSplitBlock;
+    for (uint64_t base = p0 + blockIdx.x * kStep; base < p1; base += gridDim.x * kStep) {
+        uint32_t id[kIn];
 #pragma unroll
-            for (uint32_t z = 0; z < kIn; z++) {
-                const OffT q = q0 + (OffT)(z * kSplitBlock);
-                id[z] = q < p1 ? colInd[q] : 0u;
-            }
-#pragma unroll
-            for (uint32_t z = 0; z < kIn; z++)
-                if (q0 + (OffT)(z * kSplitBlock) < p1) atomicAdd(&s_cnt[part_of(id[z])], 1u);
+        for (uint32_t z = 0; z < kIn; z++) {
+            const uint64_t q = base + z * kSplitBlock + threadIdx.x;
+            id[z] = q < p1 ? colInd[q] : 0u;
         }
-        for (uint64_t v0 = c0 + threadIdx.x; v0 < c1; v0 += 4 * kSplitBlock) {
-            uint32_t id[4];
-            bool has[4];
 #pragma unroll
-            for (uint32_t z = 0; z < 4; z++) {
-                const uint64_t v = v0 + z * kSplitBlock;
-                OffT rb = 0, e = 0;
-                if (v < c1) {
-                    rb = rowPtr[v];
-                    e = rowPtr[v + 1];
-                }
-                has[z] = e > rb;
-                id[z] = has[z] ? colInd[e - 1] : 0u;
-            }
-#pragma unroll
-            for (uint32_t z = 0; z < 4; z++)
-                if (has[z]) atomicSub(&s_cnt[part_of(id[z])], 1u);
-        }
-        if (clip) {
-            const uint64_t w_lo = S.w_lo, w_hi = S.w_hi;
-            for (int z = 0; z < 2; z++) {
-                const uint64_t ve = z == 0 ? v_lo : v_hi;
-                if (ve < c0 || ve >= c1 || (z == 1 && v_hi == v_lo)) continue;  // block-uniform
-                const OffT rb = rowPtr[ve], e = rowPtr[ve + 1];
-                const uint64_t ws = S.ws_full[ve];
-                for (OffT j = rb + threadIdx.x; j + 1 < e; j += kSplitBlock) {
-                    OffT lo, hi;
-                    clip_tail<OffT>(j, e, rb, ws, w_lo, w_hi, lo, hi);
-                    if (lo >= hi) atomicSub(&s_cnt[part_of(colInd[j])], 1u);
-                }
+        for (uint32_t z = 0; z < kIn; z++) {
+            const uint64_t q = base + z * kSplitBlock + threadIdx.x;
+            const uint32_t part = q < p1 ? part_of(id[z]) : kSentinel;
+            const uint32_t next = (uint32_t)__shfl_down((int)part, 1, kWave);
+            const bool last = lane == kWave - 1 || next != part;
+            const uint64_t ends = __ballot(last);
+            if (last && part != kSentinel) {
+                const uint64_t below = ends & ((1ull << lane) - 1);  // run ends before this lane
+                const uint32_t first = below ? 64u - (uint32_t)__builtin_clzll(below) : 0u;
+                atomicAdd(&s_cnt[part], lane + 1 - first);
             }
         }
     }
     __syncthreads();
-    for (uint32_t i = threadIdx.x; i < parts; i += kSplitBlock) S.hist1[b * parts + i] = s_cnt[i];
-}
-
-// Vertices with at least this many in-edges are taken by a whole wave.
-constexpr uint32_t kSplitBigVertex = kWave;
-
-// First level of the transposition.  Block b takes vertex chunk b (clipped
-// to the counted vertices); a wave takes 64 consecutive vertices:
-//  * a vertex with kSplitBigVertex or more in-edges is taken by the whole
-//    wave in turn: the lanes load its ids 64 consecutive positions at a
-//    time, four loads in flight;
-//  * the others' in-edges are scanned and dealt to the lanes 64 at a time
-//    (a lane finds its vertex by a binary lifting over the scanned counts),
-//    four such rounds together so that their loads are in flight at once.
-// Every in-edge (its tail clipped at the ends of the counted range; empty
-// ones dropped) gets its key -- w - thr for a top row w, else rows +
-// rowPtr[w] / kSlabSpan -- and belongs to the part key / kSplitPart.  With
-// hist1 holding each part's records in earlier chunks (k_split_l1count,
-// then the offset scans) and part_base its first record, each in-edge takes
-// the next record slot of its part (an LDS cursor), and its key and record
-// are stored there.  The count saw the same in-edges in the same chunks.
-template <typename OffT>
-__global__ __launch_bounds__(kSplitBlock) void k_split_l1(const GraphDesc *__restrict__ desc,
-                                                          const SplitDesc *__restrict__ sd) {
-    __shared__ uint32_t s_cnt[kSplitPartsMax];
-    __shared__ uint64_t s_base[kSplitPartsMax];
-    const GraphDesc &D = desc[0];
-    const SplitDesc &S = sd[0];
-    const OffT *__restrict__ rowPtr = static_cast<const OffT *>(D.rowPtr);
-    const gptr<uint32_t> colInd = to_global(D.colInd);
-    const uint64_t *__restrict__ wf = S.ws_full;
-    uint64_t *__restrict__ hist1 = S.hist1;
-    uint16_t *__restrict__ rec_id = S.rec_id;
-    TailPair<OffT> *__restrict__ rec = static_cast<TailPair<OffT> *>(S.rec);
-    uint32_t *__restrict__ rec_aux = S.rec_aux;
-    const uint32_t n = D.n, thr = D.thr, rows = S.rows, parts = S.parts;
-    const uint32_t b = blockIdx.x;
-    for (uint32_t i = threadIdx.x; i < parts; i += kSplitBlock) {
-        s_cnt[i] = 0u;
-        s_base[i] = S.part_base[i] + hist1[b * parts + i];
-    }
-    __syncthreads();
-
-    const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x >> 6;
-
-    // The in-edge of an act lane stored at its part's next record slot.  The lanes of a wave that share a part take consecutive
-    // slots, and a chunk's few part cursors stay in the L2 cache, so the
-    // stores leave in whole lines.
-    auto take = [&](bool act, uint32_t key, OffT first, OffT hi, uint32_t aux) {
-        if (!act) return;
-        const uint32_t q = key / kSplitPart;
-        const uint64_t p = s_base[q] + atomicAdd(&s_cnt[q], 1u);
-        rec_id[p] = (uint16_t)(key & (kSplitPart - 1));
-        rec[p] = TailPair<OffT>{first, hi};
-        if (key >= rows) rec_aux[p] = aux;
-    };
-    // key of middle vertex id, given rowPtr[id] for a list row
-    auto key_of = [&](uint32_t id, OffT rp) -> uint32_t {
-        return id >= thr ? id - thr : rows + (uint32_t)((uint64_t)rp / kSlabSpan);
-    };
-    // slab_aux of a list row: adj+(id) = colInd[rp, rp1)
-    auto aux_of = [&](OffT rp, OffT rp1) -> uint32_t {
-        const uint64_t len = (uint64_t)(rp1 - rp);
-        return (uint32_t)((uint64_t)rp % kSlabSpan) | ((len <= kSlabRowMax ? (uint32_t)len : kSlabAuxLong) << 13);
-    };
-
-    const bool clip = S.clip != 0;
-    const uint32_t v_lo = S.v_lo, v_hi = S.v_hi;
-    const uint64_t w_lo = S.w_lo, w_hi = S.w_hi;
-    const cptr<uint64_t> ie_pre = to_const(static_cast<const uint64_t *>(S.ie_pre));
-    uint64_t c0 = uni32(chunk_start(ie_pre, n, b, S.chunks)), c1 = uni32(chunk_start(ie_pre, n, b + 1, S.chunks));
-    if (clip) {
-        c0 = c0 > v_lo ? c0 : v_lo;
-        c1 = c1 < (uint64_t)v_hi + 1 ? c1 : (uint64_t)v_hi + 1;
-    }
-    constexpr uint32_t kWaves = kSplitBlock / kWave;
-    for (uint64_t g = c0 + (uint64_t)wv * kWave; g < c1; g += (uint64_t)kWaves * kWave) {
-        const uint64_t v = g + lane;
-        OffT e = 0, rb = 0;
-        uint32_t cnt = 0;
-        bool edge = false;
-        uint64_t wsv = 0;
-        if (v < c1) {
-            rb = rowPtr[v];
-            e = rowPtr[v + 1];
-            cnt = (uint32_t)in_edges_of((uint64_t)(e - rb));
-            edge = clip && (v == v_lo || v == v_hi);
-            if (edge) wsv = wf[v];
-        }
-        // big vertices, one at a time by the whole wave
-        uint64_t big = __ballot(cnt >= kSplitBigVertex);
-        while (big) {
-            const uint32_t src = (uint32_t)__builtin_ctzll(big);
-            big &= big - 1;
-            const OffT vrb = (OffT)readlane_u64((uint64_t)rb, src);
-            const OffT vend = vrb + (OffT)(uint32_t)__builtin_amdgcn_readlane((int)cnt, (int)src);
-            const OffT ve = (OffT)readlane_u64((uint64_t)e, src);
-            const bool vedge = __builtin_amdgcn_readlane((int)edge, (int)src) != 0;
-            const uint64_t vws = readlane_u64(wsv, src);
-            for (OffT jb = vrb; jb < vend; jb += 4 * kWave) {
-                uint32_t ids[4];
-                OffT rp[4], rp1[4];
-#pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    const OffT j = jb + (OffT)(u * kWave) + lane;
-                    ids[u] = j < vend ? colInd[j] : 0u;
-                }
-#pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    const OffT j = jb + (OffT)(u * kWave) + lane;
-                    rp[u] = rp1[u] = 0;
-                    if (j < vend && ids[u] < thr) {
-                        rp[u] = rowPtr[ids[u]];
-                        rp1[u] = rowPtr[ids[u] + 1];
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    const OffT j = jb + (OffT)(u * kWave) + lane;
-                    OffT lo = j + 1, hi = ve;
-                    if (vedge && j < vend) clip_tail<OffT>(j, ve, vrb, vws, w_lo, w_hi, lo, hi);
-                    const bool top = ids[u] >= thr;
-                    take(j < vend && lo < hi, key_of(ids[u], rp[u]), top ? lo : j, hi, aux_of(rp[u], rp1[u]));
-                }
-            }
-        }
-        if (cnt >= kSplitBigVertex) cnt = 0;
-        // the other vertices' in-edges, dealt to the lanes
-        uint32_t incl = cnt;
-#pragma unroll
-        for (int o = 1; o < kWave; o <<= 1) {
-            const uint32_t y = (uint32_t)__shfl_up((int)incl, o, kWave);
-            if ((int)lane >= o) incl += y;
-        }
-        const uint32_t tot = uni32((uint32_t)__shfl((int)incl, kWave - 1, kWave));
-        const uint32_t excl = incl - cnt;
-        const bool any_edge = __ballot(edge) != 0;  // wave-uniform
-        // kDeal rounds of 64 in-edges at a time, so that their colInd and
-        // rowPtr loads are in flight together
-        constexpr uint32_t kDeal = 4;
-        for (uint32_t base = 0; base < tot; base += kDeal * kWave) {
-            OffT j[kDeal], lo[kDeal], hi[kDeal];
-            bool act[kDeal];
-#pragma unroll
-            for (uint32_t u = 0; u < kDeal; u++) {
-                const uint32_t idx = base + u * kWave + lane;
-                // the lane's vertex: the rightmost whose first in-edge is <= idx
-                uint32_t pos = 0;
-#pragma unroll
-                for (uint32_t st = kWave / 2; st > 0; st >>= 1) {
-                    const uint32_t c = pos + st;
-                    const uint32_t x = (uint32_t)__shfl((int)excl, (int)(c & (kWave - 1)), kWave);
-                    if (c < (uint32_t)kWave && x <= idx) pos = c;
-                }
-                const OffT rbv = shfl_off(rb, pos);
-                j[u] = rbv + (OffT)(idx - (uint32_t)__shfl((int)excl, (int)pos, kWave));
-                const OffT ev = shfl_off(e, pos);
-                lo[u] = j[u] + 1;
-                hi[u] = ev;
-                if (any_edge) {
-                    const bool ed = __shfl((int)edge, (int)pos, kWave) != 0;
-                    const uint64_t wv0 = shfl_u64(wsv, pos);
-                    if (ed) clip_tail<OffT>(j[u], ev, rbv, wv0, w_lo, w_hi, lo[u], hi[u]);
-                }
-                act[u] = idx < tot && lo[u] < hi[u];
-            }
-            uint32_t id[kDeal];
-#pragma unroll
-            for (uint32_t u = 0; u < kDeal; u++) id[u] = act[u] ? colInd[j[u]] : 0u;
-            OffT rp[kDeal], rp1[kDeal];
-#pragma unroll
-            for (uint32_t u = 0; u < kDeal; u++) {
-                rp[u] = rp1[u] = 0;
-                if (act[u] && id[u] < thr) {
-                    rp[u] = rowPtr[id[u]];
-                    rp1[u] = rowPtr[id[u] + 1];
-                }
-            }
-#pragma unroll
-            for (uint32_t u = 0; u < kDeal; u++)
-                take(act[u], key_of(id[u], rp[u]), id[u] >= thr ? lo[u] : j[u], hi[u], aux_of(rp[u], rp1[u]));
-        }
-    }
+    for (uint32_t i = threadIdx.x; i < parts; i += kSplitBlock)
+        if (s_cnt[i]) atomicAdd(reinterpret_cast<unsigned long long *>(&S.part_tot[i]), (unsigned long long)s_cnt[i]);
 }
 
 // Exclusive scan over the kSplitBlock threads of a block; the block's sum
@@ -533,66 +330,272 @@ __device__ __forceinline__ uint64_t split_block_scan(uint64_t x, uint64_t *s_w, 
     return off + inc - x;
 }
 
-// Block q (a part), thread c (a chunk): hist1[c][q] becomes the part's
-// records in earlier chunks, and part_tot[q] its total.
-__global__ __launch_bounds__(kSplitBlock) void k_split_l1cols(const SplitDesc *__restrict__ sd) {
-    __shared__ uint64_t s_w[kSplitBlock / kWave];
-    const SplitDesc &S = sd[0];
-    const uint32_t q = blockIdx.x, c = threadIdx.x, parts = S.parts;
-    uint64_t *__restrict__ hist1 = S.hist1;
-    const uint64_t x = c < S.chunks ? hist1[(uint64_t)c * parts + q] : 0;
-    uint64_t tot;
-    const uint64_t ex = split_block_scan(x, s_w, tot);
-    if (c < S.chunks) hist1[(uint64_t)c * parts + q] = ex;
-    if (c == 0) S.part_tot[q] = tot;
-}
-
-// One block, thread per part: part_base and c2base (kSplitChunk2 records per
-// second-level block) as prefixes of the part totals.
-__global__ __launch_bounds__(kBlock) void k_split_l1bases(const SplitDesc *__restrict__ sd) {
+// One block, thread per part: part_base as the prefix of the part sizes.
+__global__ __launch_bounds__(kBlock) void k_split_partbase(const SplitDesc *__restrict__ sd) {
     __shared__ uint64_t s_tot[kWavesPerBlock];
     static_assert(kSplitPartsMax <= (uint32_t)kBlock, "a part per thread");
     const SplitDesc &S = sd[0];
     const uint32_t q = threadIdx.x, parts = S.parts;
-    const uint64_t t = q < parts ? S.part_tot[q] : 0, nb = (t + kSplitChunk2 - 1) / kSplitChunk2;
-    uint64_t tt, tb;
-    const uint64_t et = block_excl_scan(t, s_tot, tt);
-    const uint64_t eb = block_excl_scan(nb, s_tot, tb);
-    if (q < parts) {
-        S.part_base[q] = et;
-        S.c2base[q] = (uint32_t)eb;
+    uint64_t tt;
+    const uint64_t et = block_excl_scan(q < parts ? S.part_tot[q] : 0, s_tot, tt);
+    if (q < parts) S.part_base[q] = et;
+}
+
+// Exclusive prefix of the n counts in s_cnt (a multiple of 64, at most
+// 2048) into s_off by the first wave of a block.
+__device__ __forceinline__ void wave_prefix(const uint32_t *s_cnt, uint32_t *s_off, uint32_t n) {
+    const uint32_t lane = threadIdx.x, per = n / kWave;
+    uint32_t sum = 0;
+    for (uint32_t z = 0; z < per; z++) sum += s_cnt[lane * per + z];
+    uint32_t incl = sum;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        const uint32_t y = (uint32_t)__shfl_up((int)incl, o, kWave);
+        if ((int)lane >= o) incl += y;
     }
-    if (q == 0) {
-        S.part_base[parts] = tt;
-        S.c2base[parts] = (uint32_t)tb;
+    uint32_t run = incl - sum;
+    for (uint32_t z = 0; z < per; z++) {
+        s_off[lane * per + z] = run;
+        run += s_cnt[lane * per + z];
     }
 }
 
-// Second and third levels.  Level 2 groups each part's A records by
-// sub-part into B; level 3 groups each sub-part's B records by key into ie.
-// A level's input bucket b (a part, or a sub-part) holds records
-// [base_in[b], base_in[b+1]) and is split into blocks of kChunk records
-// (its blocks start at cbase[b]); an output bucket is one of the kF
-// sub-parts of a part, or one of the kSplitSub keys of a sub-part.
-// k_split_level_count counts a block's records per output bucket into
-// hist[c][0..kF); k_split_level_scatter (hist then holding, per output
-// bucket, the records of the input bucket's earlier blocks) places each
-// record at the next slot of its output bucket.  Blocks stride over the
+// First level of the transposition.  The counted vertices' in-edges in
+// order, [K0, K1) of the in-edge prefix ie_pre, are cut into tiles of kT
+// that the blocks take in turn, so every block has the same work however the
+// in-edges fall on the vertices, and the tiles in flight are neighbours: a
+// part's records, and in the end a row's in-edges, stay nearly in the order
+// of their vertices, which the row kernel's reads of the tails need (with a
+// contiguous share of the tiles per block it took 19.2 instead of 16.4 ms on
+// R-MAT-24).  Per tile:
+//  1. the vertices that own its in-edges, read kSplitBlock at a time, mark
+//     their first slot and leave their row's position and end there; a
+//     running maximum over the marks tells each in-edge its vertex's slot;
+//  2. every in-edge loads its id (consecutive positions, so coalesced),
+//     clips its tail at the ends of the counted range (an empty one is
+//     dropped) and gets its key -- w - thr for a top row w, else rows +
+//     rowPtr[w] / kSlabSpan -- and the part key >> part_shift;
+//  3. the tile is ranked per part (LDS atomics), takes its slots of every
+//     part with one global atomic per part, and leaves sorted by part
+//     through LDS, a part's records as consecutive lanes of one store.
+// Bound by the chain of loads and barriers of a tile (two blocks a CU), then
+// by the records' 10 bytes written.  R-MAT-20: part sizes and records in
+// 0.16 ms against 0.36 with vertex chunks counted and dealt to waves, whose
+// lanes stored straight to 32,768-key parts; R-MAT-22 0.62 against 0.90;
+// R-MAT-24 2.5 against 2.7, and its parts are small enough to leave out a
+// level (the levels after: 2.8 against 3.9 ms).
+template <typename OffT>
+__global__ __launch_bounds__(kSplitBlock) void k_split_l1(const GraphDesc *__restrict__ desc,
+                                                          const SplitDesc *__restrict__ sd) {
+    constexpr uint32_t kT = LevelTile<OffT>::kT, kPer = kT / kSplitBlock;
+    constexpr uint32_t kWaves = kSplitBlock / kWave;
+    // step 1's slots and step 3's staged pairs share their memory
+    union SlotOrPair {
+        struct {
+            OffT j0, e;  // position of in-edge slot 0 as if in this row, and the row's end
+        } v;
+        TailPair<OffT> t;
+    };
+    __shared__ SlotOrPair s_x[kT];
+    __shared__ uint16_t s_mark[kT];
+    __shared__ uint16_t s_key[kT];
+    __shared__ uint8_t s_part[kT];
+    __shared__ uint32_t s_cnt[kSplitPartsMax], s_off[kSplitPartsMax];
+    __shared__ uint64_t s_base[kSplitPartsMax];
+    __shared__ uint32_t s_w[kWaves];
+    static_assert(kSplitPartsMax <= 256 && kT <= 65536, "8-bit parts, 16-bit slots");
+    const GraphDesc &D = desc[0];
+    const SplitDesc &S = sd[0];
+    const OffT *__restrict__ rowPtr = static_cast<const OffT *>(D.rowPtr);
+    const gptr<uint32_t> colInd = to_global(D.colInd);
+    const uint64_t *__restrict__ iep = S.ie_pre;
+    uint16_t *__restrict__ rec_id = S.rec_id;
+    TailPair<OffT> *__restrict__ rec = static_cast<TailPair<OffT> *>(S.rec);
+    uint32_t *__restrict__ rec_aux = S.rec_aux;
+    const uint32_t thr = D.thr, rows = S.rows, parts = S.parts, shift = S.part_shift;
+    const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x >> 6;
+    const bool clip = S.clip != 0;
+    const uint32_t v_lo = S.v_lo, v_hi = S.v_hi;
+    if (v_lo > v_hi) return;  // nothing counted
+    const uint64_t w_lo = S.w_lo, w_hi = S.w_hi;
+    // the end vertices' rows, whose tails the range may clip
+    const OffT rl0 = rowPtr[v_lo], rl1 = rowPtr[(uint64_t)v_lo + 1], rh0 = rowPtr[v_hi], rh1 = rowPtr[(uint64_t)v_hi + 1];
+    const uint64_t K0 = iep[v_lo], K1 = iep[(uint64_t)v_hi + 1];
+    const uint64_t tiles = (K1 - K0 + kT - 1) / kT;
+    const uint32_t list_part = rows >> shift;  // the first part with list keys
+    for (uint64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        uint64_t vb = S.tile_v[tile];
+        const uint64_t t0 = K0 + tile * kT, t1 = t0 + kT < K1 ? t0 + kT : K1;
+        const uint32_t nt = (uint32_t)(t1 - t0);
+        __syncthreads();  // the previous tile is written out
+        for (uint32_t i = threadIdx.x; i < kT / 2; i += kSplitBlock) reinterpret_cast<uint32_t *>(s_mark)[i] = 0u;
+        if (threadIdx.x < kSplitPartsMax) s_cnt[threadIdx.x] = 0u;
+        __syncthreads();
+        for (;;) {  // windows of kSplitBlock vertices from vb, up to the one holding t1 - 1
+            const uint64_t v = vb + threadIdx.x, vn = vb + kSplitBlock;
+            const uint64_t next = vn > v_hi ? t1 : iep[vn];
+            if (v <= v_hi) {
+                const uint64_t a = iep[v], z = iep[v + 1];
+                const OffT rb = rowPtr[v], re = rowPtr[v + 1];
+                if (z > a && z > t0 && a < t1) {
+                    const uint32_t at = a > t0 ? (uint32_t)(a - t0) : 0u;
+                    s_mark[at] = (uint16_t)at;
+                    s_x[at].v.j0 = rb - (OffT)(a - t0);  // modulo the width where a < t0
+                    s_x[at].v.e = re;
+                }
+            }
+            if (next >= t1) break;  // block-uniform
+            vb = vn;
+        }
+        __syncthreads();
+        // running maximum of the marks: kPer consecutive slots a thread
+        {
+            uint32_t x[kPer], mx = 0;
+#pragma unroll
+            for (uint32_t z = 0; z < kPer; z++) {
+                const uint32_t y = s_mark[threadIdx.x * kPer + z];
+                mx = y > mx ? y : mx;
+                x[z] = mx;
+            }
+            uint32_t run = mx;
+#pragma unroll
+            for (int o = 1; o < kWave; o <<= 1) {
+                const uint32_t y = (uint32_t)__shfl_up((int)run, o, kWave);
+                run = (int)lane >= o && y > run ? y : run;
+            }
+            if (lane == kWave - 1) s_w[wv] = run;
+            uint32_t before = (uint32_t)__shfl_up((int)run, 1, kWave);
+            before = lane ? before : 0u;
+            __syncthreads();
+            for (uint32_t w = 0; w < wv; w++) before = s_w[w] > before ? s_w[w] : before;
+#pragma unroll
+            for (uint32_t z = 0; z < kPer; z++) s_mark[threadIdx.x * kPer + z] = (uint16_t)(x[z] > before ? x[z] : before);
+        }
+        __syncthreads();
+        OffT j[kPer], e[kPer];
+        uint32_t id[kPer];
+#pragma unroll
+        for (uint32_t u = 0; u < kPer; u++) {
+            const uint32_t i = threadIdx.x + u * kSplitBlock;
+            j[u] = e[u] = 0;
+            id[u] = 0;
+            if (i < nt) {
+                const uint32_t p = s_mark[i];
+                j[u] = s_x[p].v.j0 + (OffT)i;
+                e[u] = s_x[p].v.e;
+                id[u] = colInd[j[u]];
+            }
+        }
+        OffT rp[kPer], rp1[kPer];
+#pragma unroll
+        for (uint32_t u = 0; u < kPer; u++) {
+            const uint32_t i = threadIdx.x + u * kSplitBlock;
+            rp[u] = rp1[u] = 0;
+            if (i < nt && id[u] < thr) {
+                rp[u] = rowPtr[id[u]];
+                rp1[u] = rowPtr[(uint64_t)id[u] + 1];
+            }
+        }
+        uint32_t key[kPer], rank[kPer], aux[kPer];
+        TailPair<OffT> t[kPer];
+#pragma unroll
+        for (uint32_t u = 0; u < kPer; u++) {
+            const uint32_t i = threadIdx.x + u * kSplitBlock;
+            key[u] = kSentinel;
+            if (i >= nt) continue;
+            OffT lo = j[u] + 1, hi = e[u];
+            if (clip) {
+                if (j[u] >= rl0 && j[u] < rl1) clip_tail<OffT>(j[u], e[u], rl0, S.ws_full[v_lo], w_lo, w_hi, lo, hi);
+                else if (j[u] >= rh0 && j[u] < rh1) clip_tail<OffT>(j[u], e[u], rh0, S.ws_full[v_hi], w_lo, w_hi, lo, hi);
+                if (lo >= hi) continue;
+            }
+            const bool top = id[u] >= thr;
+            key[u] = top ? id[u] - thr : rows + (uint32_t)((uint64_t)rp[u] / kSlabSpan);
+            t[u] = TailPair<OffT>{top ? lo : j[u], hi};
+            const uint64_t len = (uint64_t)(rp1[u] - rp[u]);
+            aux[u] = (uint32_t)((uint64_t)rp[u] % kSlabSpan) | ((len <= kSlabRowMax ? (uint32_t)len : kSlabAuxLong) << 13);
+            rank[u] = atomicAdd(&s_cnt[key[u] >> shift], 1u);
+        }
+        __syncthreads();  // s_x's rows are read, the counts are done
+        uint64_t slot = 0;
+        if (threadIdx.x < parts) {
+            const uint32_t c = s_cnt[threadIdx.x];
+            if (c)
+                slot = S.part_base[threadIdx.x] +
+                       atomicAdd(reinterpret_cast<unsigned long long *>(&S.part_cnt[threadIdx.x]), (unsigned long long)c);
+        }
+        if (wv == kWaves - 1) {  // another wave than the atomics'
+            constexpr uint32_t kQ = kSplitPartsMax / kWave;
+            uint32_t v[kQ], sum = 0;
+#pragma unroll
+            for (uint32_t z = 0; z < kQ; z++) {
+                v[z] = s_cnt[lane * kQ + z];
+                sum += v[z];
+            }
+            uint32_t run = sum;
+#pragma unroll
+            for (int o = 1; o < kWave; o <<= 1) {
+                const uint32_t y = (uint32_t)__shfl_up((int)run, o, kWave);
+                if ((int)lane >= o) run += y;
+            }
+            run -= sum;
+#pragma unroll
+            for (uint32_t z = 0; z < kQ; z++) {
+                s_off[lane * kQ + z] = run;
+                run += v[z];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t u = 0; u < kPer; u++) {
+            if (key[u] == kSentinel) continue;
+            const uint32_t q = key[u] >> shift, at = s_off[q] + rank[u];
+            rank[u] = at;
+            s_x[at].t = t[u];
+            s_key[at] = (uint16_t)(key[u] & ((1u << shift) - 1));
+            s_part[at] = (uint8_t)q;
+        }
+        if (threadIdx.x < parts) s_base[threadIdx.x] = slot;
+        __syncthreads();
+        const uint32_t kept = s_off[kSplitPartsMax - 1] + s_cnt[kSplitPartsMax - 1];
+        for (uint32_t i = threadIdx.x; i < kept; i += kSplitBlock) {
+            const uint32_t q = s_part[i];
+            const uint64_t p = s_base[q] + (i - s_off[q]);
+            rec_id[p] = s_key[i];
+            rec[p] = s_x[i].t;
+        }
+        const uint32_t lists = s_off[list_part];  // sorted by part: the list keys are at the end
+        if (lists < kept) {  // block-uniform
+            __syncthreads();
+            uint32_t *s_aux = reinterpret_cast<uint32_t *>(s_x);
+#pragma unroll
+            for (uint32_t u = 0; u < kPer; u++)
+                if (key[u] != kSentinel) s_aux[rank[u]] = aux[u];
+            __syncthreads();
+            for (uint32_t i = lists + threadIdx.x; i < kept; i += kSplitBlock) {
+                const uint32_t q = s_part[i];
+                if ((q << shift) + s_key[i] >= rows) rec_aux[s_base[q] + (i - s_off[q])] = s_aux[i];
+            }
+        }
+    }
+}
+
+// Later levels.  With up to kSplitPartsMax << kSplitFinalMax keys, a part
+// has at most 1 << kSplitFinalMax keys and the final level groups its A
+// records by key into ie.  With more, level 2 first groups each part's A
+// records by sub-part of kSplitSub keys into B and the final level groups
+// each sub-part's B records by key.
+// A level's input bucket b holds the records [base[b], base[b] + cnt[b]) and
+// is split into blocks of S.chunk records (its blocks start at cbase[b]); an
+// output bucket is one of the kF sub-parts of a part, or one of the keys of
+// the bucket.  k_split_level_count counts a block's records per output
+// bucket into hist[c][0..kF); k_split_level_scatter (hist then holding, per
+// output bucket, the records of the input bucket's earlier blocks) places
+// each record at the next slot of its output bucket.  Blocks stride over the
 // level's blocks.
 constexpr int kLevelRecords = 4;  // records per thread per step, loads issued together
 // Most blocks a level launches (they stride over its blocks of records).
 constexpr uint32_t kLevelGridMax = 2048;
-
-// A level's input keys are the keys within their input bucket (15 bits in
-// A, 8 in B): key = b * kUnit + local.
-template <int kLevel>
-struct SplitLevel {
-    static constexpr uint32_t kF = kLevel == 2 ? kSplitFan2 : kSplitSub;
-    static constexpr uint32_t kShift = kLevel == 2 ? kSplitSubShift : 0u;
-    static constexpr uint32_t kChunk = kLevel == 2 ? kSplitChunk2 : kSplitChunk3;
-    static constexpr uint32_t kUnit = kLevel == 2 ? kSplitPart : kSplitSub;
-    using KeyIn = typename std::conditional<kLevel == 2, uint16_t, uint8_t>::type;
-};
 
 // The last b in [0, nb) with cbase[b] <= c (cbase[0] = 0 <= c).
 __device__ __forceinline__ uint32_t bucket_of_block(const uint32_t *cbase, uint32_t nb, uint32_t c) {
@@ -605,23 +608,44 @@ __device__ __forceinline__ uint32_t bucket_of_block(const uint32_t *cbase, uint3
     return lo;
 }
 
-template <typename OffT, int kLevel>
+// What a level reads and writes.  KeyIn: 16-bit keys within a part (A) or
+// 8-bit ones within a sub-part (B); kFinal: grouped by key, else by
+// sub-part; kF output buckets (level 2: at most kSplitFan2).
+template <typename KeyIn, bool kFinal, uint32_t kF>
+struct SplitLevel {
+    static constexpr bool kFromA = sizeof(KeyIn) == 2;
+    const SplitDesc &S;
+    __device__ __forceinline__ explicit SplitLevel(const SplitDesc &s) : S(s) {}
+    __device__ __forceinline__ uint32_t buckets() const { return kFromA ? S.parts : S.subs; }
+    __device__ __forceinline__ const uint64_t *base() const { return kFromA ? S.part_base : S.sub_base; }
+    __device__ __forceinline__ uint64_t count(uint32_t b) const { return kFromA ? S.part_cnt[b] : S.sub_tot[b]; }
+    __device__ __forceinline__ const uint32_t *cbase() const { return kFinal ? S.c3base : S.c2base; }
+    __device__ __forceinline__ uint32_t *hist() const { return kFinal ? S.hist3 : S.hist2; }
+    __device__ __forceinline__ const KeyIn *keys() const {
+        return reinterpret_cast<const KeyIn *>(kFromA ? (const void *)S.rec_id : (const void *)S.rec_id2);
+    }
+    __device__ __forceinline__ const void *pairs() const { return kFromA ? S.rec : S.rec2; }
+    __device__ __forceinline__ const uint32_t *aux() const { return kFromA ? S.rec_aux : S.rec_aux2; }
+    // keys of an input bucket
+    __device__ __forceinline__ uint32_t unit_shift() const { return kFromA ? S.part_shift : kSplitSubShift; }
+    __device__ __forceinline__ uint32_t bucket(uint32_t key) const { return kFinal ? key : key >> kSplitSubShift; }
+    // output buckets of an input bucket: kF of them in hist, `fan` in the tables
+    __device__ __forceinline__ uint32_t fan() const { return kFinal ? kF : 1u << (S.part_shift - kSplitSubShift); }
+};
+
+template <typename KeyIn, bool kFinal, uint32_t kF>
 __global__ __launch_bounds__(kSplitBlock) void k_split_level_count(const SplitDesc *__restrict__ sd) {
-    using L = SplitLevel<kLevel>;
-    constexpr uint32_t kF = L::kF;
     __shared__ uint32_t s_cnt[kF];
-    const SplitDesc &S = sd[0];
-    const uint32_t nb = kLevel == 2 ? S.parts : S.subs;
-    const uint64_t *__restrict__ base_in = kLevel == 2 ? S.part_base : S.sub_base;
-    const uint32_t *__restrict__ cbase = kLevel == 2 ? S.c2base : S.c3base;
-    uint32_t *__restrict__ hist = kLevel == 2 ? S.hist2 : S.hist3;
-    const typename L::KeyIn *__restrict__ key_in =
-        reinterpret_cast<const typename L::KeyIn *>(kLevel == 2 ? (const void *)S.rec_id : (const void *)S.rec_id2);
+    const SplitLevel<KeyIn, kFinal, kF> L(sd[0]);
+    const uint32_t nb = L.buckets(), chunk = L.S.chunk;
+    const uint64_t *__restrict__ base_in = L.base();
+    const uint32_t *__restrict__ cbase = L.cbase();
+    const KeyIn *__restrict__ key_in = L.keys();
     const uint32_t nblk = cbase[nb];
     for (uint32_t c = blockIdx.x; c < nblk; c += gridDim.x) {
         const uint32_t b = bucket_of_block(cbase, nb, c);
-        const uint64_t k0 = base_in[b] + (uint64_t)(c - cbase[b]) * L::kChunk;
-        const uint64_t kq = base_in[b + 1], k1 = k0 + L::kChunk < kq ? k0 + L::kChunk : kq;
+        const uint64_t k0 = base_in[b] + (uint64_t)(c - cbase[b]) * chunk;
+        const uint64_t kq = base_in[b] + L.count(b), k1 = k0 + chunk < kq ? k0 + chunk : kq;
         __syncthreads();  // the previous block's LDS reads are done
         for (uint32_t i = threadIdx.x; i < kF; i += kSplitBlock) s_cnt[i] = 0u;
         __syncthreads();
@@ -635,66 +659,58 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_level_count(const SplitDe
             }
 #pragma unroll
             for (int u = 0; u < kU; u++)
-                if (key[u] != kSentinel) atomicAdd(&s_cnt[(key[u] >> L::kShift) & (kF - 1)], 1u);
+                if (key[u] != kSentinel) atomicAdd(&s_cnt[L.bucket(key[u])], 1u);
         }
         __syncthreads();
-        uint32_t *__restrict__ h = hist + (uint64_t)c * kF;
+        uint32_t *__restrict__ h = L.hist() + (uint64_t)c * kF;
         for (uint32_t i = threadIdx.x; i < kF; i += kSplitBlock) h[i] = s_cnt[i];
     }
 }
-
-// Records a level's scatter stages in LDS per tile: 4096 with 4-byte
-// offsets, 2048 with 8-byte ones (32 + 8 KB of pairs and words either way).
-template <typename OffT>
-struct LevelTile {
-    static constexpr uint32_t kT = sizeof(OffT) == 4 ? 4096 : 2048;
-};
 
 // The scatter of a level.  hist[c] holds, per output bucket, the input
 // bucket's records in blocks before c.  The block takes its records in tiles
 // of kT: each tile is ranked per output bucket (LDS atomics), staged in LDS
 // sorted by output bucket, and written out in that order, so that the
 // records of one output bucket in a tile -- kT / kF of them on average --
-// leave as consecutive lanes of one store to consecutive addresses.
-template <typename OffT, int kLevel>
+// leave as consecutive lanes of one store to consecutive addresses.  The
+// list records' slab words go through the same LDS after the pairs, in
+// buckets that hold list keys only.
+template <typename OffT, typename KeyIn, bool kFinal, uint32_t kF>
 __global__ __launch_bounds__(kSplitBlock) void k_split_level_scatter(const SplitDesc *__restrict__ sd) {
-    using L = SplitLevel<kLevel>;
-    constexpr uint32_t kF = L::kF;
     constexpr uint32_t kT = LevelTile<OffT>::kT;
     constexpr uint32_t kPerThread = kT / kSplitBlock;
     __shared__ uint64_t s_base[kF];  // next output slot of each output bucket
     __shared__ uint32_t s_tcnt[kF];  // the tile's records per output bucket
     __shared__ uint32_t s_toff[kF];  // their exclusive prefix: each bucket's first staged slot
-    __shared__ uint32_t st_key[kT];
+    __shared__ uint16_t st_key[kT];
     __shared__ TailPair<OffT> st_rec[kT];
-    __shared__ uint32_t st_aux[kT];
-    const SplitDesc &S = sd[0];
-    const uint32_t rows = S.rows, keys = S.keys;
-    const uint32_t nb = kLevel == 2 ? S.parts : S.subs;
-    const uint64_t *__restrict__ base_in = kLevel == 2 ? S.part_base : S.sub_base;
-    const uint32_t *__restrict__ cbase = kLevel == 2 ? S.c2base : S.c3base;
-    const uint32_t *__restrict__ hist = kLevel == 2 ? S.hist2 : S.hist3;
-    const typename L::KeyIn *__restrict__ key_in =
-        reinterpret_cast<const typename L::KeyIn *>(kLevel == 2 ? (const void *)S.rec_id : (const void *)S.rec_id2);
-    const TailPair<OffT> *__restrict__ rec_in = static_cast<const TailPair<OffT> *>(kLevel == 2 ? S.rec : S.rec2);
-    const uint32_t *__restrict__ aux_in = kLevel == 2 ? S.rec_aux : S.rec_aux2;
+    const SplitLevel<KeyIn, kFinal, kF> L(sd[0]);
+    const SplitDesc &S = L.S;
+    const uint32_t rows = S.rows, keys = S.keys, nb = L.buckets(), chunk = S.chunk, fan = L.fan();
+    const uint64_t *__restrict__ base_in = L.base();
+    const uint32_t *__restrict__ cbase = L.cbase();
+    const uint32_t *__restrict__ hist = L.hist();
+    const KeyIn *__restrict__ key_in = L.keys();
+    const TailPair<OffT> *__restrict__ rec_in = static_cast<const TailPair<OffT> *>(L.pairs());
+    const uint32_t *__restrict__ aux_in = L.aux();
     uint8_t *__restrict__ key_out = S.rec_id2;  // level 2 only
-    TailPair<OffT> *__restrict__ rec_out = static_cast<TailPair<OffT> *>(kLevel == 2 ? S.rec2 : S.ie);
-    uint32_t *__restrict__ aux_out = kLevel == 2 ? S.rec_aux2 : S.ie_aux;
+    TailPair<OffT> *__restrict__ rec_out = static_cast<TailPair<OffT> *>(kFinal ? S.ie : S.rec2);
+    uint32_t *__restrict__ aux_out = kFinal ? S.ie_aux : S.rec_aux2;
     const OffT *__restrict__ rp_in = static_cast<const OffT *>(S.rp_in);
-    const uint32_t lane = threadIdx.x & (kWave - 1);
-    auto bucket = [](uint32_t key) { return (key >> L::kShift) & (kF - 1); };
     const uint32_t nblk = cbase[nb];
     for (uint32_t c = blockIdx.x; c < nblk; c += gridDim.x) {
         const uint32_t b = bucket_of_block(cbase, nb, c);
-        const uint64_t k0 = base_in[b] + (uint64_t)(c - cbase[b]) * L::kChunk;
-        const uint64_t kq = base_in[b + 1], k1 = k0 + L::kChunk < kq ? k0 + L::kChunk : kq;
+        const uint64_t k0 = base_in[b] + (uint64_t)(c - cbase[b]) * chunk;
+        const uint64_t kq = base_in[b] + L.count(b), k1 = k0 + chunk < kq ? k0 + chunk : kq;
+        const uint32_t first_key = b << L.unit_shift();
+        const bool lists = (uint64_t)first_key + (1u << L.unit_shift()) > rows;  // block-uniform
         const uint32_t *__restrict__ h = hist + (uint64_t)c * kF;
         __syncthreads();  // the previous block's LDS reads are done
         for (uint32_t i = threadIdx.x; i < kF; i += kSplitBlock) {
             // first slot of output bucket i: a sub-part's first record, or a key's first in-edge
-            const uint32_t o = b * kF + i;
-            const uint64_t ob = kLevel == 2 ? S.sub_base[o] : o < keys ? (uint64_t)rp_in[o] : 0;
+            uint64_t ob = 0;
+            if (kFinal) ob = first_key + i < keys ? (uint64_t)rp_in[first_key + i] : 0;
+            else if (i < fan) ob = S.sub_base[b * fan + i];
             s_base[i] = ob + h[i];
         }
         for (uint64_t t0 = k0; t0 < k1; t0 += kT) {  // block-uniform
@@ -709,42 +725,22 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_level_scatter(const Split
                 aux[u] = 0u;
                 if (key[u] != kSentinel) {
                     t[u] = rec_in[k];
-                    if (b * L::kUnit + key[u] >= rows) aux[u] = aux_in[k];  // a list record
+                    if (lists && first_key + key[u] >= rows) aux[u] = aux_in[k];  // a list record
                 }
             }
 #pragma unroll
             for (uint32_t u = 0; u < kPerThread; u++)
-                if (key[u] != kSentinel) rank[u] = atomicAdd(&s_tcnt[bucket(key[u])], 1u);
+                if (key[u] != kSentinel) rank[u] = atomicAdd(&s_tcnt[L.bucket(key[u])], 1u);
             __syncthreads();
-            if (threadIdx.x < kWave) {  // exclusive prefix of the tile's bucket counts, kF / 64 per lane
-                constexpr uint32_t kPer = kF / kWave;
-                uint32_t v[kPer], sum = 0;
-#pragma unroll
-                for (uint32_t z = 0; z < kPer; z++) {
-                    v[z] = s_tcnt[lane * kPer + z];
-                    sum += v[z];
-                }
-                uint32_t incl = sum;
-#pragma unroll
-                for (int o = 1; o < kWave; o <<= 1) {
-                    const uint32_t y = (uint32_t)__shfl_up((int)incl, o, kWave);
-                    if ((int)lane >= o) incl += y;
-                }
-                uint32_t run = incl - sum;
-#pragma unroll
-                for (uint32_t z = 0; z < kPer; z++) {
-                    s_toff[lane * kPer + z] = run;
-                    run += v[z];
-                }
-            }
+            if (threadIdx.x < kWave) wave_prefix(s_tcnt, s_toff, kF);
             __syncthreads();
 #pragma unroll
             for (uint32_t u = 0; u < kPerThread; u++) {
                 if (key[u] == kSentinel) continue;
-                const uint32_t at = s_toff[bucket(key[u])] + rank[u];
-                st_key[at] = key[u];
+                const uint32_t at = s_toff[L.bucket(key[u])] + rank[u];
+                rank[u] = at;
+                st_key[at] = (uint16_t)key[u];
                 st_rec[at] = t[u];
-                st_aux[at] = aux[u];
             }
             __syncthreads();
             const uint32_t nt = (uint32_t)(k1 - t0 < kT ? k1 - t0 : kT);
@@ -752,54 +748,66 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_level_scatter(const Split
             for (uint32_t u = 0; u < kPerThread; u++) {
                 const uint32_t i = threadIdx.x + u * kSplitBlock;
                 if (i >= nt) continue;
-                const uint32_t k = st_key[i], q = bucket(k);  // the key within the input bucket
+                const uint32_t k = st_key[i], q = L.bucket(k);  // the key within the input bucket
                 const uint64_t p = s_base[q] + (i - s_toff[q]);
-                if (kLevel == 2) key_out[p] = (uint8_t)(k & (kSplitSub - 1));
+                if (!kFinal) key_out[p] = (uint8_t)(k & (kSplitSub - 1));
                 rec_out[p] = st_rec[i];
-                if (b * L::kUnit + k >= rows) aux_out[p] = st_aux[i];
             }
             __syncthreads();
+            if (lists) {
+                uint32_t *st_aux = reinterpret_cast<uint32_t *>(st_rec);
+#pragma unroll
+                for (uint32_t u = 0; u < kPerThread; u++)
+                    if (key[u] != kSentinel) st_aux[rank[u]] = aux[u];
+                __syncthreads();
+#pragma unroll
+                for (uint32_t u = 0; u < kPerThread; u++) {
+                    const uint32_t i = threadIdx.x + u * kSplitBlock;
+                    if (i >= nt) continue;
+                    const uint32_t k = st_key[i], q = L.bucket(k);
+                    if (first_key + k >= rows) aux_out[s_base[q] + (i - s_toff[q])] = st_aux[i];
+                }
+                __syncthreads();
+            }
             for (uint32_t i = threadIdx.x; i < kF; i += kSplitBlock) s_base[i] += s_tcnt[i];
         }
     }
 }
 
-// Thread per output bucket o = b*kF + i of a level: the column prefix of
-// hist over input bucket b's blocks (hist[c][i] becomes o's records in b's
-// earlier blocks) and o's total (sub_tot, or key_tot at level 3).
-template <int kLevel>
-__global__ __launch_bounds__(kBlock) void k_split_levelcols(const SplitDesc *__restrict__ sd) {
-    constexpr uint32_t kF = SplitLevel<kLevel>::kF;
+// Thread per key o of the final level: the column prefix of hist3 over its
+// input bucket's blocks (hist3[c][i] becomes the key's records in the
+// bucket's earlier blocks) and the key's total into key_tot.
+__global__ __launch_bounds__(kBlock) void k_split_levelcols3(const SplitDesc *__restrict__ sd) {
     const SplitDesc &S = sd[0];
     const uint32_t o = blockIdx.x * kBlock + threadIdx.x;
-    if (o >= (kLevel == 2 ? S.subs : S.keys)) return;
-    const uint32_t b = o / kF, i = o % kF;
-    const uint32_t *__restrict__ cbase = kLevel == 2 ? S.c2base : S.c3base;
-    uint32_t *__restrict__ hist = kLevel == 2 ? S.hist2 : S.hist3;
+    if (o >= S.keys) return;
+    const uint32_t sh = S.final_shift, b = o >> sh, i = o & ((1u << sh) - 1);
+    const uint32_t *__restrict__ cbase = S.c3base;
+    uint32_t *__restrict__ hist = S.hist3;
     uint32_t s = 0;
     const uint32_t c1 = cbase[b + 1];
     for (uint32_t c = cbase[b]; c < c1; c += 8) {  // eight loads in flight
         uint32_t x[8];
 #pragma unroll
-        for (uint32_t z = 0; z < 8; z++) x[z] = c + z < c1 ? hist[(uint64_t)(c + z) * kF + i] : 0u;
+        for (uint32_t z = 0; z < 8; z++) x[z] = c + z < c1 ? hist[((uint64_t)(c + z) << sh) + i] : 0u;
 #pragma unroll
         for (uint32_t z = 0; z < 8; z++) {
-            if (c + z < c1) hist[(uint64_t)(c + z) * kF + i] = s;
+            if (c + z < c1) hist[((uint64_t)(c + z) << sh) + i] = s;
             s += x[z];
         }
     }
-    (kLevel == 2 ? S.sub_tot : S.key_tot)[o] = s;
+    S.key_tot[o] = s;
 }
 
-// The second level's column prefixes, as k_split_levelcols<2>, with one
-// block per part: the part's blocks are cut into kSplitBlock / kSplitFan2
-// segments whose column sums are taken in parallel first (a part spans
-// hundreds of blocks, which one thread per column walked in turn).
+// The second level's column prefixes, one block per part: the part's blocks
+// are cut into kSplitBlock / kSplitFan2 segments whose column sums are taken
+// in parallel first (a part spans hundreds of blocks).
 __global__ __launch_bounds__(kSplitBlock) void k_split_levelcols2(const SplitDesc *__restrict__ sd) {
     constexpr uint32_t kF = kSplitFan2, kSeg = kSplitBlock / kF;
     __shared__ uint32_t s_sum[kSeg][kF];
     const SplitDesc &S = sd[0];
     const uint32_t b = blockIdx.x, i = threadIdx.x % kF, sg = threadIdx.x / kF;
+    const uint32_t fan = 1u << (S.part_shift - kSplitSubShift);
     const uint32_t cb0 = S.c2base[b], nb = S.c2base[b + 1] - cb0;
     const uint32_t per = (nb + kSeg - 1) / kSeg;
     const uint32_t s0 = cb0 + (sg * per < nb ? sg * per : nb), s1 = cb0 + ((sg + 1) * per < nb ? (sg + 1) * per : nb);
@@ -822,23 +830,25 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_levelcols2(const SplitDes
         hist[(uint64_t)c * kF + i] = pre;
         pre += x;
     }
-    if (sg == 0) S.sub_tot[b * kF + i] = tot;
+    if (sg == 0 && i < fan) S.sub_tot[b * fan + i] = tot;
 }
 
-// One block: sub_base = exclusive prefix of the sub-part totals (the
-// sub-parts in key order, so each part's sub-parts start at its own base)
-// and c3base = exclusive prefix of their third-level blocks.
-__global__ __launch_bounds__(kSplitBlock) void k_split_subscan(const SplitDesc *__restrict__ sd) {
+// One block: the blocks of a level's input buckets, c2base or c3base as the
+// prefix of ceil(count / chunk); with the sub-parts also sub_base, the
+// prefix of their totals (in key order).
+template <bool kSubs>
+__global__ __launch_bounds__(kSplitBlock) void k_split_bases(const SplitDesc *__restrict__ sd) {
     constexpr int kWaves = kSplitBlock / kWave;
     __shared__ uint64_t s_r[kWaves], s_b[kWaves];
     const SplitDesc &S = sd[0];
-    const uint32_t subs = S.subs;
+    const uint32_t nb = kSubs ? S.subs : S.parts, chunk = S.chunk;
+    uint32_t *__restrict__ cbase = kSubs || S.part_shift == S.final_shift ? S.c3base : S.c2base;
     const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x >> 6;
     uint64_t cr = 0, cb = 0;
-    for (uint32_t base = 0; base < subs; base += kSplitBlock) {
+    for (uint32_t base = 0; base < nb; base += kSplitBlock) {
         const uint32_t i = base + threadIdx.x;
-        const uint64_t x = i < subs ? S.sub_tot[i] : 0;
-        const uint64_t y = (x + kSplitChunk3 - 1) / kSplitChunk3;
+        const uint64_t x = i < nb ? (kSubs ? (uint64_t)S.sub_tot[i] : S.part_cnt[i]) : 0;
+        const uint64_t y = (x + chunk - 1) / chunk;
         const uint64_t ix = wave_incl_scan(x), iy = wave_incl_scan(y);
         if (lane == kWave - 1) {
             s_r[wv] = ix;
@@ -854,17 +864,14 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_subscan(const SplitDesc *
             ay += s_b[w];
         }
         __syncthreads();
-        if (i < subs) {
-            S.sub_base[i] = cr + ox + ix - x;
-            S.c3base[i] = (uint32_t)(cb + oy + iy - y);
+        if (i < nb) {
+            if (kSubs) S.sub_base[i] = cr + ox + ix - x;
+            cbase[i] = (uint32_t)(cb + oy + iy - y);
         }
         cr += ax;
         cb += ay;
     }
-    if (threadIdx.x == 0) {
-        S.sub_base[subs] = cr;
-        S.c3base[subs] = (uint32_t)cb;
-    }
+    if (threadIdx.x == 0) cbase[nb] = (uint32_t)cb;
 }
 
 // Block b: the in-edges of keys [b*kKeyChunk, (b+1)*kKeyChunk) into
@@ -993,12 +1000,11 @@ __device__ __forceinline__ void chunk_fields(u32x4 d, uint32_t *f, std::integer_
     ((f[I] = chunk_field<B, I>(d)), ...);
 }
 
-// Packs colInd into S.rec2 (free once the third level has grouped its
-// records): a block takes kBlock chunks at a time, loads their P * kBlock
+// Packs colInd into S.packed (the memory of the final level's input pairs): a block takes kBlock chunks at a time, loads their P * kBlock
 // ids into LDS with coalesced 4-byte loads, and each thread packs one chunk
 // from LDS (stride P words: no bank conflicts for odd P, two-way for P = 6
 // and 8) into one 16-byte store.  Positions past m pack as 0.  Writes
-// ceil(m / P) * 16 bytes, within rec2's cap * 2o bytes (and the 256-byte
+// ceil(m / P) * 16 bytes, within the cap * 2o bytes there (and the 256-byte
 // rounding of every workspace piece).
 template <int L>
 __device__ __forceinline__ void pack_chunks(const GraphDesc &D, uint64_t m, u32x4 *__restrict__ dst,
@@ -1041,7 +1047,7 @@ __global__ __launch_bounds__(kBlock) void k_split_pack(const GraphDesc *__restri
     const GraphDesc &D = desc[0];
     const SplitDesc &S = sd[0];
     const uint64_t m = (uint64_t) static_cast<const OffT *>(D.rowPtr)[D.n];
-    u32x4 *__restrict__ dst = static_cast<u32x4 *>(S.rec2);
+    u32x4 *__restrict__ dst = static_cast<u32x4 *>(S.packed);
     switch (pack_layout(S.rows)) {  // block-uniform
         case 0: pack_chunks<0>(D, m, dst, s_ids); break;
         case 1: pack_chunks<1>(D, m, dst, s_ids); break;
@@ -1112,7 +1118,7 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *
     const SplitDesc &S = sd[0];
     const cptr<OffT> rowPtrU = to_const(static_cast<const OffT *>(D.rowPtr));
     const gptr<uint32_t> colInd = to_global(D.colInd);
-    const gptr<u32x4> packed = to_global(static_cast<const u32x4 *>(S.rec2));
+    const gptr<u32x4> packed = to_global(static_cast<const u32x4 *>(S.packed));
     const cptr<OffT> rp_in = to_const(static_cast<const OffT *>(S.rp_in));
     const cptr<OffT> ieU = to_const(static_cast<const OffT *>(S.ie));
     const gptr<OffT> ieG = to_global(static_cast<const OffT *>(S.ie));
@@ -1425,51 +1431,90 @@ hipError_t launch_split_range(const GraphDesc *desc, SplitDesc *sd, int ob, hipS
     return WTC_LAUNCH_OFF(ob, k_split_range, dim3(1), dim3(kSplitPartsMax), 0, st, desc, sd);
 }
 
-hipError_t launch_split_transpose(const GraphDesc *desc, const SplitDesc *sd, int ob, uint32_t chunks,
-                                  uint32_t c2cap, uint32_t c3cap, uint32_t parts, uint32_t keys, uint64_t *key_part,
-                                  uint64_t *meta, unsigned long long *counts, hipStream_t st) {
-    if (keys == 0 || chunks == 0 || c2cap == 0 || c3cap == 0 || parts == 0 || parts > kSplitPartsMax)
-        return hipErrorInvalidValue;
-    const dim3 blk(kSplitBlock), g1(chunks);
-    const dim3 g2(c2cap < kLevelGridMax ? c2cap : kLevelGridMax), g3(c3cap < kLevelGridMax ? c3cap : kLevelGridMax);
-    const dim3 gk((keys + kBlock - 1) / kBlock);
+namespace {
+
+template <typename OffT, typename KeyIn, bool kFinal, uint32_t kF>
+hipError_t launch_level_count(const SplitDesc *sd, uint32_t grid, hipStream_t st) {
+    k_split_level_count<KeyIn, kFinal, kF><<<dim3(grid), dim3(kSplitBlock), 0, st>>>(sd);
+    return hipGetLastError();
+}
+
+template <typename OffT, typename KeyIn, bool kFinal, uint32_t kF>
+hipError_t launch_level_scatter(const SplitDesc *sd, uint32_t grid, hipStream_t st) {
+    k_split_level_scatter<OffT, KeyIn, kFinal, kF><<<dim3(grid), dim3(kSplitBlock), 0, st>>>(sd);
+    return hipGetLastError();
+}
+
+// The final level's count or scatter: from B, or from A by a part's keys.
+template <typename OffT>
+hipError_t launch_final(bool scatter, bool from_b, uint32_t shift, const SplitDesc *sd, uint32_t grid, hipStream_t st) {
+    if (from_b)
+        return scatter ? launch_level_scatter<OffT, uint8_t, true, kSplitSub>(sd, grid, st)
+                       : launch_level_count<OffT, uint8_t, true, kSplitSub>(sd, grid, st);
+    switch (shift) {
+        case 8:
+            return scatter ? launch_level_scatter<OffT, uint16_t, true, 256>(sd, grid, st)
+                           : launch_level_count<OffT, uint16_t, true, 256>(sd, grid, st);
+        case 9:
+            return scatter ? launch_level_scatter<OffT, uint16_t, true, 512>(sd, grid, st)
+                           : launch_level_count<OffT, uint16_t, true, 512>(sd, grid, st);
+        case 10:
+            return scatter ? launch_level_scatter<OffT, uint16_t, true, 1024>(sd, grid, st)
+                           : launch_level_count<OffT, uint16_t, true, 1024>(sd, grid, st);
+        case 11:
+            return scatter ? launch_level_scatter<OffT, uint16_t, true, 2048>(sd, grid, st)
+                           : launch_level_count<OffT, uint16_t, true, 2048>(sd, grid, st);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+template <typename OffT>
+hipError_t transpose(const GraphDesc *desc, const SplitDesc *sd, const SplitGrids &g, uint64_t *key_part, uint64_t *meta,
+                     unsigned long long *counts, hipStream_t st) {
+    const dim3 blk(kSplitBlock);
+    const uint32_t g2 = g.c2cap < kLevelGridMax ? g.c2cap : kLevelGridMax;
+    const uint32_t g3 = g.c3cap < kLevelGridMax ? g.c3cap : kLevelGridMax;
+    const bool three = g.part_shift != g.final_shift;
     hipError_t e;
-#define WTC_SPLIT_LAUNCH(KERNEL, GRID, BLOCK, ...)                                             \
-    do {                                                                                       \
-        if (ob == 8) KERNEL<uint64_t, __VA_ARGS__><<<GRID, BLOCK, 0, st>>>(sd);                \
-        else KERNEL<uint32_t, __VA_ARGS__><<<GRID, BLOCK, 0, st>>>(sd);                        \
-        if ((e = hipGetLastError()) != hipSuccess) return e;                                   \
-    } while (0)
-    if (ob == 8) k_split_l1count<uint64_t><<<g1, blk, 0, st>>>(desc, sd);
-    else k_split_l1count<uint32_t><<<g1, blk, 0, st>>>(desc, sd);
+    k_split_parthist<OffT><<<dim3(g.chunks), blk, 0, st>>>(desc, sd);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    k_split_l1cols<<<dim3(parts), blk, 0, st>>>(sd);
+    k_split_partbase<<<dim3(1), dim3(kBlock), 0, st>>>(sd);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    k_split_l1bases<<<dim3(1), dim3(kBlock), 0, st>>>(sd);
+    k_split_l1<OffT><<<dim3(g.chunks), blk, 0, st>>>(desc, sd);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    if (ob == 8) k_split_l1<uint64_t><<<g1, blk, 0, st>>>(desc, sd);
-    else k_split_l1<uint32_t><<<g1, blk, 0, st>>>(desc, sd);
+    k_split_bases<false><<<dim3(1), blk, 0, st>>>(sd);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    WTC_SPLIT_LAUNCH(k_split_level_count, g2, blk, 2);
-    k_split_levelcols2<<<dim3(parts), blk, 0, st>>>(sd);
+    if (three) {
+        if ((e = launch_level_count<OffT, uint16_t, false, kSplitFan2>(sd, g2, st)) != hipSuccess) return e;
+        k_split_levelcols2<<<dim3(g.parts), blk, 0, st>>>(sd);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        k_split_bases<true><<<dim3(1), blk, 0, st>>>(sd);
+        if ((e = hipGetLastError()) != hipSuccess) return e;
+        if ((e = launch_level_scatter<OffT, uint16_t, false, kSplitFan2>(sd, g2, st)) != hipSuccess) return e;
+    }
+    if ((e = launch_final<OffT>(false, three, g.final_shift, sd, g3, st)) != hipSuccess) return e;
+    k_split_levelcols3<<<dim3((g.keys + kBlock - 1) / kBlock), dim3(kBlock), 0, st>>>(sd);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    k_split_subscan<<<dim3(1), blk, 0, st>>>(sd);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    WTC_SPLIT_LAUNCH(k_split_level_scatter, g2, blk, 2);
-    WTC_SPLIT_LAUNCH(k_split_level_count, g3, blk, 3);
-    k_split_levelcols<3><<<gk, dim3(kBlock), 0, st>>>(sd);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    const dim3 gkb((keys + kKeyChunk - 1) / kKeyChunk);
+    const dim3 gkb((g.keys + kKeyChunk - 1) / kKeyChunk);
     k_split_keysum<<<gkb, blk, 0, st>>>(sd);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if ((e = launch_scan_partials(key_part, gkb.x, st)) != hipSuccess) return e;
-    if (ob == 8) k_split_keyscan<uint64_t><<<gkb, blk, 0, st>>>(sd, meta, counts);
-    else k_split_keyscan<uint32_t><<<gkb, blk, 0, st>>>(sd, meta, counts);
+    k_split_keyscan<OffT><<<gkb, blk, 0, st>>>(sd, meta, counts);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    WTC_SPLIT_LAUNCH(k_split_level_scatter, g3, blk, 3);
-#undef WTC_SPLIT_LAUNCH
-    // the packed top ids, over B's pairs (the third level has read them)
-    return WTC_LAUNCH_OFF(ob, k_split_pack, dim3(kPackGrid), dim3(kBlock), 0, st, desc, sd);
+    if ((e = launch_final<OffT>(true, three, g.final_shift, sd, g3, st)) != hipSuccess) return e;
+    // the packed top ids, over the final level's input pairs
+    k_split_pack<OffT><<<dim3(kPackGrid), dim3(kBlock), 0, st>>>(desc, sd);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_split_transpose(const GraphDesc *desc, const SplitDesc *sd, int ob, const SplitGrids &g,
+                                  uint64_t *key_part, uint64_t *meta, unsigned long long *counts, hipStream_t st) {
+    if (g.keys == 0 || g.chunks == 0 || g.c3cap == 0 || g.parts == 0 || g.parts > kSplitPartsMax)
+        return hipErrorInvalidValue;
+    return ob == 8 ? transpose<uint64_t>(desc, sd, g, key_part, meta, counts, st)
+                   : transpose<uint32_t>(desc, sd, g, key_part, meta, counts, st);
 }
 
 size_t split_rows_lds(uint32_t rows) { return (size_t)(((rows + 31) / 32 + 1) & ~1u) * sizeof(uint32_t) + sizeof(uint64_t); }
