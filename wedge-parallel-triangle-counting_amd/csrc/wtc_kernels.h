@@ -101,7 +101,8 @@ enum : int {
 // kSplitFinalMax keys and the second level groups by key; beyond that (up to
 // kSplitPartsMax << kSplitPartMax keys), parts are first grouped by sub-part
 // of kSplitSub keys (at most kSplitFan2 a part).  kSplitBlock: threads per
-// transposition block; kSplitTile: in-edges per tile of the row kernel.
+// transposition block; a tile of the row kernel is kSplitTileMinWork to
+// kSplitTile units of work, an in-edge being one and a row kSplitRowCost.
 constexpr uint32_t kSplitPartMax = 15;
 constexpr uint32_t kSplitPartsMax = 256;
 constexpr uint32_t kSplitFinalMin = 8, kSplitFinalMax = 11;
@@ -113,7 +114,8 @@ static_assert(kSplitPartMax <= 16 && kSplitSubShift <= 8, "A keys fit 16 bits, B
 // few as kSplitChunkMin for small graphs, so that the levels fill the GPU.
 constexpr uint32_t kSplitChunkMax = 65536, kSplitChunkMin = 8192;
 constexpr int kSplitBlock = 1024;
-constexpr uint32_t kSplitTile = 1024;
+constexpr uint32_t kSplitTile = 1024, kSplitTileMinWork = 128;
+constexpr uint32_t kSplitRowCost = 32;
 // Keys per block of the key-offset scan (four per thread).
 constexpr uint32_t kKeyChunk = 4 * kSplitBlock;
 // Slabs of the list rows (middle vertex below thr): slab s holds the rows

@@ -1057,13 +1057,12 @@ __global__ __launch_bounds__(kBlock) void k_split_pack(const GraphDesc *__restri
 }
 
 // Lanes per in-edge tail in the row kernel (a wave takes kWave / kSplitLanes
-// in-edges per step) and 16-byte chunks per lane per step.  Tails average
+// in-edges per step), a 16-byte chunk per lane per step.  Tails average
 // ~180 ids on R-MAT-24 (median 86), and a step lasts as long as its longest
 // tail: 8 lanes of one chunk keep 80% of the id slots busy, 16 lanes of two
 // chunks 57%.  Measured on R-MAT-24: 18.2 ms at 8 x 1, 19.0 at 8 x 2, 18.8
 // at 16 x 1, 19.1 at 4 x 1, 22.1 at 16 x 2.
 constexpr int kSplitLanes = 8;
-constexpr int kSplitChunks = 1;
 
 // Counts the hits of the P packed ids of chunk c of a tail.  base = Pc - lo
 // (mod 2^32): position Pc + z is in the tail iff base + z < len.  Every
@@ -1100,14 +1099,39 @@ __device__ __forceinline__ uint32_t rows_chunk_hits(const uint32_t *s_bits, u32x
     return __builtin_popcount(hm & vm);
 }
 
-// Persistent blocks take tiles of kSplitTile consecutive in-edges (in row
-// order) from one counter.  Per row of a tile: adj+(w) set as bits (u - thr)
-// in LDS, the tile's in-edges of the row dealt to the waves (kLanes lanes
-// per in-edge), and each tail streamed through the bitmap from the packed
-// ids (k_split_pack) by 16-byte chunks of P ids (6 to 8, PackLayout), kCh
-// chunks per lane per step and the next step's chunks loaded before this
-// step's are counted; then the row's bits cleared.
-template <typename OffT, int kWaves, int kLanes, int kCh, int kLayout>
+// Rightmost r in [0, hi] with f(r) <= t for a non-decreasing f with f(0) <=
+// t, by a whole wave: 64 probes a round.
+template <class F>
+__device__ __forceinline__ uint32_t wave_rightmost_le(uint32_t hi, uint64_t t, F f) {
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    uint32_t lo = 0;  // f(lo) <= t
+    while (lo < hi) {
+        const uint32_t step = (hi - lo + kWave - 1) / kWave;
+        const uint64_t at = (uint64_t)lo + (uint64_t)(lane + 1) * step;
+        const bool le = at <= hi && f((uint32_t)at) <= t;
+        const uint32_t k = (uint32_t)__builtin_popcountll(__ballot(le));  // a prefix of the lanes
+        const uint64_t end = (uint64_t)lo + (uint64_t)(k + 1) * step - 1;
+        lo += k * step;
+        hi = end < hi ? (uint32_t)end : hi;
+    }
+    return uni32(lo);
+}
+
+// Persistent blocks take tiles of the rows' work from one counter.  The work
+// of a row is kSplitRowCost for its bitmap and one unit per in-edge, so a
+// tile is up to `tile` in-edges of few rows, or fewer in-edges where rows
+// have few each: tiles of in-edges alone left blocks with hundreds of such
+// rows to the end, one chain of loads and barriers after another (a quarter
+// of R-MAT-21's wedges: 1.75 ms).
+// Per row of a tile the block puts adj+(w) into an LDS bitmap as bits u -
+// thr, its waves take the row's in-edges in the tile (kLanes lanes each),
+// and each tail is streamed through the bitmap from the packed ids
+// (k_split_pack) by 16-byte chunks of P ids (6 to 8, PackLayout), the next
+// chunk loaded before this one is counted, and the next in-edges' bounds
+// before these are streamed.  A row's ids are loaded while the row before is
+// streamed; its bits go in as the other row's go out, all by exclusive or,
+// so a row takes two barriers.
+template <typename OffT, int kWaves, int kLanes, int kLayout>
 __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *__restrict__ desc,
                                                                const SplitDesc *__restrict__ sd,
                                                                uint64_t *__restrict__ meta,
@@ -1116,51 +1140,115 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *
     extern __shared__ uint32_t s_bits[];
     const GraphDesc &D = desc[0];
     const SplitDesc &S = sd[0];
-    const cptr<OffT> rowPtrU = to_const(static_cast<const OffT *>(D.rowPtr));
+    const gptr<OffT> rowPtr = to_global(static_cast<const OffT *>(D.rowPtr));
     const gptr<uint32_t> colInd = to_global(D.colInd);
     const gptr<u32x4> packed = to_global(static_cast<const u32x4 *>(S.packed));
-    const cptr<OffT> rp_in = to_const(static_cast<const OffT *>(S.rp_in));
-    const cptr<OffT> ieU = to_const(static_cast<const OffT *>(S.ie));
+    const gptr<OffT> rp_in = to_global(static_cast<const OffT *>(S.rp_in));
     const gptr<OffT> ieG = to_global(static_cast<const OffT *>(S.ie));
     const uint32_t thr = D.thr, rows = S.rows;
+    constexpr uint32_t kThreads = kWave * kWaves;
     constexpr uint32_t kPer = kWave / kLanes;  // in-edges a wave takes per step
+    constexpr uint32_t kHold = 2;              // ids of a row a thread keeps
     const uint32_t words = (rows + 31) >> 5;
     uint64_t &s_tile = *reinterpret_cast<uint64_t *>(s_bits + ((words + 1) & ~1u));
-    for (uint32_t i = threadIdx.x; i < words; i += kWave * kWaves) s_bits[i] = 0;
-    const uint64_t K = (uint64_t)rp_in[rows];
+    for (uint32_t i = threadIdx.x; i < words; i += kThreads) s_bits[i] = 0;
+    const uint64_t K = uni((uint64_t)rp_in[rows]), work = K + (uint64_t)kSplitRowCost * rows;
+    // about eight tiles a block, of kSplitTileMinWork to kSplitTile
+    uint64_t tile = work / (8ull * gridDim.x);
+    tile = tile < kSplitTileMinWork ? kSplitTileMinWork : tile > kSplitTile ? kSplitTile : tile;
     const uint32_t lane = threadIdx.x & (kWave - 1), wv = uni32(threadIdx.x >> 6);
     const uint32_t sub = lane / kLanes, sl = lane % kLanes;
     unsigned long long *const ctr = reinterpret_cast<unsigned long long *>(meta + kMetaRows);
     uint64_t hits = 0, checked = 0;
-    for (;;) {
-        __syncthreads();  // the previous tile's s_tile reads and bit clears are done
-        if (threadIdx.x == 0) s_tile = atomicAdd(ctr, 1ull);
-        __syncthreads();
-        const uint64_t k0 = uni64(s_tile) * kSplitTile;
-        if (k0 >= K) break;  // block-uniform
-        const uint64_t k1 = k0 + kSplitTile < K ? k0 + kSplitTile : K;
-        uint64_t k = k0;
-        while (k < k1) {
-            const uint32_t r = uni32(rightmost_le(rp_in, 0u, rows - 1, k));  // the row holding in-edge k
-            const uint64_t re = (uint64_t)rp_in[r + 1];
-            const uint64_t kend = re < k1 ? re : k1;
-            const uint32_t w = thr + r;
-            const OffT ab = rowPtrU[w], ae = rowPtrU[w + 1];
-            for (OffT i = ab + threadIdx.x; i < ae; i += kWave * kWaves) {
-                const uint32_t c = colInd[i] - thr;
-                atomicOr(&s_bits[c >> 5], 1u << (c & 31u));
+    // the row in the bitmap: adj+ = colInd[pb, pe), its first ids in held[]
+    OffT pb = 0, pe = 0;
+    uint32_t held[kHold] = {0, 0};
+    auto flip = [&](uint32_t u) { atomicXor(&s_bits[(u - thr) >> 5], 1u << ((u - thr) & 31u)); };
+    if (threadIdx.x == 0) s_tile = atomicAdd(ctr, 1ull);
+    __syncthreads();
+    uint64_t t = uni64(s_tile);
+    while (t * tile < work) {  // block-uniform
+        const uint64_t t0 = t * tile, t1 = t0 + tile < work ? t0 + tile : work;
+        __syncthreads();  // s_tile is read
+        if (threadIdx.x == 0) s_tile = atomicAdd(ctr, 1ull);  // the next tile, read at this one's end
+        // row r's work is [rp_in[r] + r*kSplitRowCost, rp_in[r + 1] + (r + 1)*kSplitRowCost)
+        const uint32_t r0 = wave_rightmost_le(rows - 1, t0, [&](uint32_t r) {
+            return (uint64_t)rp_in[r] + (uint64_t)kSplitRowCost * r;
+        });
+        // lane l: in-edge and adjacency bounds of row r0 + l (a tile has fewer than 63 rows)
+        static_assert(kSplitTile / kSplitRowCost + 2 < kWave, "a tile's rows fit a wave");
+        const uint32_t rl = r0 + lane < rows ? r0 + lane : rows;
+        const OffT my_in = rp_in[rl], my_adj = rowPtr[(uint64_t)thr + rl];
+        // the tile's in-edges [ka, kz) and adjacency [ab, ae) of row r0 + x
+        auto row_bounds = [&](uint32_t x, uint64_t &ka, uint64_t &kz, OffT &ab, OffT &ae) {
+            const uint64_t b = readlane_u64((uint64_t)my_in, x), e = readlane_u64((uint64_t)my_in, x + 1);
+            const uint64_t c = (uint64_t)kSplitRowCost * (r0 + x + 1);
+            ka = t0 > b + c ? t0 - c : b;
+            kz = t1 < e + c ? (t1 > b + c ? t1 - c : b) : e;
+            ab = (OffT)readlane_u64((uint64_t)my_adj, x);
+            ae = (OffT)readlane_u64((uint64_t)my_adj, x + 1);
+        };
+        // the next row from x on with in-edges in the tile, or kSentinel
+        auto next_row = [&](uint32_t x) -> uint32_t {
+            for (; r0 + x < rows; x++) {
+                uint64_t ka, kz;
+                OffT ab, ae;
+                row_bounds(x, ka, kz, ab, ae);
+                if ((uint64_t)readlane_u64((uint64_t)my_in, x) + (uint64_t)kSplitRowCost * (r0 + x) >= t1) break;
+                if (ka < kz) return x;
             }
+            return kSentinel;
+        };
+        uint32_t x = next_row(0);
+        uint64_t k = 0, kend = 0;
+        OffT ab = 0, ae = 0;
+        uint32_t ids[kHold] = {0, 0};
+        if (x != kSentinel) {
+            row_bounds(x, k, kend, ab, ae);
+#pragma unroll
+            for (uint32_t z = 0; z < kHold; z++) {
+                const OffT i = ab + threadIdx.x + z * kThreads;
+                if (i < ae) ids[z] = colInd[i];
+            }
+        }
+        while (x != kSentinel) {  // block-uniform
+            // this row's bits in, the row before's out
+#pragma unroll
+            for (uint32_t z = 0; z < kHold; z++) {
+                if (pb + threadIdx.x + z * kThreads < pe) flip(held[z]);
+                if (ab + threadIdx.x + z * kThreads < ae) flip(ids[z]);
+                held[z] = ids[z];
+            }
+            for (OffT i = pb + threadIdx.x + kHold * kThreads; i < pe; i += kThreads) flip(colInd[i]);
+            for (OffT i = ab + threadIdx.x + kHold * kThreads; i < ae; i += kThreads) flip(colInd[i]);
+            pb = ab;
+            pe = ae;
+            const uint64_t ck = k, ckend = kend;
             __syncthreads();
+            // the next row's ids, on their way while this row is streamed
+            x = next_row(x + 1);
+            if (x != kSentinel) {
+                row_bounds(x, k, kend, ab, ae);
+#pragma unroll
+                for (uint32_t z = 0; z < kHold; z++) {
+                    const OffT i = ab + threadIdx.x + z * kThreads;
+                    if (i < ae) ids[z] = colInd[i];
+                }
+            }
             uint32_t h = 0;
-            for (uint64_t x0 = k + (uint64_t)wv * kPer; x0 < kend; x0 += (uint64_t)kWaves * kPer) {
-                // kPer in-edges per step, kLanes lanes each
-                OffT lo = 0, hi = 0;
-                if (kPer == 1) {
-                    lo = uni(ieU[2 * x0]);
-                    hi = uni(ieU[2 * x0 + 1]);
-                } else if (x0 + sub < kend) {
-                    lo = ieG[2 * (x0 + sub)];
-                    hi = ieG[2 * (x0 + sub) + 1];
+            uint64_t x0 = ck + (uint64_t)wv * kPer;
+            OffT lo = 0, hi = 0;
+            if (x0 + sub < ckend) {
+                lo = ieG[2 * (x0 + sub)];
+                hi = ieG[2 * (x0 + sub) + 1];
+            }
+            while (x0 < ckend) {
+                // the bounds of the step after this one
+                x0 += (uint64_t)kWaves * kPer;
+                OffT nlo = 0, nhi = 0;
+                if (x0 + sub < ckend) {
+                    nlo = ieG[2 * (x0 + sub)];
+                    nhi = ieG[2 * (x0 + sub) + 1];
                 }
                 if (sl == 0) checked += (uint64_t)(hi - lo);
                 // chunk c holds positions [Pc, Pc + P); a tail is shorter
@@ -1169,38 +1257,25 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *
                 const uint32_t len = (uint32_t)(hi - lo);
                 const OffT c_end = hi / P + (hi % P != 0 ? 1 : 0);
                 OffT c = lo / P + sl;
-                u32x4 cur[kCh];
-#pragma unroll
-                for (int q = 0; q < kCh; q++) {
-                    cur[q] = u32x4{0u, 0u, 0u, 0u};
-                    if (c + (OffT)(q * kLanes) < c_end) cur[q] = packed[c + (OffT)(q * kLanes)];
-                }
+                u32x4 cur = u32x4{0u, 0u, 0u, 0u};
+                if (c < c_end) cur = packed[c];
                 while (c < c_end) {
-                    const OffT cn = c + (OffT)(kCh * kLanes);
-                    // the next chunks, or chunk c again past the tail's end
+                    const OffT cn = c + (OffT)kLanes;
+                    // the next chunk, or chunk c again past the tail's end
                     // (loaded unconditionally; a chunk past c_end is not counted)
-                    u32x4 nxt[kCh];
-#pragma unroll
-                    for (int q = 0; q < kCh; q++) {
-                        const OffT cq = cn + (OffT)(q * kLanes);
-                        nxt[q] = packed[cq < c_end ? cq : c];
-                    }
-                    const uint32_t base = (uint32_t)(P * c - lo);
-#pragma unroll
-                    for (int q = 0; q < kCh; q++)
-                        if (q == 0 || c + (OffT)(q * kLanes) < c_end)
-                            h += rows_chunk_hits<kLayout>(s_bits, cur[q], base + P * q * kLanes, len);
-#pragma unroll
-                    for (int q = 0; q < kCh; q++) cur[q] = nxt[q];
+                    const u32x4 nxt = packed[cn < c_end ? cn : c];
+                    h += rows_chunk_hits<kLayout>(s_bits, cur, (uint32_t)(P * c - lo), len);
+                    cur = nxt;
                     c = cn;
                 }
+                lo = nlo;
+                hi = nhi;
             }
             hits += h;
             __syncthreads();
-            for (OffT i = ab + threadIdx.x; i < ae; i += kWave * kWaves) s_bits[(colInd[i] - thr) >> 5] = 0u;
-            __syncthreads();
-            k = kend;
         }
+        __syncthreads();  // the next tile is there, also after a tile without in-edges
+        t = uni64(s_tile);
     }
     hits = wave_sum(hits);
     checked = wave_sum(checked);
@@ -1521,8 +1596,8 @@ size_t split_rows_lds(uint32_t rows) { return (size_t)(((rows + 31) / 32 + 1) & 
 
 template <int W, int L>
 static const void *split_rows_fn(int ob) {
-    return ob == 8 ? reinterpret_cast<const void *>(&k_split_rows<uint64_t, W, kSplitLanes, kSplitChunks, L>)
-                   : reinterpret_cast<const void *>(&k_split_rows<uint32_t, W, kSplitLanes, kSplitChunks, L>);
+    return ob == 8 ? reinterpret_cast<const void *>(&k_split_rows<uint64_t, W, kSplitLanes, L>)
+                   : reinterpret_cast<const void *>(&k_split_rows<uint32_t, W, kSplitLanes, L>);
 }
 
 template <int L>
