@@ -731,6 +731,9 @@ def offsets_u64_leg(ctx, g, W, spread, a, steps, warmup, expect):
             counts.append(c)
             stats.append(st.as_dict())
         el = time.perf_counter() - t0
+        if stats[-1]["split"]:  # the row kernel's share (the rest is the dense part's)
+            dense_w, dense_e = ctx.debug_split()
+            row_w, row_e = stats[-1]["top_wedges"] - dense_w, stats[-1]["in_edges"] - dense_e
     finally:
         dg8.free()
     _, b_min8 = g.alg_bytes(8)
@@ -745,7 +748,7 @@ def offsets_u64_leg(ctx, g, W, spread, a, steps, warmup, expect):
         # in-edge records of 2*4 B when every position fits 32 bits (the split
         # count then runs on a 4-byte copy of the offsets), else 2*8 B
         rec_bytes = 8.0 if g.m < 0xFFFFFFFF else 16.0
-        dom_bytes = split_id_bytes(min(a, g.n)) * stats[-1]["top_wedges"] + rec_bytes * stats[-1]["in_edges"]
+        dom_bytes = split_id_bytes(min(a, g.n)) * row_w + rec_bytes * row_e
         out["kernel_ms"]["split_rows"] = rows_ms
         out["kernel_ms"]["split_slabs"] = statistics.median(s["list_ms"] for s in stats)
         out["roofline"] = {"kernel": "k_split_rows", "achieved": dom_bytes / (rows_ms / 1e3) / 1e9, "unit": "GB/s",
@@ -929,7 +932,8 @@ def main():
         # probe itself is an LDS read) and every in-edge's (lo, hi) record of
         # 2*ob bytes
         dom, dom_ms = "k_split_rows", statistics.median(s["rows_ms"] for s in stats)
-        top_w, in_e = stats[-1]["top_wedges"], stats[-1]["in_edges"]
+        dense_w, dense_e = ctx.debug_split()  # counted by the dense part, not the row kernel
+        top_w, in_e = stats[-1]["top_wedges"] - dense_w, stats[-1]["in_edges"] - dense_e
         id_bytes = split_id_bytes(min(args.a, dg.n))
         dom_bytes = id_bytes * top_w + 2.0 * ob * in_e
         dom_units = {"wedges_checked": top_w, "in_edges": in_e, "bytes_per_wedge": id_bytes,

@@ -196,9 +196,9 @@ typedef struct wtc_dgraph wtc_dgraph; /* oriented CSR resident in HBM    */
 typedef struct {
     double prefix_ms;  /* wedge prefix scan + setup (split count: its two
                           prefixes and range map)                             */
-    double bitmap_ms;  /* bitmap clear + build (split count: the counting
-                          sort of the in-edges by middle vertex and the
-                          packing of the top tails' ids)                      */
+    double bitmap_ms;  /* bitmap clear + build (split count: the dense part,
+                          the counting sort of the other in-edges by middle
+                          vertex and the packing of the top tails' ids)       */
     double count_ms;   /* counting kernel(s) (split count: row + slab kernels) */
     double total_ms;   /* first launch to count back on the host             */
     uint64_t wedges;   /* W counted                                          */
@@ -207,10 +207,10 @@ typedef struct {
     uint32_t small_graphs; /* graphs counted by the small-graph kernel       */
     uint32_t split;    /* 1: counted by the split count                      */
     double rows_ms;    /* split count: its row kernel alone                  */
-    uint64_t top_wedges; /* split count: wedges probed in LDS (w in the top rows) */
-    uint64_t in_edges; /* split count: in-edge tails the row kernel streamed */
+    uint64_t top_wedges; /* split count: wedges with w in the top rows (row kernel, dense part) */
+    uint64_t in_edges; /* split count: in-edges of the top rows */
     double list_ms;    /* split count: its slab kernel alone (w below the top rows) */
-    uint64_t list_in_edges; /* split count: in-edge tails the slab kernel streamed */
+    uint64_t list_in_edges; /* split count: the other in-edges */
 } wtc_count_stats;
 
 int wtc_device_count(int *count);
@@ -237,7 +237,9 @@ int wtc_ctx_set_tuning(wtc_ctx *ctx, int probe_ways, uint32_t lds_chunk, int wav
  *                     ranks (the reference's bitmap probes, tc.cu:262-272)
  *                     are counted against adj+(w) held as a bitmap row in
  *                     LDS (their tails streamed from a copy of colInd
- *                     packed to 16-21 bits per id), the rest (sorted-list
+ *                     packed to 16-21 bits per id; where a row has many ids
+ *                     among the last ranks, its wedges there as a masked
+ *                     product of bit matrices), the rest (sorted-list
  *                     probes, tc.cu:273-286) against hash sets of adj+(w)
  *                     in LDS.  No a*a/8-byte bitmap in HBM; about 27 or 43
  *                     bytes per edge of workspace (4- or 8-byte offsets)
@@ -337,6 +339,11 @@ int wtc_count_noalloc(const void *d_row_ptr, uint32_t offset_bytes, const uint32
  * the bitmap words (tc.cu:329-346) left by the last count on `ctx`. */
 int wtc_ctx_debug_prefix(wtc_ctx *ctx, uint64_t n, uint64_t *wedge_sum, uint64_t *tree);
 int wtc_ctx_debug_bitmap(wtc_ctx *ctx, uint64_t words, uint32_t *out);
+/* What the dense part of the last split count on `ctx` took (the wedges among
+ * the last ranks counted as a product of bit matrices) of that count's
+ * top_wedges and in_edges; the row kernel took the rest.  WTC_ERR_ARG if the
+ * last count was no split count. */
+int wtc_ctx_debug_split(wtc_ctx *ctx, uint64_t *dense_top_wedges, uint64_t *dense_top_in_edges);
 /* Copies `bytes` (rounded down to 16) between two fresh device buffers `reps`
  * times with a plain streaming kernel; *ms = average per copy.  The byte
  * count is known exactly, so profiler HBM counters read on it calibrate the

@@ -157,6 +157,9 @@ struct SplitLayout {
     size_t wsfull, tile_v, part_base, part_cnt, c2base, hist2, sub_base, c3base, hist3, sub_tot, list_bid, slab_row, key_tot;
     size_t part_tot, key_part;
     size_t recid, rec, recaux, recid2, rec2, recaux2, rpin, rp32, total;
+    size_t dense_cnt, dense_sums, dense_r, dense_b, dense_list;  // the last three within the records
+    uint64_t dense_list_off[kDenseClasses];
+    uint32_t dense_classes;
     uint32_t slabs, subs, chunk;
     SplitGrids g;
     uint64_t cap;
@@ -229,7 +232,34 @@ SplitLayout split_plan(uint32_t n, uint64_t m, uint32_t rows, int ob_in) {
     L.recid2 = take(three ? (size_t)L.cap * sizeof(uint8_t) : 0);
     L.rec2 = take((size_t)L.cap * pair);
     L.recaux2 = take((size_t)L.cap * sizeof(uint32_t));
+    const size_t rec_end = off;
     L.rpin = take(((size_t)L.g.keys + 1) * (size_t)ob);
+    L.dense_cnt = take(kDenseClasses * sizeof(uint32_t));
+    L.dense_sums = take(kDenseSums * sizeof(uint64_t));
+    // The dense part runs before the transposition, in the records' memory:
+    // R, the class rows (a row of K / 8 bytes has K / kDenseSparsest ids or
+    // more, so kDenseSparsest / 8 bytes an edge, and a class's padding of
+    // 128 rows) and the lists.  As many classes as fit, R taking no more than
+    // a byte an edge: a wider class finds so few rows in a graph of that size
+    // (R-MAT-20: one at 16,384 columns) that its tiles are mostly padding.
+    for (L.dense_classes = kDenseClasses; L.dense_classes > 0; L.dense_classes--) {
+        const uint64_t core = (uint64_t)kDenseCore0 << (L.dense_classes - 1);
+        size_t at = L.rec;
+        auto put = [&](size_t bytes) {
+            const size_t x = at;
+            at = (at + bytes + 255) & ~(size_t)255;
+            return x;
+        };
+        L.dense_r = put(core * core / 8);
+        L.dense_b = put(L.cap * (kDenseSparsest / 8) + 2 * (core / 8) * 128);  // the classes' rows: < 2 core / 8 bytes
+        uint64_t entries = 0;
+        for (uint32_t q = 0; q < L.dense_classes; q++) {
+            L.dense_list_off[q] = entries;
+            entries += L.cap * kDenseSparsest / ((uint64_t)kDenseCore0 << q) + 1;
+        }
+        L.dense_list = put(entries * sizeof(uint2));
+        if (at <= rec_end && core * core / 8 <= L.cap) break;
+    }
     L.rp32 = narrow ? take(((size_t)n + 1) * sizeof(uint32_t)) : 0;
     L.total = off;
     return L;
@@ -239,9 +269,19 @@ SplitLayout split_plan(uint32_t n, uint64_t m, uint32_t rows, int ob_in) {
 
 size_t split_workspace_bytes(uint32_t n, uint64_t m, uint32_t rows, int ob) { return split_plan(n, m, rows, ob).total; }
 
-int split_layout(SplitDesc *sd, SplitGrids *grids, char *base, uint32_t n, uint64_t m, uint32_t rows, int ob,
-                 uint32_t **rp32) {
+int split_layout(SplitDesc *sd, DenseDesc *dd, SplitGrids *grids, char *base, uint32_t n, uint64_t m, uint32_t rows,
+                 int ob, uint32_t **rp32) {
     const SplitLayout L = split_plan(n, m, rows, ob);
+    dd->R = base + L.dense_r;
+    dd->B = base + L.dense_b;
+    dd->list = reinterpret_cast<uint2 *>(base + L.dense_list);
+    dd->cnt = reinterpret_cast<uint32_t *>(base + L.dense_cnt);
+    dd->sums = reinterpret_cast<uint64_t *>(base + L.dense_sums);
+    for (uint32_t q = 0; q < L.dense_classes; q++) dd->list_off[q] = L.dense_list_off[q];
+    dd->classes = L.dense_classes;
+    dd->core = L.dense_classes ? kDenseCore0 << (L.dense_classes - 1) : 0;
+    dd->edge = kDenseEdgeCost;
+    dd->wedge = kDenseWedgeCost;
     *grids = L.g;
     if (rp32) *rp32 = L.rp32 ? reinterpret_cast<uint32_t *>(base + L.rp32) : nullptr;
     sd->rows = rows;
@@ -346,13 +386,14 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
     if (blocks > 0x7fffffffULL) return WTC_ERR_RANGE;
     const bool single = G == 1;
     if (ws_n) WTC_HIPC(s.ws.ensure(ws_n * sizeof(uint64_t)));
-    WTC_HIPC(s.partials.ensure((split ? 2 : 1) * blocks * sizeof(uint64_t)));
+    WTC_HIPC(s.partials.ensure(blocks * sizeof(uint64_t)));
     if (single) WTC_HIPC(s.tree.ensure(kTreeSize * sizeof(uint64_t)));
     // descriptors, then the block list of the small-graph kernel
     if (small_parts > 0x7fffffffULL) return WTC_ERR_RANGE;
     const size_t list_bytes = (size_t)G * sizeof(GraphDesc) + (size_t)small_parts * sizeof(SmallPart);
     const size_t split_off = (list_bytes + 255) & ~(size_t)255;
-    const size_t desc_bytes = split ? split_off + sizeof(SplitDesc) : list_bytes;
+    const size_t dense_off = split_off + sizeof(SplitDesc);
+    const size_t desc_bytes = split ? dense_off + sizeof(DenseDesc) : list_bytes;
     WTC_HIPC(s.desc.ensure(desc_bytes));
     WTC_HIPC(s.out.ensure((size_t)(kMetaSlots + G) * sizeof(uint64_t)));
     if (bm_words) WTC_HIPC(s.bm.ensure(bm_words * sizeof(uint32_t)));
@@ -376,6 +417,7 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
         blk_off += prefix_blocks(d.n);
     }
     SplitDesc sd{};
+    DenseDesc dd{};
     int split_ob = ob;
     const uint64_t *split_rp_src = nullptr;
     uint32_t *split_rp_dst = nullptr;
@@ -386,7 +428,7 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
             base = s.sp.as<char>();
         }
         uint32_t *rp32 = nullptr;
-        split_ob = split_layout(&sd, &plan->split_grids, base, hd[0].n, m[0], split_rows, ob, &rp32);
+        split_ob = split_layout(&sd, &dd, &plan->split_grids, base, hd[0].n, m[0], split_rows, ob, &rp32);
         if (rp32) {  // the split kernels read the 4-byte copy the count starts by making
             split_rp_src = static_cast<const uint64_t *>(hd[0].rowPtr);
             split_rp_dst = rp32;
@@ -396,7 +438,10 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
         WTC_HIPC(split_slabs_grid(split_ob, t.num_cus, &s.slabs_grid));
     }
     std::memcpy(s.h_desc.p, hd.data(), (size_t)G * sizeof(GraphDesc));
-    if (split) std::memcpy(s.h_desc.as<char>() + split_off, &sd, sizeof(SplitDesc));
+    if (split) {
+        std::memcpy(s.h_desc.as<char>() + split_off, &sd, sizeof(SplitDesc));
+        std::memcpy(s.h_desc.as<char>() + dense_off, &dd, sizeof(DenseDesc));
+    }
     SmallPart *h_parts = reinterpret_cast<SmallPart *>(s.h_desc.as<GraphDesc>() + G);
     for (uint32_t g = 0, k = 0; g < G; g++) {
         if (hd[g].mode != kModeSmall) continue;
@@ -432,6 +477,9 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
     plan->small_lds = std::min((small_words * 4u + 255u) & ~255u, t.small_words_max * 4u);
     plan->split = split;
     plan->split_off = split_off;
+    plan->dense_off = dense_off;
+    plan->dense_core = dd.core;
+    plan->num_cus = t.num_cus;
     plan->split_rows = split_rows;
     plan->split_key_part = sd.key_part;
     plan->split_wpb = t.split_wpb;
@@ -454,8 +502,12 @@ int launch_set(Slot &s, const SetPlan &p, bool timed) {
         if (p.split_rp_dst) WTC_HIPC(launch_split_narrow_offsets(p.split_rp_src, p.split_rp_dst, p.split_rp_n, s.stream));
         WTC_HIPC(launch_split_prefix(ddesc, sd, ob, p.blocks, s.partials.as<uint64_t>(), s.stream));
         WTC_HIPC(launch_split_range(ddesc, sd, ob, s.stream));
+        const DenseDesc *dd = reinterpret_cast<const DenseDesc *>(s.desc.as<char>() + p.dense_off);
+        WTC_HIPC(launch_dense_class(ddesc, sd, dd, ob, (uint32_t)(p.split_rp_n - 1), p.blocks, s.partials.as<uint64_t>(), dcounts, s.stream));
+        WTC_HIPC(launch_split_inscan(ddesc, sd, p.blocks, s.partials.as<uint64_t>(), s.stream));
         if (timed) WTC_HIPC(hipEventRecord(s.ev[1], s.stream));
-        WTC_HIPC(launch_split_transpose(ddesc, sd, ob, p.split_grids, p.split_key_part, meta, dcounts, s.stream));
+        if (p.dense_core) WTC_HIPC(launch_dense_count(ddesc, dd, ob, p.dense_core, p.num_cus, dcounts, s.stream));
+        WTC_HIPC(launch_split_transpose(ddesc, sd, dd, ob, p.split_grids, p.split_key_part, meta, s.stream));
         if (timed) WTC_HIPC(hipEventRecord(s.ev[2], s.stream));
         WTC_HIPC(launch_split_rows(ddesc, sd, ob, p.split_rows, p.split_wpb, meta, dcounts, s.rows_grid,
                                    s.stream));
@@ -886,6 +938,16 @@ int wtc_dgraph_count(wtc_ctx *c, wtc_dgraph *dg, uint32_t spread, uint32_t a, ui
     WTC_HIPC(hipSetDevice(c->device));
     std::vector<GraphDesc> hd{make_desc(dg->rowPtr.p, dg->colInd.as<uint32_t>(), dg->n, spread, a, w_begin, w_end)};
     return run_set(c, dg->ob, hd, triangles, st, nullptr, &dg->m);
+}
+
+// The wedges and in-edges of the last split count on this context that its
+// dense part took, of those the stats give for the top rows.
+int wtc_ctx_debug_split(wtc_ctx *c, uint64_t *dense_top_wedges, uint64_t *dense_top_in_edges) {
+    if (!c || !c->slot.split || !c->slot.h_out.p) return WTC_ERR_ARG;
+    const uint64_t *h = c->slot.h_out.as<uint64_t>();
+    if (dense_top_wedges) *dense_top_wedges = h[kMetaDenseTopWedges];
+    if (dense_top_in_edges) *dense_top_in_edges = h[kMetaDenseTopEdges];
+    return WTC_OK;
 }
 
 // Copies the wedge prefix and search tree left by the last single-graph count

@@ -172,7 +172,9 @@ struct SetPlan {
     size_t desc_bytes = 0;
     // split count: SplitDesc at byte split_off of the descriptor buffer
     bool split = false;
-    size_t split_off = 0;
+    size_t split_off = 0, dense_off = 0;  // bytes of the SplitDesc and DenseDesc
+    uint32_t dense_core = 0;              // columns of the dense part's largest class (0: none)
+    int num_cus = 0;
     uint32_t split_rows = 0;
     SplitGrids split_grids;
     uint32_t split_wpb = 8;
@@ -211,7 +213,7 @@ size_t split_workspace_bytes(uint32_t n, uint64_t m, uint32_t rows, int ob);
 // whose positions fit 32 bits, split_narrow) and, through rp32, where the
 // count copies its row offsets to 4 bytes (null when not narrowed).
 bool split_narrow(int ob, uint64_t m);
-int split_layout(SplitDesc *sd, SplitGrids *grids, char *base, uint32_t n, uint64_t m, uint32_t rows, int ob,
+int split_layout(SplitDesc *sd, DenseDesc *dd, SplitGrids *grids, char *base, uint32_t n, uint64_t m, uint32_t rows, int ob,
                  uint32_t **rp32 = nullptr);
 // Waits for the slot (or, if it is done, does not wait) and reads results.
 int finish_set(Slot &s, uint64_t *counts, uint64_t *wedges, RunTimes *rt);

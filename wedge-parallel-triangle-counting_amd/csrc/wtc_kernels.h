@@ -91,6 +91,9 @@ enum : int {
     kMetaListWedges = 6,
     kMetaAllEdges = 7,
     kMetaNext = 8,
+    // split count: what its dense part took of the top rows' totals
+    kMetaDenseTopWedges = 8,
+    kMetaDenseTopEdges = 9,
     kMetaSlots = 16
 };
 
@@ -143,7 +146,7 @@ constexpr uint32_t kSlabTile = 1024;
 // range cuts at the front: [clip_lo, hi)).
 struct SplitDesc {
     uint64_t *ws_full;    // n+1: the full wedge prefix
-    uint64_t *ie_pre;     // n+1: prefix of the in-edges (positions of adj+(v) but the last) of each row
+    uint64_t *ie_pre;     // n+1: prefix of the in-edges of each row (its first positions)
     uint32_t *tile_v;     // first-level tiles: the vertex each starts in
     uint64_t *part_base;  // parts: first record slot of each part
     uint64_t *part_cnt;   // parts: records of each part so far
@@ -192,5 +195,36 @@ struct SplitDesc {
 constexpr uint32_t kSlabAuxLong = 0x1fffu;
 static_assert(kSlabSpan <= 8192 && kSlabRowMax < kSlabAuxLong, "slab_aux fields");
 static_assert(sizeof(SplitDesc) % 8 == 0, "SplitDesc alignment");
+
+// The dense part of a split count (wtc_dense.hip).  Class q holds the
+// vertices whose wedges among the last kDenseCore0 << q ranks are counted as
+// a product of bit matrices.
+constexpr uint32_t kDenseCore0 = 512;
+constexpr uint32_t kDenseClasses = 6;
+// A class's rows hold at least one id per this many columns.  At 64 the rows
+// between cost as much as they save (R-MAT-20 1.31 ms either way, R-MAT-22
+// 4.12 against 4.21, R-MAT-24 20.4 against 20.6).
+constexpr uint32_t kDenseSparsest = 32;
+// What the other kernels take for an in-edge and a wedge, in multiply-adds of
+// the product (3.1e15 a second on R-MAT-24): 24 ps for the transposition and
+// the row kernel's start of a tail, 0.34 ps for a probed id.  Twice or half
+// as much moves R-MAT-20 to R-MAT-26 by less than 1% (half: R-MAT-22 6%).
+constexpr float kDenseEdgeCost = 75000.0f, kDenseWedgeCost = 1050.0f;
+// sums[]: the dense in-edges whose middle vertex is a top row, their wedges,
+// all dense in-edges, and the product's work counter.
+enum : uint32_t { kDenseTopEdges = 0, kDenseTopWedges = 1, kDenseEdges = 2, kDenseNext = 3, kDenseSums = 4 };
+
+struct DenseDesc {
+    void *R;                             // core x core bits: the rows of the last `core` ranks
+    void *B;                             // the listed rows' bits, class by class
+    uint2 *list;                         // (vertex, ids in its class's columns) per class
+    uint32_t *cnt;                       // kDenseClasses: listed vertices
+    uint64_t *sums;                      // kDenseSums
+    uint64_t list_off[kDenseClasses];    // first list entry of each class
+    uint32_t classes;                    // classes in use (0: no dense part)
+    uint32_t core;                       // columns of the largest class
+    float edge, wedge;                   // cost of an in-edge and a wedge elsewhere, in multiply-adds here
+};
+static_assert(sizeof(DenseDesc) % 8 == 0, "DenseDesc alignment");
 
 }  // namespace wtc

@@ -54,7 +54,18 @@ hipError_t count_grid(int kernel, int ob, uint32_t staged, int ways, int wpb, in
 hipError_t launch_count(int kernel, const GraphDesc *desc, uint32_t G, int ob, const uint64_t *tree, uint64_t *meta,
                         unsigned long long *counts, uint32_t max_spread, uint32_t chunk, int ways, int wpb,
                         uint32_t work, uint32_t grid, hipStream_t st);
-// Split count (wtc_split.hip).  partials holds 2*nblocks entries.
+// Dense part of the split count (wtc_dense.hip): the vertices' classes and
+// the in-edges left to the other kernels (into ie_pre, as counts, and the
+// nblocks sums of part_in); zeroes counts[0].
+hipError_t launch_dense_class(const GraphDesc *desc, const SplitDesc *sd, const DenseDesc *dd, int ob, uint32_t n,
+                              uint32_t nblocks, uint64_t *part_in, unsigned long long *counts, hipStream_t st);
+// The listed rows' dense wedges added to counts[0].
+hipError_t launch_dense_count(const GraphDesc *desc, const DenseDesc *dd, int ob, uint32_t core, int num_cus,
+                              unsigned long long *counts, hipStream_t st);
+// ie_pre from the counts and block sums of launch_dense_class.
+hipError_t launch_split_inscan(const GraphDesc *desc, const SplitDesc *sd, uint32_t nblocks, uint64_t *part_in,
+                               hipStream_t st);
+// Split count (wtc_split.hip).  partials holds nblocks entries.
 hipError_t launch_split_prefix(const GraphDesc *desc, const SplitDesc *sd, int ob, uint32_t nblocks,
                                uint64_t *partials, hipStream_t st);
 // The counted range's ends and the in-edge it cuts at the front.
@@ -62,16 +73,15 @@ hipError_t launch_split_range(const GraphDesc *desc, SplitDesc *sd, int ob, hipS
 // dst[i] = src[i] for i < count (8-byte row offsets below 2^32 to 4 bytes).
 hipError_t launch_split_narrow_offsets(const uint64_t *src, uint32_t *dst, uint64_t count, hipStream_t st);
 // The counting sort of the in-edges by key (key_part = the SplitDesc's
-// key_part, on the device); zeroes the tile counters, the wedge tallies and
-// counts[0].
+// key_part, on the device); zeroes the tile counters and the wedge tallies.
 struct SplitGrids {
     uint32_t chunks = 0;          // blocks of the first level
     uint32_t c2cap = 0, c3cap = 0;  // bounds of the second and final levels' blocks
     uint32_t parts = 0, keys = 0;
     uint32_t part_shift = 0, final_shift = 0;  // equal: two levels, else three
 };
-hipError_t launch_split_transpose(const GraphDesc *desc, const SplitDesc *sd, int ob, const SplitGrids &g,
-                                  uint64_t *key_part, uint64_t *meta, unsigned long long *counts, hipStream_t st);
+hipError_t launch_split_transpose(const GraphDesc *desc, const SplitDesc *sd, const DenseDesc *dd, int ob,
+                                  const SplitGrids &g, uint64_t *key_part, uint64_t *meta, hipStream_t st);
 // Waves per block of the row kernel: 4, 8 or 16.
 bool valid_split_waves(int wpb);
 // LDS bytes of the row kernel's bitmap for `rows` top rows.

@@ -23,9 +23,14 @@
 // numbering, tc.cu:203-212) holds the in-edges of the vertices between its
 // ends, with the tails of the two end vertices clipped.
 //
-// Pipeline on one stream: k_split_partials, k_scan_partials (twice) and
-// k_split_scan (the full wedge prefix and the in-edge prefix);
-// k_split_range; the transposition, a counting sort by key: k_split_parthist
+// Where a row has many ids among the last ranks, its wedges there are counted
+// as a product of bit matrices instead (wtc_dense.hip): those in-edges are at
+// the row's end, and the rest of this file sees rows without them.
+//
+// Pipeline on one stream: k_split_partials, k_scan_partials and k_split_scan
+// (the full wedge prefix); k_split_range; k_dense_class, k_scan_partials and
+// k_split_inscan (the prefix of the in-edges left); k_dense_rows and
+// k_dense_mm; the transposition, a counting sort by key: k_split_parthist
 // and k_split_partbase (part sizes), k_split_l1 (records bucketed by part),
 // k_split_bases; with many keys k_split_level_count, k_split_levelcols2,
 // k_split_bases and k_split_level_scatter to sub-parts; then
@@ -61,72 +66,48 @@ __device__ __forceinline__ uint64_t row_base(uint64_t i, uint64_t d) { return i 
 
 // --------------------------------------------------------------- prefixes
 
-// In-edges of a row of out-degree d: every position but the last.
-__device__ __forceinline__ uint64_t in_edges_of(uint64_t d) { return d ? d - 1 : 0; }
-
-// Block b: vertices [b*kScanChunk, (b+1)*kScanChunk): the sums of the full
-// order's wedges and of the in-edges.
+// Block b: vertices [b*kScanChunk, (b+1)*kScanChunk): the sum of the full
+// order's wedges.
 template <typename OffT>
 __global__ __launch_bounds__(kBlock) void k_split_partials(const GraphDesc *__restrict__ desc,
-                                                           uint64_t *__restrict__ part_full,
-                                                           uint64_t *__restrict__ part_in) {
-    __shared__ uint64_t s_f[kWavesPerBlock], s_i[kWavesPerBlock];
+                                                           uint64_t *__restrict__ part_full) {
+    __shared__ uint64_t s_f[kWavesPerBlock];
     const GraphDesc &D = desc[0];
     const OffT *__restrict__ rowPtr = static_cast<const OffT *>(D.rowPtr);
     const uint32_t n = D.n;
     const uint64_t base = (uint64_t)blockIdx.x * kScanChunk;
-    uint64_t af = 0, ai = 0;
+    uint64_t af = 0;
     for (int k = 0; k < kScanItems; k++) {
         const uint64_t v = base + (uint64_t)k * kBlock + threadIdx.x;
-        if (v < n) {
-            const uint64_t d = (uint64_t)(rowPtr[v + 1] - rowPtr[v]);
-            af += binom2_d(d);
-            ai += in_edges_of(d);
-        }
+        if (v < n) af += binom2_d((uint64_t)(rowPtr[v + 1] - rowPtr[v]));
     }
     af = wave_sum(af);
-    ai = wave_sum(ai);
-    if ((threadIdx.x & (kWave - 1)) == 0) {
-        s_f[threadIdx.x >> 6] = af;
-        s_i[threadIdx.x >> 6] = ai;
-    }
+    if ((threadIdx.x & (kWave - 1)) == 0) s_f[threadIdx.x >> 6] = af;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        part_full[blockIdx.x] = s_f[0] + s_f[1] + s_f[2] + s_f[3];
-        part_in[blockIdx.x] = s_i[0] + s_i[1] + s_i[2] + s_i[3];
-    }
+    if (threadIdx.x == 0) part_full[blockIdx.x] = s_f[0] + s_f[1] + s_f[2] + s_f[3];
 }
 
-// ws_full and ie_pre from the scanned block partials, and slab_row.
+// ws_full from the scanned block partials, and slab_row.
 template <typename OffT>
 __global__ __launch_bounds__(kBlock) void k_split_scan(const GraphDesc *__restrict__ desc,
                                                        const SplitDesc *__restrict__ sd,
-                                                       const uint64_t *__restrict__ part_full,
-                                                       const uint64_t *__restrict__ part_in) {
+                                                       const uint64_t *__restrict__ part_full) {
     __shared__ uint64_t s_tot[kWavesPerBlock];
     const GraphDesc &D = desc[0];
     const OffT *__restrict__ rowPtr = static_cast<const OffT *>(D.rowPtr);
     uint64_t *__restrict__ wf = sd->ws_full;
-    uint64_t *__restrict__ wi = sd->ie_pre;
     uint32_t *__restrict__ slab_row = sd->slab_row;
     const uint32_t n = D.n, thr = D.thr, slabs = sd->slabs;
-    uint64_t cf = part_full[blockIdx.x], ci = part_in[blockIdx.x];
+    uint64_t cf = part_full[blockIdx.x];
     const uint64_t base = (uint64_t)blockIdx.x * kScanChunk;
     for (int k = 0; k < kScanItems; k++) {
         if (base + (uint64_t)k * kBlock >= n) break;  // block-uniform
         const uint64_t v = base + (uint64_t)k * kBlock + threadIdx.x;
-        uint64_t xf = 0, xi = 0;
-        if (v < n) {
-            const uint64_t d = (uint64_t)(rowPtr[v + 1] - rowPtr[v]);
-            xf = binom2_d(d);
-            xi = in_edges_of(d);
-        }
-        uint64_t tf, ti;
+        const uint64_t xf = v < n ? binom2_d((uint64_t)(rowPtr[v + 1] - rowPtr[v])) : 0;
+        uint64_t tf;
         const uint64_t ef = block_excl_scan(xf, s_tot, tf);
-        const uint64_t ei = block_excl_scan(xi, s_tot, ti);
         if (v < n) {
             wf[v] = cf + ef;
-            wi[v] = ci + ei;
             if (v <= thr) {  // the slabs whose first row is v: rowPtr[v - 1] < s*kSlabSpan <= rowPtr[v]
                 const uint64_t s_hi = (uint64_t)rowPtr[v] / kSlabSpan;
                 for (uint64_t s = v ? (uint64_t)rowPtr[v - 1] / kSlabSpan + 1 : 0; s <= s_hi && s <= slabs; s++)
@@ -134,12 +115,29 @@ __global__ __launch_bounds__(kBlock) void k_split_scan(const GraphDesc *__restri
             }
         }
         cf += tf;
-        ci += ti;
     }
-    if (blockIdx.x == (n - 1) / kScanChunk && threadIdx.x == 0) {
-        wf[n] = cf;
-        wi[n] = ci;
+    if (blockIdx.x == (n - 1) / kScanChunk && threadIdx.x == 0) wf[n] = cf;
+}
+
+// ie_pre: its counts of in-edges (k_dense_class) become their prefix.
+__global__ __launch_bounds__(kBlock) void k_split_inscan(const GraphDesc *__restrict__ desc,
+                                                         const SplitDesc *__restrict__ sd,
+                                                         const uint64_t *__restrict__ part_in) {
+    __shared__ uint64_t s_tot[kWavesPerBlock];
+    uint64_t *__restrict__ wi = sd->ie_pre;
+    const uint32_t n = desc[0].n;
+    uint64_t ci = part_in[blockIdx.x];
+    const uint64_t base = (uint64_t)blockIdx.x * kScanChunk;
+    for (int k = 0; k < kScanItems; k++) {
+        if (base + (uint64_t)k * kBlock >= n) break;  // block-uniform
+        const uint64_t v = base + (uint64_t)k * kBlock + threadIdx.x;
+        const uint64_t x = v < n ? wi[v] : 0;
+        uint64_t t;
+        const uint64_t ex = block_excl_scan(x, s_tot, t);
+        if (v < n) wi[v] = ci + ex;
+        ci += t;
     }
+    if (blockIdx.x == (n - 1) / kScanChunk && threadIdx.x == 0) wi[n] = ci;
 }
 
 // Thread 0: the counted range of the full order, its end vertices, and the
@@ -239,7 +237,7 @@ struct LevelTile {
 
 // First-level part sizes, as an upper bound: every position of the counted
 // vertices' rows in its id's part (the in-edges are all of them but each
-// row's last, and fewer where the range clips a row).  Positions in order
+// row's last or its dense ones, and fewer where the range clips a row).  Positions in order
 // run through a row's ascending ids, so neighbouring lanes mostly share a
 // part: one LDS atomic per run of equal parts instead of one per id, which
 // with few parts all fell on the same counters (R-MAT-20: 112 us).  A list
@@ -897,14 +895,14 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_keysum(const SplitDesc *_
 // Block b (key_part then holding the exclusive prefix of the key blocks):
 // rp_in of its keys; the block of key `rows` puts the top rows' in-edges
 // into meta, the last block rp_in[keys] and the rest of meta (tile counters
-// and wedge tallies zeroed, the counted wedges and all in-edges) and
-// counts[0] = 0.
+// and wedge tallies zeroed, the counted wedges and all in-edges).
 template <typename OffT>
 __global__ __launch_bounds__(kSplitBlock) void k_split_keyscan(const SplitDesc *__restrict__ sd,
-                                                               uint64_t *__restrict__ meta,
-                                                               unsigned long long *__restrict__ counts) {
+                                                               const DenseDesc *__restrict__ dd,
+                                                               uint64_t *__restrict__ meta) {
     __shared__ uint64_t s_w[kSplitBlock / kWave];
     const SplitDesc &S = sd[0];
+    const uint64_t *__restrict__ dense = dd->sums;  // the dense in-edges and wedges are in the totals
     const uint32_t keys = S.keys, rows = S.rows;
     OffT *__restrict__ rp = static_cast<OffT *>(S.rp_in);
     const uint64_t i0 = (uint64_t)blockIdx.x * kKeyChunk + 4ull * threadIdx.x;
@@ -920,20 +918,21 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_keyscan(const SplitDesc *
 #pragma unroll
     for (uint32_t z = 0; z < 4; z++) {
         if (i0 + z < keys) rp[i0 + z] = (OffT)at;
-        if (i0 + z == rows) meta[kMetaInEdges] = at;
+        if (i0 + z == rows) meta[kMetaInEdges] = at + dense[kDenseTopEdges];
         at += v[z];
     }
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
         const uint64_t all = S.key_part[blockIdx.x] + tot;
         rp[keys] = (OffT)all;
-        if (rows >= keys) meta[kMetaInEdges] = all;
+        if (rows >= keys) meta[kMetaInEdges] = all + dense[kDenseTopEdges];
         meta[kMetaRows] = 0;
         meta[kMetaSlabs] = 0;
-        meta[kMetaTopWedges] = 0;
+        meta[kMetaTopWedges] = dense[kDenseTopWedges];
+        meta[kMetaDenseTopWedges] = dense[kDenseTopWedges];
+        meta[kMetaDenseTopEdges] = dense[kDenseTopEdges];
         meta[kMetaListWedges] = 0;
         meta[kMetaWedges] = S.w_hi - S.w_lo;
-        meta[kMetaAllEdges] = all;
-        counts[0] = 0;
+        meta[kMetaAllEdges] = all + dense[kDenseEdges];
     }
 }
 
@@ -1479,13 +1478,18 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
 hipError_t launch_split_prefix(const GraphDesc *desc, const SplitDesc *sd, int ob, uint32_t nblocks,
                                uint64_t *partials, hipStream_t st) {
     if (nblocks == 0) return hipSuccess;
-    uint64_t *pf = partials, *pi = partials + nblocks;
-    hipError_t e = WTC_LAUNCH_OFF(ob, k_split_partials, dim3(nblocks), dim3(kBlock), 0, st, desc, pf, pi);
+    hipError_t e = WTC_LAUNCH_OFF(ob, k_split_partials, dim3(nblocks), dim3(kBlock), 0, st, desc, partials);
     if (e != hipSuccess) return e;
-    if ((e = launch_scan_partials(pf, nblocks, st)) != hipSuccess) return e;
-    if ((e = launch_scan_partials(pi, nblocks, st)) != hipSuccess) return e;
-    return WTC_LAUNCH_OFF(ob, k_split_scan, dim3(nblocks), dim3(kBlock), 0, st, desc, sd, (const uint64_t *)pf,
-                          (const uint64_t *)pi);
+    if ((e = launch_scan_partials(partials, nblocks, st)) != hipSuccess) return e;
+    return WTC_LAUNCH_OFF(ob, k_split_scan, dim3(nblocks), dim3(kBlock), 0, st, desc, sd, (const uint64_t *)partials);
+}
+
+hipError_t launch_split_inscan(const GraphDesc *desc, const SplitDesc *sd, uint32_t nblocks, uint64_t *part_in,
+                               hipStream_t st) {
+    hipError_t e = launch_scan_partials(part_in, nblocks, st);
+    if (e != hipSuccess) return e;
+    k_split_inscan<<<dim3(nblocks), dim3(kBlock), 0, st>>>(desc, sd, part_in);
+    return hipGetLastError();
 }
 
 // 8-byte row offsets that all fit 32 bits, copied to 4 bytes.
@@ -1544,8 +1548,8 @@ hipError_t launch_final(bool scatter, bool from_b, uint32_t shift, const SplitDe
 }
 
 template <typename OffT>
-hipError_t transpose(const GraphDesc *desc, const SplitDesc *sd, const SplitGrids &g, uint64_t *key_part, uint64_t *meta,
-                     unsigned long long *counts, hipStream_t st) {
+hipError_t transpose(const GraphDesc *desc, const SplitDesc *sd, const DenseDesc *dd, const SplitGrids &g,
+                     uint64_t *key_part, uint64_t *meta, hipStream_t st) {
     const dim3 blk(kSplitBlock);
     const uint32_t g2 = g.c2cap < kLevelGridMax ? g.c2cap : kLevelGridMax;
     const uint32_t g3 = g.c3cap < kLevelGridMax ? g.c3cap : kLevelGridMax;
@@ -1574,7 +1578,7 @@ hipError_t transpose(const GraphDesc *desc, const SplitDesc *sd, const SplitGrid
     k_split_keysum<<<gkb, blk, 0, st>>>(sd);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if ((e = launch_scan_partials(key_part, gkb.x, st)) != hipSuccess) return e;
-    k_split_keyscan<OffT><<<gkb, blk, 0, st>>>(sd, meta, counts);
+    k_split_keyscan<OffT><<<gkb, blk, 0, st>>>(sd, dd, meta);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if ((e = launch_final<OffT>(true, three, g.final_shift, sd, g3, st)) != hipSuccess) return e;
     // the packed top ids, over the final level's input pairs
@@ -1584,12 +1588,12 @@ hipError_t transpose(const GraphDesc *desc, const SplitDesc *sd, const SplitGrid
 
 }  // namespace
 
-hipError_t launch_split_transpose(const GraphDesc *desc, const SplitDesc *sd, int ob, const SplitGrids &g,
-                                  uint64_t *key_part, uint64_t *meta, unsigned long long *counts, hipStream_t st) {
+hipError_t launch_split_transpose(const GraphDesc *desc, const SplitDesc *sd, const DenseDesc *dd, int ob,
+                                  const SplitGrids &g, uint64_t *key_part, uint64_t *meta, hipStream_t st) {
     if (g.keys == 0 || g.chunks == 0 || g.c3cap == 0 || g.parts == 0 || g.parts > kSplitPartsMax)
         return hipErrorInvalidValue;
-    return ob == 8 ? transpose<uint64_t>(desc, sd, g, key_part, meta, counts, st)
-                   : transpose<uint32_t>(desc, sd, g, key_part, meta, counts, st);
+    return ob == 8 ? transpose<uint64_t>(desc, sd, dd, g, key_part, meta, st)
+                   : transpose<uint32_t>(desc, sd, dd, g, key_part, meta, st);
 }
 
 size_t split_rows_lds(uint32_t rows) { return (size_t)(((rows + 31) / 32 + 1) & ~1u) * sizeof(uint32_t) + sizeof(uint64_t); }

@@ -152,6 +152,7 @@ _sig = {
                                    C.c_uint64, C.c_uint64, _P, _P]),
     "wtc_ctx_debug_prefix": (C.c_int, [_P, C.c_uint64, _P, _P]),
     "wtc_ctx_debug_bitmap": (C.c_int, [_P, C.c_uint64, _P]),
+    "wtc_ctx_debug_split": (C.c_int, [_P, C.POINTER(C.c_uint64), C.POINTER(C.c_uint64)]),
     "wtc_debug_decode": (C.c_int, [_P, _P, _P, C.c_uint64, _P, _P]),
     "wtc_debug_copy": (C.c_int, [_P, C.c_uint64, C.c_int, C.POINTER(C.c_double)]),
     "wtc_ctx_set_tuning": (C.c_int, [_P, C.c_int, C.c_uint32, C.c_int]),
@@ -522,6 +523,12 @@ class Context:
         _check(_lib.wtc_debug_decode(self._p, d.ctypes.data, iv.ctypes.data, d.size, w.ctypes.data, u.ctypes.data),
                "debug_decode")
         return w, u
+
+    def debug_split(self):
+        """(wedges, in-edges) of the last split count's top rows that its dense part took."""
+        w, e = C.c_uint64(), C.c_uint64()
+        _check(_lib.wtc_ctx_debug_split(self._p, C.byref(w), C.byref(e)), "debug_split")
+        return int(w.value), int(e.value)
 
     def debug_bitmap(self, words: int) -> np.ndarray:
         out = np.zeros(max(words, 1), dtype=np.uint32)
