@@ -456,14 +456,17 @@ def tune_sweep(args):
         # bitmap rows past 2^18 only for the split count (one row in LDS, no a*a/8 bytes in HBM);
         # 65,536 is the largest a whose packed ids take 16 bits
         split_alens = sorted(set([x for x in alens if x] + [x for x in (65536, 524288, 1048576) if x <= n32 and W > 0]))
-        best = best_walk = None
+        best = best_walk = best_staged = None
         base = wtc.Tuned(0, 0, wtc.KERNEL_WALK, 4, 4, 8)
-        kernels = (wtc.KERNEL_SPLIT,) if big else (wtc.KERNEL_WALK, wtc.KERNEL_STAGED, wtc.KERNEL_SPLIT)
+        kernels = (wtc.KERNEL_SPLIT,) if big else (wtc.KERNEL_WALK, wtc.KERNEL_STAGED, wtc.KERNEL_SPLIT,
+                                                   wtc.KERNEL_ROWS)
         spreads = {wtc.KERNEL_WALK: (2, 4, 8, 16, 32, 64, 128), wtc.KERNEL_STAGED: (2, 4, 8, 16, 32),
-                   wtc.KERNEL_SPLIT: (12,)}
+                   wtc.KERNEL_SPLIT: (12,), wtc.KERNEL_ROWS: (8,)}
         for kernel in kernels:
             for a in (split_alens if kernel == wtc.KERNEL_SPLIT else alens):
                 if kernel == wtc.KERNEL_SPLIT and (a == 0 or (big and a < 131072)):
+                    continue
+                if kernel == wtc.KERNEL_ROWS and a:  # it has no bitmap
                     continue
                 # (the split count has no spread: one value stands in its row of the table)
                 log(f"tune {workload}: kernel {kernel} a {a}")
@@ -478,13 +481,17 @@ def tune_sweep(args):
                             best = (ms, t)
                         if kernel == wtc.KERNEL_WALK and (best_walk is None or ms < best_walk[0]):
                             best_walk = (ms, t)
+                        if kernel == wtc.KERNEL_STAGED and (best_staged is None or ms < best_staged[0]):
+                            best_staged = (ms, t)
         ms0, t0 = best
         log(f"tune {workload}: stage 1 best {ms0:.3f} ms {t0.as_dict()}")
-        split = t0.kernel == wtc.KERNEL_SPLIT
+        split, by_rows = t0.kernel == wtc.KERNEL_SPLIT, t0.kernel == wtc.KERNEL_ROWS
         # stage 2: the block shape of the winner; a split row also keeps the
         # walk's best spread and block shape, which the walk takes where the
-        # split count does not apply (a = 0, a set of graphs)
-        walk0 = (best_walk[1] if best_walk else None) if split else t0
+        # split count does not apply (a = 0, a set of graphs), and a rows row
+        # the staged kernel's best spread, bitmap length and block shape, for
+        # wedge ranges
+        walk0 = (best_walk[1] if best_walk else None) if split else best_staged[1] if by_rows else t0
         walk_best = None
         if walk0 is not None and not big:  # (graphs built on the GPU: the split count only)
             for waves in (2, 4, 8):
@@ -505,12 +512,17 @@ def tune_sweep(args):
                 w = walk_best[1]
                 best = (best[0], wtc.Tuned(w.spread, best[1].adjacency_matrix_len, wtc.KERNEL_SPLIT, w.waves_per_block,
                                            w.probe_ways, best[1].split_waves))
+        elif by_rows:
+            w = walk_best[1]
+            best = (best[0], wtc.Tuned(w.spread, w.adjacency_matrix_len, wtc.KERNEL_ROWS, w.waves_per_block, w.probe_ways,
+                                       8))
         elif walk_best and walk_best[0] < best[0]:
             best = walk_best
         dg.free()
         ms, t = best
         a = t.adjacency_matrix_len
-        kname = {wtc.KERNEL_WALK: "walk", wtc.KERNEL_STAGED: "staged", wtc.KERNEL_SPLIT: "split"}[t.kernel]
+        kname = {wtc.KERNEL_WALK: "walk", wtc.KERNEL_STAGED: "staged", wtc.KERNEL_SPLIT: "split",
+                 wtc.KERNEL_ROWS: "rows"}[t.kernel]
         row = ("alone", family_skew, int(math.floor(math.log2(W))) if W else 0, t.spread, 1 if a else 0, a, kname,
                t.waves_per_block, t.probe_ways, t.split_waves, ms, workload)
         log(f"tune {workload}: n={n} m={m} W={W} -> {row}")
@@ -543,9 +555,18 @@ def tune_sweep(args):
                         ms = statistics.median(ts)
                         if best is None or ms < best[0]:
                             best = (ms, sp, waves, ways, kernel)
+        # the row count in its place when it is faster (the shape stays for wedge ranges)
+        ctx.use_tuned(wtc.Tuned(8, 0, wtc.KERNEL_ROWS, best[2], best[3], 8))
+        ts = []
+        for _ in range(4):
+            t0 = time.perf_counter()
+            b.count([8] * len(graphs), [0] * len(graphs))
+            ts.append((time.perf_counter() - t0) * 1e3)
+        if statistics.median(ts[1:]) < best[0]:
+            best = (statistics.median(ts[1:]),) + best[1:4] + (wtc.KERNEL_ROWS,)
         b.free()
         ms, sp, waves, ways, kernel = best
-        kname = "staged" if kernel == wtc.KERNEL_STAGED else "walk"
+        kname = {wtc.KERNEL_WALK: "walk", wtc.KERNEL_STAGED: "staged", wtc.KERNEL_ROWS: "rows"}[kernel]
         rows.append(("batch", "any", 0, sp, 0, 0, kname, waves, ways, 8, ms, f"batch{args.tune_batch}"))
         log(f"tune batch: {rows[-1]}")
     ctx.close()
@@ -769,7 +790,7 @@ def main():
     ap.add_argument("--ways", type=int, default=None, help="probes advanced together per lane (default: autotuner)")
     ap.add_argument("--chunk", type=int, default=12, help="wedges per lane staged in LDS per phase (staged kernel)")
     ap.add_argument("--waves", type=int, default=None, help="waves per counting block, 1/2/4/8 (default: autotuner)")
-    ap.add_argument("--kernel", type=int, default=None, help="0 walk, 1 staged, 2 split (default: autotuner)")
+    ap.add_argument("--kernel", type=int, default=None, help="0 walk, 1 staged, 2 split, 3 rows (default: autotuner)")
     ap.add_argument("--split-waves", type=int, default=None, help="waves per row-kernel block, 4/8/16 (default: autotuner)")
     ap.add_argument("--builder", choices=("auto", "host", "device"), default="auto",
                     help="build the oriented CSR on the host or on the GPU (auto: GPU from scale 26)")

@@ -246,10 +246,17 @@ int wtc_ctx_set_tuning(wtc_ctx *ctx, int probe_ways, uint32_t lds_chunk, int wav
  *                     instead.  Batches, a = 0, a row of a bits that does
  *                     not fit a block's LDS and colInd not 16-byte aligned:
  *                     the row walk.  Same count for every wedge range.
+ *   WTC_KERNEL_ROWS   whole graphs, alone or in sets: every edge v -> w
+ *                     closes |adj+(v) and adj+(w)| triangles; the rows of v
+ *                     of 512 edges at a time hashed into LDS, adj+(w)
+ *                     streamed through them.  No prefix, no bitmap (the
+ *                     spread and bitmap length have no effect), two
+ *                     launches.  Wedge ranges: WTC_KERNEL_STAGED.
  * Default WTC_KERNEL_WALK or $WTC_COUNT_KERNEL. */
 #define WTC_KERNEL_WALK 0
 #define WTC_KERNEL_STAGED 1
 #define WTC_KERNEL_SPLIT 2
+#define WTC_KERNEL_ROWS 3
 int wtc_ctx_set_count_kernel(wtc_ctx *ctx, int kernel);
 /* How the counting kernels hand out work: the wedge order is cut into tiles
  * of 64*s wedges, and a wave takes up to tiles_per_grab consecutive tiles

@@ -16,7 +16,7 @@
 //   spread       s
 //   a_div/a_cap  a = min(a_cap, n / a_div rounded up to a multiple of 32);
 //                a_div = 0: a = 0
-//   kernel       walk, staged or split (WTC_KERNEL_*)
+//   kernel       walk, staged, split or rows (WTC_KERNEL_*)
 //   waves ways   the counting block's waves and probes in flight per lane
 //   split_waves  waves per block of the split count's row kernel
 //
@@ -73,6 +73,7 @@ int parse_kernel(const std::string &k) {
     if (k == "staged") return WTC_KERNEL_STAGED;
     if (k == "split") return WTC_KERNEL_SPLIT;
     if (k == "walk") return WTC_KERNEL_WALK;
+    if (k == "rows") return WTC_KERNEL_ROWS;
     return -1;
 }
 

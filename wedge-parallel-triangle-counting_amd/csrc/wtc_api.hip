@@ -363,6 +363,22 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
         small_parts += small_parts_of(W[g]);
         small_words = std::max(small_words, (uint32_t)words);
     }
+    // The row count takes whole graphs (every wedge of each); it needs no
+    // prefix and no bitmap.
+    const bool want_rows = t.kernel == kKernelRows || (t.rows_else && t.kernel == kKernelSplit);
+    bool rows_ok = want_rows && m && !all_small &&
+                   !(G == 1 && split_eligible(t, hd[0], m[0]) && (!t.split_needs_base || split_base));
+    for (uint32_t g = 0; g < G && rows_ok; g++)
+        rows_ok = hd[g].mode == kModeTiles && hd[g].w_begin == 0 && hd[g].w_end == UINT64_MAX;
+    uint64_t rows_tiles = 0;
+    for (uint32_t g = 0; g < G && rows_ok; g++) {
+        hd[g].bm_rows = 0;
+        hd[g].bm_words = 0;
+        hd[g].bitmap = nullptr;
+        hd[g].wcount = m[g];
+        hd[g].tile_base = rows_tiles;
+        rows_tiles += (m[g] + kRowsTile - 1) / kRowsTile;
+    }
     // The split count takes a single graph with a bitmap length whose colInd
     // is 16-byte aligned (its slab kernel loads four ids at a time); its top
     // rows then need no bitmap in HBM.
@@ -378,7 +394,7 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
     for (const auto &d : hd) {
         if (d.n == 0 || d.spread == 0) return WTC_ERR_ARG;
         if (d.mode == kModeTiles) max_spread = std::max(max_spread, d.spread);
-        if (!d.ws && !split) ws_n += (uint64_t)d.n + 1;  // the split count keeps its prefixes in its workspace
+        if (!d.ws && !split && !rows_ok) ws_n += (uint64_t)d.n + 1;  // the split count keeps its prefixes in its workspace
         if (d.bm_rows && !d.bitmap) bm_words += bm_words_for(d.a);
         rows += d.bm_rows;
         blocks += prefix_blocks(d.n);
@@ -386,8 +402,8 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
     if (blocks > 0x7fffffffULL) return WTC_ERR_RANGE;
     const bool single = G == 1;
     if (ws_n) WTC_HIPC(s.ws.ensure(ws_n * sizeof(uint64_t)));
-    WTC_HIPC(s.partials.ensure(blocks * sizeof(uint64_t)));
-    if (single) WTC_HIPC(s.tree.ensure(kTreeSize * sizeof(uint64_t)));
+    if (!rows_ok) WTC_HIPC(s.partials.ensure(blocks * sizeof(uint64_t)));
+    if (single && !rows_ok) WTC_HIPC(s.tree.ensure(kTreeSize * sizeof(uint64_t)));
     // descriptors, then the block list of the small-graph kernel
     if (small_parts > 0x7fffffffULL) return WTC_ERR_RANGE;
     const size_t list_bytes = (size_t)G * sizeof(GraphDesc) + (size_t)small_parts * sizeof(SmallPart);
@@ -403,7 +419,7 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
     for (auto &d : hd) {
         d.bm_clear_base = clear_off;
         clear_off += d.bm_rows ? bm_words_for(d.a) : 0;
-        if (!d.ws && !split) {
+        if (!d.ws && !split && !rows_ok) {
             d.ws = s.ws.as<uint64_t>() + ws_off;
             ws_off += (uint64_t)d.n + 1;
         }
@@ -451,13 +467,17 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
 
     const int oi = ob == 8 ? 1 : 0;
     const uint32_t staged = std::min<uint32_t>(max_spread, t.chunk);
-    // a set the split count does not take uses the row walk
-    const int kernel = t.kernel == kKernelStaged ? kKernelStaged : kKernelWalk;
+    // a set the split count does not take uses the row walk, a range the row
+    // count does not take the staged kernel
+    const int kernel = t.kernel == kKernelStaged || t.kernel == kKernelRows ? kKernelStaged : kKernelWalk;
     uint32_t &gc = t.grid_cache[kernel == kKernelWalk ? 0 : 1][oi][ways_index(t.ways)][wpb_index(t.wpb)][staged];
-    if (!gc) WTC_HIPC(count_grid(kernel, ob, staged, t.ways, t.wpb, t.num_cus, &gc));
+    if (!gc && !rows_ok) WTC_HIPC(count_grid(kernel, ob, staged, t.ways, t.wpb, t.num_cus, &gc));
+    uint32_t &rg = t.rows_grid[oi];
+    if (rows_ok && !rg) WTC_HIPC(rows_grid(ob, t.num_cus, &rg));
     s.G = G;
-    s.grid = gc;
+    s.grid = rows_ok ? rg : gc;
     s.split = split;
+    s.rows = rows_ok;
     s.small = small_n;
     plan->G = G;
     plan->ob = ob;
@@ -475,6 +495,9 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
     plan->small_count = (uint32_t)small_parts;
     plan->tile_graphs = G - small_n;
     plan->small_lds = std::min((small_words * 4u + 255u) & ~255u, t.small_words_max * 4u);
+    plan->by_rows = rows_ok;
+    plan->rows_tiles = rows_tiles;
+    plan->rows_grid = rg;
     plan->split = split;
     plan->split_off = split_off;
     plan->dense_off = dense_off;
@@ -490,10 +513,19 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
     return WTC_OK;
 }
 
-int launch_set(Slot &s, const SetPlan &p, bool timed) {
+int launch_set(Slot &s, const SetPlan &p, bool timed, bool desc_ready) {
     uint64_t *meta = s.out.as<uint64_t>();
     unsigned long long *dcounts = reinterpret_cast<unsigned long long *>(meta + kMetaSlots);
     GraphDesc *ddesc = s.desc.as<GraphDesc>();
+    if (p.by_rows) {
+        if (timed) WTC_HIPC(hipEventRecord(s.ev[0], s.stream));
+        WTC_HIPC(launch_rows(desc_ready ? nullptr : s.h_desc.as<uint64_t>(), ddesc, p.G, p.ob, p.rows_tiles, meta, dcounts,
+                             p.rows_grid, s.stream));
+        if (timed) WTC_HIPC(hipEventRecord(s.ev[3], s.stream));
+        WTC_HIPC(hipMemcpyAsync(s.h_out.p, meta, (size_t)(kMetaSlots + p.G) * sizeof(uint64_t), hipMemcpyDeviceToHost,
+                                s.stream));
+        return WTC_OK;
+    }
     uint64_t *tree = p.single ? s.tree.as<uint64_t>() : nullptr;
     if (p.split) {
         SplitDesc *sd = reinterpret_cast<SplitDesc *>(s.desc.as<char>() + p.split_off);
@@ -536,14 +568,18 @@ int launch_set(Slot &s, const SetPlan &p, bool timed) {
     return WTC_OK;
 }
 
+// Most descriptors (128 bytes each) a kernel reads across the bus itself.
+constexpr uint32_t kRowsFetchMax = 64;
+
 int enqueue_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, const uint64_t *m, const uint64_t *W,
                 char *split_base) {
     SetPlan p;
     int rc = stage_set(s, t, ob, hd, &p, m, W, split_base);
     if (rc) return rc;
-    WTC_HIPC(hipMemcpyAsync(s.desc.p, s.h_desc.p, p.desc_bytes, hipMemcpyHostToDevice,
-                            s.stream));
-    return launch_set(s, p, true);
+    // a row count of few graphs reads its descriptors from the pinned memory
+    const bool fetch = p.by_rows && kRowsFetchMax >= p.G;
+    if (!fetch) WTC_HIPC(hipMemcpyAsync(s.desc.p, s.h_desc.p, p.desc_bytes, hipMemcpyHostToDevice, s.stream));
+    return launch_set(s, p, true, !fetch);
 }
 
 uint32_t default_small_words() {
@@ -568,7 +604,10 @@ int finish_set(Slot &s, uint64_t *counts, uint64_t *wedges, RunTimes *rt) {
     const uint64_t *h = s.h_out.as<uint64_t>();
     for (uint32_t g = 0; g < s.G; g++) counts[g] = h[kMetaSlots + g];
     if (wedges) *wedges = h[kMetaWedges];
-    if (rt) {
+    if (rt && s.rows) {
+        rt->rows = true;
+        WTC_HIPC(hipEventElapsedTime(&rt->count_ms, s.ev[0], s.ev[3]));
+    } else if (rt) {
         WTC_HIPC(hipEventElapsedTime(&rt->prefix_ms, s.ev[0], s.ev[1]));
         WTC_HIPC(hipEventElapsedTime(&rt->bitmap_ms, s.ev[1], s.ev[2]));
         WTC_HIPC(hipEventElapsedTime(&rt->count_ms, s.ev[2], s.ev[3]));
@@ -591,6 +630,11 @@ namespace {
 bool valid_ways(int w) { return w == 1 || w == 2 || w == 4 || w == 8; }
 bool valid_waves(int v) { return valid_count_waves(v); }
 
+static_assert(kKernelWalk == WTC_KERNEL_WALK && kKernelStaged == WTC_KERNEL_STAGED &&
+                  kKernelSplit == WTC_KERNEL_SPLIT && kKernelRows == WTC_KERNEL_ROWS,
+              "the ABI's kernel numbers");
+bool valid_kernel(int k) { return k >= kKernelWalk && k <= kKernelRows; }
+
 // Default probes per lane for new contexts: WTC_PROBE_WAYS (1, 2, 4 or 8),
 // else 4.
 int default_probe_ways() {
@@ -608,11 +652,11 @@ int default_count_waves() {
 }
 
 // Default counting kernel for new contexts: WTC_COUNT_KERNEL (0 row walk,
-// 1 staged, 2 split), else the row walk.
+// 1 staged, 2 split, 3 rows), else the row walk.
 int default_count_kernel() {
     const char *e = std::getenv("WTC_COUNT_KERNEL");
     const int v = e ? std::atoi(e) : kKernelWalk;
-    return v == kKernelStaged || v == kKernelSplit ? v : kKernelWalk;
+    return v == kKernelStaged || v == kKernelSplit || v == kKernelRows ? v : kKernelWalk;
 }
 
 int set_device(int dev) {
@@ -690,10 +734,9 @@ namespace {
 // context.
 int apply_tuned(wtc_ctx *c, const wtc_tuned &t) {
     if (!valid_ways(t.probe_ways) || !valid_waves(t.waves_per_block) || !valid_split_waves(t.split_waves) ||
-        (t.kernel != WTC_KERNEL_WALK && t.kernel != WTC_KERNEL_STAGED && t.kernel != WTC_KERNEL_SPLIT))
+        !valid_kernel(t.kernel))
         return WTC_ERR_ARG;
-    c->tune.kernel = t.kernel == WTC_KERNEL_WALK ? kKernelWalk : t.kernel == WTC_KERNEL_STAGED ? kKernelStaged
-                                                                                              : kKernelSplit;
+    c->tune.kernel = t.kernel;
     c->tune.ways = t.probe_ways;
     c->tune.wpb = t.waves_per_block;
     c->tune.split_wpb = t.split_waves;
@@ -838,10 +881,8 @@ int wtc_ctx_set_work_split(wtc_ctx *c, uint32_t tiles_per_grab, int deal_to_xcds
 }
 
 int wtc_ctx_set_count_kernel(wtc_ctx *c, int kernel) {
-    if (!c || (kernel != WTC_KERNEL_WALK && kernel != WTC_KERNEL_STAGED && kernel != WTC_KERNEL_SPLIT))
-        return WTC_ERR_ARG;
-    c->tune.kernel = kernel == WTC_KERNEL_WALK ? kKernelWalk : kernel == WTC_KERNEL_STAGED ? kKernelStaged
-                                                                                          : kKernelSplit;
+    if (!c || !valid_kernel(kernel)) return WTC_ERR_ARG;
+    c->tune.kernel = kernel;
     return WTC_OK;
 }
 
@@ -1215,7 +1256,7 @@ int batch_capture(wtc_ctx *c, wtc_batch *b, const std::vector<uint32_t> &s, cons
                             hipMemcpyHostToDevice, st));
     WTC_HIPC(hipStreamSynchronize(st));
     WTC_HIPC(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-    rc = launch_set(b->slot, b->plan, false);
+    rc = launch_set(b->slot, b->plan, false, true);
     hipGraph_t graph = nullptr;
     const hipError_t ec = hipStreamEndCapture(st, &graph);
     if (rc == WTC_OK && ec != hipSuccess) rc = hip_fail("batch capture", ec);

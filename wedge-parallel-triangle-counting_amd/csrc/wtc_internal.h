@@ -92,6 +92,7 @@ struct Slot {
     uint32_t rows_grid = 0;   // row-kernel grid of the last split count
     uint32_t slabs_grid = 0;  // slab-kernel grid of the last split count
     bool split = false;       // the last enqueue was a split count
+    bool rows = false;        // the last enqueue was a row count
     uint32_t small = 0;   // graphs of the last enqueue taken by the small-graph kernel
     int create();
     void release_device();  // frees the device workspace (keeps stream/events)
@@ -103,7 +104,9 @@ struct Tuning {
     int num_cus = 0;
     int ways = 4;         // probes advanced together per lane
     int wpb = 4;          // waves per counting block: 1, 2, 4 or 8
-    int kernel = 0;       // kKernelWalk, kKernelStaged or kKernelSplit
+    int kernel = 0;       // kKernelWalk, kKernelStaged, kKernelSplit or kKernelRows
+    bool rows_else = false;  // whole graphs the split count does not take: by the row count
+    uint32_t rows_grid[2] = {0, 0};  // the row count's grid by offset width
     int split_wpb = 8;    // waves per block of the split count's row kernel
     // the process context of the tc_GPU drop-ins takes the autotuner's
     // kernel and block shape per graph unless $WTC_COUNT_KERNEL names one
@@ -144,7 +147,7 @@ int init_small_graphs(Tuning &t, const hipDeviceProp_t &prop, uint32_t want);
 struct RunTimes {
     float prefix_ms = 0, bitmap_ms = 0, count_ms = 0;
     float rows_ms = 0, list_ms = 0;  // split count: its row and slab kernels
-    bool split = false;
+    bool split = false, rows = false;
     uint64_t top_wedges = 0, in_edges = 0, list_in_edges = 0;
 };
 
@@ -171,6 +174,9 @@ struct SetPlan {
     uint32_t tile_graphs = 0;  // graphs counted by the wedge-parallel kernel
     size_t desc_bytes = 0;
     // split count: SplitDesc at byte split_off of the descriptor buffer
+    bool by_rows = false;     // the row count
+    uint64_t rows_tiles = 0;
+    uint32_t rows_grid = 0;
     bool split = false;
     size_t split_off = 0, dense_off = 0;  // bytes of the SplitDesc and DenseDesc
     uint32_t dense_core = 0;              // columns of the dense part's largest class (0: none)
@@ -195,7 +201,9 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
 // Enqueues the set's kernels and the copy of meta + counts to the host; no
 // host-to-device copies, allocations or memsets, so it can be captured into
 // a graph once the descriptors are on the device.  timed: record ev[0..3].
-int launch_set(Slot &s, const SetPlan &p, bool timed);
+// desc_ready: the descriptors are on the device (else a row count fetches
+// them itself, and any other set's caller has enqueued their copy).
+int launch_set(Slot &s, const SetPlan &p, bool timed, bool desc_ready);
 // stage_set + descriptors to the device + launch_set: the whole device
 // pipeline for a graph set on the slot's stream and the copy of its counts
 // into the slot's pinned buffer; returns without waiting.  All graphs of a

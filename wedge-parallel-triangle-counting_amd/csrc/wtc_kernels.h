@@ -45,6 +45,9 @@ enum : uint32_t {
 // Count of a graph whose CSR failed the device-side check.
 constexpr unsigned long long kCountInvalid = ~0ull;
 
+// Edges per tile of the row count (wtc_rows.hip).
+constexpr uint32_t kRowsTile = 512;
+
 // One graph of a graph set.  A graph set is any number of oriented CSRs
 // resident in HBM (ids local to each graph, row offsets relative to the
 // graph's own colInd); one count launch covers all of them.  A single graph
@@ -68,9 +71,9 @@ struct GraphDesc {
     uint32_t thr;            // bitmap threshold max(n,a) - a (a = 0: n)
     uint32_t bm_rows;        // min(n, a)
     uint32_t mode;           // kModeTiles, kModeSmall or kModeInvalid
-    // device-filled by the setup kernel
+    // device-filled by the setup kernel (the row count: host-filled)
     uint64_t wbase;          // first counted wedge (graph-local index)
-    uint64_t wcount;         // wedges counted
+    uint64_t wcount;         // wedges counted (the row count: edges)
     uint64_t tile_base;      // first tile of this graph
 };
 static_assert(sizeof(GraphDesc) == 128, "GraphDesc layout");

@@ -43,7 +43,15 @@ bool valid_count_waves(int wpb);
 // in-edges grouped by middle vertex: the top-a rows against one LDS bitmap
 // row, the rest against LDS windows of colInd; wtc_split.hip); any other set
 // with it by k_walk.
-enum : int { kKernelWalk = 0, kKernelStaged = 1, kKernelSplit = 2 };
+// kKernelRows: whole graphs, alone or in sets, counted edge by edge against
+// hashed rows (wtc_rows.hip); wedge ranges with it by k_count.
+enum : int { kKernelWalk = 0, kKernelStaged = 1, kKernelSplit = 2, kKernelRows = 3 };
+// Row count: its persistent grid, and the count of a set whose descriptors
+// hold tile_base and wcount (edges); host_desc, when given, is pinned memory
+// the descriptors are read from first.
+hipError_t rows_grid(int ob, int num_cus, uint32_t *grid);
+hipError_t launch_rows(const uint64_t *host_desc, GraphDesc *desc, uint32_t G, int ob, uint64_t tiles, uint64_t *meta,
+                       unsigned long long *counts, uint32_t grid, hipStream_t st);
 // `ways`: independent probes each lane advances together (1, 2, 4 or 8; for
 // k_walk, the steps in flight); `wpb`: waves per block; `staged` = min(max
 // spread, chunk) (k_count's LDS staging).

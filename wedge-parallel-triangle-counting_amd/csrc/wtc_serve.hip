@@ -375,9 +375,10 @@ int wtc_server_create(int device, const wtc_server_config *cfg, wtc_server **out
     s->tune.chunk = s->cfg.lds_chunk;
     s->tune.wpb = s->cfg.waves_per_block;
     // a request whose graph the autotuner counts by the split count runs
-    // alone with its workspace from the pool; sets of several graphs walk
+    // alone with its workspace from the pool, any other set by the row count
     s->tune.kernel = kKernelSplit;
     s->tune.split_needs_base = true;
+    s->tune.rows_else = true;
     int rc = init_small_graphs(s->tune, prop, s->cfg.small_graph_words < 0    ? 0u
                                               : s->cfg.small_graph_words == 0 ? default_small_words()
                                                                               : (uint32_t)s->cfg.small_graph_words);

@@ -1098,24 +1098,6 @@ __device__ __forceinline__ uint32_t rows_chunk_hits(const uint32_t *s_bits, u32x
     return __builtin_popcount(hm & vm);
 }
 
-// Rightmost r in [0, hi] with f(r) <= t for a non-decreasing f with f(0) <=
-// t, by a whole wave: 64 probes a round.
-template <class F>
-__device__ __forceinline__ uint32_t wave_rightmost_le(uint32_t hi, uint64_t t, F f) {
-    const uint32_t lane = threadIdx.x & (kWave - 1);
-    uint32_t lo = 0;  // f(lo) <= t
-    while (lo < hi) {
-        const uint32_t step = (hi - lo + kWave - 1) / kWave;
-        const uint64_t at = (uint64_t)lo + (uint64_t)(lane + 1) * step;
-        const bool le = at <= hi && f((uint32_t)at) <= t;
-        const uint32_t k = (uint32_t)__builtin_popcountll(__ballot(le));  // a prefix of the lanes
-        const uint64_t end = (uint64_t)lo + (uint64_t)(k + 1) * step - 1;
-        lo += k * step;
-        hi = end < hi ? (uint32_t)end : hi;
-    }
-    return uni32(lo);
-}
-
 // Persistent blocks take tiles of the rows' work from one counter.  The work
 // of a row is kSplitRowCost for its bitmap and one unit per in-edge, so a
 // tile is up to `tile` in-edges of few rows, or fewer in-edges where rows

@@ -412,7 +412,7 @@ def tc_arrow_gpu_big(g: CSR, spread: int, a: int, t: Optional[GpuTime] = None) -
 
 WEDGE_OUTGOING, WEDGE_ARROW, WEDGE_MIXED = 0, 1, 2
 PARALLEL_VERTEX, PARALLEL_EDGE = 0, 1
-KERNEL_WALK, KERNEL_STAGED, KERNEL_SPLIT = 0, 1, 2
+KERNEL_WALK, KERNEL_STAGED, KERNEL_SPLIT, KERNEL_ROWS = 0, 1, 2, 3
 
 
 def _baseline_call(fn32, fn64, g: CSR, a: int, style: int, t: Optional[GpuTime], big: bool) -> int:
@@ -484,9 +484,10 @@ class Context:
         _check(_lib.wtc_ctx_set_tuning(self._p, probe_ways, lds_chunk, waves_per_block), "set_tuning")
 
     def set_count_kernel(self, kernel: int):
-        """KERNEL_WALK (0), KERNEL_STAGED (1) or KERNEL_SPLIT (2: a single graph
-        with a > 0 counts its top-a wedges by middle vertex against an LDS
-        bitmap row, the rest by the walk); counts do not depend on it."""
+        """KERNEL_WALK (0), KERNEL_STAGED (1), KERNEL_SPLIT (2: a single graph
+        with a > 0 counts its wedges grouped by middle vertex) or KERNEL_ROWS
+        (3: whole graphs edge by edge against hashed rows); counts do not
+        depend on it."""
         _check(_lib.wtc_ctx_set_count_kernel(self._p, kernel), "set_count_kernel")
 
     def use_tuned(self, t: "Tuned"):
