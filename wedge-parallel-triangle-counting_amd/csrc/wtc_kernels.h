@@ -133,7 +133,7 @@ constexpr uint32_t kSlabSpan = 2048;
 constexpr uint32_t kSlabRowMax = 1024;
 constexpr uint32_t kSlabWin = kSlabSpan + kSlabRowMax;
 constexpr uint32_t kSlabWays = 4;
-constexpr uint32_t kSlabTile = 1024;
+constexpr uint32_t kSlabTile = 1024, kSlabTileMin = 128, kSlabCost = 48;  // a tile's work; a slab's share of it
 
 // Workspace and device-filled state of a split count.  The top rows are the
 // ranks [thr, n) of the graph's GraphDesc; OffT arrays use the set's offset

@@ -1266,14 +1266,18 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *
 
 // ---------------------------------------------------------------- list part
 
-// Bucket of id u in a row's region of len buckets (multiplicative hash).
+// Bucket of id u in a row's region of len buckets (multiplicative hash; twelve
+// reversed bits of u scaled to len, all in full-rate instructions, were slower:
+// more ids per bucket, R-MAT-26's list part 37.3 ms against 36.0).
 __device__ __forceinline__ uint32_t slab_bucket(uint32_t u, uint32_t len) {
     return __umulhi(u * 0x9e3779b1u, len);
 }
 
-// Persistent blocks take tiles of kSlabTile consecutive list in-edges (in
-// slab order) from one counter.  A tile's in-edges of one slab form a
-// segment.  Per segment, the block hashes into LDS every row of the slab the
+// Persistent blocks take tiles of the slabs' work from one counter: a slab's
+// work is kSlabCost for its rows and one unit per in-edge, in tiles of at most
+// kSlabTile, as in the row kernel (with tiles of in-edges alone, those over
+// the many slabs with few in-edges took 0.45 ms on R-MAT-20 however few the
+// list rows were).  A tile's in-edges of one slab form a segment.  Per segment, the block hashes into LDS every row of the slab the
 // segment's in-edges name that is not there yet (the table is kept while
 // the next segment stays in the slab; a wave per row clears its buckets and
 // inserts its ids): the row starting at window position st with len
@@ -1312,18 +1316,27 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
     unsigned long long *const ctr = reinterpret_cast<unsigned long long *>(meta + kMetaSlabs);
     uint32_t cur = kSentinel;  // slab in s_tab (block-uniform)
     uint64_t hits = 0, checked = 0;
+    const uint64_t work = L1 - L0 + (uint64_t)kSlabCost * (keys - rows);
+    uint64_t tile = work / (8ull * gridDim.x);
+    tile = tile < kSlabTileMin ? kSlabTileMin : tile > kSlabTile ? kSlabTile : tile;
     for (;;) {
         __syncthreads();
         if (threadIdx.x == 0) s_tile = atomicAdd(ctr, 1ull);
         __syncthreads();
-        const uint64_t k0 = L0 + uni64(s_tile) * kSlabTile;
-        if (k0 >= L1) break;  // block-uniform
-        const uint64_t k1 = k0 + kSlabTile < L1 ? k0 + kSlabTile : L1;
-        uint64_t k = k0;
-        while (k < k1) {
-            const uint32_t key = uni32(rightmost_le(rp_in, rows, keys - 1, k));  // the key holding in-edge k
-            const uint64_t re = (uint64_t)rp_in[key + 1];
-            const uint64_t kend = re < k1 ? re : k1;
+        const uint64_t t0 = uni64(s_tile) * tile;
+        if (t0 >= work || L0 == L1) break;  // block-uniform
+        const uint64_t t1 = t0 + tile < work ? t0 + tile : work;
+        // slab y's work is [rp_in[rows + y] - L0 + y*kSlabCost, rp_in[rows + y + 1] - L0 + (y + 1)*kSlabCost)
+        const uint32_t y0 = wave_rightmost_le(keys - rows - 1, t0, [&](uint32_t y) {
+            return (uint64_t)rp_in[rows + y] - L0 + (uint64_t)kSlabCost * y;
+        });
+        for (uint32_t key = rows + y0; key < keys; key++) {
+            const uint64_t c = (uint64_t)kSlabCost * (key - rows + 1);  // in-edges after this much of the work
+            const uint64_t kb = (uint64_t)rp_in[key] - L0, ke = (uint64_t)rp_in[key + 1] - L0;
+            if (kb + c - kSlabCost >= t1) break;  // block-uniform
+            const uint64_t k = L0 + (t0 > kb + c ? t0 - c : kb);
+            const uint64_t kend = L0 + (t1 < ke + c ? (t1 > kb + c ? t1 - c : kb) : ke);
+            if (k >= kend) continue;
             const uint32_t slab = key - rows;
             const uint64_t wb = (uint64_t)slab * kSlabSpan;  // window start in colInd
             // the rows this segment names that the table lacks
@@ -1446,7 +1459,6 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
                 }
             }
             hits += h;
-            k = kend;
         }
     }
     hits = wave_sum(hits);
