@@ -154,8 +154,8 @@ namespace {
 // Byte offsets of the pieces of a split count's workspace in one buffer
 // (each on a 256-byte boundary), and the buffer's size.
 struct SplitLayout {
-    size_t wsfull, tile_v, part_base, part_cnt, c2base, hist2, sub_base, c3base, hist3, sub_tot, list_bid, slab_row, key_tot;
-    size_t part_tot, key_part;
+    size_t wsfull, tile_v, part_base, part_cnt, c2base, hist2, sub_base, c3base, hist3, sub_tot, list_bid, key_tot;
+    size_t part_tot, tally, key_part;
     size_t recid, rec, recaux, recid2, rec2, recaux2, rpin, rp32, total;
     size_t dense_cnt, dense_sums, dense_r, dense_b, dense_list;  // the last three within the records
     uint64_t dense_list_off[kDenseClasses];
@@ -222,8 +222,8 @@ SplitLayout split_plan(uint32_t n, uint64_t m, uint32_t rows, int ob_in) {
     L.hist3 = take(((size_t)L.g.c3cap << L.g.final_shift) * sizeof(uint32_t));
     L.sub_tot = take((size_t)L.subs * sizeof(uint32_t));
     L.list_bid = take((size_t)L.g.parts * sizeof(uint32_t));
-    L.slab_row = take(((size_t)L.slabs + 1) * sizeof(uint32_t));
     L.part_tot = take((size_t)L.g.parts * sizeof(uint64_t));
+    L.tally = take(2 * sizeof(uint64_t));
     L.key_part = take(((size_t)L.g.keys / kKeyChunk + 2) * sizeof(uint64_t));
     L.key_tot = take((size_t)L.g.keys * sizeof(uint32_t));
     L.recid = take((size_t)L.cap * sizeof(uint16_t));
@@ -292,6 +292,7 @@ int split_layout(SplitDesc *sd, DenseDesc *dd, SplitGrids *grids, char *base, ui
     sd->final_shift = L.g.final_shift;
     sd->subs = L.subs;
     sd->chunk = L.chunk;
+    sd->far_ids = split_far_ids(rows);
     sd->cap = L.cap;
     sd->ws_full = reinterpret_cast<uint64_t *>(base + L.wsfull);
     sd->ie_pre = sd->ws_full + (size_t)n + 1;
@@ -305,8 +306,8 @@ int split_layout(SplitDesc *sd, DenseDesc *dd, SplitGrids *grids, char *base, ui
     sd->hist3 = reinterpret_cast<uint32_t *>(base + L.hist3);
     sd->sub_tot = reinterpret_cast<uint32_t *>(base + L.sub_tot);
     sd->list_bid = reinterpret_cast<uint32_t *>(base + L.list_bid);
-    sd->slab_row = reinterpret_cast<uint32_t *>(base + L.slab_row);
     sd->part_tot = reinterpret_cast<uint64_t *>(base + L.part_tot);
+    sd->tally = reinterpret_cast<uint64_t *>(base + L.tally);
     sd->key_part = reinterpret_cast<uint64_t *>(base + L.key_part);
     sd->key_tot = reinterpret_cast<uint32_t *>(base + L.key_tot);
     sd->rec_id = reinterpret_cast<uint16_t *>(base + L.recid);

@@ -144,9 +144,8 @@ constexpr uint32_t kSlabTile = 1024, kSlabTileMin = 128, kSlabCost = 48;  // a t
 // key (the pairs, and a list record's slab_aux), in the arrays of the level
 // before the last: B's when there is no B.  A record's position names its
 // part (in A) or sub-part (in B), so A keeps the key's low part_shift bits
-// and B its low 8.  A top record's pair is the tail [lo, hi) of colInd; a list
-// record's is (j, hi), its tail [j + 1, hi) (the one in-edge whose tail the
-// range cuts at the front: [clip_lo, hi)).
+// and B its low 8.  A top record's pair is its tail's first packed chunk and
+// number of chunks; a list record's is (j, hi), its tail [j + 1, hi) of colInd.
 struct SplitDesc {
     uint64_t *ws_full;    // n+1: the full wedge prefix
     uint64_t *ie_pre;     // n+1: prefix of the in-edges of each row (its first positions)
@@ -160,8 +159,8 @@ struct SplitDesc {
     uint32_t *hist3;      // c3cap << final_shift: final-level counts, then column prefixes
     uint32_t *sub_tot;    // subs: records of each sub-part
     uint32_t *list_bid;   // parts: the first list vertex w whose key lies in each part (0 up to the first list part)
-    uint32_t *slab_row;   // slabs+1: the first vertex w with rowPtr[w] >= s*kSlabSpan (set for s*kSlabSpan <= rowPtr[thr])
     uint64_t *part_tot;   // parts: record slots of each part (>= its records)
+    uint64_t *tally;      // 2: wedges of the top rows' and of the list rows' in-edges
     uint64_t *key_part;   // key blocks: in-edges of each block of kKeyChunk keys, then their prefix
     uint32_t *key_tot;    // keys: in-edges of each key
     uint16_t *rec_id;     // cap: A keys within their part
@@ -173,7 +172,7 @@ struct SplitDesc {
     void *rp_in;          // keys+1 OffT: first in-edge of each key
     void *ie;             // the records' pairs grouped by key: rec2 (two levels) or rec (three)
     uint32_t *ie_aux;     // the list records' slab_aux words, beside ie
-    void *packed;         // the packed top ids: over the pairs that ie is not in
+    void *packed;         // 3 cap / 4 chunks of 16 bytes, the packed top ids: over the pairs (and slab words) that ie is not in
     uint64_t cap;         // records each array holds (>= the in-edges)
     uint32_t rows;        // top rows: n - thr
     uint32_t keys;        // rows + slabs
@@ -183,12 +182,16 @@ struct SplitDesc {
     uint32_t subs;        // sub-parts (three levels)
     uint32_t slabs;       // slabs of the list rows: ceil(m / kSlabSpan)
     uint32_t chunk;       // records per block of the second and final levels
+    uint32_t far_ids;     // ids per far chunk of the packed top ids
     // device-filled by the range kernel
     uint64_t w_lo, w_hi;  // the counted wedges of the full order, clamped to [0, W]
-    uint64_t clip_j;      // the in-edge whose tail the range cuts at the front (~0: none)
-    uint64_t clip_lo;     // that tail's first position
+    uint64_t cut_j[2];    // in-edges whose tail the range cuts, and what it leaves of
+    uint64_t cut_lo[2];   // them: positions [cut_lo, cut_hi) of colInd
+    uint64_t cut_hi[2];
     uint32_t v_lo, v_hi;  // vertices holding w_lo and w_hi - 1 (v_lo > v_hi: none)
     uint32_t clip;        // 1 unless [w_lo, w_hi) is the whole order
+    uint32_t cuts;        // cut tails: up to two
+    uint32_t cut_top;     // those of top rows
     uint32_t pad_;
 };
 

@@ -54,13 +54,41 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 template <typename OffT>
 struct TailPair {
-    OffT lo, hi;  // a top record: colInd positions [lo, hi) of one in-edge's tail;
-                  // a list record: (j, hi), the tail [j + 1, hi)
+    OffT lo, hi;  // a top record: the tail's first packed chunk, and its chunks (pack_count);
+                  // a list record: (j, hi), the tail [j + 1, hi) of colInd
 };
 
 // Wedges before row i of a vertex of out-degree d in its row-major order
 // (row r holds d - 1 - r wedges).
 __device__ __forceinline__ uint64_t row_base(uint64_t i, uint64_t d) { return i * (d - 1) - binom2_d(i); }
+
+// The packed copy of the top ids (k_split_pack).  A row is held from its top
+// id down, so that the tail of each of its in-edges is a prefix of it: ids as
+// x = n - u, first those with x <= kPackNear in 16-bit fields (near chunks),
+// then the rest in wider ones (far chunks).
+constexpr uint32_t kPackNear = 65528, kPackNearIds = 8;
+constexpr uint32_t kPackAlign = 16;  // rows of this many ids start on a 128-byte line
+
+// Chunk slots before those of the row that starts at position p: three for
+// four ids.  A row's chunks start at its first slot, on a 128-byte line in
+// rows of kPackAlign ids or more: of its d - 1 tail ids there are at most (d -
+// 1) / 6 + 2 chunks and not more than d - 1, so with the alignment's 7 they
+// fit.
+template <typename T>
+__device__ __forceinline__ T pack_slot(T p) {
+    return p - (p >> 2);
+}
+template <typename OffT>
+__device__ __forceinline__ OffT pack_row(OffT rb, OffT re) {
+    const OffT c = pack_slot(rb);
+    return re - rb >= kPackAlign ? (c + 7) & ~(OffT)7 : c;
+}
+
+// A tail's near and far chunks in one word (at most 8,191 and 349,526).
+__device__ __forceinline__ uint32_t pack_count(uint32_t near, uint32_t far) { return near | (far << 13); }
+
+// x / q for the far chunks' ids, 6 or 7 (block-uniform).
+__device__ __forceinline__ uint32_t pack_div(uint32_t x, uint32_t q) { return q == 7 ? x / 7 : x / 6; }
 
 }  // namespace
 
@@ -87,7 +115,7 @@ __global__ __launch_bounds__(kBlock) void k_split_partials(const GraphDesc *__re
     if (threadIdx.x == 0) part_full[blockIdx.x] = s_f[0] + s_f[1] + s_f[2] + s_f[3];
 }
 
-// ws_full from the scanned block partials, and slab_row.
+// ws_full from the scanned block partials.
 template <typename OffT>
 __global__ __launch_bounds__(kBlock) void k_split_scan(const GraphDesc *__restrict__ desc,
                                                        const SplitDesc *__restrict__ sd,
@@ -96,8 +124,7 @@ __global__ __launch_bounds__(kBlock) void k_split_scan(const GraphDesc *__restri
     const GraphDesc &D = desc[0];
     const OffT *__restrict__ rowPtr = static_cast<const OffT *>(D.rowPtr);
     uint64_t *__restrict__ wf = sd->ws_full;
-    uint32_t *__restrict__ slab_row = sd->slab_row;
-    const uint32_t n = D.n, thr = D.thr, slabs = sd->slabs;
+    const uint32_t n = D.n;
     uint64_t cf = part_full[blockIdx.x];
     const uint64_t base = (uint64_t)blockIdx.x * kScanChunk;
     for (int k = 0; k < kScanItems; k++) {
@@ -108,11 +135,6 @@ __global__ __launch_bounds__(kBlock) void k_split_scan(const GraphDesc *__restri
         const uint64_t ef = block_excl_scan(xf, s_tot, tf);
         if (v < n) {
             wf[v] = cf + ef;
-            if (v <= thr) {  // the slabs whose first row is v: rowPtr[v - 1] < s*kSlabSpan <= rowPtr[v]
-                const uint64_t s_hi = (uint64_t)rowPtr[v] / kSlabSpan;
-                for (uint64_t s = v ? (uint64_t)rowPtr[v - 1] / kSlabSpan + 1 : 0; s <= s_hi && s <= slabs; s++)
-                    slab_row[s] = (uint32_t)v;
-            }
         }
         cf += tf;
     }
@@ -141,8 +163,8 @@ __global__ __launch_bounds__(kBlock) void k_split_inscan(const GraphDesc *__rest
 }
 
 // Thread 0: the counted range of the full order, its end vertices, and the
-// one in-edge whose tail the range cuts at the front (row i0 of v_lo holding
-// wedge w_lo: its tail starts w_lo - base(i0) ids in).  Thread q < parts:
+// in-edges whose tails the range cuts (row i0 of v_lo holding wedge w_lo: its
+// tail starts w_lo - base(i0) ids in; likewise the one of wedge w_hi - 1).  Thread q < parts:
 // list_bid[q], the first list vertex w (below thr) whose key rows +
 // rowPtr[w] / kSlabSpan lies in part q or later (keys grow with w), and the
 // part's counters zeroed.
@@ -177,8 +199,9 @@ __global__ __launch_bounds__(kSplitPartsMax) void k_split_range(const GraphDesc 
     const uint64_t lo = D.w_begin < W ? D.w_begin : W, hi = D.w_end < W ? D.w_end : W;
     S.w_lo = lo;
     S.w_hi = hi;
-    S.clip_j = ~0ull;
-    S.clip_lo = 0;
+    S.cuts = 0;
+    S.cut_top = 0;
+    S.tally[0] = S.tally[1] = 0;
     if (lo == 0 && hi == W) {  // the whole order: nothing clipped
         S.clip = 0;
         S.v_lo = 0;
@@ -191,40 +214,50 @@ __global__ __launch_bounds__(kSplitPartsMax) void k_split_range(const GraphDesc 
         S.v_hi = 0;
         return;
     }
-    const uint32_t v = rightmost_le(wf, 0u, n - 1, lo);
-    S.v_lo = v;
-    S.v_hi = rightmost_le(wf, 0u, n - 1, hi - 1);
-    const uint64_t rb = (uint64_t)rowPtr[v], d = (uint64_t)rowPtr[v + 1] - rb, off = lo - wf[v];
-    uint64_t s = 0, e = d - 1;  // the last i in [0, d - 2] with row_base(i) <= off
-    while (e - s > 1) {
-        const uint64_t mid = s + ((e - s) >> 1);
-        if (row_base(mid, d) <= off) s = mid;
-        else e = mid;
+    const uint32_t v[2] = {rightmost_le(wf, 0u, n - 1, lo), rightmost_le(wf, 0u, n - 1, hi - 1)};
+    S.v_lo = v[0];
+    S.v_hi = v[1];
+    // the in-edges that hold the range's first and last wedge, and the
+    // positions [b, e) of their tails that the range leaves
+    uint64_t j[2], b[2], e[2], end[2];
+    for (int z = 0; z < 2; z++) {
+        const uint64_t rb = (uint64_t)rowPtr[v[z]], d = (uint64_t)rowPtr[(uint64_t)v[z] + 1] - rb;
+        const uint64_t off = (z ? hi - 1 : lo) - wf[v[z]];
+        uint64_t s = 0, t = d - 1;  // the last i in [0, d - 2] with row_base(i) <= off
+        while (t - s > 1) {
+            const uint64_t mid = s + ((t - s) >> 1);
+            if (row_base(mid, d) <= off) s = mid;
+            else t = mid;
+        }
+        j[z] = rb + s;
+        end[z] = rb + d;
+        b[z] = j[z] + 1 + (z ? 0 : off - row_base(s, d));
+        e[z] = z ? j[z] + 1 + (off + 1 - row_base(s, d)) : end[z];
     }
-    S.clip_j = rb + s;
-    S.clip_lo = rb + s + 1 + (off - row_base(s, d));
+    if (j[0] == j[1]) e[0] = e[1];
+    for (int z = 0; z < 2; z++) {
+        if ((z && j[0] == j[1]) || (b[z] == j[z] + 1 && e[z] == end[z])) continue;
+        const bool top = to_global(D.colInd)[j[z]] >= D.thr;
+        S.cut_j[S.cuts] = j[z];
+        S.cut_lo[S.cuts] = b[z];
+        S.cut_hi[S.cuts] = e[z];
+        S.cuts++;
+        S.cut_top += top;
+        S.tally[top ? 0 : 1] += e[z] - b[z];
+    }
 }
 
 // ------------------------------------------------------------ transposition
 
-// Clips the tail [j+1, e) of in-edge j of an end vertex of the counted
-// range (row start rb, full-order base ws) to its wedges in [w_lo, w_hi):
-// the tail ids of row i = j - rb are the wedges [base, base + L) of the full
-// order (tc.cu:203-212 numbering).  Returns the clipped [lo, hi) (lo == hi:
-// none).
+// Whether the tail [j+1, e) of in-edge j of an end vertex of the counted
+// range (row start rb, full-order base ws) lies wholly in the range: the tail
+// ids of row i = j - rb are the wedges [base, base + L) of the full order
+// (tc.cu:203-212 numbering).  At most one tail is cut at each end of the
+// range; the row kernel counts those by themselves.
 template <typename OffT>
-__device__ __forceinline__ void clip_tail(OffT j, OffT e, OffT rb, uint64_t ws, uint64_t w_lo, uint64_t w_hi,
-                                          OffT &lo, OffT &hi) {
-    const uint64_t d = (uint64_t)(e - rb), i = (uint64_t)(j - rb);
-    const uint64_t bse = ws + row_base(i, d), L = (uint64_t)(e - j - 1);
-    const uint64_t a = bse > w_lo ? bse : w_lo;
-    const uint64_t z = bse + L < w_hi ? bse + L : w_hi;
-    lo = j + 1;
-    hi = lo;
-    if (a < z) {
-        lo = j + 1 + (OffT)(a - bse);
-        hi = j + 1 + (OffT)(z - bse);
-    }
+__device__ __forceinline__ bool whole_tail(OffT j, OffT e, OffT rb, uint64_t ws, uint64_t w_lo, uint64_t w_hi) {
+    const uint64_t bse = ws + row_base((uint64_t)(j - rb), (uint64_t)(e - rb));
+    return bse >= w_lo && bse + (uint64_t)(e - j - 1) <= w_hi;
 }
 
 // Records staged in LDS per tile of a scatter: 4096 with 4-byte offsets,
@@ -339,22 +372,39 @@ __global__ __launch_bounds__(kBlock) void k_split_partbase(const SplitDesc *__re
     if (q < parts) S.part_base[q] = et;
 }
 
-// Exclusive prefix of the n counts in s_cnt (a multiple of 64, at most
-// 2048) into s_off by the first wave of a block.
-__device__ __forceinline__ void wave_prefix(const uint32_t *s_cnt, uint32_t *s_off, uint32_t n) {
-    const uint32_t lane = threadIdx.x, per = n / kWave;
-    uint32_t sum = 0;
-    for (uint32_t z = 0; z < per; z++) sum += s_cnt[lane * per + z];
-    uint32_t incl = sum;
+// Exclusive prefix of the kN counts in s_cnt into s_off by a block of
+// kSplitBlock threads (s_w: a word per wave); s_cnt is final and s_off and s_w
+// free on entry, s_off is whole after the next barrier.
+template <uint32_t kN>
+__device__ __forceinline__ void block_prefix(const uint32_t *s_cnt, uint32_t *s_off, uint32_t *s_w) {
+    constexpr uint32_t kPer = kN > (uint32_t)kSplitBlock ? kN / kSplitBlock : 1;
+    constexpr uint32_t kWaves = kN / kPer / kWave;  // those that hold counts
+    static_assert(kN % (kPer * kWave) == 0 && kWaves * kWave <= (uint32_t)kSplitBlock, "whole waves of counts");
+    const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x >> 6;
+    uint32_t v[kPer], sum = 0, incl = 0;
+    if (wv < kWaves) {
 #pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-        const uint32_t y = (uint32_t)__shfl_up((int)incl, o, kWave);
-        if ((int)lane >= o) incl += y;
+        for (uint32_t z = 0; z < kPer; z++) {
+            v[z] = s_cnt[threadIdx.x * kPer + z];
+            sum += v[z];
+        }
+        incl = sum;
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) {
+            const uint32_t y = (uint32_t)__shfl_up((int)incl, o, kWave);
+            incl += (int)lane >= o ? y : 0u;
+        }
+        if (lane == kWave - 1) s_w[wv] = incl;
     }
-    uint32_t run = incl - sum;
-    for (uint32_t z = 0; z < per; z++) {
-        s_off[lane * per + z] = run;
-        run += s_cnt[lane * per + z];
+    __syncthreads();
+    if (wv < kWaves) {
+        uint32_t run = incl - sum;
+        for (uint32_t w = 0; w < wv; w++) run += s_w[w];
+#pragma unroll
+        for (uint32_t z = 0; z < kPer; z++) {
+            s_off[threadIdx.x * kPer + z] = run;
+            run += v[z];
+        }
     }
 }
 
@@ -370,8 +420,8 @@ __device__ __forceinline__ void wave_prefix(const uint32_t *s_cnt, uint32_t *s_o
 //     their first slot and leave their row's position and end there; a
 //     running maximum over the marks tells each in-edge its vertex's slot;
 //  2. every in-edge loads its id (consecutive positions, so coalesced),
-//     clips its tail at the ends of the counted range (an empty one is
-//     dropped) and gets its key -- w - thr for a top row w, else rows +
+//     is dropped where the counted range does not hold its whole tail, and
+//     gets its key -- w - thr for a top row w, else rows +
 //     rowPtr[w] / kSlabSpan -- and the part key >> part_shift;
 //  3. the tile is ranked per part (LDS atomics), takes its slots of every
 //     part with one global atomic per part, and leaves sorted by part
@@ -390,11 +440,15 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_l1(const GraphDesc *__res
     // step 1's slots and step 3's staged pairs share their memory
     union SlotOrPair {
         struct {
-            OffT j0, e;  // position of in-edge slot 0 as if in this row, and the row's end
+            OffT rb, e;     // the row's bounds
+            uint32_t near;  // its near ids (set where a far in-edge is in the tile)
         } v;
         TailPair<OffT> t;
     };
     __shared__ SlotOrPair s_x[kT];
+    __shared__ uint64_t s_front;  // in-edges of the tile's first row before the tile
+    __shared__ unsigned long long s_tally[2];
+    __shared__ uint32_t s_open;  // the last row's far in-edges reach the tile's end
     __shared__ uint16_t s_mark[kT];
     __shared__ uint16_t s_key[kT];
     __shared__ uint8_t s_part[kT];
@@ -421,6 +475,11 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_l1(const GraphDesc *__res
     const uint64_t K0 = iep[v_lo], K1 = iep[(uint64_t)v_hi + 1];
     const uint64_t tiles = (K1 - K0 + kT - 1) / kT;
     const uint32_t list_part = rows >> shift;  // the first part with list keys
+    // the top ids below far_end are far
+    const uint32_t far_ids = S.far_ids, far_end = D.n > kPackNear ? D.n - kPackNear : 0;
+    const bool far_top = far_end > thr;
+    uint64_t tops = 0, rest = 0;  // wedges of the top and of the list in-edges
+    if (threadIdx.x < 2) s_tally[threadIdx.x] = 0;
     for (uint64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
         uint64_t vb = S.tile_v[tile];
         const uint64_t t0 = K0 + tile * kT, t1 = t0 + kT < K1 ? t0 + kT : K1;
@@ -428,6 +487,7 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_l1(const GraphDesc *__res
         __syncthreads();  // the previous tile is written out
         for (uint32_t i = threadIdx.x; i < kT / 2; i += kSplitBlock) reinterpret_cast<uint32_t *>(s_mark)[i] = 0u;
         if (threadIdx.x < kSplitPartsMax) s_cnt[threadIdx.x] = 0u;
+        if (threadIdx.x == 0) s_open = 0;
         __syncthreads();
         for (;;) {  // windows of kSplitBlock vertices from vb, up to the one holding t1 - 1
             const uint64_t v = vb + threadIdx.x, vn = vb + kSplitBlock;
@@ -438,8 +498,10 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_l1(const GraphDesc *__res
                 if (z > a && z > t0 && a < t1) {
                     const uint32_t at = a > t0 ? (uint32_t)(a - t0) : 0u;
                     s_mark[at] = (uint16_t)at;
-                    s_x[at].v.j0 = rb - (OffT)(a - t0);  // modulo the width where a < t0
+                    s_x[at].v.rb = rb;
                     s_x[at].v.e = re;
+                    s_x[at].v.near = 0;
+                    if (at == 0) s_front = t0 - a;
                 }
             }
             if (next >= t1) break;  // block-uniform
@@ -470,18 +532,20 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_l1(const GraphDesc *__res
             for (uint32_t z = 0; z < kPer; z++) s_mark[threadIdx.x * kPer + z] = (uint16_t)(x[z] > before ? x[z] : before);
         }
         __syncthreads();
-        OffT j[kPer], e[kPer];
-        uint32_t id[kPer];
+        const OffT front = (OffT)s_front;
+        auto position = [&](uint32_t i) -> OffT {  // of in-edge slot i in colInd
+            const uint32_t p = s_mark[i];
+            return s_x[p].v.rb + (OffT)(i - p) + (p ? 0 : front);
+        };
+        uint32_t id[kPer], nid[kPer];
 #pragma unroll
         for (uint32_t u = 0; u < kPer; u++) {
             const uint32_t i = threadIdx.x + u * kSplitBlock;
-            j[u] = e[u] = 0;
-            id[u] = 0;
+            id[u] = nid[u] = 0;
             if (i < nt) {
-                const uint32_t p = s_mark[i];
-                j[u] = s_x[p].v.j0 + (OffT)i;
-                e[u] = s_x[p].v.e;
-                id[u] = colInd[j[u]];
+                const OffT j = position(i);
+                id[u] = colInd[j];
+                nid[u] = colInd[j + 1];  // an in-edge is not its row's last
             }
         }
         OffT rp[kPer], rp1[kPer];
@@ -494,22 +558,62 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_l1(const GraphDesc *__res
                 rp1[u] = rowPtr[(uint64_t)id[u] + 1];
             }
         }
+        // a row's near ids are those after its last far one: where two
+        // neighbours show it; of a row whose far in-edges reach the tile's
+        // end, by a search
+        if (far_top) {  // block-uniform
+#pragma unroll
+            for (uint32_t u = 0; u < kPer; u++) {
+                const uint32_t i = threadIdx.x + u * kSplitBlock;
+                if (i >= nt || id[u] < thr || id[u] >= far_end) continue;
+                if (nid[u] >= far_end) s_x[s_mark[i]].v.near = (uint32_t)(s_x[s_mark[i]].v.e - position(i) - 1);
+                else if (i == nt - 1) s_open = 1;
+            }
+            __syncthreads();
+            if (s_open) {  // block-uniform
+                if (wv == 0) {
+                    const OffT re = s_x[s_mark[nt - 1]].v.e, at = position(nt - 1);
+                    const uint32_t last = wave_rightmost_le((uint32_t)(re - at - 1), (uint64_t)far_end - 1,
+                                                            [&](uint32_t x) { return (uint64_t)colInd[at + x]; });
+                    if (lane == 0) s_x[s_mark[nt - 1]].v.near = (uint32_t)(re - at - 1 - last);
+                }
+                __syncthreads();
+            }
+        }
+        uint32_t cut = 0;  // bit u: in-edge u is not wholly in the range
+        if (clip) {
+#pragma unroll 1
+            for (uint32_t u = 0; u < kPer; u++) {
+                const uint32_t i = threadIdx.x + u * kSplitBlock;
+                if (i >= nt) continue;
+                const OffT j = position(i), e = s_x[s_mark[i]].v.e;
+                const bool in = j >= rl0 && j < rl1   ? whole_tail<OffT>(j, e, rl0, S.ws_full[v_lo], w_lo, w_hi)
+                                : j >= rh0 && j < rh1 ? whole_tail<OffT>(j, e, rh0, S.ws_full[v_hi], w_lo, w_hi)
+                                                      : true;
+                cut |= in ? 0u : 1u << u;
+            }
+        }
         uint32_t key[kPer], rank[kPer], aux[kPer];
         TailPair<OffT> t[kPer];
 #pragma unroll
         for (uint32_t u = 0; u < kPer; u++) {
             const uint32_t i = threadIdx.x + u * kSplitBlock;
             key[u] = kSentinel;
-            if (i >= nt) continue;
-            OffT lo = j[u] + 1, hi = e[u];
-            if (clip) {
-                if (j[u] >= rl0 && j[u] < rl1) clip_tail<OffT>(j[u], e[u], rl0, S.ws_full[v_lo], w_lo, w_hi, lo, hi);
-                else if (j[u] >= rh0 && j[u] < rh1) clip_tail<OffT>(j[u], e[u], rh0, S.ws_full[v_hi], w_lo, w_hi, lo, hi);
-                if (lo >= hi) continue;
-            }
+            if (i >= nt || (cut >> u & 1u)) continue;
+            const uint32_t p = s_mark[i];
+            const OffT j = position(i), rb = s_x[p].v.rb, e = s_x[p].v.e;
             const bool top = id[u] >= thr;
             key[u] = top ? id[u] - thr : rows + (uint32_t)((uint64_t)rp[u] / kSlabSpan);
-            t[u] = TailPair<OffT>{top ? lo : j[u], hi};
+            const uint32_t tail = (uint32_t)(e - j - 1);
+            if (top) {
+                tops += tail;
+                const uint32_t near = id[u] < far_end ? s_x[p].v.near : tail;
+                t[u].lo = pack_row<OffT>(rb, e);
+                t[u].hi = pack_count((near + kPackNearIds - 1) / kPackNearIds, pack_div(tail - near + far_ids - 1, far_ids));
+            } else {
+                rest += tail;
+                t[u] = TailPair<OffT>{j, e};
+            }
             const uint64_t len = (uint64_t)(rp1[u] - rp[u]);
             aux[u] = (uint32_t)((uint64_t)rp[u] % kSlabSpan) | ((len <= kSlabRowMax ? (uint32_t)len : kSlabAuxLong) << 13);
             rank[u] = atomicAdd(&s_cnt[key[u] >> shift], 1u);
@@ -576,6 +680,14 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_l1(const GraphDesc *__res
             }
         }
     }
+    tops = wave_sum(tops);
+    rest = wave_sum(rest);
+    __syncthreads();  // s_tally is zeroed, also without a tile
+    if (lane == 0 && tops) atomicAdd(&s_tally[0], (unsigned long long)tops);
+    if (lane == 0 && rest) atomicAdd(&s_tally[1], (unsigned long long)rest);
+    __syncthreads();
+    if (threadIdx.x < 2 && s_tally[threadIdx.x])
+        atomicAdd(reinterpret_cast<unsigned long long *>(&S.tally[threadIdx.x]), s_tally[threadIdx.x]);
 }
 
 // Later levels.  With up to kSplitPartsMax << kSplitFinalMax keys, a part
@@ -674,12 +786,13 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_level_count(const SplitDe
 // list records' slab words go through the same LDS after the pairs, in
 // buckets that hold list keys only.
 template <typename OffT, typename KeyIn, bool kFinal, uint32_t kF>
-__global__ __launch_bounds__(kSplitBlock) void k_split_level_scatter(const SplitDesc *__restrict__ sd) {
+__global__ __launch_bounds__(kSplitBlock, 8) void k_split_level_scatter(const SplitDesc *__restrict__ sd) {
     constexpr uint32_t kT = LevelTile<OffT>::kT;
     constexpr uint32_t kPerThread = kT / kSplitBlock;
     __shared__ uint64_t s_base[kF];  // next output slot of each output bucket
     __shared__ uint32_t s_tcnt[kF];  // the tile's records per output bucket
     __shared__ uint32_t s_toff[kF];  // their exclusive prefix: each bucket's first staged slot
+    __shared__ uint32_t s_w[kSplitBlock / kWave];
     __shared__ uint16_t st_key[kT];
     __shared__ TailPair<OffT> st_rec[kT];
     const SplitLevel<KeyIn, kFinal, kF> L(sd[0]);
@@ -730,7 +843,7 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_level_scatter(const Split
             for (uint32_t u = 0; u < kPerThread; u++)
                 if (key[u] != kSentinel) rank[u] = atomicAdd(&s_tcnt[L.bucket(key[u])], 1u);
             __syncthreads();
-            if (threadIdx.x < kWave) wave_prefix(s_tcnt, s_toff, kF);
+            block_prefix<kF>(s_tcnt, s_toff, s_w);
             __syncthreads();
 #pragma unroll
             for (uint32_t u = 0; u < kPerThread; u++) {
@@ -918,40 +1031,50 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_keyscan(const SplitDesc *
 #pragma unroll
     for (uint32_t z = 0; z < 4; z++) {
         if (i0 + z < keys) rp[i0 + z] = (OffT)at;
-        if (i0 + z == rows) meta[kMetaInEdges] = at + dense[kDenseTopEdges];
+        if (i0 + z == rows) meta[kMetaInEdges] = at + dense[kDenseTopEdges] + S.cut_top;
         at += v[z];
     }
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
         const uint64_t all = S.key_part[blockIdx.x] + tot;
         rp[keys] = (OffT)all;
-        if (rows >= keys) meta[kMetaInEdges] = all + dense[kDenseTopEdges];
+        if (rows >= keys) meta[kMetaInEdges] = all + dense[kDenseTopEdges] + S.cut_top;
         meta[kMetaRows] = 0;
         meta[kMetaSlabs] = 0;
-        meta[kMetaTopWedges] = dense[kDenseTopWedges];
+        meta[kMetaTopWedges] = S.tally[0] + dense[kDenseTopWedges];
         meta[kMetaDenseTopWedges] = dense[kDenseTopWedges];
         meta[kMetaDenseTopEdges] = dense[kDenseTopEdges];
-        meta[kMetaListWedges] = 0;
+        meta[kMetaListWedges] = S.tally[1];
         meta[kMetaWedges] = S.w_hi - S.w_lo;
-        meta[kMetaAllEdges] = all + dense[kDenseEdges];
+        meta[kMetaAllEdges] = all + dense[kDenseEdges] + S.cuts;
     }
 }
 
 // ------------------------------------------------------------- top-a part
 
 // The top rows' tails as packed ids.  A top in-edge v -> w (w >= thr) has a
-// tail of ids above w, so each of them lies in [thr, n) and its offset x =
-// u - thr is below rows (the a-bit row must fit a block's LDS, so rows <=
-// 2^21).  The packed array is a sequence of 16-byte chunks; chunk c holds
-// the fields of colInd positions [Pc, Pc + P) in bits [Bi, Bi + B), i < P,
-// with the fewest bits B the graph's rows allow: the row kernel streams 16/P
-// bytes per tail id instead of 4.  Layouts (PackLayout<L>):
+// tail of ids above w, which is a prefix of row v from the top; x = n - u of
+// each is below rows (the a-bit row must fit a block's LDS, so rows <= 2^21).
+// Each counted row's tail ids (all but its lowest) are packed as 16-byte
+// chunks: kPackNearIds near ids to a chunk, then P far ones in fields of the
+// fewest bits B that the graph's rows allow, and the end of a row's last near
+// and last far chunk with 0.  So the row kernel streams 2 or 16/P bytes per
+// tail id instead of 4, long rows by whole lines, and every field of a tail's
+// chunks can be looked up in the bitmap of adj+(w) with nothing masked off: a
+// chunk's ids past the tail are at most w, adj+(w) holds ids above w only,
+// and no id has x = 0.
+// The row kernel is bound by the 128-byte lines that it misses L2 for (every
+// one of them: 7.0 TB/s on R-MAT-24).  With rows in colInd's order, 7 ids a
+// chunk cut at fixed positions and the ends masked, a tail of R-MAT-24 touched
+// 3.3 lines and a lookup took 10.4 vector instructions; now 2.7 and 6.7.  Row
+// kernel 10.3 -> 8.4 ms there, 59.9 -> 48.2 on R-MAT-26; packing 0.39 -> 0.73
+// and 1.6 -> 2.6.
+// Layouts of the far chunks (PackLayout<L>):
 //   0: P = 6, B = 21, rows <= 2^19, field (x >> 5) << 7 | (x & 31): bits
 //      [5, 21) are the LDS byte address of x's bitmap word and bits [0, 5)
 //      its bit, so that the row kernel takes both with one extract;
 //   1: P = 6, B = 21, rows <= 2^21, field x;
 //   2: P = 7, B = 18, rows <= 2^18, field x;
-//   3: P = 8, B = 16, rows <= 2^16, field x.
-// An id below thr (never in a top tail) packs as 0.
+//   3: near chunks only, rows <= kPackNear (P = 8, B = 16: the near fields).
 template <int L>
 struct PackLayout;
 template <>
@@ -975,11 +1098,12 @@ struct PackLayout<3> {
     static constexpr bool kAddr = false;
 };
 constexpr uint32_t kPackRowsMax = 1u << 21;
-constexpr uint32_t kPackGrid = 4096;  // blocks of the packing kernel (grid-stride)
+constexpr uint32_t kPackTile = 8192;  // slots a block packs at a time
+constexpr uint32_t kPackGrid = 2048;  // blocks of the packing kernel (eight a CU)
 
 // The layout of a graph with `rows` top rows (rows <= kPackRowsMax).
 __host__ __device__ __forceinline__ int pack_layout(uint32_t rows) {
-    return rows <= (1u << 16) ? 3 : rows <= (1u << 18) ? 2 : rows <= (1u << 19) ? 0 : 1;
+    return rows <= kPackNear ? 3 : rows <= (1u << 18) ? 2 : rows <= (1u << 19) ? 0 : 1;
 }
 
 // Field i of a chunk, shifted down so that its bits start at bit 0 (bits
@@ -999,80 +1123,145 @@ __device__ __forceinline__ void chunk_fields(u32x4 d, uint32_t *f, std::integer_
     ((f[I] = chunk_field<B, I>(d)), ...);
 }
 
-// Packs colInd into S.packed (the memory of the final level's input pairs): a block takes kBlock chunks at a time, loads their P * kBlock
-// ids into LDS with coalesced 4-byte loads, and each thread packs one chunk
-// from LDS (stride P words: no bank conflicts for odd P, two-way for P = 6
-// and 8) into one 16-byte store.  Positions past m pack as 0.  Writes
-// ceil(m / P) * 16 bytes, within the cap * 2o bytes there (and the 256-byte
-// rounding of every workspace piece).
+// The chunk of the cnt (1 to P) ids that end at position end of colInd, from
+// the last one down.
 template <int L>
-__device__ __forceinline__ void pack_chunks(const GraphDesc &D, uint64_t m, u32x4 *__restrict__ dst,
-                                            uint32_t *s_ids) {
+__device__ __forceinline__ u32x4 pack_chunk(gptr<uint32_t> colInd, uint64_t end, uint32_t cnt, uint32_t n,
+                                            uint32_t thr) {
     using PL = PackLayout<L>;
     constexpr int P = PL::P, B = PL::B;
-    const gptr<uint32_t> colInd = to_global(D.colInd);
-    const uint32_t thr = D.thr;
-    const uint64_t chunks = (m + P - 1) / P;
-    for (uint64_t g0 = (uint64_t)blockIdx.x * kBlock; g0 < chunks; g0 += (uint64_t)gridDim.x * kBlock) {
-        const uint64_t q0 = g0 * P;
+    typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));
+    uint32_t id[8];
+    if (end >= 8) {
+        const u32x4u x = *reinterpret_cast<gptr<u32x4u>>(colInd + (end - 4));
+        const u32x4u y = *reinterpret_cast<gptr<u32x4u>>(colInd + (end - 8));
 #pragma unroll
-        for (int z = 0; z < P; z++) {
-            const uint64_t q = q0 + (uint64_t)z * kBlock + threadIdx.x;
-            s_ids[z * kBlock + threadIdx.x] = q < m ? colInd[q] : 0u;
-        }
-        __syncthreads();
-        const uint64_t t = g0 + threadIdx.x;
-        if (t < chunks) {
-            uint32_t d[4] = {0u, 0u, 0u, 0u};
+        for (int z = 0; z < 8; z++) id[z] = z < 4 ? x[3 - z] : y[7 - z];
+    } else {
 #pragma unroll
-            for (int i = 0; i < P; i++) {
-                const uint32_t u = s_ids[P * threadIdx.x + i];
-                const uint32_t x = u >= thr ? u - thr : 0u;
-                const uint32_t f = PL::kAddr ? ((x >> 5) << 7) | (x & 31u) : x;
-                const int bit = B * i, k = bit / 32, sh = bit % 32;
-                d[k] |= f << sh;
-                if (sh + B > 32) d[k + 1] |= f >> (32 - sh);
-            }
-            dst[t] = u32x4{d[0], d[1], d[2], d[3]};
-        }
-        __syncthreads();
+        for (int z = 0; z < 8; z++) id[z] = (uint32_t)z < cnt ? colInd[end - 1 - z] : 0u;
     }
+    uint32_t d[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int z = 0; z < P; z++) {
+        const uint32_t x = (uint32_t)z < cnt && id[z] > thr ? n - id[z] : 0u;  // below rows
+        const uint32_t f = PL::kAddr ? ((x >> 5) << 7) | (x & 31u) : x;
+        const int bit = B * z, k = bit / 32, sh = bit % 32;
+        d[k] |= f << sh;
+        if (sh + B > 32) d[k + 1] |= f >> (32 - sh);
+    }
+    return u32x4{d[0], d[1], d[2], d[3]};
 }
 
+// Packs the counted rows into S.packed (the memory of the final level's
+// input pairs and slab words).  Blocks take tiles of kPackTile chunk slots in
+// turn, and the rows with slots in the tile kBlock at a time: a thread finds
+// its row's near ids by a binary search and with them its chunks in the tile,
+// whose prefix over the block deals them out; a thread finds a chunk's row in
+// the prefix, loads the ids by two 16-byte loads of any alignment and packs
+// them.  Chunks of ids up to thr only are left unwritten: no tail holds them.
 template <typename OffT>
 __global__ __launch_bounds__(kBlock) void k_split_pack(const GraphDesc *__restrict__ desc,
                                                        const SplitDesc *__restrict__ sd) {
-    __shared__ uint32_t s_ids[8 * kBlock];
+    __shared__ OffT s_re[kBlock], s_at[kBlock];  // a row's end; slot of its chunk 0 less the prefix
+    __shared__ uint32_t s_tail[kBlock], s_near[kBlock], s_pre[kBlock], s_skip[kBlock];
+    __shared__ uint32_t s_w[kWavesPerBlock];
     const GraphDesc &D = desc[0];
     const SplitDesc &S = sd[0];
-    const uint64_t m = (uint64_t) static_cast<const OffT *>(D.rowPtr)[D.n];
+    const gptr<OffT> rowPtr = to_global(static_cast<const OffT *>(D.rowPtr));
+    const gptr<uint32_t> colInd = to_global(D.colInd);
     u32x4 *__restrict__ dst = static_cast<u32x4 *>(S.packed);
-    switch (pack_layout(S.rows)) {  // block-uniform
-        case 0: pack_chunks<0>(D, m, dst, s_ids); break;
-        case 1: pack_chunks<1>(D, m, dst, s_ids); break;
-        case 2: pack_chunks<2>(D, m, dst, s_ids); break;
-        default: pack_chunks<3>(D, m, dst, s_ids); break;
+    const uint32_t v_lo = S.v_lo, v_hi = S.v_hi, n = D.n, thr = D.thr, P = S.far_ids;
+    if (v_lo > v_hi) return;  // nothing counted
+    const uint32_t near_end = n > kPackNear ? n - kPackNear : 0;  // ids from here on are near
+    const int layout = pack_layout(S.rows);
+    const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x >> 6;
+    const uint64_t c0 = pack_slot((uint64_t)rowPtr[v_lo]), c1 = pack_slot((uint64_t)rowPtr[(uint64_t)v_hi + 1]);
+    const uint64_t tiles = (c1 - c0 + kPackTile - 1) / kPackTile;
+    for (uint64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const uint64_t s0 = c0 + tile * kPackTile, s1 = s0 + kPackTile < c1 ? s0 + kPackTile : c1;
+        uint64_t vb = v_lo + wave_rightmost_le(v_hi - v_lo, s0, [&](uint32_t x) { return pack_slot((uint64_t)rowPtr[(uint64_t)v_lo + x]); });
+        for (;;) {  // windows of kBlock vertices from vb
+            const uint64_t v = vb + threadIdx.x, vn = vb + kBlock;
+            const bool more = vn <= v_hi && pack_slot((uint64_t)rowPtr[vn]) < s1;
+            uint32_t cnt = 0, near = 0, tail = 0, skip = 0;
+            OffT re = 0, c = 0;
+            if (v <= v_hi) {
+                const OffT rb = rowPtr[v];
+                re = rowPtr[v + 1];
+                c = pack_row<OffT>(rb, re);
+                if (re - rb >= 2 && c < s1 && pack_slot(re) > s0 && colInd[re - 1] > thr) {
+                    tail = (uint32_t)(re - rb - 1);
+                    OffT lo = rb + 1, hi = re;  // the first near one of the tail ids
+                    while (lo < hi) {
+                        const OffT mid = lo + ((hi - lo) >> 1);
+                        if (colInd[mid] < near_end) lo = mid + 1;
+                        else hi = mid;
+                    }
+                    near = (uint32_t)(re - lo);
+                    const uint32_t far = layout == 3 ? 0u : pack_div(tail - near + P - 1, P);
+                    const uint64_t z = (uint64_t)c + (near + kPackNearIds - 1) / kPackNearIds + far;
+                    skip = c < s0 ? (uint32_t)(s0 - c) : 0u;
+                    const uint64_t e = z < s1 ? z : s1;
+                    cnt = e > c + skip ? (uint32_t)(e - c - skip) : 0u;
+                }
+            }
+            uint32_t incl = cnt;
+#pragma unroll
+            for (int o = 1; o < kWave; o <<= 1) {
+                const uint32_t y = (uint32_t)__shfl_up((int)incl, o, kWave);
+                incl += (int)lane >= o ? y : 0u;
+            }
+            if (lane == kWave - 1) s_w[wv] = incl;
+            __syncthreads();  // also: the previous window is packed
+            uint32_t before = 0, total = 0;
+#pragma unroll
+            for (uint32_t w = 0; w < (uint32_t)kWavesPerBlock; w++) {
+                before += w < wv ? s_w[w] : 0u;
+                total += s_w[w];
+            }
+            s_pre[threadIdx.x] = before + incl - cnt;
+            s_skip[threadIdx.x] = skip;
+            s_near[threadIdx.x] = near;
+            s_tail[threadIdx.x] = tail;
+            s_re[threadIdx.x] = re;
+            s_at[threadIdx.x] = c;
+            __syncthreads();
+            for (uint32_t t = threadIdx.x; t < total; t += kBlock) {
+                uint32_t r = 0;  // the last row with s_pre[r] <= t
+#pragma unroll
+                for (uint32_t o = kBlock / 2; o > 0; o >>= 1) r += s_pre[r + o] <= t ? o : 0u;
+                const uint32_t q = t - s_pre[r] + s_skip[r], near_r = s_near[r], tail_r = s_tail[r];
+                const uint32_t qn = (near_r + kPackNearIds - 1) / kPackNearIds;
+                const bool is_near = q < qn;
+                const uint32_t first = is_near ? kPackNearIds * q : near_r + P * (q - qn);
+                const uint32_t left = (is_near ? near_r : tail_r) - first;
+                const uint64_t end = (uint64_t)s_re[r] - first;
+                if (colInd[end - 1] <= thr) continue;
+                const uint64_t at = (uint64_t)s_at[r] + q;
+                if (is_near) dst[at] = pack_chunk<3>(colInd, end, left < kPackNearIds ? left : kPackNearIds, n, thr);
+                else if (layout == 2) dst[at] = pack_chunk<2>(colInd, end, left < P ? left : P, n, thr);
+                else if (layout == 0) dst[at] = pack_chunk<0>(colInd, end, left < P ? left : P, n, thr);
+                else dst[at] = pack_chunk<1>(colInd, end, left < P ? left : P, n, thr);
+            }
+            if (!more) break;  // block-uniform
+            vb = vn;
+            __syncthreads();  // s_w is read
+        }
+        __syncthreads();
     }
 }
 
 // Lanes per in-edge tail in the row kernel (a wave takes kWave / kSplitLanes
-// in-edges per step), a 16-byte chunk per lane per step.  Tails average
-// ~180 ids on R-MAT-24 (median 86), and a step lasts as long as its longest
-// tail: 8 lanes of one chunk keep 80% of the id slots busy, 16 lanes of two
-// chunks 57%.  Measured on R-MAT-24: 18.2 ms at 8 x 1, 19.0 at 8 x 2, 18.8
-// at 16 x 1, 19.1 at 4 x 1, 22.1 at 16 x 2.
+// in-edges per step), a 16-byte chunk per lane: eight take a line at a time.
 constexpr int kSplitLanes = 8;
 
-// Counts the hits of the P packed ids of chunk c of a tail.  base = Pc - lo
-// (mod 2^32): position Pc + z is in the tail iff base + z < len.  Every
-// packed field names a bit of the row bitmap, so all P are looked up (word
-// and bit straight from the fields: a field's bit offset is its low 5
-// bits), the hits gathered as a P-bit mask and the positions outside the
-// tail masked off at the end.  An address field's bits [5, 21) are the byte
-// offset of its word in the bitmap.
+// The hits of the P packed ids of a chunk.  Every field names a bit of the
+// row bitmap (word and bit straight from the fields: a field's bit offset is
+// its low 5 bits), and those outside the tail name bits that are not set.  An
+// address field's bits [5, 21) are the byte offset of its word in the bitmap.
 template <int L>
-__device__ __forceinline__ uint32_t rows_chunk_hits(const uint32_t *s_bits, u32x4 ch, uint32_t base,
-                                                    uint32_t len) {
+__device__ __forceinline__ uint32_t rows_chunk_hits(const uint32_t *s_bits, u32x4 ch) {
     using PL = PackLayout<L>;
     constexpr int P = PL::P, B = PL::B;
     uint32_t f[P];
@@ -1080,22 +1269,33 @@ __device__ __forceinline__ uint32_t rows_chunk_hits(const uint32_t *s_bits, u32x
     uint32_t wrd[P];
 #pragma unroll
     for (int z = 0; z < P; z++) {
-        if (PL::kAddr) {
-            const uint32_t addr = __builtin_amdgcn_ubfe(f[z], 5u, 16u);
-            wrd[z] = *reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(s_bits) + addr);
-        } else {
-            wrd[z] = s_bits[__builtin_amdgcn_ubfe(f[z], 5u, (uint32_t)B - 5u)];
-        }
+        const uint32_t addr = PL::kAddr ? __builtin_amdgcn_ubfe(f[z], 5u, 16u) : (f[z] >> 3) & (((1u << (B - 5)) - 1) << 2);
+        wrd[z] = *reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(s_bits) + addr);
     }
-    uint32_t hm = 0;
+    uint32_t h = 0;
 #pragma unroll
-    for (int z = 0; z < P; z++) hm |= __builtin_amdgcn_ubfe(wrd[z], f[z], 1u) << z;
-    // valid z: [lc, hc) with lc = -base when base is negative (the tail's
-    // first chunk), hc = min(len - base, P)
-    const uint32_t lc = base > 0xfffffff0u ? 0u - base : 0u;
-    const uint32_t rem = len - base, hc = rem < (uint32_t)P ? rem : (uint32_t)P;
-    const uint32_t vm = ((1u << hc) - 1u) & (0xffffffffu << lc);
-    return __builtin_popcount(hm & vm);
+    for (int z = 0; z < P; z++) h += __builtin_amdgcn_ubfe(wrd[z], f[z], 1u);
+    return h;
+}
+
+// The hits of a tail's `chunks` chunks from `at` on (each lane's own first
+// one), kLanes lanes to a tail, this one's number sl.
+template <int L, int kLanes>
+__device__ __forceinline__ uint32_t rows_tail_hits(const uint32_t *s_bits, gptr<u32x4> at, uint32_t chunks, uint32_t sl) {
+    if (chunks <= sl) return 0;
+    uint32_t left = (chunks - sl + kLanes - 1) / kLanes, h = 0;  // the lane's chunks
+    u32x4 a = at[0], b;
+    for (;;) {  // two chunks a turn, each loaded before the one before is counted
+        if (left > 1) b = at[kLanes];
+        h += rows_chunk_hits<L>(s_bits, a);
+        if (left <= 1) break;
+        if (left > 2) a = at[2 * kLanes];
+        h += rows_chunk_hits<L>(s_bits, b);
+        if (left <= 2) break;
+        left -= 2;
+        at += 2 * kLanes;
+    }
+    return h;
 }
 
 // Persistent blocks take tiles of the rows' work from one counter.  The work
@@ -1104,10 +1304,10 @@ __device__ __forceinline__ uint32_t rows_chunk_hits(const uint32_t *s_bits, u32x
 // have few each: tiles of in-edges alone left blocks with hundreds of such
 // rows to the end, one chain of loads and barriers after another (a quarter
 // of R-MAT-21's wedges: 1.75 ms).
-// Per row of a tile the block puts adj+(w) into an LDS bitmap as bits u -
-// thr, its waves take the row's in-edges in the tile (kLanes lanes each),
+// Per row of a tile the block puts adj+(w) into an LDS bitmap as bits n -
+// u, its waves take the row's in-edges in the tile (kLanes lanes each),
 // and each tail is streamed through the bitmap from the packed ids
-// (k_split_pack) by 16-byte chunks of P ids (6 to 8, PackLayout), the next
+// (k_split_pack) by 16-byte chunks of 6 to 8 ids, the next
 // chunk loaded before this one is counted, and the next in-edges' bounds
 // before these are streamed.  A row's ids are loaded while the row before is
 // streamed; its bits go in as the other row's go out, all by exclusive or,
@@ -1126,7 +1326,7 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *
     const gptr<u32x4> packed = to_global(static_cast<const u32x4 *>(S.packed));
     const gptr<OffT> rp_in = to_global(static_cast<const OffT *>(S.rp_in));
     const gptr<OffT> ieG = to_global(static_cast<const OffT *>(S.ie));
-    const uint32_t thr = D.thr, rows = S.rows;
+    const uint32_t n = D.n, thr = D.thr, rows = S.rows;
     constexpr uint32_t kThreads = kWave * kWaves;
     constexpr uint32_t kPer = kWave / kLanes;  // in-edges a wave takes per step
     constexpr uint32_t kHold = 2;              // ids of a row a thread keeps
@@ -1140,11 +1340,29 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *
     const uint32_t lane = threadIdx.x & (kWave - 1), wv = uni32(threadIdx.x >> 6);
     const uint32_t sub = lane / kLanes, sl = lane % kLanes;
     unsigned long long *const ctr = reinterpret_cast<unsigned long long *>(meta + kMetaRows);
-    uint64_t hits = 0, checked = 0;
+    uint64_t hits = 0;
+    // the tails that the ends of a range cut: searched by one block
+    if (blockIdx.x == 0) {
+        for (uint32_t z = 0; z < S.cuts; z++) {
+            const uint32_t w = colInd[S.cut_j[z]];
+            const OffT wb = rowPtr[w], we = rowPtr[(uint64_t)w + 1];
+            for (uint64_t q = S.cut_lo[z] + threadIdx.x; q < S.cut_hi[z]; q += kThreads) {
+                const uint32_t u = colInd[q];
+                OffT lb = wb, n_ = we - wb;
+                while (n_ > 0) {
+                    const OffT half = n_ >> 1;
+                    const bool less = colInd[lb + half] < u;
+                    lb = less ? lb + half + 1 : lb;
+                    n_ = less ? n_ - half - 1 : half;
+                }
+                hits += lb < we && colInd[lb] == u ? 1u : 0u;
+            }
+        }
+    }
     // the row in the bitmap: adj+ = colInd[pb, pe), its first ids in held[]
     OffT pb = 0, pe = 0;
     uint32_t held[kHold] = {0, 0};
-    auto flip = [&](uint32_t u) { atomicXor(&s_bits[(u - thr) >> 5], 1u << ((u - thr) & 31u)); };
+    auto flip = [&](uint32_t u) { atomicXor(&s_bits[(n - u) >> 5], 1u << ((n - u) & 31u)); };
     if (threadIdx.x == 0) s_tile = atomicAdd(ctr, 1ull);
     __syncthreads();
     uint64_t t = uni64(s_tile);
@@ -1205,6 +1423,7 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *
             pb = ab;
             pe = ae;
             const uint64_t ck = k, ckend = kend;
+            const bool far = rows - (r0 + x) > kPackNear;  // the row's tails have far ids
             __syncthreads();
             // the next row's ids, on their way while this row is streamed
             x = next_row(x + 1);
@@ -1218,7 +1437,7 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *
             }
             uint32_t h = 0;
             uint64_t x0 = ck + (uint64_t)wv * kPer;
-            OffT lo = 0, hi = 0;
+            OffT lo = 0, hi = 0;  // a tail's first chunk, its chunks
             if (x0 + sub < ckend) {
                 lo = ieG[2 * (x0 + sub)];
                 hi = ieG[2 * (x0 + sub) + 1];
@@ -1231,24 +1450,10 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *
                     nlo = ieG[2 * (x0 + sub)];
                     nhi = ieG[2 * (x0 + sub) + 1];
                 }
-                if (sl == 0) checked += (uint64_t)(hi - lo);
-                // chunk c holds positions [Pc, Pc + P); a tail is shorter
-                // than 2^32 positions
-                constexpr uint32_t P = PackLayout<kLayout>::P;
-                const uint32_t len = (uint32_t)(hi - lo);
-                const OffT c_end = hi / P + (hi % P != 0 ? 1 : 0);
-                OffT c = lo / P + sl;
-                u32x4 cur = u32x4{0u, 0u, 0u, 0u};
-                if (c < c_end) cur = packed[c];
-                while (c < c_end) {
-                    const OffT cn = c + (OffT)kLanes;
-                    // the next chunk, or chunk c again past the tail's end
-                    // (loaded unconditionally; a chunk past c_end is not counted)
-                    const u32x4 nxt = packed[cn < c_end ? cn : c];
-                    h += rows_chunk_hits<kLayout>(s_bits, cur, (uint32_t)(P * c - lo), len);
-                    cur = nxt;
-                    c = cn;
-                }
+                const gptr<u32x4> at = packed + lo + sl;
+                const uint32_t near = (uint32_t)hi & 8191u;
+                h += rows_tail_hits<3, kLanes>(s_bits, at, near, sl);
+                if (kLayout != 3 && far) h += rows_tail_hits<kLayout, kLanes>(s_bits, at + near, (uint32_t)hi >> 13, sl);
                 lo = nlo;
                 hi = nhi;
             }
@@ -1259,9 +1464,7 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *
         t = uni64(s_tile);
     }
     hits = wave_sum(hits);
-    checked = wave_sum(checked);
     if (lane == 0 && hits) atomicAdd(&counts[0], (unsigned long long)hits);
-    if (lane == 0 && checked) atomicAdd(reinterpret_cast<unsigned long long *>(meta + kMetaTopWedges), checked);
 }
 
 // ---------------------------------------------------------------- list part
@@ -1309,13 +1512,11 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
     const gptr<uint32_t> auxG = to_global(static_cast<const uint32_t *>(S.ie_aux));
     const uint32_t rows = S.rows, keys = S.keys;
     const uint64_t L0 = (uint64_t)rp_in[rows], L1 = (uint64_t)rp_in[keys];
-    const OffT clip_j = (OffT)S.clip_j, clip_lo = (OffT)S.clip_lo;
-    const bool clipped = S.clip_j != ~0ull;
     constexpr uint32_t kThreads = kWave * kWaves;
     const uint32_t lane = threadIdx.x & (kWave - 1), wv = uni32(threadIdx.x >> 6);
     unsigned long long *const ctr = reinterpret_cast<unsigned long long *>(meta + kMetaSlabs);
     uint32_t cur = kSentinel;  // slab in s_tab (block-uniform)
-    uint64_t hits = 0, checked = 0;
+    uint64_t hits = 0;
     const uint64_t work = L1 - L0 + (uint64_t)kSlabCost * (keys - rows);
     uint64_t tile = work / (8ull * gridDim.x);
     tile = tile < kSlabTileMin ? kSlabTileMin : tile > kSlabTile ? kSlabTile : tile;
@@ -1384,10 +1585,8 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
                     hi = ieG[2 * x + 1];
                     aux = auxG[x];
                 }
-                OffT lo = j + 1;
-                if (clipped && j == clip_j) lo = clip_lo;
+                const OffT lo = j + 1;
                 if (x >= kend) hi = lo;  // nothing to stream
-                if (sl == 0) checked += (uint64_t)(hi - lo);
                 const uint32_t st = aux & kSlabAuxLong, len = aux >> 13;
                 if (len == 0) continue;  // adj+(w) is empty: no triangle
                 OffT gb = 0, ge = 0;  // adj+(w) in HBM for a long row
@@ -1462,9 +1661,7 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
         }
     }
     hits = wave_sum(hits);
-    checked = wave_sum(checked);
     if (lane == 0 && hits) atomicAdd(&counts[0], (unsigned long long)hits);
-    if (lane == 0 && checked) atomicAdd(reinterpret_cast<unsigned long long *>(meta + kMetaListWedges), checked);
 }
 
 // ---------------------------------------------------------------- launches
@@ -1589,6 +1786,8 @@ hipError_t launch_split_transpose(const GraphDesc *desc, const SplitDesc *sd, co
     return ob == 8 ? transpose<uint64_t>(desc, sd, dd, g, key_part, meta, st)
                    : transpose<uint32_t>(desc, sd, dd, g, key_part, meta, st);
 }
+
+uint32_t split_far_ids(uint32_t rows) { return pack_layout(rows) == 2 ? PackLayout<2>::P : PackLayout<0>::P; }
 
 size_t split_rows_lds(uint32_t rows) { return (size_t)(((rows + 31) / 32 + 1) & ~1u) * sizeof(uint32_t) + sizeof(uint64_t); }
 
