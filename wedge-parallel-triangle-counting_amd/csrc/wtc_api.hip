@@ -326,10 +326,11 @@ int split_layout(SplitDesc *sd, DenseDesc *dd, SplitGrids *grids, char *base, ui
 }
 
 // A bitmap length whose row does not fit one block's LDS (or a graph whose
-// keys overflow the transposition's parts) is counted by the row walk
+// keys overflow the transposition's parts, or whose ids the slab kernel's hash
+// sets could not hold) is counted by the row walk
 // against the bitmap in HBM, as the reference does.
 bool split_eligible(const Tuning &t, const GraphDesc &d, uint64_t m) {
-    return t.kernel == kKernelSplit && d.mode == kModeTiles && d.a > 0 && d.bm_rows > 0 &&
+    return t.kernel == kKernelSplit && d.mode == kModeTiles && d.a > 0 && d.bm_rows > 0 && d.n <= kSlabFree &&
            (uint64_t)d.bm_rows + split_slabs(m) <= (uint64_t)kSplitPartsMax << kSplitPartMax &&
            split_rows_lds(d.bm_rows) <= t.lds_bytes && (reinterpret_cast<uintptr_t>(d.colInd) & 15u) == 0;
 }

@@ -133,6 +133,9 @@ constexpr uint32_t kSlabSpan = 2048;
 constexpr uint32_t kSlabRowMax = 1024;
 constexpr uint32_t kSlabWin = kSlabSpan + kSlabRowMax;
 constexpr uint32_t kSlabWays = 4;
+constexpr uint32_t kSlabLong = 72;  // list tails are streamed by eight lanes where they hold this many ids on average
+constexpr uint32_t kSlabFree = 0x7fffffffu;  // a free slot (ids are below it)
+constexpr uint32_t kSlabMore = 0x80000000u;  // on a bucket's last slot: ids of the bucket are in the next, too
 constexpr uint32_t kSlabTile = 1024, kSlabTileMin = 128, kSlabCost = 48;  // a tile's work; a slab's share of it
 
 // Workspace and device-filled state of a split count.  The top rows are the

@@ -1469,30 +1469,74 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *
 
 // ---------------------------------------------------------------- list part
 
-// Bucket of id u in a row's region of len buckets (multiplicative hash; twelve
-// reversed bits of u scaled to len, all in full-rate instructions, were slower:
-// more ids per bucket, R-MAT-26's list part 37.3 ms against 36.0).
-__device__ __forceinline__ uint32_t slab_bucket(uint32_t u, uint32_t len) {
-    return __umulhi(u * 0x9e3779b1u, len);
+// Bucket of id u in a row's region of `len8 >> 8` buckets: a multiplicative
+// hash of u's low 24 bits, in 24-bit multiplications (32-bit ones take four
+// times as long, and the compiler makes them of a product that it needs the
+// low bits of only).
+__device__ __forceinline__ uint32_t slab_bucket(uint32_t u, uint32_t len8) {
+    uint32_t h, b;
+    asm("v_mul_u32_u24_e32 %0, %1, %2" : "=v"(h) : "s"(0x9e3779u), "v"(u));
+    asm("v_mul_hi_u32_u24_e32 %0, %1, %2" : "=v"(b) : "v"(h), "v"(len8));
+    return b;
+}
+
+// How many of four ids are in the row whose buckets start at st (len of
+// them); the ids from number `left` on are not counted.  Each id's first
+// bucket is read for all four at once, one 16-byte LDS read each; the slots are
+// compared without branches, and only a bucket marked full goes on to the
+// next.
+__device__ __forceinline__ uint32_t slab_hits(const u32x4 *tab4, const uint32_t (&u)[4], uint32_t left, uint32_t st,
+                                              uint32_t len) {
+    uint32_t bk[4], h = 0;
+    u32x4 v[4];
+#pragma unroll
+    for (int z = 0; z < 4; z++) {
+        bk[z] = st + slab_bucket(u[z], len << 8);
+        v[z] = tab4[bk[z]];
+    }
+#pragma unroll
+    for (int z = 0; z < 4; z++) {
+        const bool in = left > (uint32_t)z;
+        const bool f = (v[z][0] == u[z]) | (v[z][1] == u[z]) | (v[z][2] == u[z]) | ((v[z][3] & ~kSlabMore) == u[z]);
+        h += (in & f) ? 1u : 0u;
+        if (in & !f & ((int)v[z][3] < 0)) {
+            uint32_t b2 = bk[z];
+            for (;;) {
+                b2 = b2 + 1 == st + len ? st : b2 + 1;
+                const u32x4 w = tab4[b2];
+                const bool f2 = (w[0] == u[z]) | (w[1] == u[z]) | (w[2] == u[z]) | ((w[3] & ~kSlabMore) == u[z]);
+                h += f2 ? 1u : 0u;
+                if (f2 | ((int)w[3] >= 0)) break;
+            }
+        }
+    }
+    return h;
 }
 
 // Persistent blocks take tiles of the slabs' work from one counter: a slab's
 // work is kSlabCost for its rows and one unit per in-edge, in tiles of at most
 // kSlabTile, as in the row kernel (with tiles of in-edges alone, those over
 // the many slabs with few in-edges took 0.45 ms on R-MAT-20 however few the
-// list rows were).  A tile's in-edges of one slab form a segment.  Per segment, the block hashes into LDS every row of the slab the
-// segment's in-edges name that is not there yet (the table is kept while
-// the next segment stays in the slab; a wave per row clears its buckets and
-// inserts its ids): the row starting at window position st with len
-// entries owns the buckets [st, st + len) of kSlabWays slots each, so a
-// quarter of its slots are filled and a lookup nearly always ends in its
-// first bucket (one 16-byte LDS read).  Then the segment's in-edges are
-// dealt to the waves, kLanes lanes each; each tail is streamed by 16-byte
-// loads, two in flight per lane, and each id u looked up in adj+(w) by
-// linear probing from its hash bucket, or by a binary search in HBM for a
-// row longer than kSlabRowMax.
+// list rows were; half or twice as large tiles cost R-MAT-24 12% and 22%).
+// A tile's in-edges of one slab form a segment.  Per segment, the block hashes
+// into LDS every row of the slab the segment's in-edges name that is not there
+// yet (the table is kept while the next segment stays in the slab; a wave per
+// row clears its buckets and inserts its ids): the row starting at window
+// position st with len entries owns the buckets [st, st + len) of kSlabWays
+// slots each, so a quarter of its slots are filled; an id whose bucket is full
+// marks it and goes to the next.  Then the segment's in-edges are dealt to the
+// waves, 4 or 8 lanes each, the next step's first ids and the bounds of the
+// one after on their way while this one's tails are streamed and looked up
+// (slab_hits; by a binary search in HBM for a row longer than kSlabRowMax).
+// No one unit is full (R-MAT-26: vector instructions 54%, lines from beyond
+// L2 60%, LDS 37%): bound by the chain of a segment at the 24 waves a CU that
+// the tables leave.  Against a hash by 32-bit multiplications, full buckets
+// not marked (a wave met a full one in 7 of 10 lookups, now one in 5) and
+// loads not ahead of the tables: R-MAT-26 36.2 -> 27.8 ms, R-MAT-24 2.61 ->
+// 2.08, R-MAT-22 0.43 -> 0.37.  Eight lanes where tails are long: R-MAT-26
+// (~90 ids) 27.8 against 30.1 with four, R-MAT-24 (49 ids) 2.16 against 2.06.
 // Same alignment and slack needs as the row kernel.
-template <typename OffT, int kWaves, int kLanes>
+template <typename OffT, int kWaves>
 __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc *__restrict__ desc,
                                                                 const SplitDesc *__restrict__ sd,
                                                                 uint64_t *__restrict__ meta,
@@ -1515,6 +1559,9 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
     constexpr uint32_t kThreads = kWave * kWaves;
     const uint32_t lane = threadIdx.x & (kWave - 1), wv = uni32(threadIdx.x >> 6);
     unsigned long long *const ctr = reinterpret_cast<unsigned long long *>(meta + kMetaSlabs);
+    // lanes to a tail: a turn of four takes 16 ids, of eight 32
+    const uint32_t lanes = S.tally[1] > (uint64_t)kSlabLong * (L1 - L0) ? 8u : 4u;
+    const uint32_t per = kWave / lanes, deal = kWaves * per, step = 4 * lanes, sub = lane / lanes, sl = lane % lanes;
     uint32_t cur = kSentinel;  // slab in s_tab (block-uniform)
     uint64_t hits = 0;
     const uint64_t work = L1 - L0 + (uint64_t)kSlabCost * (keys - rows);
@@ -1540,6 +1587,33 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
             if (k >= kend) continue;
             const uint32_t slab = key - rows;
             const uint64_t wb = (uint64_t)slab * kSlabSpan;  // window start in colInd
+            // the segment's in-edges are dealt to the waves, `lanes` lanes each;
+            // the first two steps' and the first tails' first ids are on their
+            // way while the table is built
+            struct Edge {
+                OffT j, hi;
+                uint32_t aux;
+                __device__ __forceinline__ OffT first(uint32_t l) const { return ((j + 1) & ~(OffT)3) + 4 * l; }
+                __device__ __forceinline__ bool hashed() const { return (aux >> 13) != 0 && (aux >> 13) != kSlabAuxLong; }
+            };
+            auto edge = [&](uint64_t x) -> Edge {
+                Edge e{0, 0, 0u};
+                if (x < kend) {
+                    e.j = ieG[2 * x];
+                    e.hi = ieG[2 * x + 1];
+                    e.aux = auxG[x];
+                }
+                return e;
+            };
+            auto head = [&](const Edge &e) -> u32x4 {
+                const OffT q = e.first(sl);
+                u32x4 r = {0u, 0u, 0u, 0u};
+                if (e.hashed() && q < e.hi) r = *reinterpret_cast<gptr<u32x4>>(colInd + q);
+                return r;
+            };
+            uint64_t x0 = k + (uint64_t)wv * per + sub;
+            Edge ed = edge(x0), en = edge(x0 + deal);
+            u32x4 ids = head(ed);
             // the rows this segment names that the table lacks
             __syncthreads();  // the previous segment's lookups are done
             if (slab != cur)
@@ -1555,107 +1629,78 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
             }
             __syncthreads();
             // a wave per new row: its buckets cleared, then its ids inserted
-            // (one wave's LDS operations stay in order)
+            // (one wave's LDS operations stay in order), the next row's first
+            // ids loaded before
             const uint32_t nnew = s_nnew;
-            for (uint32_t r = wv; r < nnew; r += kWaves) {
-                const uint32_t aux = s_new[r], st = aux & kSlabAuxLong, len = aux >> 13;
-                for (uint32_t i = lane; i < len; i += kWave)
-                    reinterpret_cast<uint4 *>(s_tab)[st + i] = make_uint4(kSentinel, kSentinel, kSentinel, kSentinel);
-                for (uint32_t i = lane; i < len; i += kWave) {
-                    const uint32_t u = colInd[wb + st + i];
-                    uint32_t bk = st + slab_bucket(u, len);
-                    for (bool done = false; !done;) {
-                        for (uint32_t z = 0; z < kSlabWays && !done; z++)
-                            done = atomicCAS(&s_tab[bk * kSlabWays + z], kSentinel, u) == kSentinel;
-                        bk = bk + 1 == st + len ? st : bk + 1;
+            {
+                uint32_t aux = wv < nnew ? s_new[wv] : 0u;
+                uint32_t u = lane < aux >> 13 ? colInd[wb + (aux & kSlabAuxLong) + lane] : 0u;
+                for (uint32_t r = wv; r < nnew; r += kWaves) {
+                    const uint32_t naux = r + kWaves < nnew ? s_new[r + kWaves] : 0u;
+                    const uint32_t nu = lane < naux >> 13 ? colInd[wb + (naux & kSlabAuxLong) + lane] : 0u;
+                    const uint32_t st = aux & kSlabAuxLong, len = aux >> 13;
+                    for (uint32_t i = lane; i < len; i += kWave)
+                        reinterpret_cast<uint4 *>(s_tab)[st + i] = make_uint4(kSlabFree, kSlabFree, kSlabFree, kSlabFree);
+                    for (uint32_t i = lane; i < len; i += kWave) {
+                        if (i >= kWave) u = colInd[wb + st + i];
+                        uint32_t bk = st + slab_bucket(u, len << 8);
+                        for (;;) {
+                            uint32_t z = 0;
+                            while (z < kSlabWays && atomicCAS(&s_tab[bk * kSlabWays + z], kSlabFree, u) != kSlabFree) z++;
+                            if (z < kSlabWays) break;
+                            atomicOr(&s_tab[bk * kSlabWays + kSlabWays - 1], kSlabMore);  // full: on to the next
+                            bk = bk + 1 == st + len ? st : bk + 1;
+                        }
                     }
+                    aux = naux;
+                    u = nu;
                 }
             }
             __syncthreads();
-            // the segment's in-edges dealt to the waves, kLanes lanes each
-            constexpr uint32_t kPer = kWave / kLanes;
-            const uint32_t sub = lane / kLanes, sl = lane % kLanes;
             uint32_t h = 0;
-            for (uint64_t x0 = k + (uint64_t)wv * kPer; x0 < kend; x0 += (uint64_t)kWaves * kPer) {
-                const uint64_t x = x0 + sub;
-                OffT j = 0, hi = 0;
-                uint32_t aux = 0;
-                if (x < kend) {
-                    j = ieG[2 * x];
-                    hi = ieG[2 * x + 1];
-                    aux = auxG[x];
-                }
-                const OffT lo = j + 1;
-                if (x >= kend) hi = lo;  // nothing to stream
-                const uint32_t st = aux & kSlabAuxLong, len = aux >> 13;
-                if (len == 0) continue;  // adj+(w) is empty: no triangle
-                OffT gb = 0, ge = 0;  // adj+(w) in HBM for a long row
-                if (len == kSlabAuxLong) {
-                    const uint32_t w = colInd[j];
-                    gb = rowPtr[w];
-                    ge = rowPtr[w + 1];
-                }
-                for (OffT q = (lo & ~(OffT)3) + 4 * sl; q < hi; q += 8 * kLanes) {  // two loads in flight
-                    const OffT q1 = q + 4 * kLanes;
-                    const u32x4 a = *reinterpret_cast<gptr<u32x4>>(colInd + q);
-                    u32x4 b = {0u, 0u, 0u, 0u};
-                    if (q1 < hi) b = *reinterpret_cast<gptr<u32x4>>(colInd + q1);
-                    const uint32_t ua[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-                    if (len != kSlabAuxLong) {
-                        // each id's first bucket read for all eight at once (one 16-byte LDS
-                        // read each; a position outside the tail reads the row's first
-                        // bucket and is not counted), the four slots compared without
-                        // branches; slots fill in order, so a free last slot ends the chain,
-                        // and only a full bucket without the id goes on to the next
-                        const u32x4 *tab4 = reinterpret_cast<const u32x4 *>(s_tab);
-                        uint32_t bk[8];
-                        bool in[8];
-                        u32x4 v[8];
-#pragma unroll
-                        for (int z = 0; z < 8; z++) {
-                            const OffT t = (z < 4 ? q : q1) + (OffT)(z & 3);
-                            in[z] = t >= lo && t < hi;
-                            bk[z] = st + slab_bucket(ua[z], len);
-                            v[z] = tab4[in[z] ? bk[z] : st];
-                        }
-#pragma unroll
-                        for (int z = 0; z < 8; z++) {
-                            const uint32_t u = ua[z];
-                            const bool f = (v[z][0] == u) | (v[z][1] == u) | (v[z][2] == u) | (v[z][3] == u);
-                            h += (in[z] & f) ? 1u : 0u;
-                            if (in[z] & !f & (v[z][3] != kSentinel)) {
-                                uint32_t b2 = bk[z] + 1 == st + len ? st : bk[z] + 1;
-                                for (;;) {
-                                    const u32x4 w2 = tab4[b2];
-                                    const bool f2 = (w2[0] == u) | (w2[1] == u) | (w2[2] == u) | (w2[3] == u);
-                                    h += f2 ? 1u : 0u;
-                                    if (f2 | (w2[3] == kSentinel)) break;
-                                    b2 = b2 + 1 == st + len ? st : b2 + 1;
-                                }
-                            }
-                        }
-                        continue;
+            for (; x0 - sub < kend; x0 += deal) {
+                const Edge e2 = edge(x0 + 2 * deal);
+                const u32x4 nids = head(en);
+                const uint32_t st = ed.aux & kSlabAuxLong, len = ed.aux >> 13;
+                const OffT lo = ed.j + 1;
+                OffT q = ed.first(sl);
+                if (ed.hashed() && q < ed.hi) {
+                    uint32_t left = (uint32_t)(ed.hi - q);
+                    u32x4 a = ids;
+                    if (q < lo) {  // ids before the tail: 0 is in no row
+                        a[0] = 0u;
+                        a[1] = lo - q > 1 ? 0u : a[1];
+                        a[2] = lo - q > 2 ? 0u : a[2];
                     }
-                    // a long row: adj+(w) searched in HBM
-#pragma unroll
-                    for (int z = 0; z < 8; z++) {
-                        const OffT t = (z < 4 ? q : q1) + (OffT)(z & 3);
-                        if (t < lo || t >= hi) continue;
-                        const uint32_t u = ua[z];
-                        OffT lb = gb, n_ = ge - gb;
+                    gptr<uint32_t> p = colInd + q;
+                    for (;;) {
+                        u32x4 b = a;
+                        if (left > step) b = *reinterpret_cast<gptr<u32x4>>(p + step);
+                        const uint32_t u[4] = {a[0], a[1], a[2], a[3]};
+                        h += slab_hits(reinterpret_cast<const u32x4 *>(s_tab), u, left, st, len);
+                        if (left <= step) break;
+                        left -= step;
+                        p += step;
+                        a = b;
+                    }
+                } else if (len == kSlabAuxLong) {  // a long row: adj+(w) searched in HBM
+                    const uint32_t w = colInd[ed.j];
+                    OffT gb = rowPtr[w], ge = rowPtr[(uint64_t)w + 1];
+                    for (q = lo + sl; q < ed.hi; q += (OffT)lanes) {
+                        const uint32_t u = colInd[q];
+                        OffT n_ = ge - gb;
                         while (n_ > 0) {
                             const OffT half = n_ >> 1;
-                            if (colInd[lb + half] < u) {
-                                lb += half + 1;
-                                n_ -= half + 1;
-                            } else {
-                                n_ = half;
-                            }
+                            const bool less = colInd[gb + half] < u;
+                            gb = less ? gb + half + 1 : gb;
+                            n_ = less ? n_ - half - 1 : half;
                         }
-                        gb = lb;  // the lane's next id is larger
-                        h += lb < ge && colInd[lb] == u ? 1u : 0u;
+                        h += gb < ge && colInd[gb] == u ? 1u : 0u;  // the lane's next id is larger
                     }
                 }
+                ed = en;
+                en = e2;
+                ids = nids;
             }
             hits += h;
         }
@@ -1841,15 +1886,12 @@ hipError_t launch_split_rows(const GraphDesc *desc, const SplitDesc *sd, int ob,
     return hipLaunchKernel(fn, dim3(grid), dim3(wpb * kWave), args, split_rows_lds(rows), st);
 }
 
-// The slab kernel's block: 8 waves, 4 lanes per in-edge tail (list tails
-// are short: ~50 ids on R-MAT-24; 2.53 ms there at 4 lanes, 2.71 at 2, 2.73
-// at 8).
+// The slab kernel's block (three to a CU by their LDS).
 constexpr int kSlabWaves = 8;
-constexpr int kSlabLanes = 4;
 
 static const void *split_slabs_kernel(int ob) {
-    return ob == 8 ? reinterpret_cast<const void *>(&k_split_slabs<uint64_t, kSlabWaves, kSlabLanes>)
-                   : reinterpret_cast<const void *>(&k_split_slabs<uint32_t, kSlabWaves, kSlabLanes>);
+    return ob == 8 ? reinterpret_cast<const void *>(&k_split_slabs<uint64_t, kSlabWaves>)
+                   : reinterpret_cast<const void *>(&k_split_slabs<uint32_t, kSlabWaves>);
 }
 
 hipError_t split_slabs_grid(int ob, int num_cus, uint32_t *grid) {
