@@ -223,7 +223,7 @@ SplitLayout split_plan(uint32_t n, uint64_t m, uint32_t rows, int ob_in) {
     L.sub_tot = take((size_t)L.subs * sizeof(uint32_t));
     L.list_bid = take((size_t)L.g.parts * sizeof(uint32_t));
     L.part_tot = take((size_t)L.g.parts * sizeof(uint64_t));
-    L.tally = take(2 * sizeof(uint64_t));
+    L.tally = take(sizeof(uint64_t));
     L.key_part = take(((size_t)L.g.keys / kKeyChunk + 2) * sizeof(uint64_t));
     L.key_tot = take((size_t)L.g.keys * sizeof(uint32_t));
     L.recid = take((size_t)L.cap * sizeof(uint16_t));

@@ -163,7 +163,7 @@ struct SplitDesc {
     uint32_t *sub_tot;    // subs: records of each sub-part
     uint32_t *list_bid;   // parts: the first list vertex w whose key lies in each part (0 up to the first list part)
     uint64_t *part_tot;   // parts: record slots of each part (>= its records)
-    uint64_t *tally;      // 2: wedges of the top rows' and of the list rows' in-edges
+    uint64_t *tally;      // 1: wedges of the top rows' in-edges
     uint64_t *key_part;   // key blocks: in-edges of each block of kKeyChunk keys, then their prefix
     uint32_t *key_tot;    // keys: in-edges of each key
     uint16_t *rec_id;     // cap: A keys within their part

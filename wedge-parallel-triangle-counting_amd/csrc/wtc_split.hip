@@ -201,7 +201,7 @@ __global__ __launch_bounds__(kSplitPartsMax) void k_split_range(const GraphDesc 
     S.w_hi = hi;
     S.cuts = 0;
     S.cut_top = 0;
-    S.tally[0] = S.tally[1] = 0;
+    S.tally[0] = 0;
     if (lo == 0 && hi == W) {  // the whole order: nothing clipped
         S.clip = 0;
         S.v_lo = 0;
@@ -243,7 +243,7 @@ __global__ __launch_bounds__(kSplitPartsMax) void k_split_range(const GraphDesc 
         S.cut_hi[S.cuts] = e[z];
         S.cuts++;
         S.cut_top += top;
-        S.tally[top ? 0 : 1] += e[z] - b[z];
+        if (top) S.tally[0] += e[z] - b[z];
     }
 }
 
@@ -426,14 +426,15 @@ __device__ __forceinline__ void block_prefix(const uint32_t *s_cnt, uint32_t *s_
 //  3. the tile is ranked per part (LDS atomics), takes its slots of every
 //     part with one global atomic per part, and leaves sorted by part
 //     through LDS, a part's records as consecutive lanes of one store.
-// Bound by the chain of loads and barriers of a tile (two blocks a CU), then
-// by the records' 10 bytes written.  R-MAT-20: part sizes and records in
-// 0.16 ms against 0.36 with vertex chunks counted and dealt to waves, whose
-// lanes stored straight to 32,768-key parts; R-MAT-22 0.62 against 0.90;
-// R-MAT-24 2.5 against 2.7, and its parts are small enough to leave out a
-// level (the levels after: 2.8 against 3.9 ms).
+// Bound by the chain of loads and barriers of a tile, so held to 64 registers
+// for two blocks a CU (with one, 96 registers: R-MAT-24 1.92 against 1.52 ms,
+// R-MAT-26 10.4 against 8.4), then by the records' 10 bytes written.  R-MAT-20:
+// part sizes and records in 0.12 ms against 0.36 with vertex chunks counted and
+// dealt to waves, whose lanes stored straight to 32,768-key parts; R-MAT-22
+// 0.53 against 0.90; R-MAT-24 1.9 against 2.7, and its parts are small enough
+// to leave out a level.
 template <typename OffT>
-__global__ __launch_bounds__(kSplitBlock) void k_split_l1(const GraphDesc *__restrict__ desc,
+__global__ __launch_bounds__(kSplitBlock, 8) void k_split_l1(const GraphDesc *__restrict__ desc,
                                                           const SplitDesc *__restrict__ sd) {
     constexpr uint32_t kT = LevelTile<OffT>::kT, kPer = kT / kSplitBlock;
     constexpr uint32_t kWaves = kSplitBlock / kWave;
@@ -447,7 +448,7 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_l1(const GraphDesc *__res
     };
     __shared__ SlotOrPair s_x[kT];
     __shared__ uint64_t s_front;  // in-edges of the tile's first row before the tile
-    __shared__ unsigned long long s_tally[2];
+    __shared__ unsigned long long s_tally;
     __shared__ uint32_t s_open;  // the last row's far in-edges reach the tile's end
     __shared__ uint16_t s_mark[kT];
     __shared__ uint16_t s_key[kT];
@@ -465,23 +466,24 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_l1(const GraphDesc *__res
     TailPair<OffT> *__restrict__ rec = static_cast<TailPair<OffT> *>(S.rec);
     uint32_t *__restrict__ rec_aux = S.rec_aux;
     const uint32_t thr = D.thr, rows = S.rows, parts = S.parts, shift = S.part_shift;
-    const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x >> 6;
+    const uint32_t lane = threadIdx.x & (kWave - 1), wv = uni32(threadIdx.x >> 6);
     const bool clip = S.clip != 0;
     const uint32_t v_lo = S.v_lo, v_hi = S.v_hi;
     if (v_lo > v_hi) return;  // nothing counted
     const uint64_t w_lo = S.w_lo, w_hi = S.w_hi;
     // the end vertices' rows, whose tails the range may clip
-    const OffT rl0 = rowPtr[v_lo], rl1 = rowPtr[(uint64_t)v_lo + 1], rh0 = rowPtr[v_hi], rh1 = rowPtr[(uint64_t)v_hi + 1];
-    const uint64_t K0 = iep[v_lo], K1 = iep[(uint64_t)v_hi + 1];
+    const OffT rl0 = uni(rowPtr[v_lo]), rl1 = uni(rowPtr[(uint64_t)v_lo + 1]);
+    const OffT rh0 = uni(rowPtr[v_hi]), rh1 = uni(rowPtr[(uint64_t)v_hi + 1]);
+    const uint64_t K0 = uni64(iep[v_lo]), K1 = uni64(iep[(uint64_t)v_hi + 1]);
     const uint64_t tiles = (K1 - K0 + kT - 1) / kT;
     const uint32_t list_part = rows >> shift;  // the first part with list keys
     // the top ids below far_end are far
-    const uint32_t far_ids = S.far_ids, far_end = D.n > kPackNear ? D.n - kPackNear : 0;
-    const bool far_top = far_end > thr;
-    uint64_t tops = 0, rest = 0;  // wedges of the top and of the list in-edges
-    if (threadIdx.x < 2) s_tally[threadIdx.x] = 0;
+    const uint32_t far_ids = S.far_ids, far_end = uni32(D.n > kPackNear ? D.n - kPackNear : 0u);
+    const uint32_t far_rows = far_end > thr ? far_end - thr : 0;
+    uint64_t tops = 0;  // wedges of the top in-edges
+    if (threadIdx.x == 0) s_tally = 0;
     for (uint64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        uint64_t vb = S.tile_v[tile];
+        uint64_t vb = uni32(S.tile_v[tile]);
         const uint64_t t0 = K0 + tile * kT, t1 = t0 + kT < K1 ? t0 + kT : K1;
         const uint32_t nt = (uint32_t)(t1 - t0);
         __syncthreads();  // the previous tile is written out
@@ -491,7 +493,7 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_l1(const GraphDesc *__res
         __syncthreads();
         for (;;) {  // windows of kSplitBlock vertices from vb, up to the one holding t1 - 1
             const uint64_t v = vb + threadIdx.x, vn = vb + kSplitBlock;
-            const uint64_t next = vn > v_hi ? t1 : iep[vn];
+            const uint64_t next = vn > v_hi ? t1 : uni64(iep[vn]);
             if (v <= v_hi) {
                 const uint64_t a = iep[v], z = iep[v + 1];
                 const OffT rb = rowPtr[v], re = rowPtr[v + 1];
@@ -532,7 +534,7 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_l1(const GraphDesc *__res
             for (uint32_t z = 0; z < kPer; z++) s_mark[threadIdx.x * kPer + z] = (uint16_t)(x[z] > before ? x[z] : before);
         }
         __syncthreads();
-        const OffT front = (OffT)s_front;
+        const OffT front = (OffT)uni64(s_front);
         auto position = [&](uint32_t i) -> OffT {  // of in-edge slot i in colInd
             const uint32_t p = s_mark[i];
             return s_x[p].v.rb + (OffT)(i - p) + (p ? 0 : front);
@@ -558,14 +560,21 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_l1(const GraphDesc *__res
                 rp1[u] = rowPtr[(uint64_t)id[u] + 1];
             }
         }
+        uint32_t key[kPer], aux[kPer];
+#pragma unroll
+        for (uint32_t u = 0; u < kPer; u++) {
+            key[u] = id[u] >= thr ? id[u] - thr : rows + (uint32_t)((uint64_t)rp[u] / kSlabSpan);
+            const uint64_t len = (uint64_t)(rp1[u] - rp[u]);
+            aux[u] = (uint32_t)((uint64_t)rp[u] % kSlabSpan) | ((len <= kSlabRowMax ? (uint32_t)len : kSlabAuxLong) << 13);
+        }
         // a row's near ids are those after its last far one: where two
         // neighbours show it; of a row whose far in-edges reach the tile's
         // end, by a search
-        if (far_top) {  // block-uniform
+        if (far_rows) {  // block-uniform
 #pragma unroll
             for (uint32_t u = 0; u < kPer; u++) {
                 const uint32_t i = threadIdx.x + u * kSplitBlock;
-                if (i >= nt || id[u] < thr || id[u] >= far_end) continue;
+                if (i >= nt || key[u] >= far_rows) continue;
                 if (nid[u] >= far_end) s_x[s_mark[i]].v.near = (uint32_t)(s_x[s_mark[i]].v.e - position(i) - 1);
                 else if (i == nt - 1) s_open = 1;
             }
@@ -593,29 +602,26 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_l1(const GraphDesc *__res
                 cut |= in ? 0u : 1u << u;
             }
         }
-        uint32_t key[kPer], rank[kPer], aux[kPer];
+        uint32_t rank[kPer];
         TailPair<OffT> t[kPer];
 #pragma unroll
         for (uint32_t u = 0; u < kPer; u++) {
             const uint32_t i = threadIdx.x + u * kSplitBlock;
-            key[u] = kSentinel;
-            if (i >= nt || (cut >> u & 1u)) continue;
+            if (i >= nt || (cut >> u & 1u)) {
+                key[u] = kSentinel;
+                continue;
+            }
             const uint32_t p = s_mark[i];
-            const OffT j = position(i), rb = s_x[p].v.rb, e = s_x[p].v.e;
-            const bool top = id[u] >= thr;
-            key[u] = top ? id[u] - thr : rows + (uint32_t)((uint64_t)rp[u] / kSlabSpan);
+            const OffT j = position(i), e = s_x[p].v.e;
             const uint32_t tail = (uint32_t)(e - j - 1);
-            if (top) {
+            if (key[u] < rows) {
                 tops += tail;
-                const uint32_t near = id[u] < far_end ? s_x[p].v.near : tail;
-                t[u].lo = pack_row<OffT>(rb, e);
+                const uint32_t near = key[u] < far_rows ? s_x[p].v.near : tail;
+                t[u].lo = pack_row<OffT>(s_x[p].v.rb, e);
                 t[u].hi = pack_count((near + kPackNearIds - 1) / kPackNearIds, pack_div(tail - near + far_ids - 1, far_ids));
             } else {
-                rest += tail;
-                t[u] = TailPair<OffT>{j, e};
+                                t[u] = TailPair<OffT>{j, e};
             }
-            const uint64_t len = (uint64_t)(rp1[u] - rp[u]);
-            aux[u] = (uint32_t)((uint64_t)rp[u] % kSlabSpan) | ((len <= kSlabRowMax ? (uint32_t)len : kSlabAuxLong) << 13);
             rank[u] = atomicAdd(&s_cnt[key[u] >> shift], 1u);
         }
         __syncthreads();  // s_x's rows are read, the counts are done
@@ -681,13 +687,10 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_l1(const GraphDesc *__res
         }
     }
     tops = wave_sum(tops);
-    rest = wave_sum(rest);
     __syncthreads();  // s_tally is zeroed, also without a tile
-    if (lane == 0 && tops) atomicAdd(&s_tally[0], (unsigned long long)tops);
-    if (lane == 0 && rest) atomicAdd(&s_tally[1], (unsigned long long)rest);
+    if (lane == 0 && tops) atomicAdd(&s_tally, (unsigned long long)tops);
     __syncthreads();
-    if (threadIdx.x < 2 && s_tally[threadIdx.x])
-        atomicAdd(reinterpret_cast<unsigned long long *>(&S.tally[threadIdx.x]), s_tally[threadIdx.x]);
+    if (threadIdx.x == 0 && s_tally) atomicAdd(reinterpret_cast<unsigned long long *>(S.tally), s_tally);
 }
 
 // Later levels.  With up to kSplitPartsMax << kSplitFinalMax keys, a part
@@ -777,6 +780,17 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_level_count(const SplitDe
     }
 }
 
+// Records of a scatter's tile: twice LevelTile's (one block a CU by LDS) where
+// a bucket gets four or fewer of a tile.  Writes of less than 64 bytes pass L2
+// one by one, some 54 a nanosecond, and bound the kernel: R-MAT-24 (2,048
+// buckets) 2.02 -> 1.74 ms with tiles of 8,192, R-MAT-22 (1,024) 0.42 -> 0.35,
+// R-MAT-20 (512) 0.068 either way.
+template <typename OffT, uint32_t kF>
+struct ScatterTile {
+    static constexpr bool kTwo = kF < 1024;  // two blocks a CU
+    static constexpr uint32_t kT = LevelTile<OffT>::kT * (kTwo ? 1 : 2);
+};
+
 // The scatter of a level.  hist[c] holds, per output bucket, the input
 // bucket's records in blocks before c.  The block takes its records in tiles
 // of kT: each tile is ranked per output bucket (LDS atomics), staged in LDS
@@ -786,8 +800,9 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_level_count(const SplitDe
 // list records' slab words go through the same LDS after the pairs, in
 // buckets that hold list keys only.
 template <typename OffT, typename KeyIn, bool kFinal, uint32_t kF>
-__global__ __launch_bounds__(kSplitBlock, 8) void k_split_level_scatter(const SplitDesc *__restrict__ sd) {
-    constexpr uint32_t kT = LevelTile<OffT>::kT;
+__global__ __launch_bounds__(kSplitBlock, (ScatterTile<OffT, kF>::kTwo ? 8 : 4)) void k_split_level_scatter(
+    const SplitDesc *__restrict__ sd) {
+    constexpr uint32_t kT = ScatterTile<OffT, kF>::kT;
     constexpr uint32_t kPerThread = kT / kSplitBlock;
     __shared__ uint64_t s_base[kF];  // next output slot of each output bucket
     __shared__ uint32_t s_tcnt[kF];  // the tile's records per output bucket
@@ -1043,7 +1058,7 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_keyscan(const SplitDesc *
         meta[kMetaTopWedges] = S.tally[0] + dense[kDenseTopWedges];
         meta[kMetaDenseTopWedges] = dense[kDenseTopWedges];
         meta[kMetaDenseTopEdges] = dense[kDenseTopEdges];
-        meta[kMetaListWedges] = S.tally[1];
+        meta[kMetaListWedges] = S.w_hi - S.w_lo - S.tally[0] - dense[kDenseTopWedges];
         meta[kMetaWedges] = S.w_hi - S.w_lo;
         meta[kMetaAllEdges] = all + dense[kDenseEdges] + S.cuts;
     }
@@ -1560,7 +1575,7 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
     const uint32_t lane = threadIdx.x & (kWave - 1), wv = uni32(threadIdx.x >> 6);
     unsigned long long *const ctr = reinterpret_cast<unsigned long long *>(meta + kMetaSlabs);
     // lanes to a tail: a turn of four takes 16 ids, of eight 32
-    const uint32_t lanes = S.tally[1] > (uint64_t)kSlabLong * (L1 - L0) ? 8u : 4u;
+    const uint32_t lanes = uni64(meta[kMetaListWedges]) > (uint64_t)kSlabLong * (L1 - L0) ? 8u : 4u;
     const uint32_t per = kWave / lanes, deal = kWaves * per, step = 4 * lanes, sub = lane / lanes, sl = lane % lanes;
     uint32_t cur = kSentinel;  // slab in s_tab (block-uniform)
     uint64_t hits = 0;
