@@ -330,7 +330,7 @@ int split_layout(SplitDesc *sd, DenseDesc *dd, SplitGrids *grids, char *base, ui
 // sets could not hold) is counted by the row walk
 // against the bitmap in HBM, as the reference does.
 bool split_eligible(const Tuning &t, const GraphDesc &d, uint64_t m) {
-    return t.kernel == kKernelSplit && d.mode == kModeTiles && d.a > 0 && d.bm_rows > 0 && d.n <= kSlabFree &&
+    return t.kernel == kKernelSplit && d.mode == kModeTiles && d.a > 0 && d.bm_rows > 0 && d.n <= kSetIdsEnd &&
            (uint64_t)d.bm_rows + split_slabs(m) <= (uint64_t)kSplitPartsMax << kSplitPartMax &&
            split_rows_lds(d.bm_rows) <= t.lds_bytes && (reinterpret_cast<uintptr_t>(d.colInd) & 15u) == 0;
 }
@@ -371,15 +371,19 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
     bool rows_ok = want_rows && m && !all_small &&
                    !(G == 1 && split_eligible(t, hd[0], m[0]) && (!t.split_needs_base || split_base));
     for (uint32_t g = 0; g < G && rows_ok; g++)
-        rows_ok = hd[g].mode == kModeTiles && hd[g].w_begin == 0 && hd[g].w_end == UINT64_MAX;
-    uint64_t rows_tiles = 0;
+        rows_ok = hd[g].mode == kModeTiles && hd[g].n <= kSetIdsEnd && hd[g].w_begin == 0 && hd[g].w_end == UINT64_MAX;
+    uint64_t rows_tiles = 0, rows_edges = 0;
+    uint32_t &rg = t.rows_grid[ob == 8 ? 1 : 0];
+    if (rows_ok && !rg) WTC_HIPC(rows_grid(ob, t.num_cus, &rg));
+    for (uint32_t g = 0; g < G && rows_ok; g++) rows_edges += m[g];
+    const uint32_t tile_edges = rows_ok ? rows_tile_edges(rows_edges, rg) : kRowsTile;
     for (uint32_t g = 0; g < G && rows_ok; g++) {
         hd[g].bm_rows = 0;
         hd[g].bm_words = 0;
         hd[g].bitmap = nullptr;
         hd[g].wcount = m[g];
         hd[g].tile_base = rows_tiles;
-        rows_tiles += (m[g] + kRowsTile - 1) / kRowsTile;
+        rows_tiles += (m[g] + tile_edges - 1) / tile_edges;
     }
     // The split count takes a single graph with a bitmap length whose colInd
     // is 16-byte aligned (its slab kernel loads four ids at a time); its top
@@ -474,8 +478,6 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
     const int kernel = t.kernel == kKernelStaged || t.kernel == kKernelRows ? kKernelStaged : kKernelWalk;
     uint32_t &gc = t.grid_cache[kernel == kKernelWalk ? 0 : 1][oi][ways_index(t.ways)][wpb_index(t.wpb)][staged];
     if (!gc && !rows_ok) WTC_HIPC(count_grid(kernel, ob, staged, t.ways, t.wpb, t.num_cus, &gc));
-    uint32_t &rg = t.rows_grid[oi];
-    if (rows_ok && !rg) WTC_HIPC(rows_grid(ob, t.num_cus, &rg));
     s.G = G;
     s.grid = rows_ok ? rg : gc;
     s.split = split;
@@ -500,6 +502,7 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
     plan->by_rows = rows_ok;
     plan->rows_tiles = rows_tiles;
     plan->rows_grid = rg;
+    plan->rows_tile_edges = tile_edges;
     plan->split = split;
     plan->split_off = split_off;
     plan->dense_off = dense_off;
@@ -521,11 +524,10 @@ int launch_set(Slot &s, const SetPlan &p, bool timed, bool desc_ready) {
     GraphDesc *ddesc = s.desc.as<GraphDesc>();
     if (p.by_rows) {
         if (timed) WTC_HIPC(hipEventRecord(s.ev[0], s.stream));
-        WTC_HIPC(launch_rows(desc_ready ? nullptr : s.h_desc.as<uint64_t>(), ddesc, p.G, p.ob, p.rows_tiles, meta, dcounts,
-                             p.rows_grid, s.stream));
+        WTC_HIPC(launch_rows(desc_ready ? nullptr : s.h_desc.as<uint64_t>(), ddesc, p.G, p.ob, p.rows_tiles, p.rows_tile_edges,
+                             meta, dcounts, p.rows_grid, s.stream));
         if (timed) WTC_HIPC(hipEventRecord(s.ev[3], s.stream));
-        WTC_HIPC(hipMemcpyAsync(s.h_out.p, meta, (size_t)(kMetaSlots + p.G) * sizeof(uint64_t), hipMemcpyDeviceToHost,
-                                s.stream));
+        WTC_HIPC(launch_publish(meta, s.h_out.as<uint64_t>(), kMetaSlots + p.G, s.stream));
         return WTC_OK;
     }
     uint64_t *tree = p.single ? s.tree.as<uint64_t>() : nullptr;
@@ -548,8 +550,7 @@ int launch_set(Slot &s, const SetPlan &p, bool timed, bool desc_ready) {
         if (timed) WTC_HIPC(hipEventRecord(s.ev[4], s.stream));
         WTC_HIPC(launch_split_slabs(ddesc, sd, ob, meta, dcounts, s.slabs_grid, s.stream));
         if (timed) WTC_HIPC(hipEventRecord(s.ev[3], s.stream));
-        WTC_HIPC(hipMemcpyAsync(s.h_out.p, meta, (size_t)(kMetaSlots + p.G) * sizeof(uint64_t),
-                                hipMemcpyDeviceToHost, s.stream));
+        WTC_HIPC(launch_publish(meta, s.h_out.as<uint64_t>(), kMetaSlots + p.G, s.stream));
         return WTC_OK;
     }
     if (timed) WTC_HIPC(hipEventRecord(s.ev[0], s.stream));
@@ -565,8 +566,7 @@ int launch_set(Slot &s, const SetPlan &p, bool timed, bool desc_ready) {
                               p.work, s.grid,
                               s.stream));
     if (timed) WTC_HIPC(hipEventRecord(s.ev[3], s.stream));
-    WTC_HIPC(hipMemcpyAsync(s.h_out.p, meta, (size_t)(kMetaSlots + p.G) * sizeof(uint64_t), hipMemcpyDeviceToHost,
-                            s.stream));
+    WTC_HIPC(launch_publish(meta, s.h_out.as<uint64_t>(), kMetaSlots + p.G, s.stream));
     return WTC_OK;
 }
 
@@ -574,14 +574,14 @@ int launch_set(Slot &s, const SetPlan &p, bool timed, bool desc_ready) {
 constexpr uint32_t kRowsFetchMax = 64;
 
 int enqueue_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, const uint64_t *m, const uint64_t *W,
-                char *split_base) {
+                char *split_base, bool timed) {
     SetPlan p;
     int rc = stage_set(s, t, ob, hd, &p, m, W, split_base);
     if (rc) return rc;
     // a row count of few graphs reads its descriptors from the pinned memory
     const bool fetch = p.by_rows && kRowsFetchMax >= p.G;
     if (!fetch) WTC_HIPC(hipMemcpyAsync(s.desc.p, s.h_desc.p, p.desc_bytes, hipMemcpyHostToDevice, s.stream));
-    return launch_set(s, p, true, !fetch);
+    return launch_set(s, p, timed, !fetch);
 }
 
 uint32_t default_small_words() {
@@ -677,11 +677,14 @@ int set_device(int dev) {
 int run_set(wtc_ctx *c, int ob, std::vector<GraphDesc> &hd, uint64_t *counts, wtc_count_stats *st,
             RunTimes *rt_out = nullptr, const uint64_t *m = nullptr, const uint64_t *wedges = nullptr) {
     auto t0 = std::chrono::steady_clock::now();
-    int rc = enqueue_set(c->slot, c->tune, ob, hd, m, wedges);
+    // events between the kernels only for a caller who reads their times: each
+    // holds the next kernel back by some 5 us
+    const bool timed = st || rt_out;
+    int rc = enqueue_set(c->slot, c->tune, ob, hd, m, wedges, nullptr, timed);
     if (rc) return rc;
     RunTimes rt;
     uint64_t W = 0;
-    rc = finish_set(c->slot, counts, &W, &rt);
+    rc = finish_set(c->slot, counts, &W, timed ? &rt : nullptr);
     auto t1 = std::chrono::steady_clock::now();
     if (rc) return rc;
     if (rt_out) *rt_out = rt;
@@ -798,7 +801,7 @@ int tc_gpu_impl(uint32_t n, uint64_t m, const OffT *rowPtr, const uint32_t *colI
     uint64_t cnt = 0;
     RunTimes rt;
     const uint64_t m64 = m;
-    rc = run_set(c, (int)sizeof(OffT), hd, &cnt, nullptr, &rt, &m64);
+    rc = run_set(c, (int)sizeof(OffT), hd, &cnt, nullptr, t ? &rt : nullptr, &m64);
     cleanup();
     if (rc) return rc;
     if (t) {

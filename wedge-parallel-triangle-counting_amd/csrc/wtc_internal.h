@@ -177,6 +177,7 @@ struct SetPlan {
     bool by_rows = false;     // the row count
     uint64_t rows_tiles = 0;
     uint32_t rows_grid = 0;
+    uint32_t rows_tile_edges = 0;
     bool split = false;
     size_t split_off = 0, dense_off = 0;  // bytes of the SplitDesc and DenseDesc
     uint32_t dense_core = 0;              // columns of the dense part's largest class (0: none)
@@ -209,7 +210,7 @@ int launch_set(Slot &s, const SetPlan &p, bool timed, bool desc_ready);
 // into the slot's pinned buffer; returns without waiting.  All graphs of a
 // set share the row-offset width ob.
 int enqueue_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, const uint64_t *m = nullptr,
-                const uint64_t *W = nullptr, char *split_base = nullptr);
+                const uint64_t *W = nullptr, char *split_base = nullptr, bool timed = true);
 // The split count (a single graph with a bitmap length; wtc_split.hip):
 // whether the tuning takes it for a graph, its workspace's device bytes for
 // a graph of n vertices, m edges and `rows` top rows at offset width ob, and

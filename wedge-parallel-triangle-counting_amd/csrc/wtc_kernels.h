@@ -46,7 +46,7 @@ enum : uint32_t {
 constexpr unsigned long long kCountInvalid = ~0ull;
 
 // Edges per tile of the row count (wtc_rows.hip).
-constexpr uint32_t kRowsTile = 512;
+constexpr uint32_t kRowsTile = 512, kRowsTileMin = 256;
 
 // One graph of a graph set.  A graph set is any number of oriented CSRs
 // resident in HBM (ids local to each graph, row offsets relative to the
@@ -127,12 +127,12 @@ constexpr uint32_t kKeyChunk = 4 * kSplitBlock;
 // Slabs of the list rows (middle vertex below thr): slab s holds the rows
 // whose adjacency starts in colInd[s*kSlabSpan, (s+1)*kSlabSpan).  The slab
 // kernel hashes colInd[s*kSlabSpan, +kSlabWin) into LDS, one bucket of
-// kSlabWays slots per position, which covers every such row of out-degree
+// four slots per position, which covers every such row of out-degree
 // <= kSlabRowMax (longer rows are searched in HBM).
 constexpr uint32_t kSlabSpan = 2048;
 constexpr uint32_t kSlabRowMax = 1024;
 constexpr uint32_t kSlabWin = kSlabSpan + kSlabRowMax;
-constexpr uint32_t kSlabWays = 4;
+constexpr uint32_t kSetIdsEnd = 0x7fffffffu;  // the LDS sets of ids (wtc_set.h) hold ids below this
 constexpr uint32_t kSlabLong = 72;  // list tails are streamed by eight lanes where they hold this many ids on average
 constexpr uint32_t kSlabFree = 0x7fffffffu;  // a free slot (ids are below it)
 constexpr uint32_t kSlabMore = 0x80000000u;  // on a bucket's last slot: ids of the bucket are in the next, too

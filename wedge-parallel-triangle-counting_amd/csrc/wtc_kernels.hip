@@ -1281,6 +1281,19 @@ hipError_t launch_prefix(const GraphDesc *desc, uint32_t G, int ob, uint32_t nbl
                           (const uint64_t *)partials);
 }
 
+// The results to the host's pinned memory: a kernel, since a copy of a few
+// words waits several microseconds between the kernels and the host.
+__global__ __launch_bounds__(kBlock) void k_publish(const uint64_t *__restrict__ src, uint64_t *__restrict__ dst,
+                                                    uint32_t words) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < words) dst[i] = src[i];
+}
+
+hipError_t launch_publish(const uint64_t *src, uint64_t *host_dst, uint32_t words, hipStream_t st) {
+    k_publish<<<dim3((words + kBlock - 1) / kBlock), dim3(kBlock), 0, st>>>(src, host_dst, words);
+    return hipGetLastError();
+}
+
 hipError_t launch_setup(GraphDesc *desc, uint32_t G, uint64_t *tree, uint64_t *meta, unsigned long long *counts,
                         hipStream_t st) {
     k_setup<<<dim3(1), dim3(kBlock), 0, st>>>(desc, G, tree, meta, counts);

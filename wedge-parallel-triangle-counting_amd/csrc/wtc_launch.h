@@ -18,6 +18,8 @@ uint32_t prefix_blocks(uint32_t n);
 // partials holds nblocks entries.
 hipError_t launch_prefix(const GraphDesc *desc, uint32_t G, int ob, uint32_t nblocks, uint64_t *partials,
                          hipStream_t st);
+// Copies the results (words of 8 bytes) to the host's pinned memory.
+hipError_t launch_publish(const uint64_t *src, uint64_t *host_dst, uint32_t words, hipStream_t st);
 hipError_t launch_setup(GraphDesc *desc, uint32_t G, uint64_t *tree, uint64_t *meta, unsigned long long *counts,
                         hipStream_t st);
 // Clears every graph's bitmap (clear_words = sum of their word counts, laid
@@ -50,8 +52,11 @@ enum : int { kKernelWalk = 0, kKernelStaged = 1, kKernelSplit = 2, kKernelRows =
 // hold tile_base and wcount (edges); host_desc, when given, is pinned memory
 // the descriptors are read from first.
 hipError_t rows_grid(int ob, int num_cus, uint32_t *grid);
-hipError_t launch_rows(const uint64_t *host_desc, GraphDesc *desc, uint32_t G, int ob, uint64_t tiles, uint64_t *meta,
-                       unsigned long long *counts, uint32_t grid, hipStream_t st);
+// Edges per tile (at most kRowsTile) of a set of `edges` edges.
+uint32_t rows_tile_edges(uint64_t edges, uint32_t grid);
+hipError_t launch_rows(const uint64_t *host_desc, GraphDesc *desc, uint32_t G, int ob, uint64_t tiles,
+                       uint32_t tile_edges, uint64_t *meta, unsigned long long *counts, uint32_t grid,
+                       hipStream_t st);
 // `ways`: independent probes each lane advances together (1, 2, 4 or 8; for
 // k_walk, the steps in flight); `wpb`: waves per block; `staged` = min(max
 // spread, chunk) (k_count's LDS staging).

@@ -297,7 +297,7 @@ bool schedule(wtc_server *s) {
             if (r->split) break;  // alone
         }
         if (hd.empty()) break;
-        const int rc = enqueue_set(x.slot, s->tune, 4, hd, hm.data(), hw.data(), split_base);
+        const int rc = enqueue_set(x.slot, s->tune, 4, hd, hm.data(), hw.data(), split_base, false);
         x.batch_id = ++s->batches;
         for (SrvReq *r : x.reqs) {
             r->batch_graphs = (uint32_t)hd.size();

@@ -44,13 +44,11 @@
 #include "wtc_dev.h"
 #include "wtc_kernels.h"
 #include "wtc_launch.h"
+#include "wtc_set.h"
 
 namespace wtc {
 
 namespace {
-
-// Four ids loaded by one 16-byte load.
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 template <typename OffT>
 struct TailPair {
@@ -1484,50 +1482,6 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *
 
 // ---------------------------------------------------------------- list part
 
-// Bucket of id u in a row's region of `len8 >> 8` buckets: a multiplicative
-// hash of u's low 24 bits, in 24-bit multiplications (32-bit ones take four
-// times as long, and the compiler makes them of a product that it needs the
-// low bits of only).
-__device__ __forceinline__ uint32_t slab_bucket(uint32_t u, uint32_t len8) {
-    uint32_t h, b;
-    asm("v_mul_u32_u24_e32 %0, %1, %2" : "=v"(h) : "s"(0x9e3779u), "v"(u));
-    asm("v_mul_hi_u32_u24_e32 %0, %1, %2" : "=v"(b) : "v"(h), "v"(len8));
-    return b;
-}
-
-// How many of four ids are in the row whose buckets start at st (len of
-// them); the ids from number `left` on are not counted.  Each id's first
-// bucket is read for all four at once, one 16-byte LDS read each; the slots are
-// compared without branches, and only a bucket marked full goes on to the
-// next.
-__device__ __forceinline__ uint32_t slab_hits(const u32x4 *tab4, const uint32_t (&u)[4], uint32_t left, uint32_t st,
-                                              uint32_t len) {
-    uint32_t bk[4], h = 0;
-    u32x4 v[4];
-#pragma unroll
-    for (int z = 0; z < 4; z++) {
-        bk[z] = st + slab_bucket(u[z], len << 8);
-        v[z] = tab4[bk[z]];
-    }
-#pragma unroll
-    for (int z = 0; z < 4; z++) {
-        const bool in = left > (uint32_t)z;
-        const bool f = (v[z][0] == u[z]) | (v[z][1] == u[z]) | (v[z][2] == u[z]) | ((v[z][3] & ~kSlabMore) == u[z]);
-        h += (in & f) ? 1u : 0u;
-        if (in & !f & ((int)v[z][3] < 0)) {
-            uint32_t b2 = bk[z];
-            for (;;) {
-                b2 = b2 + 1 == st + len ? st : b2 + 1;
-                const u32x4 w = tab4[b2];
-                const bool f2 = (w[0] == u[z]) | (w[1] == u[z]) | (w[2] == u[z]) | ((w[3] & ~kSlabMore) == u[z]);
-                h += f2 ? 1u : 0u;
-                if (f2 | ((int)w[3] >= 0)) break;
-            }
-        }
-    }
-    return h;
-}
-
 // Persistent blocks take tiles of the slabs' work from one counter: a slab's
 // work is kSlabCost for its rows and one unit per in-edge, in tiles of at most
 // kSlabTile, as in the row kernel (with tiles of in-edges alone, those over
@@ -1537,12 +1491,12 @@ __device__ __forceinline__ uint32_t slab_hits(const u32x4 *tab4, const uint32_t 
 // into LDS every row of the slab the segment's in-edges name that is not there
 // yet (the table is kept while the next segment stays in the slab; a wave per
 // row clears its buckets and inserts its ids): the row starting at window
-// position st with len entries owns the buckets [st, st + len) of kSlabWays
+// position st with len entries owns the buckets [st, st + len) of kSetWays
 // slots each, so a quarter of its slots are filled; an id whose bucket is full
 // marks it and goes to the next.  Then the segment's in-edges are dealt to the
 // waves, 4 or 8 lanes each, the next step's first ids and the bounds of the
 // one after on their way while this one's tails are streamed and looked up
-// (slab_hits; by a binary search in HBM for a row longer than kSlabRowMax).
+// (set_hits; by a binary search in HBM for a row longer than kSlabRowMax).
 // No one unit is full (R-MAT-26: vector instructions 54%, lines from beyond
 // L2 60%, LDS 37%): bound by the chain of a segment at the 24 waves a CU that
 // the tables leave.  Against a hash by 32-bit multiplications, full buckets
@@ -1557,7 +1511,7 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
                                                                 uint64_t *__restrict__ meta,
                                                                 unsigned long long *__restrict__ counts) {
     constexpr uint32_t kRefWords = kSlabSpan / 32;
-    __shared__ __align__(16) uint32_t s_tab[kSlabWin * kSlabWays];
+    __shared__ __align__(16) uint32_t s_tab[kSlabWin * kSetWays];
     __shared__ uint32_t s_ref[kRefWords];  // rows (by start position) hashed so far
     __shared__ uint32_t s_new[kSlabTile];  // slab_aux words of the rows a segment adds
     __shared__ uint32_t s_nnew;
@@ -1655,17 +1609,10 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
                     const uint32_t nu = lane < naux >> 13 ? colInd[wb + (naux & kSlabAuxLong) + lane] : 0u;
                     const uint32_t st = aux & kSlabAuxLong, len = aux >> 13;
                     for (uint32_t i = lane; i < len; i += kWave)
-                        reinterpret_cast<uint4 *>(s_tab)[st + i] = make_uint4(kSlabFree, kSlabFree, kSlabFree, kSlabFree);
+                        reinterpret_cast<uint4 *>(s_tab)[st + i] = make_uint4(kSetFree, kSetFree, kSetFree, kSetFree);
                     for (uint32_t i = lane; i < len; i += kWave) {
                         if (i >= kWave) u = colInd[wb + st + i];
-                        uint32_t bk = st + slab_bucket(u, len << 8);
-                        for (;;) {
-                            uint32_t z = 0;
-                            while (z < kSlabWays && atomicCAS(&s_tab[bk * kSlabWays + z], kSlabFree, u) != kSlabFree) z++;
-                            if (z < kSlabWays) break;
-                            atomicOr(&s_tab[bk * kSlabWays + kSlabWays - 1], kSlabMore);  // full: on to the next
-                            bk = bk + 1 == st + len ? st : bk + 1;
-                        }
+                        set_insert(s_tab, st, len, u);
                     }
                     aux = naux;
                     u = nu;
@@ -1692,7 +1639,7 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
                         u32x4 b = a;
                         if (left > step) b = *reinterpret_cast<gptr<u32x4>>(p + step);
                         const uint32_t u[4] = {a[0], a[1], a[2], a[3]};
-                        h += slab_hits(reinterpret_cast<const u32x4 *>(s_tab), u, left, st, len);
+                        h += set_hits(s_tab, u, left, st, len);
                         if (left <= step) break;
                         left -= step;
                         p += step;

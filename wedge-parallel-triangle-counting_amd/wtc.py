@@ -581,9 +581,9 @@ class DeviceGraph:
 
     def count(self, spread: int, a: int, w_begin: int = 0, w_end: int = 2 ** 64 - 1, stats: bool = False):
         cnt = C.c_uint64()
-        st = CountStats()
-        _check(_lib.wtc_dgraph_count(self.ctx._p, self._p, spread, a, w_begin, w_end, C.byref(cnt), C.byref(st)),
-               "dgraph_count")
+        st = CountStats() if stats else None  # without: no events between the kernels
+        _check(_lib.wtc_dgraph_count(self.ctx._p, self._p, spread, a, w_begin, w_end, C.byref(cnt),
+                                     C.byref(st) if stats else None), "dgraph_count")
         return (int(cnt.value), st) if stats else int(cnt.value)
 
     def count_baseline(self, parallelism: int, style: int, a: int, stats: bool = False):
