@@ -417,7 +417,7 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
     const size_t dense_off = split_off + sizeof(SplitDesc);
     const size_t desc_bytes = split ? dense_off + sizeof(DenseDesc) : list_bytes;
     WTC_HIPC(s.desc.ensure(desc_bytes));
-    WTC_HIPC(s.out.ensure((size_t)(kMetaSlots + G) * sizeof(uint64_t)));
+    WTC_HIPC(s.out.ensure((size_t)(lines_at(G) + kLines * kLineWords) * sizeof(uint64_t)));
     if (bm_words) WTC_HIPC(s.bm.ensure(bm_words * sizeof(uint32_t)));
     WTC_HIPC(s.h_desc.ensure(desc_bytes));
     WTC_HIPC(s.h_out.ensure((size_t)(kMetaSlots + G) * sizeof(uint64_t)));
@@ -521,13 +521,14 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
 int launch_set(Slot &s, const SetPlan &p, bool timed, bool desc_ready) {
     uint64_t *meta = s.out.as<uint64_t>();
     unsigned long long *dcounts = reinterpret_cast<unsigned long long *>(meta + kMetaSlots);
+    uint64_t *lines = meta + lines_at(p.G);  // used by the row and the split count
     GraphDesc *ddesc = s.desc.as<GraphDesc>();
     if (p.by_rows) {
         if (timed) WTC_HIPC(hipEventRecord(s.ev[0], s.stream));
         WTC_HIPC(launch_rows(desc_ready ? nullptr : s.h_desc.as<uint64_t>(), ddesc, p.G, p.ob, p.rows_tiles, p.rows_tile_edges,
-                             meta, dcounts, p.rows_grid, s.stream));
+                             meta, dcounts, lines, p.rows_grid, s.stream));
         if (timed) WTC_HIPC(hipEventRecord(s.ev[3], s.stream));
-        WTC_HIPC(launch_publish(meta, s.h_out.as<uint64_t>(), kMetaSlots + p.G, s.stream));
+        WTC_HIPC(launch_publish(meta, lines, s.h_out.as<uint64_t>(), kMetaSlots + p.G, s.stream));
         return WTC_OK;
     }
     uint64_t *tree = p.single ? s.tree.as<uint64_t>() : nullptr;
@@ -539,18 +540,18 @@ int launch_set(Slot &s, const SetPlan &p, bool timed, bool desc_ready) {
         WTC_HIPC(launch_split_prefix(ddesc, sd, ob, p.blocks, s.partials.as<uint64_t>(), s.stream));
         WTC_HIPC(launch_split_range(ddesc, sd, ob, s.stream));
         const DenseDesc *dd = reinterpret_cast<const DenseDesc *>(s.desc.as<char>() + p.dense_off);
-        WTC_HIPC(launch_dense_class(ddesc, sd, dd, ob, (uint32_t)(p.split_rp_n - 1), p.blocks, s.partials.as<uint64_t>(), dcounts, s.stream));
+        WTC_HIPC(launch_dense_class(ddesc, sd, dd, ob, (uint32_t)(p.split_rp_n - 1), p.blocks, s.partials.as<uint64_t>(), dcounts,
+                                    lines, s.stream));
         WTC_HIPC(launch_split_inscan(ddesc, sd, p.blocks, s.partials.as<uint64_t>(), s.stream));
         if (timed) WTC_HIPC(hipEventRecord(s.ev[1], s.stream));
-        if (p.dense_core) WTC_HIPC(launch_dense_count(ddesc, dd, ob, p.dense_core, p.num_cus, dcounts, s.stream));
+        if (p.dense_core) WTC_HIPC(launch_dense_count(ddesc, dd, ob, p.dense_core, p.num_cus, lines, s.stream));
         WTC_HIPC(launch_split_transpose(ddesc, sd, dd, ob, p.split_grids, p.split_key_part, meta, s.stream));
         if (timed) WTC_HIPC(hipEventRecord(s.ev[2], s.stream));
-        WTC_HIPC(launch_split_rows(ddesc, sd, ob, p.split_rows, p.split_wpb, meta, dcounts, s.rows_grid,
-                                   s.stream));
+        WTC_HIPC(launch_split_rows(ddesc, sd, ob, p.split_rows, p.split_wpb, lines, s.rows_grid, s.stream));
         if (timed) WTC_HIPC(hipEventRecord(s.ev[4], s.stream));
-        WTC_HIPC(launch_split_slabs(ddesc, sd, ob, meta, dcounts, s.slabs_grid, s.stream));
+        WTC_HIPC(launch_split_slabs(ddesc, sd, ob, meta, lines, s.slabs_grid, s.stream));
         if (timed) WTC_HIPC(hipEventRecord(s.ev[3], s.stream));
-        WTC_HIPC(launch_publish(meta, s.h_out.as<uint64_t>(), kMetaSlots + p.G, s.stream));
+        WTC_HIPC(launch_publish(meta, lines, s.h_out.as<uint64_t>(), kMetaSlots + p.G, s.stream));
         return WTC_OK;
     }
     if (timed) WTC_HIPC(hipEventRecord(s.ev[0], s.stream));
@@ -566,7 +567,7 @@ int launch_set(Slot &s, const SetPlan &p, bool timed, bool desc_ready) {
                               p.work, s.grid,
                               s.stream));
     if (timed) WTC_HIPC(hipEventRecord(s.ev[3], s.stream));
-    WTC_HIPC(launch_publish(meta, s.h_out.as<uint64_t>(), kMetaSlots + p.G, s.stream));
+    WTC_HIPC(launch_publish(meta, nullptr, s.h_out.as<uint64_t>(), kMetaSlots + p.G, s.stream));
     return WTC_OK;
 }
 

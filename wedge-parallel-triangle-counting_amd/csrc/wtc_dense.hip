@@ -71,15 +71,17 @@ __device__ __forceinline__ uint64_t dense_base(const uint32_t *cnt, uint32_t q) 
 
 }  // namespace
 
-// Zeroes the counters of a dense count and the nblocks sums of part_in.
+// Zeroes the counters of a split count and the nblocks sums of part_in.
 __global__ __launch_bounds__(kBlock) void k_dense_init(const DenseDesc *__restrict__ dd, uint64_t *__restrict__ part_in,
-                                                       uint32_t nblocks, unsigned long long *__restrict__ counts) {
+                                                       uint32_t nblocks, unsigned long long *__restrict__ counts,
+                                                       uint64_t *__restrict__ lines) {
     const DenseDesc &N = dd[0];
     for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < nblocks; i += gridDim.x * kBlock) part_in[i] = 0ull;
     if (blockIdx.x != 0) return;
     if (threadIdx.x < kDenseClasses) N.cnt[threadIdx.x] = 0u;
     if (threadIdx.x < kDenseSums) N.sums[threadIdx.x] = 0ull;
     if (threadIdx.x == 0) counts[0] = 0ull;
+    for (uint32_t i = threadIdx.x; i < kLines * kLineWords; i += kBlock) lines[i] = 0ull;
 }
 
 // A thread takes a vertex (the rows worth a class lie together at the last
@@ -336,7 +338,7 @@ __device__ __forceinline__ i32x8 dense_operand_w(uint32_t x) {
 // Counts are exact: the sums are whole numbers up to 2^15 in 32-bit floats, a
 // unit's total per lane below 2^22.
 __global__ __launch_bounds__(kBlock, 2) void k_dense_mm(const DenseDesc *__restrict__ dd,
-                                                        unsigned long long *__restrict__ counts) {
+                                                        uint64_t *__restrict__ lines) {
     const DenseDesc &N = dd[0];
     const uint32_t nq = N.classes, lane = threadIdx.x & (kWave - 1), wv = uni32(threadIdx.x >> 6);
     static_assert(kWavesPerBlock == 4, "a wave per 64 of a unit's 256 core rows");
@@ -493,22 +495,23 @@ __global__ __launch_bounds__(kBlock, 2) void k_dense_mm(const DenseDesc *__restr
         __syncthreads();  // the waves stay near each other, for the cache
     }
     total = wave_sum(total);
-    if (lane == 0 && total) atomicAdd(counts, (unsigned long long)total);
+    if (lane == 0 && total) line_add(lines, kLineHits, total);
 }
 
 // ---------------------------------------------------------------- launches
 
 hipError_t launch_dense_class(const GraphDesc *desc, const SplitDesc *sd, const DenseDesc *dd, int ob, uint32_t n,
-                              uint32_t nblocks, uint64_t *part_in, unsigned long long *counts, hipStream_t st) {
+                              uint32_t nblocks, uint64_t *part_in, unsigned long long *counts, uint64_t *lines,
+                              hipStream_t st) {
     const uint32_t ib = (nblocks + kBlock - 1) / kBlock;
-    k_dense_init<<<dim3(ib < 64 ? ib : 64), dim3(kBlock), 0, st>>>(dd, part_in, nblocks, counts);
+    k_dense_init<<<dim3(ib < 64 ? ib : 64), dim3(kBlock), 0, st>>>(dd, part_in, nblocks, counts, lines);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     return WTC_LAUNCH_OFF(ob, k_dense_class, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, desc, sd, dd, part_in);
 }
 
 hipError_t launch_dense_count(const GraphDesc *desc, const DenseDesc *dd, int ob, uint32_t core, int num_cus,
-                              unsigned long long *counts, hipStream_t st) {
+                              uint64_t *lines, hipStream_t st) {
     const uint32_t cus = (uint32_t)(num_cus > 0 ? num_cus : 1);
     // a block's LDS holds 32 rows: 64 KB for 16,384 columns, 8 KB for 2,048
     constexpr uint32_t kShort = 3;
@@ -521,7 +524,7 @@ hipError_t launch_dense_count(const GraphDesc *desc, const DenseDesc *dd, int ob
         e = WTC_LAUNCH_OFF(ob, k_dense_rows, dim3(cus * per_cu), dim3(kRowsThreads), lds, st, desc, dd, kShort, kDenseClasses, true);
         if (e != hipSuccess) return e;
     }
-    k_dense_mm<<<dim3(cus * 2), dim3(kBlock), 0, st>>>(dd, counts);
+    k_dense_mm<<<dim3(cus * 2), dim3(kBlock), 0, st>>>(dd, lines);
     return hipGetLastError();
 }
 

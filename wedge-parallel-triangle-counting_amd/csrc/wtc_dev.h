@@ -141,6 +141,20 @@ __device__ __forceinline__ uint32_t rightmost_le(P ws, uint32_t lo, uint32_t hi,
     return s - 1;
 }
 
+// Adds x to word `word` of the block's sum line.
+__device__ __forceinline__ void line_add(uint64_t *lines, uint32_t word, uint64_t x) {
+    atomicAdd(reinterpret_cast<unsigned long long *>(&lines[(blockIdx.x % kSumLines) * kLineWords + word]),
+              (unsigned long long)x);
+}
+
+// The next tile of `of` counters at line `first`, for one thread of a block
+// (a counter for each block at most: every one needs blocks).
+__device__ __forceinline__ uint64_t line_tile(uint64_t *lines, uint32_t first, uint32_t of) {
+    of = of < gridDim.x ? of : gridDim.x;
+    const uint32_t c = blockIdx.x % of;
+    return c + of * atomicAdd(reinterpret_cast<unsigned long long *>(&lines[(first + c) * kLineWords]), 1ull);
+}
+
 // Rightmost r in [0, hi] with f(r) <= t for a non-decreasing f with f(0) <=
 // t, by a whole wave: 64 probes a round.
 template <class F>

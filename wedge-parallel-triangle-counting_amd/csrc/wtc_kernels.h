@@ -80,17 +80,14 @@ static_assert(sizeof(GraphDesc) == 128, "GraphDesc layout");
 
 // meta[] slots written by the setup kernel
 // (kMetaNext..kMetaNext+7: per-XCD work counters of the counting kernel).
-// The split count: kMetaRows and kMetaSlabs, tile counters of its row and
-// slab kernels; kMetaTopWedges and kMetaListWedges, the wedges each of them
-// checked; kMetaInEdges, the top rows' in-edges; kMetaAllEdges, every
+// The split count: kMetaTopWedges and kMetaListWedges, the wedges of its row
+// and its slab kernel; kMetaInEdges, the top rows' in-edges; kMetaAllEdges, every
 // grouped in-edge.
 enum : int {
     kMetaTiles = 0,
     kMetaWedges = 1,
-    kMetaRows = 2,
     kMetaTopWedges = 3,
     kMetaInEdges = 4,
-    kMetaSlabs = 5,
     kMetaListWedges = 6,
     kMetaAllEdges = 7,
     kMetaNext = 8,
@@ -99,6 +96,23 @@ enum : int {
     kMetaDenseTopEdges = 9,
     kMetaSlots = 16
 };
+
+// Sums and tile counters that every block adds to.  Atomics to one 128-byte
+// line take 12.1 ns each, one after another, wherever in the line and from
+// however many blocks; to 64 lines 0.3 ns.  With one line for all, the row
+// kernel's 18,432 tile grabs on R-MAT-20 took 0.22 ms of its 0.45 and its
+// 8,192 waves' counts another 0.1.  So they are spread over lines by the block's
+// number and summed when they are read (k_publish), and a block takes its tiles
+// from its line's counter, which holds every kTileLines-th tile.
+constexpr uint32_t kLineWords = 16;                 // 8-byte words of a line
+constexpr uint32_t kSumLines = 64, kTileLines = 16;
+constexpr uint32_t kLineRows = kSumLines, kLineSlabs = kLineRows + kTileLines;  // first tile counters of the two kernels
+constexpr uint32_t kLines = kLineSlabs + kTileLines;
+constexpr uint32_t kLineHits = 0, kLineWedges = 1;  // a sum line's words
+// Where they start behind meta and the counts of G graphs, in words.
+__host__ __device__ constexpr uint32_t lines_at(uint32_t G) {
+    return (kMetaSlots + G + kLineWords - 1) / kLineWords * kLineWords;
+}
 
 // Split count of one graph (wtc_split.hip).  The in-edges are grouped by key
 // in counting-sort levels: by part of 1 << part_shift keys, at most

@@ -1281,16 +1281,27 @@ hipError_t launch_prefix(const GraphDesc *desc, uint32_t G, int ob, uint32_t nbl
                           (const uint64_t *)partials);
 }
 
-// The results to the host's pinned memory: a kernel, since a copy of a few
-// words waits several microseconds between the kernels and the host.
-__global__ __launch_bounds__(kBlock) void k_publish(const uint64_t *__restrict__ src, uint64_t *__restrict__ dst,
-                                                    uint32_t words) {
+// The results (meta, then the counts) to the host's pinned memory, the sum
+// lines, if any, added to the wedges and to the first count: a kernel, since a
+// copy of a few words waits several microseconds between the kernels and the
+// host.
+__global__ __launch_bounds__(kBlock) void k_publish(const uint64_t *__restrict__ src, const uint64_t *__restrict__ lines,
+                                                    uint64_t *__restrict__ dst, uint32_t words) {
+    static_assert(kSumLines == (uint32_t)kWave, "a sum line per lane");
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i < words) dst[i] = src[i];
+    uint64_t x = i < words ? src[i] : 0;
+    if (lines && i < (uint32_t)kWave) {  // the wave that holds meta and the first count
+        static_assert(kMetaSlots < kWave, "meta and a count in the first wave");
+        const uint64_t hits = wave_sum(lines[i * kLineWords + kLineHits]);
+        const uint64_t wedges = wave_sum(lines[i * kLineWords + kLineWedges]);
+        if (i == (uint32_t)kMetaSlots) x += hits;
+        if (i == (uint32_t)kMetaWedges) x += wedges;
+    }
+    if (i < words) dst[i] = x;
 }
 
-hipError_t launch_publish(const uint64_t *src, uint64_t *host_dst, uint32_t words, hipStream_t st) {
-    k_publish<<<dim3((words + kBlock - 1) / kBlock), dim3(kBlock), 0, st>>>(src, host_dst, words);
+hipError_t launch_publish(const uint64_t *src, const uint64_t *lines, uint64_t *host_dst, uint32_t words, hipStream_t st) {
+    k_publish<<<dim3((words + kBlock - 1) / kBlock), dim3(kBlock), 0, st>>>(src, lines, host_dst, words);
     return hipGetLastError();
 }
 

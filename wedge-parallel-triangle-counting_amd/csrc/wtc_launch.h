@@ -18,8 +18,9 @@ uint32_t prefix_blocks(uint32_t n);
 // partials holds nblocks entries.
 hipError_t launch_prefix(const GraphDesc *desc, uint32_t G, int ob, uint32_t nblocks, uint64_t *partials,
                          hipStream_t st);
-// Copies the results (words of 8 bytes) to the host's pinned memory.
-hipError_t launch_publish(const uint64_t *src, uint64_t *host_dst, uint32_t words, hipStream_t st);
+// Copies the results (words of 8 bytes: meta and counts) to the host's pinned
+// memory; lines, when given, are the sum lines that they are completed by.
+hipError_t launch_publish(const uint64_t *src, const uint64_t *lines, uint64_t *host_dst, uint32_t words, hipStream_t st);
 hipError_t launch_setup(GraphDesc *desc, uint32_t G, uint64_t *tree, uint64_t *meta, unsigned long long *counts,
                         hipStream_t st);
 // Clears every graph's bitmap (clear_words = sum of their word counts, laid
@@ -55,7 +56,7 @@ hipError_t rows_grid(int ob, int num_cus, uint32_t *grid);
 // Edges per tile (at most kRowsTile) of a set of `edges` edges.
 uint32_t rows_tile_edges(uint64_t edges, uint32_t grid);
 hipError_t launch_rows(const uint64_t *host_desc, GraphDesc *desc, uint32_t G, int ob, uint64_t tiles,
-                       uint32_t tile_edges, uint64_t *meta, unsigned long long *counts, uint32_t grid,
+                       uint32_t tile_edges, uint64_t *meta, unsigned long long *counts, uint64_t *lines, uint32_t grid,
                        hipStream_t st);
 // `ways`: independent probes each lane advances together (1, 2, 4 or 8; for
 // k_walk, the steps in flight); `wpb`: waves per block; `staged` = min(max
@@ -69,12 +70,13 @@ hipError_t launch_count(int kernel, const GraphDesc *desc, uint32_t G, int ob, c
                         uint32_t work, uint32_t grid, hipStream_t st);
 // Dense part of the split count (wtc_dense.hip): the vertices' classes and
 // the in-edges left to the other kernels (into ie_pre, as counts, and the
-// nblocks sums of part_in); zeroes counts[0].
+// nblocks sums of part_in); zeroes counts[0] and the lines.
 hipError_t launch_dense_class(const GraphDesc *desc, const SplitDesc *sd, const DenseDesc *dd, int ob, uint32_t n,
-                              uint32_t nblocks, uint64_t *part_in, unsigned long long *counts, hipStream_t st);
-// The listed rows' dense wedges added to counts[0].
+                              uint32_t nblocks, uint64_t *part_in, unsigned long long *counts, uint64_t *lines,
+                              hipStream_t st);
+// The listed rows' dense wedges added to the sum lines.
 hipError_t launch_dense_count(const GraphDesc *desc, const DenseDesc *dd, int ob, uint32_t core, int num_cus,
-                              unsigned long long *counts, hipStream_t st);
+                              uint64_t *lines, hipStream_t st);
 // ie_pre from the counts and block sums of launch_dense_class.
 hipError_t launch_split_inscan(const GraphDesc *desc, const SplitDesc *sd, uint32_t nblocks, uint64_t *part_in,
                                hipStream_t st);
@@ -86,7 +88,7 @@ hipError_t launch_split_range(const GraphDesc *desc, SplitDesc *sd, int ob, hipS
 // dst[i] = src[i] for i < count (8-byte row offsets below 2^32 to 4 bytes).
 hipError_t launch_split_narrow_offsets(const uint64_t *src, uint32_t *dst, uint64_t count, hipStream_t st);
 // The counting sort of the in-edges by key (key_part = the SplitDesc's
-// key_part, on the device); zeroes the tile counters and the wedge tallies.
+// key_part, on the device); fills meta.
 struct SplitGrids {
     uint32_t chunks = 0;          // blocks of the first level
     uint32_t c2cap = 0, c3cap = 0;  // bounds of the second and final levels' blocks
@@ -104,11 +106,11 @@ uint32_t split_far_ids(uint32_t rows);
 // Persistent grid of the row kernel for `rows` top rows (its LDS bitmap).
 hipError_t split_rows_grid(int ob, uint32_t rows, int wpb, int num_cus, uint32_t *grid);
 hipError_t launch_split_rows(const GraphDesc *desc, const SplitDesc *sd, int ob, uint32_t rows, int wpb,
-                             uint64_t *meta, unsigned long long *counts, uint32_t grid, hipStream_t st);
+                             uint64_t *lines, uint32_t grid, hipStream_t st);
 // Persistent grid of the slab kernel (the list rows).
 hipError_t split_slabs_grid(int ob, int num_cus, uint32_t *grid);
-hipError_t launch_split_slabs(const GraphDesc *desc, const SplitDesc *sd, int ob, uint64_t *meta,
-                              unsigned long long *counts, uint32_t grid, hipStream_t st);
+hipError_t launch_split_slabs(const GraphDesc *desc, const SplitDesc *sd, int ob, const uint64_t *meta,
+                              uint64_t *lines, uint32_t grid, hipStream_t st);
 // Blocks of the transposition's first level: two per CU (its LDS), and no
 // more than a block per 8192 edges.
 constexpr uint32_t kSplitChunksMax = 512;

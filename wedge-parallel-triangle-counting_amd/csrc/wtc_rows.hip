@@ -50,7 +50,8 @@ constexpr uint32_t kRowsBuckets = kRowsSpread * (kRowsTile + kRowsRowMax);
 // rest of a small graph's count.
 __global__ __launch_bounds__(kBlock) void k_rows_init(const uint64_t *__restrict__ host_desc, GraphDesc *__restrict__ desc,
                                                       uint32_t G, uint64_t *__restrict__ meta,
-                                                      unsigned long long *__restrict__ counts) {
+                                                      unsigned long long *__restrict__ counts,
+                                                      uint64_t *__restrict__ lines) {
     static_assert(sizeof(GraphDesc) % 8 == 0, "copied by words");
     const uint64_t step = (uint64_t)gridDim.x * kBlock, at = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
     if (host_desc)
@@ -58,6 +59,7 @@ __global__ __launch_bounds__(kBlock) void k_rows_init(const uint64_t *__restrict
             reinterpret_cast<uint64_t *>(desc)[i] = host_desc[i];
     for (uint64_t i = at; i < G; i += step) counts[i] = 0ull;
     if (at < kMetaSlots) meta[at] = 0ull;
+    for (uint64_t i = at; i < kLines * kLineWords; i += step) lines[i] = 0ull;
 }
 
 // Groups of `group` consecutive tiles of the set (D.tile_base: a graph's first
@@ -85,8 +87,8 @@ __global__ __launch_bounds__(kBlock) void k_rows_init(const uint64_t *__restrict
 template <typename OffT>
 __global__ __launch_bounds__(kRowsThreads, 6) void k_rows(const GraphDesc *__restrict__ desc, uint32_t G, uint64_t tiles,
                                                        uint32_t group, uint32_t tile_edges,
-                                                       uint64_t *__restrict__ meta,
-                                                       unsigned long long *__restrict__ counts) {
+                                                       unsigned long long *__restrict__ counts,
+                                                       uint64_t *__restrict__ lines) {
     constexpr uint32_t kT = kRowsTile;
     constexpr uint32_t kLists = 4;  // adj+(w) of up to 8, of up to 32 ids, and more; edges of a row not hashed
     __shared__ __align__(16) uint32_t s_tab[kRowsBuckets * 4];
@@ -104,17 +106,24 @@ __global__ __launch_bounds__(kRowsThreads, 6) void k_rows(const GraphDesc *__res
     uint64_t hits = 0, wedges = 0;
     if (threadIdx.x < kT / 64) s_first[1][threadIdx.x] = 0ull;
     if (threadIdx.x < kLists) s_n[1][threadIdx.x] = 0u;
-    // the block's hits of graph cur_g into its count
-    auto flush = [&]() {
-        const uint64_t t = wave_sum(hits);
+    // x summed over the block (thread 0)
+    auto block_sum = [&](uint64_t x) -> uint64_t {
+        const uint64_t t = wave_sum(x);
+        __syncthreads();
         if (lane == 0) s_sum[wv] = t;
         __syncthreads();
-        if (threadIdx.x == 0) {
-            uint64_t all = 0;
+        uint64_t all = 0;
+        if (threadIdx.x == 0)
             for (uint32_t w = 0; w < kRowsWaves; w++) all += s_sum[w];
-            if (all) atomicAdd(&counts[cur_g], (unsigned long long)all);
+        return all;
+    };
+    // the block's hits of graph cur_g into its count
+    auto flush = [&]() {
+        const uint64_t all = block_sum(hits);
+        if (threadIdx.x == 0 && all) {
+            if (G == 1) line_add(lines, kLineHits, all);
+            else atomicAdd(&counts[cur_g], (unsigned long long)all);
         }
-        __syncthreads();
         hits = 0;
     };
     // the current tile: its graph's arrays, positions [p0, p0 + nt) of m
@@ -289,8 +298,8 @@ __global__ __launch_bounds__(kRowsThreads, 6) void k_rows(const GraphDesc *__res
         }
     }
     if (cur_g != kSentinel) flush();  // block-uniform
-    wedges = wave_sum(wedges);
-    if (lane == 0 && wedges) atomicAdd(reinterpret_cast<unsigned long long *>(&meta[kMetaWedges]), (unsigned long long)wedges);
+    wedges = block_sum(wedges);
+    if (threadIdx.x == 0 && wedges) line_add(lines, kLineWedges, wedges);
 }
 
 // ---------------------------------------------------------------- launches
@@ -310,10 +319,11 @@ hipError_t rows_grid(int ob, int num_cus, uint32_t *grid) {
 uint32_t rows_tile_edges(uint64_t edges, uint32_t grid) { return edges <= 256ull * grid ? kRowsTileMin : kRowsTile; }
 
 hipError_t launch_rows(const uint64_t *host_desc, GraphDesc *desc, uint32_t G, int ob, uint64_t tiles, uint32_t tile_edges,
-                       uint64_t *meta, unsigned long long *counts, uint32_t grid, hipStream_t st) {
+                       uint64_t *meta, unsigned long long *counts, uint64_t *lines, uint32_t grid,
+                       hipStream_t st) {
     if (G == 0 || grid == 0) return hipErrorInvalidValue;
     const uint64_t ib = ((uint64_t)G * (sizeof(GraphDesc) / 8) + kBlock - 1) / kBlock;
-    k_rows_init<<<dim3((uint32_t)(ib < 256 ? ib : 256)), dim3(kBlock), 0, st>>>(host_desc, desc, G, meta, counts);
+    k_rows_init<<<dim3((uint32_t)(ib < 256 ? ib : 256)), dim3(kBlock), 0, st>>>(host_desc, desc, G, meta, counts, lines);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || tiles == 0) return e;
     // up to four tiles in a row, with several turns for every block
@@ -321,7 +331,7 @@ hipError_t launch_rows(const uint64_t *host_desc, GraphDesc *desc, uint32_t G, i
     group = group < 1 ? 1 : group > 4 ? 4 : group;
     const uint64_t groups = (tiles + group - 1) / group;
     return WTC_LAUNCH_OFF(ob, k_rows, dim3(groups < grid ? (uint32_t)groups : grid), dim3(kRowsThreads), 0, st, desc, G,
-                          tiles, (uint32_t)group, tile_edges, meta, counts);
+                          tiles, (uint32_t)group, tile_edges, counts, lines);
 }
 
 }  // namespace wtc

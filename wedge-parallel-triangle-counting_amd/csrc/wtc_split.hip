@@ -1051,8 +1051,6 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_keyscan(const SplitDesc *
         const uint64_t all = S.key_part[blockIdx.x] + tot;
         rp[keys] = (OffT)all;
         if (rows >= keys) meta[kMetaInEdges] = all + dense[kDenseTopEdges] + S.cut_top;
-        meta[kMetaRows] = 0;
-        meta[kMetaSlabs] = 0;
         meta[kMetaTopWedges] = S.tally[0] + dense[kDenseTopWedges];
         meta[kMetaDenseTopWedges] = dense[kDenseTopWedges];
         meta[kMetaDenseTopEdges] = dense[kDenseTopEdges];
@@ -1328,8 +1326,7 @@ __device__ __forceinline__ uint32_t rows_tail_hits(const uint32_t *s_bits, gptr<
 template <typename OffT, int kWaves, int kLanes, int kLayout>
 __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *__restrict__ desc,
                                                                const SplitDesc *__restrict__ sd,
-                                                               uint64_t *__restrict__ meta,
-                                                               unsigned long long *__restrict__ counts) {
+                                                               uint64_t *__restrict__ lines) {
     // dynamic LDS only: the row bitmap, then the tile slot
     extern __shared__ uint32_t s_bits[];
     const GraphDesc &D = desc[0];
@@ -1350,9 +1347,12 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *
     // about eight tiles a block, of kSplitTileMinWork to kSplitTile
     uint64_t tile = work / (8ull * gridDim.x);
     tile = tile < kSplitTileMinWork ? kSplitTileMinWork : tile > kSplitTile ? kSplitTile : tile;
+    // short tiles come from sixteen counters (with one, R-MAT-20 0.45 ms instead
+    // of 0.26); full ones, 20 ns apart at the least, from one, which keeps those
+    // in flight closest (R-MAT-24 8.3 ms, two counters 8.6, eight 8.9)
+    const uint32_t of = tile < kSplitTile ? kTileLines : 1u;
     const uint32_t lane = threadIdx.x & (kWave - 1), wv = uni32(threadIdx.x >> 6);
     const uint32_t sub = lane / kLanes, sl = lane % kLanes;
-    unsigned long long *const ctr = reinterpret_cast<unsigned long long *>(meta + kMetaRows);
     uint64_t hits = 0;
     // the tails that the ends of a range cut: searched by one block
     if (blockIdx.x == 0) {
@@ -1376,13 +1376,13 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *
     OffT pb = 0, pe = 0;
     uint32_t held[kHold] = {0, 0};
     auto flip = [&](uint32_t u) { atomicXor(&s_bits[(n - u) >> 5], 1u << ((n - u) & 31u)); };
-    if (threadIdx.x == 0) s_tile = atomicAdd(ctr, 1ull);
+    if (threadIdx.x == 0) s_tile = line_tile(lines, kLineRows, of);
     __syncthreads();
     uint64_t t = uni64(s_tile);
     while (t * tile < work) {  // block-uniform
         const uint64_t t0 = t * tile, t1 = t0 + tile < work ? t0 + tile : work;
         __syncthreads();  // s_tile is read
-        if (threadIdx.x == 0) s_tile = atomicAdd(ctr, 1ull);  // the next tile, read at this one's end
+        if (threadIdx.x == 0) s_tile = line_tile(lines, kLineRows, of);  // the next tile, read at this one's end
         // row r's work is [rp_in[r] + r*kSplitRowCost, rp_in[r + 1] + (r + 1)*kSplitRowCost)
         const uint32_t r0 = wave_rightmost_le(rows - 1, t0, [&](uint32_t r) {
             return (uint64_t)rp_in[r] + (uint64_t)kSplitRowCost * r;
@@ -1477,7 +1477,7 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *
         t = uni64(s_tile);
     }
     hits = wave_sum(hits);
-    if (lane == 0 && hits) atomicAdd(&counts[0], (unsigned long long)hits);
+    if (lane == 0 && hits) line_add(lines, kLineHits, hits);
 }
 
 // ---------------------------------------------------------------- list part
@@ -1508,8 +1508,8 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *
 template <typename OffT, int kWaves>
 __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc *__restrict__ desc,
                                                                 const SplitDesc *__restrict__ sd,
-                                                                uint64_t *__restrict__ meta,
-                                                                unsigned long long *__restrict__ counts) {
+                                                                const uint64_t *__restrict__ meta,
+                                                                uint64_t *__restrict__ lines) {
     constexpr uint32_t kRefWords = kSlabSpan / 32;
     __shared__ __align__(16) uint32_t s_tab[kSlabWin * kSetWays];
     __shared__ uint32_t s_ref[kRefWords];  // rows (by start position) hashed so far
@@ -1527,7 +1527,6 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
     const uint64_t L0 = (uint64_t)rp_in[rows], L1 = (uint64_t)rp_in[keys];
     constexpr uint32_t kThreads = kWave * kWaves;
     const uint32_t lane = threadIdx.x & (kWave - 1), wv = uni32(threadIdx.x >> 6);
-    unsigned long long *const ctr = reinterpret_cast<unsigned long long *>(meta + kMetaSlabs);
     // lanes to a tail: a turn of four takes 16 ids, of eight 32
     const uint32_t lanes = uni64(meta[kMetaListWedges]) > (uint64_t)kSlabLong * (L1 - L0) ? 8u : 4u;
     const uint32_t per = kWave / lanes, deal = kWaves * per, step = 4 * lanes, sub = lane / lanes, sl = lane % lanes;
@@ -1538,7 +1537,7 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
     tile = tile < kSlabTileMin ? kSlabTileMin : tile > kSlabTile ? kSlabTile : tile;
     for (;;) {
         __syncthreads();
-        if (threadIdx.x == 0) s_tile = atomicAdd(ctr, 1ull);
+        if (threadIdx.x == 0) s_tile = line_tile(lines, kLineSlabs, kTileLines);
         __syncthreads();
         const uint64_t t0 = uni64(s_tile) * tile;
         if (t0 >= work || L0 == L1) break;  // block-uniform
@@ -1668,7 +1667,7 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
         }
     }
     hits = wave_sum(hits);
-    if (lane == 0 && hits) atomicAdd(&counts[0], (unsigned long long)hits);
+    if (lane == 0 && hits) line_add(lines, kLineHits, hits);
 }
 
 // ---------------------------------------------------------------- launches
@@ -1840,11 +1839,11 @@ hipError_t split_rows_grid(int ob, uint32_t rows, int wpb, int num_cus, uint32_t
 }
 
 hipError_t launch_split_rows(const GraphDesc *desc, const SplitDesc *sd, int ob, uint32_t rows, int wpb,
-                             uint64_t *meta, unsigned long long *counts, uint32_t grid, hipStream_t st) {
+                             uint64_t *lines, uint32_t grid, hipStream_t st) {
     if (rows == 0) return hipSuccess;
     if (!valid_split_waves(wpb) || grid == 0 || rows > kPackRowsMax) return hipErrorInvalidValue;
     const void *fn = split_rows_kernel(ob, wpb, rows);
-    void *args[] = {&desc, &sd, &meta, &counts};
+    void *args[] = {&desc, &sd, &lines};
     return hipLaunchKernel(fn, dim3(grid), dim3(wpb * kWave), args, split_rows_lds(rows), st);
 }
 
@@ -1866,10 +1865,10 @@ hipError_t split_slabs_grid(int ob, int num_cus, uint32_t *grid) {
     return hipSuccess;
 }
 
-hipError_t launch_split_slabs(const GraphDesc *desc, const SplitDesc *sd, int ob, uint64_t *meta,
-                              unsigned long long *counts, uint32_t grid, hipStream_t st) {
+hipError_t launch_split_slabs(const GraphDesc *desc, const SplitDesc *sd, int ob, const uint64_t *meta,
+                              uint64_t *lines, uint32_t grid, hipStream_t st) {
     if (grid == 0) return hipErrorInvalidValue;
-    void *args[] = {&desc, &sd, &meta, &counts};
+    void *args[] = {&desc, &sd, &meta, &lines};
     return hipLaunchKernel(split_slabs_kernel(ob), dim3(grid), dim3(kSlabWaves * kWave), args, 0, st);
 }
 
