@@ -108,6 +108,43 @@ __device__ __forceinline__ uint64_t block_excl_scan(uint64_t x, uint64_t *s_tot,
     return off + inc - x;
 }
 
+// Exclusive prefix over the kScanChunk values of a block, from `carry` on: in
+// each of four rounds a thread holds four neighbours, x[4 r .. 4 r + 3] being
+// values (r * kBlock + thread) * 4 of the block; one barrier in all (sixteen
+// rounds of one value each took 15 us a block, this 6).  Returns carry and the
+// block's values summed.
+constexpr int kScanRounds = kScanItems / 4;
+__device__ __forceinline__ uint64_t chunk_scan(uint64_t (&x)[kScanItems], uint64_t carry,
+                                               uint64_t (*s_tot)[kWavesPerBlock]) {
+    const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x >> 6;
+    uint64_t sum[kScanRounds], inc[kScanRounds];
+#pragma unroll
+    for (int r = 0; r < kScanRounds; r++) {
+        sum[r] = x[4 * r] + x[4 * r + 1] + x[4 * r + 2] + x[4 * r + 3];
+        inc[r] = wave_incl_scan(sum[r]);
+        if (lane == kWave - 1) s_tot[r][wv] = inc[r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kScanRounds; r++) {
+        uint64_t at = carry + inc[r] - sum[r];
+        for (uint32_t w = 0; w < (uint32_t)kWavesPerBlock; w++) {
+            at += w < wv ? s_tot[r][w] : 0;
+            carry += s_tot[r][w];
+        }
+#pragma unroll
+        for (int z = 0; z < 4; z++) {
+            const uint64_t y = x[4 * r + z];
+            x[4 * r + z] = at;
+            at += y;
+        }
+    }
+    return carry;
+}
+
+// Value 4 r + z of a thread in a chunk_scan, from the block's first.
+__device__ __forceinline__ uint64_t chunk_at(int r, int z) { return ((uint64_t)r * kBlock + threadIdx.x) * 4 + z; }
+
 // Global-memory views of the CSR, prefix and bitmap arrays.  Their pointers
 // are read from descriptors in memory, so without the cast the compiler must
 // treat them as generic addresses: flat loads, which also count against the

@@ -68,15 +68,22 @@ __global__ __launch_bounds__(kBlock) void k_wedge_partials(const GraphDesc *__re
 }
 
 __global__ __launch_bounds__(kBlock) void k_scan_partials(uint64_t *__restrict__ partials, uint32_t nb) {
-    __shared__ uint64_t s_tot[kWavesPerBlock];
+    __shared__ uint64_t s_tot[kScanRounds][kWavesPerBlock];
     uint64_t carry = 0;
-    for (uint32_t base = 0; base < nb; base += kBlock) {
-        const uint32_t i = base + threadIdx.x;
-        const uint64_t x = i < nb ? partials[i] : 0;
-        uint64_t tot;
-        const uint64_t ex = block_excl_scan(x, s_tot, tot);
-        if (i < nb) partials[i] = carry + ex;
-        carry += tot;
+    for (uint64_t base = 0; base < nb; base += kScanChunk) {
+        uint64_t x[kScanItems];
+#pragma unroll
+        for (int i = 0; i < kScanItems; i++) {
+            const uint64_t at = base + chunk_at(i / 4, i % 4);
+            x[i] = at < nb ? partials[at] : 0;
+        }
+        __syncthreads();  // s_tot is read
+        carry = chunk_scan(x, carry, s_tot);
+#pragma unroll
+        for (int i = 0; i < kScanItems; i++) {
+            const uint64_t at = base + chunk_at(i / 4, i % 4);
+            if (at < nb) partials[at] = x[i];
+        }
     }
 }
 

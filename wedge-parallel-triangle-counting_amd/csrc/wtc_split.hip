@@ -103,6 +103,7 @@ __global__ __launch_bounds__(kBlock) void k_split_partials(const GraphDesc *__re
     const uint32_t n = D.n;
     const uint64_t base = (uint64_t)blockIdx.x * kScanChunk;
     uint64_t af = 0;
+#pragma unroll
     for (int k = 0; k < kScanItems; k++) {
         const uint64_t v = base + (uint64_t)k * kBlock + threadIdx.x;
         if (v < n) af += binom2_d((uint64_t)(rowPtr[v + 1] - rowPtr[v]));
@@ -113,51 +114,59 @@ __global__ __launch_bounds__(kBlock) void k_split_partials(const GraphDesc *__re
     if (threadIdx.x == 0) part_full[blockIdx.x] = s_f[0] + s_f[1] + s_f[2] + s_f[3];
 }
 
-// ws_full from the scanned block partials.
+// ws_full from the scanned block partials (n + 1 values: the last is the sum).
 template <typename OffT>
 __global__ __launch_bounds__(kBlock) void k_split_scan(const GraphDesc *__restrict__ desc,
                                                        const SplitDesc *__restrict__ sd,
                                                        const uint64_t *__restrict__ part_full) {
-    __shared__ uint64_t s_tot[kWavesPerBlock];
+    __shared__ uint64_t s_tot[kScanRounds][kWavesPerBlock];
     const GraphDesc &D = desc[0];
-    const OffT *__restrict__ rowPtr = static_cast<const OffT *>(D.rowPtr);
+    const gptr<OffT> rowPtr = to_global(static_cast<const OffT *>(D.rowPtr));
     uint64_t *__restrict__ wf = sd->ws_full;
     const uint32_t n = D.n;
-    uint64_t cf = part_full[blockIdx.x];
     const uint64_t base = (uint64_t)blockIdx.x * kScanChunk;
-    for (int k = 0; k < kScanItems; k++) {
-        if (base + (uint64_t)k * kBlock >= n) break;  // block-uniform
-        const uint64_t v = base + (uint64_t)k * kBlock + threadIdx.x;
-        const uint64_t xf = v < n ? binom2_d((uint64_t)(rowPtr[v + 1] - rowPtr[v])) : 0;
-        uint64_t tf;
-        const uint64_t ef = block_excl_scan(xf, s_tot, tf);
-        if (v < n) {
-            wf[v] = cf + ef;
+    uint64_t x[kScanItems];
+#pragma unroll
+    for (int r = 0; r < kScanRounds; r++) {
+        OffT p[5];
+#pragma unroll
+        for (int z = 0; z <= 4; z++) {
+            const uint64_t v = base + chunk_at(r, z);
+            p[z] = rowPtr[v < n ? v : n];
         }
-        cf += tf;
+#pragma unroll
+        for (int z = 0; z < 4; z++) x[4 * r + z] = binom2_d((uint64_t)(p[z + 1] - p[z]));
     }
-    if (blockIdx.x == (n - 1) / kScanChunk && threadIdx.x == 0) wf[n] = cf;
+    const uint64_t sum = chunk_scan(x, part_full[blockIdx.x], s_tot);
+#pragma unroll
+    for (int i = 0; i < kScanItems; i++) {
+        const uint64_t v = base + chunk_at(i / 4, i % 4);
+        if (v <= n) wf[v] = x[i];
+    }
+    if (base + kScanChunk == n && threadIdx.x == 0) wf[n] = sum;
 }
 
 // ie_pre: its counts of in-edges (k_dense_class) become their prefix.
 __global__ __launch_bounds__(kBlock) void k_split_inscan(const GraphDesc *__restrict__ desc,
                                                          const SplitDesc *__restrict__ sd,
                                                          const uint64_t *__restrict__ part_in) {
-    __shared__ uint64_t s_tot[kWavesPerBlock];
+    __shared__ uint64_t s_tot[kScanRounds][kWavesPerBlock];
     uint64_t *__restrict__ wi = sd->ie_pre;
     const uint32_t n = desc[0].n;
-    uint64_t ci = part_in[blockIdx.x];
     const uint64_t base = (uint64_t)blockIdx.x * kScanChunk;
-    for (int k = 0; k < kScanItems; k++) {
-        if (base + (uint64_t)k * kBlock >= n) break;  // block-uniform
-        const uint64_t v = base + (uint64_t)k * kBlock + threadIdx.x;
-        const uint64_t x = v < n ? wi[v] : 0;
-        uint64_t t;
-        const uint64_t ex = block_excl_scan(x, s_tot, t);
-        if (v < n) wi[v] = ci + ex;
-        ci += t;
+    uint64_t x[kScanItems];
+#pragma unroll
+    for (int i = 0; i < kScanItems; i++) {
+        const uint64_t v = base + chunk_at(i / 4, i % 4);
+        x[i] = v < n ? wi[v] : 0;
     }
-    if (blockIdx.x == (n - 1) / kScanChunk && threadIdx.x == 0) wi[n] = ci;
+    const uint64_t sum = chunk_scan(x, part_in[blockIdx.x], s_tot);
+#pragma unroll
+    for (int i = 0; i < kScanItems; i++) {
+        const uint64_t v = base + chunk_at(i / 4, i % 4);
+        if (v <= n) wi[v] = x[i];
+    }
+    if (base + kScanChunk == n && threadIdx.x == 0) wi[n] = sum;
 }
 
 // Thread 0: the counted range of the full order, its end vertices, and the
@@ -1109,7 +1118,7 @@ struct PackLayout<3> {
     static constexpr bool kAddr = false;
 };
 constexpr uint32_t kPackRowsMax = 1u << 21;
-constexpr uint32_t kPackTile = 8192;  // slots a block packs at a time
+constexpr uint32_t kPackTile = 8192, kPackTileMin = 2048;  // slots a block packs at a time
 constexpr uint32_t kPackGrid = 2048;  // blocks of the packing kernel (eight a CU)
 
 // The layout of a graph with `rows` top rows (rows <= kPackRowsMax).
@@ -1165,7 +1174,7 @@ __device__ __forceinline__ u32x4 pack_chunk(gptr<uint32_t> colInd, uint64_t end,
 }
 
 // Packs the counted rows into S.packed (the memory of the final level's
-// input pairs and slab words).  Blocks take tiles of kPackTile chunk slots in
+// input pairs and slab words).  Blocks take tiles of chunk slots in
 // turn, and the rows with slots in the tile kBlock at a time: a thread finds
 // its row's near ids by a binary search and with them its chunks in the tile,
 // whose prefix over the block deals them out; a thread finds a chunk's row in
@@ -1188,9 +1197,13 @@ __global__ __launch_bounds__(kBlock) void k_split_pack(const GraphDesc *__restri
     const int layout = pack_layout(S.rows);
     const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x >> 6;
     const uint64_t c0 = pack_slot((uint64_t)rowPtr[v_lo]), c1 = pack_slot((uint64_t)rowPtr[(uint64_t)v_hi + 1]);
-    const uint64_t tiles = (c1 - c0 + kPackTile - 1) / kPackTile;
+    // two tiles a block, of kPackTileMin to kPackTile slots (R-MAT-20 43 us; with
+    // 8,192 slots each, for which there are fewer tiles than blocks, 79)
+    uint64_t slots = (c1 - c0) / (2ull * gridDim.x);
+    slots = slots < kPackTileMin ? kPackTileMin : slots > kPackTile ? kPackTile : slots;
+    const uint64_t tiles = (c1 - c0 + slots - 1) / slots;
     for (uint64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        const uint64_t s0 = c0 + tile * kPackTile, s1 = s0 + kPackTile < c1 ? s0 + kPackTile : c1;
+        const uint64_t s0 = c0 + tile * slots, s1 = s0 + slots < c1 ? s0 + slots : c1;
         uint64_t vb = v_lo + wave_rightmost_le(v_hi - v_lo, s0, [&](uint32_t x) { return pack_slot((uint64_t)rowPtr[(uint64_t)v_lo + x]); });
         for (;;) {  // windows of kBlock vertices from vb
             const uint64_t v = vb + threadIdx.x, vn = vb + kBlock;
@@ -1203,8 +1216,8 @@ __global__ __launch_bounds__(kBlock) void k_split_pack(const GraphDesc *__restri
                 c = pack_row<OffT>(rb, re);
                 if (re - rb >= 2 && c < s1 && pack_slot(re) > s0 && colInd[re - 1] > thr) {
                     tail = (uint32_t)(re - rb - 1);
-                    OffT lo = rb + 1, hi = re;  // the first near one of the tail ids
-                    while (lo < hi) {
+                    OffT lo = rb + 1, hi = re;  // the first near one of the tail ids (without far ones: any)
+                    while (layout != 3 && lo < hi) {
                         const OffT mid = lo + ((hi - lo) >> 1);
                         if (colInd[mid] < near_end) lo = mid + 1;
                         else hi = mid;
@@ -1264,7 +1277,9 @@ __global__ __launch_bounds__(kBlock) void k_split_pack(const GraphDesc *__restri
 }
 
 // Lanes per in-edge tail in the row kernel (a wave takes kWave / kSplitLanes
-// in-edges per step), a 16-byte chunk per lane: eight take a line at a time.
+// in-edges per step), a 16-byte chunk per lane: eight take a line at a time
+// (four: R-MAT-19 to 22 0 to 2% less, a quarter of R-MAT-21's wedges 2% and
+// R-MAT-26 1% more).
 constexpr int kSplitLanes = 8;
 
 // The hits of the P packed ids of a chunk.  Every field names a bit of the
@@ -1533,7 +1548,8 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
     uint32_t cur = kSentinel;  // slab in s_tab (block-uniform)
     uint64_t hits = 0;
     const uint64_t work = L1 - L0 + (uint64_t)kSlabCost * (keys - rows);
-    uint64_t tile = work / (8ull * gridDim.x);
+    // about four tiles a block: their chains are long (R-MAT-20 63 us, with eight 79)
+    uint64_t tile = work / (4ull * gridDim.x);
     tile = tile < kSlabTileMin ? kSlabTileMin : tile > kSlabTile ? kSlabTile : tile;
     for (;;) {
         __syncthreads();
