@@ -8,6 +8,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <thread>
 #include <string>
 #include <vector>
 
@@ -757,21 +758,34 @@ int tc_gpu_impl(uint32_t n, uint64_t m, const OffT *rowPtr, const uint32_t *colI
     int rc = check_args(spread, a);
     if (rc) return rc;
     if (!rowPtr || (m && !colInd) || !triangles || n == 0) return WTC_ERR_ARG;
-    // the whole CSR is checked on the host before anything reaches the
-    // device: an id out of range or not above its row, an unsorted row or a
-    // decreasing offset would otherwise become out-of-bounds device accesses
-    if ((rc = validate_oriented_par<OffT>(n, m, rowPtr, colInd))) return rc;
+    // the whole CSR is checked on the host before any kernel reads it: an id out
+    // of range or not above its row, an unsorted row or a decreasing offset
+    // would otherwise become out-of-bounds device accesses.  The check and the
+    // copies, which keep this thread staging, take about as long and run side by
+    // side; what the check finds comes before any error of the device.
+    int bad = WTC_OK;
+    uint64_t wedges = 0;
+    std::thread checker([&] {
+        bad = validate_oriented_par<OffT>(n, m, rowPtr, colInd);
+        if (!bad) wedges = wedge_total_par<OffT>(n, rowPtr);
+    });
+    struct Join {
+        std::thread &t;
+        ~Join() {
+            if (t.joinable()) t.join();
+        }
+    } join{checker};
+    auto checked = [&](int other) -> int {  // the check's error, or else `other`
+        if (checker.joinable()) checker.join();
+        return bad ? bad : other;
+    };
     std::lock_guard<std::mutex> lk(default_ctx_mutex());
     wtc_ctx *c;
-    if ((rc = default_context(&c))) return rc;
-    WTC_HIPC(hipSetDevice(c->device));
-    // the caller's s and a, with the autotuner's kernel and block shape for
-    // the graph's size bucket (unless $WTC_COUNT_KERNEL fixed the kernel)
-    if (c->tune.auto_shape) {
-        wtc_tuned tuned;
-        if (wtc_autotune_shape(n, m, wedge_total_par<OffT>(n, rowPtr), 0, &tuned) == WTC_OK &&
-            (rc = apply_tuned(c, tuned)))
-            return rc;
+    if ((rc = default_context(&c))) return checked(rc);
+    hipError_t e;
+    if ((e = hipSetDevice(c->device)) != hipSuccess) {
+        rc = checked(WTC_OK);
+        return rc ? rc : hip_fail("tc_gpu device", e);
     }
     hipStream_t st = c->slot.stream;
     DevBuf drow, dcol;
@@ -780,21 +794,34 @@ int tc_gpu_impl(uint32_t n, uint64_t m, const OffT *rowPtr, const uint32_t *colI
         drow.release();
         dcol.release();
     };
-    WTC_HIPC(hipEventRecord(c->slot.ev[0], st));
-    hipError_t e;
-    if ((e = drow.ensure(((size_t)n + 1) * sizeof(OffT))) != hipSuccess ||
+    if ((e = hipEventRecord(c->slot.ev[0], st)) != hipSuccess ||
+        (e = drow.ensure(((size_t)n + 1) * sizeof(OffT))) != hipSuccess ||
         (e = dcol.ensure((size_t)std::max<uint64_t>(m, 1) * sizeof(uint32_t))) != hipSuccess ||
         (e = hipMemcpyAsync(drow.p, rowPtr, ((size_t)n + 1) * sizeof(OffT), hipMemcpyHostToDevice, st)) !=
             hipSuccess ||
         (m && (e = hipMemcpyAsync(dcol.p, colInd, (size_t)m * sizeof(uint32_t), hipMemcpyHostToDevice, st)) !=
                   hipSuccess)) {
+        rc = checked(WTC_OK);
+        (void)hipStreamSynchronize(st);
         cleanup();
-        return hip_fail("tc_gpu copy", e);
+        return rc ? rc : hip_fail("tc_gpu copy", e);
     }
     if ((e = hipEventRecord(c->slot.ev[1], st)) != hipSuccess ||
         (e = hipEventSynchronize(c->slot.ev[1])) != hipSuccess) {
+        rc = checked(WTC_OK);
         cleanup();
-        return hip_fail("tc_gpu copy sync", e);
+        return rc ? rc : hip_fail("tc_gpu copy sync", e);
+    }
+    // the caller's s and a, with the autotuner's kernel and block shape for
+    // the graph's size bucket (unless $WTC_COUNT_KERNEL fixed the kernel)
+    rc = checked(WTC_OK);
+    if (!rc && c->tune.auto_shape) {
+        wtc_tuned tuned;
+        if (wtc_autotune_shape(n, m, wedges, 0, &tuned) == WTC_OK) rc = apply_tuned(c, tuned);
+    }
+    if (rc) {
+        cleanup();
+        return rc;
     }
     float copy_ms = 0;
     (void)hipEventElapsedTime(&copy_ms, c->slot.ev[0], c->slot.ev[1]);
