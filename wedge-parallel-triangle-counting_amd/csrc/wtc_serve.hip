@@ -150,12 +150,23 @@ char *pool_ptr(wtc_server *s, size_t off) { return s->pool_mem.as<char>() + off;
 
 size_t req_ws_bytes(const SrvGraph *g) { return ((size_t)g->n + 1) * sizeof(uint64_t); }
 size_t req_bm_bytes(uint32_t a) { return a ? bm_words_for(a) * sizeof(uint32_t) : 0; }
+// Graphs of fewer wedges than this are counted by the row count where the split
+// count's workspace does not fit the budget (R-MAT-18: 0.55 ms instead of 0.35).
+constexpr uint64_t kSplitOrRows = 1ull << 28;
+// What a request needs besides its graph and prefix: the split count's
+// workspace, or a bitmap.
+size_t req_extra_bytes(const SrvGraph *g, uint32_t a, bool split) {
+    return split ? split_workspace_bytes(g->n, g->m, std::min(g->n, a), 4) : req_bm_bytes(a);
+}
+bool req_fits(const wtc_server *s, const SrvGraph *g, uint32_t a, bool split) {
+    return align_up(g->bytes) + align_up(req_ws_bytes(g)) + align_up(req_extra_bytes(g, a, split)) <=
+           s->cfg.hbm_budget_bytes;
+}
 // A request takes the split count when its graph's autotuned kernel is the
-// split count and it asks for a bitmap; its bitmap bytes are then the split
-// workspace (no bitmap in HBM).
-bool req_split(const SrvGraph *g, uint32_t a) { return g->split && a > 0; }
-size_t req_extra_bytes(const SrvGraph *g, uint32_t a) {
-    return req_split(g, a) ? split_workspace_bytes(g->n, g->m, std::min(g->n, a), 4) : req_bm_bytes(a);
+// split count and it asks for a bitmap (which the split count keeps no copy of
+// in HBM).
+bool req_split(const wtc_server *s, const SrvGraph *g, uint32_t a) {
+    return g->split && a > 0 && (g->W >= kSplitOrRows || req_fits(s, g, a, true));
 }
 
 // Frees the CSRs of idle resident graphs, least recently used first, until
@@ -269,7 +280,7 @@ bool schedule(wtc_server *s) {
                 continue;
             }
             r->ws_bytes = req_ws_bytes(g);
-            r->bm_bytes = req_extra_bytes(g, r->a);
+            r->bm_bytes = req_extra_bytes(g, r->a, r->split);
             g->pins++;  // keep the graph while its own workspace is being carved out
             r->ws_off = alloc_evicting(s, r->ws_bytes, r->id);
             r->bm_off = r->bm_bytes && r->ws_off != SIZE_MAX ? alloc_evicting(s, r->bm_bytes, r->id) : SIZE_MAX;
@@ -455,8 +466,8 @@ int wtc_server_submit(wtc_server *s, uint64_t graph_id, uint32_t spread, uint32_
     auto it = s->graphs.find(graph_id);
     if (it == s->graphs.end()) return WTC_ERR_ARG;
     const SrvGraph *g = it->second;
-    if (align_up(g->bytes) + align_up(req_ws_bytes(g)) + align_up(req_extra_bytes(g, a)) > s->cfg.hbm_budget_bytes)
-        return WTC_ERR_ADMIT;
+    const bool split = req_split(s, g, a);
+    if (!req_fits(s, g, a, split)) return WTC_ERR_ADMIT;
     if (s->queue.size() >= s->cfg.queue_capacity) {
         s->stats.rejected++;
         return WTC_ERR_BUSY;
@@ -467,7 +478,7 @@ int wtc_server_submit(wtc_server *s, uint64_t graph_id, uint32_t spread, uint32_
     r->gid = graph_id;
     r->spread = spread;
     r->a = a;
-    r->split = req_split(g, a);
+    r->split = split;
     r->t_submit = Clock::now();
     s->reqs[r->id] = r;
     s->queue.push_back(r);
