@@ -25,11 +25,9 @@ import wtc  # noqa: E402
 HBM_PEAK = 8.0e12  # MI355X HBM3E, bytes/s
 
 
-def split_id_bytes(rows):
-    """Bytes the split count's row kernel reads per tail id: its packed copy
-    of colInd holds P ids per 16-byte chunk, P = 8, 7 or 6 for graphs of at
-    most 2^16, 2^18 or 2^21 top rows (the library's packing layouts)."""
-    return 16.0 / (8 if rows <= 1 << 16 else 7 if rows <= 1 << 18 else 6)
+# The least the split count's row kernel reads per tail id: eight ids among the
+# last 65,528 ranks to a 16-byte chunk (seven or six of the others).
+SPLIT_ID_BYTES = 2.0
 
 
 def log(msg):
@@ -454,8 +452,9 @@ def tune_sweep(args):
         n32 = ((n + 31) // 32) * 32
         alens = [0] + [x for x in (2048, 8192, 32768, 131072, 262144) if x <= n32 and W > 0]
         # bitmap rows past 2^18 only for the split count (one row in LDS, no a*a/8 bytes in HBM);
-        # 65,536 is the largest a whose packed ids take 16 bits
-        split_alens = sorted(set([x for x in alens if x] + [x for x in (65536, 524288, 1048576) if x <= n32 and W > 0]))
+        # 65,504 is the largest a whose packed ids all take 16 bits
+        split_alens = sorted(set([x for x in alens if x] +
+                                 [x for x in (16384, 65504, 524288, 1048576) if x <= n32 and W > 0]))
         best = best_walk = best_staged = None
         base = wtc.Tuned(0, 0, wtc.KERNEL_WALK, 4, 4, 8)
         kernels = (wtc.KERNEL_SPLIT,) if big else (wtc.KERNEL_WALK, wtc.KERNEL_STAGED, wtc.KERNEL_SPLIT,
@@ -769,7 +768,7 @@ def offsets_u64_leg(ctx, g, W, spread, a, steps, warmup, expect):
         # in-edge records of 2*4 B when every position fits 32 bits (the split
         # count then runs on a 4-byte copy of the offsets), else 2*8 B
         rec_bytes = 8.0 if g.m < 0xFFFFFFFF else 16.0
-        dom_bytes = split_id_bytes(min(a, g.n)) * row_w + rec_bytes * row_e
+        dom_bytes = SPLIT_ID_BYTES * row_w + rec_bytes * row_e
         out["kernel_ms"]["split_rows"] = rows_ms
         out["kernel_ms"]["split_slabs"] = statistics.median(s["list_ms"] for s in stats)
         out["roofline"] = {"kernel": "k_split_rows", "achieved": dom_bytes / (rows_ms / 1e3) / 1e9, "unit": "GB/s",
@@ -949,13 +948,13 @@ def main():
     if split:
         # dominant kernel: the split count's row kernel, timed by its own HIP
         # events on the count's stream.  Its algorithmic bytes: the packed id
-        # of every wedge it checks (16/P bytes; each tail id read once; the
+        # of every wedge it checks (two bytes; each tail id read once; the
         # probe itself is an LDS read) and every in-edge's (lo, hi) record of
         # 2*ob bytes
         dom, dom_ms = "k_split_rows", statistics.median(s["rows_ms"] for s in stats)
         dense_w, dense_e = ctx.debug_split()  # counted by the dense part, not the row kernel
         top_w, in_e = stats[-1]["top_wedges"] - dense_w, stats[-1]["in_edges"] - dense_e
-        id_bytes = split_id_bytes(min(args.a, dg.n))
+        id_bytes = SPLIT_ID_BYTES
         dom_bytes = id_bytes * top_w + 2.0 * ob * in_e
         dom_units = {"wedges_checked": top_w, "in_edges": in_e, "bytes_per_wedge": id_bytes,
                      "bytes_per_in_edge": 2 * ob}
