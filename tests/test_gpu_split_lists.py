@@ -40,3 +40,21 @@ def test_interleaved_cliques(gpu_ctx, monkeypatch, count, k, ob, narrow):
     finally:
         dg.free()
         gpu_ctx.set_count_kernel(wtc.KERNEL_WALK)
+
+
+@pytest.mark.parametrize("ob,narrow", [(4, "1"), (8, "0")])
+def test_rows_past_the_longest_hashed(gpu_ctx, monkeypatch, ob, narrow):
+    """A quarter of the rows too long for a hash set: searched, four ids of a
+    tail side by side, with tails of every length and alignment."""
+    monkeypatch.setenv("WTC_SPLIT_NARROW", narrow)
+    count, k = 12, 1400
+    g = _cliques(count, k, 11)
+    expect = count * k * (k - 1) * (k - 2) // 6
+    gpu_ctx.set_count_kernel(wtc.KERNEL_SPLIT)
+    dg = gpu_ctx.upload(g, offset_bytes=ob)
+    try:
+        cnt, st = dg.count(4, 32, stats=True)
+        assert cnt == expect and st.split == 1 and st.list_in_edges > st.in_edges
+    finally:
+        dg.free()
+        gpu_ctx.set_count_kernel(wtc.KERNEL_WALK)

@@ -10,9 +10,10 @@
 //    reference answers from its top-a bitmap (tc.cu:262-272).  One key per
 //    row.  A block of the row kernel holds adj+(w) as a bitmap of a bits in
 //    LDS, and its waves stream the tails of w's in-edges through it from a
-//    packed copy of colInd (ids above thr as 21-bit offsets, six per 16-byte
-//    load).  Each probe is one LDS read, and the top-a bitmap never exists
-//    in HBM: one row of it at a time in LDS instead of a*a/8 bytes.
+//    packed copy of colInd (a row's ids from its top one down, 16 to 21 bits
+//    each, six to eight per 16-byte load).  Each probe is one LDS read, and
+//    the top-a bitmap never exists in HBM: one row of it at a time in LDS
+//    instead of a*a/8 bytes.
 //  * w below thr: the sorted-list probes of tc.cu:273-286.  One key per slab
 //    of colInd (kSlabSpan positions; a row belongs to the slab its adjacency
 //    starts in).  A block of the slab kernel hashes the rows of the slab its
@@ -35,9 +36,9 @@
 // k_split_bases; with many keys k_split_level_count, k_split_levelcols2,
 // k_split_bases and k_split_level_scatter to sub-parts; then
 // k_split_level_count, k_split_levelcols3, k_split_keysum, k_scan_partials,
-// k_split_keyscan and k_split_level_scatter by key; k_split_pack (colInd as
-// ids above thr of 16 to 21 bits, over the last level's input);
-// k_split_rows (top rows); k_split_slabs (list rows).
+// k_split_keyscan and k_split_level_scatter by key; k_split_pack (the
+// packed ids, over the last level's input); k_split_rows (top rows);
+// k_split_slabs (list rows); k_publish (the sums to the host).
 #include <type_traits>
 #include <utility>
 
@@ -1519,6 +1520,9 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *
 // loads not ahead of the tables: R-MAT-26 36.2 -> 27.8 ms, R-MAT-24 2.61 ->
 // 2.08, R-MAT-22 0.43 -> 0.37.  Eight lanes where tails are long: R-MAT-26
 // (~90 ids) 27.8 against 30.1 with four, R-MAT-24 (49 ids) 2.16 against 2.06.
+// Where a is short for the graph, most list wedges name long rows and the
+// searches' chains of loads are the time (R-MAT-26 at a = 65,536: four ids a
+// lane side by side 218 ms, one after the other 308).
 // Same alignment and slack needs as the row kernel.
 template <typename OffT, int kWaves>
 __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc *__restrict__ desc,
@@ -1662,17 +1666,26 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
                     }
                 } else if (len == kSlabAuxLong) {  // a long row: adj+(w) searched in HBM
                     const uint32_t w = colInd[ed.j];
-                    OffT gb = rowPtr[w], ge = rowPtr[(uint64_t)w + 1];
-                    for (q = lo + sl; q < ed.hi; q += (OffT)lanes) {
-                        const uint32_t u = colInd[q];
-                        OffT n_ = ge - gb;
-                        while (n_ > 0) {
+                    OffT gb = rowPtr[w];
+                    const OffT ge = rowPtr[(uint64_t)w + 1];
+                    for (; q < ed.hi; q += (OffT)step) {  // four ids' halvings side by side
+                        const u32x4 a = *reinterpret_cast<gptr<u32x4>>(colInd + q);
+                        OffT at[4] = {gb, gb, gb, gb};  // the last id <= a[z], or the range's first
+                        for (OffT n_ = ge - gb; n_ > 1;) {
                             const OffT half = n_ >> 1;
-                            const bool less = colInd[gb + half] < u;
-                            gb = less ? gb + half + 1 : gb;
-                            n_ = less ? n_ - half - 1 : half;
+                            uint32_t v[4];
+#pragma unroll
+                            for (int z = 0; z < 4; z++) v[z] = colInd[at[z] + half];
+#pragma unroll
+                            for (int z = 0; z < 4; z++) at[z] = v[z] <= a[z] ? at[z] + half : at[z];
+                            n_ -= half;
                         }
-                        h += gb < ge && colInd[gb] == u ? 1u : 0u;  // the lane's next id is larger
+#pragma unroll
+                        for (int z = 0; z < 4; z++) {
+                            const OffT t = q + (OffT)z;
+                            h += t >= lo && t < ed.hi && colInd[at[z]] == a[z] ? 1u : 0u;
+                        }
+                        gb = at[3];  // the lane's next id is larger
                     }
                 }
                 ed = en;
