@@ -487,10 +487,12 @@ def tune_sweep(args):
         split, by_rows = t0.kernel == wtc.KERNEL_SPLIT, t0.kernel == wtc.KERNEL_ROWS
         # stage 2: the block shape of the winner; a split row also keeps the
         # walk's best spread and block shape, which the walk takes where the
-        # split count does not apply (a = 0, a set of graphs), and a rows row
-        # the staged kernel's best spread, bitmap length and block shape, for
-        # wedge ranges
-        walk0 = (best_walk[1] if best_walk else None) if split else best_staged[1] if by_rows else t0
+        # split count does not apply (a = 0, a set of graphs), or the staged
+        # kernel's up to 2^22 edges, whose wedge ranges without a bitmap take
+        # it; and a rows row the staged kernel's best spread, bitmap length
+        # and block shape, for wedge ranges
+        other = best_staged if by_rows or (split and dg.m <= 1 << 22) else best_walk
+        walk0 = (other[1] if other else None) if split or by_rows else t0
         walk_best = None
         if walk0 is not None and not big:  # (graphs built on the GPU: the split count only)
             for waves in (2, 4, 8):

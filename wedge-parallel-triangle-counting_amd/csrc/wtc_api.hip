@@ -336,6 +336,15 @@ bool split_eligible(const Tuning &t, const GraphDesc &d, uint64_t m) {
            split_rows_lds(d.bm_rows) <= t.lds_bytes && (reinterpret_cast<uintptr_t>(d.colInd) & 15u) == 0;
 }
 
+// Without a bitmap (a = 0) the split count has no top rows: the row count
+// takes such a graph up to kNoTopRows edges, the row walk above.  Walk and row
+// count on R-MAT graphs with a = 0: scale 18 6.7 and 0.54 ms, scale 20 (1.57e7
+// edges) 9.4 and 5.1, scale 21 (3.2e7) 17.4 and 16.7, scale 22 42 and 44.
+// Wedge ranges of it go to the staged kernel up to kNoTopStaged edges: a
+// quarter of scale 18 (3.8e6 edges) takes 0.46 ms there; from scale 19 on the
+// walk is as fast or faster (scale 20 1.88 ms against 2.06).
+constexpr uint64_t kNoTopRows = 1ull << 24, kNoTopStaged = 1ull << 22;
+
 int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *plan, const uint64_t *m,
               const uint64_t *W, char *split_base) {
     const uint32_t G = (uint32_t)hd.size();
@@ -368,7 +377,8 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
     }
     // The row count takes whole graphs (every wedge of each); it needs no
     // prefix and no bitmap.
-    const bool want_rows = t.kernel == kKernelRows || (t.rows_else && t.kernel == kKernelSplit);
+    const bool no_top = t.kernel == kKernelSplit && G == 1 && m && hd[0].a == 0 && m[0] <= kNoTopRows;
+    const bool want_rows = t.kernel == kKernelRows || no_top || (t.rows_else && t.kernel == kKernelSplit);
     bool rows_ok = want_rows && m && !all_small &&
                    !(G == 1 && split_eligible(t, hd[0], m[0]) && (!t.split_needs_base || split_base));
     for (uint32_t g = 0; g < G && rows_ok; g++)
@@ -476,7 +486,9 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
     const uint32_t staged = std::min<uint32_t>(max_spread, t.chunk);
     // a set the split count does not take uses the row walk, a range the row
     // count does not take the staged kernel
-    const int kernel = t.kernel == kKernelStaged || t.kernel == kKernelRows ? kKernelStaged : kKernelWalk;
+    const int kernel =
+        t.kernel == kKernelStaged || t.kernel == kKernelRows || (no_top && m[0] <= kNoTopStaged) ? kKernelStaged
+                                                                                                 : kKernelWalk;
     uint32_t &gc = t.grid_cache[kernel == kKernelWalk ? 0 : 1][oi][ways_index(t.ways)][wpb_index(t.wpb)][staged];
     if (!gc && !rows_ok) WTC_HIPC(count_grid(kernel, ob, staged, t.ways, t.wpb, t.num_cus, &gc));
     s.G = G;
