@@ -25,9 +25,16 @@ import wtc  # noqa: E402
 HBM_PEAK = 8.0e12  # MI355X HBM3E, bytes/s
 
 
-# The least the split count's row kernel reads per tail id: eight ids among the
-# last 65,528 ranks to a 16-byte chunk (seven or six of the others).
-SPLIT_ID_BYTES = 2.0
+def split_id_bytes(rows):
+    """Bytes per id of the split count's packed copy of colInd: P ids to a
+    16-byte chunk, P = 8, 7 or 6 for ids among the last 2^16, 2^18 or 2^21
+    ranks (the library's packing layouts)."""
+    return 16.0 / (8 if rows <= 1 << 16 else 7 if rows <= 1 << 18 else 6)
+
+
+# The least the row kernel reads per tail id, whatever the number of top rows:
+# ids among the last ranks are packed at 16 bits in every graph.
+SPLIT_ID_BYTES = split_id_bytes(1 << 16)
 
 
 def log(msg):
@@ -202,8 +209,8 @@ def small_batch_graphs(k, base_seed, n_max):
 def small_kernel_bench(ctx, k, base_seed, reps=7):
     """Kernel choice for sets of small graphs: graph-replay time of one
     resident batch counted by the small-graph kernel (CSR in LDS, one block
-    per slice of a graph) and by the wedge-parallel kernel, for batches of
-    graphs up to n = 512 and n = 1024."""
+    per slice of a graph; taken by contexts on the walk) and by the tuned
+    batch kernel, for batches of graphs up to n = 512 and n = 1024."""
     default, _ = ctx.small_graphs()
     res = {}
     try:
@@ -215,7 +222,10 @@ def small_kernel_bench(ctx, k, base_seed, reps=7):
             row = {"graphs": k, "n_max": n_max, "wedges": int(sum(g.wedges() for g in graphs))}
             counts = {}
             for name, limit in (("small_kernel", default), ("wedge_kernel", 0)):
+                ctx.use_tuned(wtc.autotune_shape(graphs[0].n, graphs[0].m, graphs[0].wedges(), batch=True))
                 ctx.set_small_graphs(limit)
+                if limit:
+                    ctx.set_count_kernel(wtc.KERNEL_WALK)
                 b = wtc.Batch(ctx, graphs)
                 b.count(spread, alen)  # capture
                 ms = []
