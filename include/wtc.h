@@ -250,7 +250,7 @@ int wtc_ctx_set_tuning(wtc_ctx *ctx, int probe_ways, uint32_t lds_chunk, int wav
  *                     closes |adj+(v) and adj+(w)| triangles; the rows of v
  *                     of 512 edges at a time hashed into LDS, adj+(w)
  *                     streamed through them.  No prefix, no bitmap (the
- *                     spread and bitmap length have no effect), two
+ *                     spread and bitmap length have no effect), three
  *                     launches.  Wedge ranges: WTC_KERNEL_STAGED.
  * Default WTC_KERNEL_WALK or $WTC_COUNT_KERNEL. */
 #define WTC_KERNEL_WALK 0

@@ -10,14 +10,15 @@
 // v's set: one 16-byte LDS read an id.  It checks the arrow wedges v -> w -> u
 // (1.2 to 4 times as many as the wedges (w, u) of v, more on skewed graphs),
 // but needs no wedge prefix, no tile search per wedge, no bitmap and no chain
-// of dependent probes: two launches a count, whatever the number of graphs.
+// of dependent probes: three launches a count (descriptors and zeroes, the count,
+// the results), whatever the number of graphs.
 //
 // Measured against the staged kernel on its tuned shape (whole call): R-MAT-12
 // 28 us instead of 146, R-MAT-16 101 instead of 329, R-MAT-18 0.55 ms instead
 // of 0.88, Erdos-Renyi n = 10^6 of degree 16 0.24 ms instead of 0.58, 256
-// Erdos-Renyi and Barabasi-Albert graphs 1.3 ms instead of 2.83.  Past 2^28
-// wedges on skewed graphs the split count is faster (R-MAT-19: 0.73 against
-// 1.7 ms).  Bound by a tile's chain of loads and barriers at the 24 waves a CU
+// Erdos-Renyi and Barabasi-Albert graphs 1.3 ms instead of 2.83.  From 2^27
+// wedges on skewed graphs the split count is faster (R-MAT-18: 0.36 against
+// 0.55 ms, R-MAT-19: 0.50 against 1.7).  Bound by a tile's chain of loads and barriers at the 24 waves a CU
 // that its registers leave, on skewed graphs by a lookup's vector instructions
 // as well.
 #include "wtc_dev.h"
