@@ -773,6 +773,9 @@ int tc_gpu_impl(uint32_t n, uint64_t m, const OffT *rowPtr, const uint32_t *colI
     int rc = check_args(spread, a);
     if (rc) return rc;
     if (!rowPtr || (m && !colInd) || !triangles || n == 0) return WTC_ERR_ARG;
+    // m ids are copied from colInd below while they are checked: first, then,
+    // that the offsets say there are as many
+    if (rowPtr[0] != 0 || (uint64_t)rowPtr[n] != m) return WTC_ERR_CSR;
     // the whole CSR is checked on the host before any kernel reads it: an id out
     // of range or not above its row, an unsorted row or a decreasing offset
     // would otherwise become out-of-bounds device accesses.  The check and the
