@@ -1,6 +1,8 @@
 """The tc_GPU drop-ins on a CSR whose offsets do not fit its edge count: such a
 call is refused from its two end offsets, before colInd, which may be shorter
 than numEdges says, is read and before anything is allocated."""
+import pytest
+
 import fake_gpu
 
 PROGRAM = """
@@ -31,3 +33,44 @@ for wide in (False, True):
 
 def test_offsets_are_checked_before_anything_is_read_or_allocated(tmp_path):
     fake_gpu.run(tmp_path, PROGRAM)
+
+
+THREADS = """
+import resource
+good = wtc.preprocess(wtc.gen_barabasi_albert(40000, 5, seed=903))  # rows for several threads
+bad = wtc.CSR(good.n, good.m, good.row_ptr.copy(), good.col_ind.copy())
+bad.col_ind[-1] = good.n
+assert wtc.tc_gpu_big(good, 5, 64) == 0
+
+
+def refused():
+    try:
+        wtc.tc_gpu_big(bad, 5, 64)
+    except wtc.WtcError as e:
+        return e.code == -10
+
+
+# room for the call's buffers, not for another thread's stack; those that ended
+# threads left behind are in use
+import threading
+ended = threading.Event()
+for _ in range(16):
+    threading.Thread(target=ended.wait, daemon=True).start()
+now = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (now + (3 << 20), -1))
+try:
+    threading.Thread(target=lambda: None).start()
+    raise SystemExit("a thread could be started")
+except RuntimeError:
+    pass
+assert wtc.tc_gpu_big(good, 5, 64) == 0
+assert refused()
+ended.set()
+"""
+
+
+@pytest.mark.parametrize("threads", [1, 4])
+def test_without_a_thread_to_check_on(tmp_path, threads):
+    """Where no thread can be started the check runs on the calling thread: no
+    exception leaves the C entry, and none ends the process."""
+    fake_gpu.run(tmp_path, THREADS, {"WTC_HOST_THREADS": str(threads)})

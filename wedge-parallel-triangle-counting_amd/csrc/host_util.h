@@ -7,6 +7,7 @@
 #include <atomic>
 #include <cstdint>
 #include <cstdlib>
+#include <exception>
 #include <new>
 #include <thread>
 #include <vector>
@@ -43,8 +44,11 @@ void par_chunks(uint64_t n, uint64_t chunk, F &&f) {
         return;
     }
     std::vector<std::thread> th;
-    th.reserve(nt - 1);
-    for (int t = 1; t < nt; t++) th.emplace_back(body, t);
+    try {
+        th.reserve(nt - 1);
+        for (int t = 1; t < nt; t++) th.emplace_back(body, t);
+    } catch (const std::exception &) {  // the threads there are, and this one, do all of it
+    }
     body(0);
     for (auto &t : th) t.join();
 }

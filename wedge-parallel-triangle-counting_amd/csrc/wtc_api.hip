@@ -7,6 +7,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <thread>
 #include <string>
@@ -780,13 +781,20 @@ int tc_gpu_impl(uint32_t n, uint64_t m, const OffT *rowPtr, const uint32_t *colI
     // of range or not above its row, an unsorted row or a decreasing offset
     // would otherwise become out-of-bounds device accesses.  The check and the
     // copies, which keep this thread staging, take about as long and run side by
-    // side; what the check finds comes before any error of the device.
+    // side (where no thread can be started, one after the other); what the
+    // check finds comes before any error of the device.
     int bad = WTC_OK;
     uint64_t wedges = 0;
-    std::thread checker([&] {
+    auto check = [&] {
         bad = validate_oriented_par<OffT>(n, m, rowPtr, colInd);
         if (!bad) wedges = wedge_total_par<OffT>(n, rowPtr);
-    });
+    };
+    std::thread checker;
+    try {
+        checker = std::thread([&] { check(); });
+    } catch (const std::exception &) {
+        check();
+    }
     struct Join {
         std::thread &t;
         ~Join() {
