@@ -285,10 +285,13 @@ __global__ __launch_bounds__(kRowsThreads) void k_dense_rows(const GraphDesc *__
         __syncthreads();
         for (uint32_t k = 0; k < kRows; k++) {
             const OffT rb0 = (OffT)readlane_u64((uint64_t)b, k), re = (OffT)readlane_u64((uint64_t)e, k);
-            for (OffT j = rb0 + lane; j < re; j += 8 * kWave) {  // eight loads in flight
+            // by the number of the id in the row: a position past a row's end
+            // may pass 2^32
+            const uint32_t len = (uint32_t)(re - rb0);
+            for (uint32_t i = lane; i < len; i += 8 * kWave) {  // eight loads in flight
                 uint32_t u[8];
 #pragma unroll
-                for (uint32_t z = 0; z < 8; z++) u[z] = j + (OffT)(z * kWave) < re ? colInd[j + (OffT)(z * kWave)] : kSentinel;
+                for (uint32_t z = 0; z < 8; z++) u[z] = i + z * kWave < len ? colInd[rb0 + (OffT)(i + z * kWave)] : kSentinel;
 #pragma unroll
                 for (uint32_t z = 0; z < 8; z++) {
                     if (u[z] == kSentinel) continue;

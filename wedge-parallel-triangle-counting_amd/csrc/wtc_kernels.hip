@@ -207,9 +207,9 @@ __global__ __launch_bounds__(kBlock) void k_bitmap_build(const GraphDesc *__rest
         uint32_t *__restrict__ bm = D.bitmap;
         const uint32_t v = D.n - D.bm_rows + (uint32_t)(r - D.row_base);
         const uint32_t a32 = D.a >> 5;
-        const OffT b = rowPtr[v], e = rowPtr[v + 1];
-        for (OffT j0 = b; j0 < e; j0 += kWave) {  // wave-uniform
-            const OffT j = j0 + lane;
+        const uint64_t b = rowPtr[v], e = rowPtr[v + 1];
+        for (uint64_t j0 = b; j0 < e; j0 += kWave) {  // wave-uniform
+            const uint64_t j = j0 + lane;
             uint64_t word = ~0ull;  // no lane's word: inactive lanes never match
             uint32_t acc = 0;
             if (j < e) {

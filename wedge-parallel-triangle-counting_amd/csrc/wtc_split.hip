@@ -1338,9 +1338,10 @@ __device__ __forceinline__ uint32_t rows_tail_hits(const uint32_t *s_bits, gptr<
 // chunk loaded before this one is counted, and the next in-edges' bounds
 // before these are streamed.  A row's ids are loaded while the row before is
 // streamed; its bits go in as the other row's go out, all by exclusive or,
-// so a row takes two barriers.
+// so a row takes two barriers.  With 4-byte offsets held to 64 registers (it
+// takes 65 by itself), for eight waves a SIMD.
 template <typename OffT, int kWaves, int kLanes, int kLayout>
-__global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *__restrict__ desc,
+__global__ __launch_bounds__(kWave * kWaves, (sizeof(OffT) == 4 ? 8 : 7)) void k_split_rows(const GraphDesc *__restrict__ desc,
                                                                const SplitDesc *__restrict__ sd,
                                                                uint64_t *__restrict__ lines) {
     // dynamic LDS only: the row bitmap, then the tile slot
@@ -1388,8 +1389,11 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *
             }
         }
     }
-    // the row in the bitmap: adj+ = colInd[pb, pe), its first ids in held[]
-    OffT pb = 0, pe = 0;
+    // the row in the bitmap: the pl ids of adj+ from colInd[pb] on, its first
+    // ones in held[] (ids by their number in the row: a position past a row's
+    // end may pass 2^32)
+    OffT pb = 0;
+    uint32_t pl = 0;
     uint32_t held[kHold] = {0, 0};
     auto flip = [&](uint32_t u) { atomicXor(&s_bits[(n - u) >> 5], 1u << ((n - u) & 31u)); };
     if (threadIdx.x == 0) s_tile = line_tile(lines, kLineRows, of);
@@ -1407,21 +1411,22 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *
         static_assert(kSplitTile / kSplitRowCost + 2 < kWave, "a tile's rows fit a wave");
         const uint32_t rl = r0 + lane < rows ? r0 + lane : rows;
         const OffT my_in = rp_in[rl], my_adj = rowPtr[(uint64_t)thr + rl];
-        // the tile's in-edges [ka, kz) and adjacency [ab, ae) of row r0 + x
-        auto row_bounds = [&](uint32_t x, uint64_t &ka, uint64_t &kz, OffT &ab, OffT &ae) {
+        // the tile's in-edges [ka, kz) and adjacency, al ids from ab on, of row r0 + x
+        auto row_bounds = [&](uint32_t x, uint64_t &ka, uint64_t &kz, OffT &ab, uint32_t &al) {
             const uint64_t b = readlane_u64((uint64_t)my_in, x), e = readlane_u64((uint64_t)my_in, x + 1);
             const uint64_t c = (uint64_t)kSplitRowCost * (r0 + x + 1);
             ka = t0 > b + c ? t0 - c : b;
             kz = t1 < e + c ? (t1 > b + c ? t1 - c : b) : e;
             ab = (OffT)readlane_u64((uint64_t)my_adj, x);
-            ae = (OffT)readlane_u64((uint64_t)my_adj, x + 1);
+            al = (uint32_t)((OffT)readlane_u64((uint64_t)my_adj, x + 1) - ab);
         };
         // the next row from x on with in-edges in the tile, or kSentinel
         auto next_row = [&](uint32_t x) -> uint32_t {
             for (; r0 + x < rows; x++) {
                 uint64_t ka, kz;
-                OffT ab, ae;
-                row_bounds(x, ka, kz, ab, ae);
+                OffT b;
+                uint32_t l;
+                row_bounds(x, ka, kz, b, l);
                 if ((uint64_t)readlane_u64((uint64_t)my_in, x) + (uint64_t)kSplitRowCost * (r0 + x) >= t1) break;
                 if (ka < kz) return x;
             }
@@ -1429,39 +1434,39 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_rows(const GraphDesc *
         };
         uint32_t x = next_row(0);
         uint64_t k = 0, kend = 0;
-        OffT ab = 0, ae = 0;
-        uint32_t ids[kHold] = {0, 0};
+        OffT ab = 0;
+        uint32_t al = 0, ids[kHold] = {0, 0};
         if (x != kSentinel) {
-            row_bounds(x, k, kend, ab, ae);
+            row_bounds(x, k, kend, ab, al);
 #pragma unroll
             for (uint32_t z = 0; z < kHold; z++) {
-                const OffT i = ab + threadIdx.x + z * kThreads;
-                if (i < ae) ids[z] = colInd[i];
+                const uint32_t i = threadIdx.x + z * kThreads;
+                if (i < al) ids[z] = colInd[ab + (OffT)i];
             }
         }
         while (x != kSentinel) {  // block-uniform
             // this row's bits in, the row before's out
 #pragma unroll
             for (uint32_t z = 0; z < kHold; z++) {
-                if (pb + threadIdx.x + z * kThreads < pe) flip(held[z]);
-                if (ab + threadIdx.x + z * kThreads < ae) flip(ids[z]);
+                if (threadIdx.x + z * kThreads < pl) flip(held[z]);
+                if (threadIdx.x + z * kThreads < al) flip(ids[z]);
                 held[z] = ids[z];
             }
-            for (OffT i = pb + threadIdx.x + kHold * kThreads; i < pe; i += kThreads) flip(colInd[i]);
-            for (OffT i = ab + threadIdx.x + kHold * kThreads; i < ae; i += kThreads) flip(colInd[i]);
+            for (uint32_t i = threadIdx.x + kHold * kThreads; i < pl; i += kThreads) flip(colInd[pb + (OffT)i]);
+            for (uint32_t i = threadIdx.x + kHold * kThreads; i < al; i += kThreads) flip(colInd[ab + (OffT)i]);
             pb = ab;
-            pe = ae;
+            pl = al;
             const uint64_t ck = k, ckend = kend;
             const bool far = rows - (r0 + x) > kPackNear;  // the row's tails have far ids
             __syncthreads();
             // the next row's ids, on their way while this row is streamed
             x = next_row(x + 1);
             if (x != kSentinel) {
-                row_bounds(x, k, kend, ab, ae);
+                row_bounds(x, k, kend, ab, al);
 #pragma unroll
                 for (uint32_t z = 0; z < kHold; z++) {
-                    const OffT i = ab + threadIdx.x + z * kThreads;
-                    if (i < ae) ids[z] = colInd[i];
+                    const uint32_t i = threadIdx.x + z * kThreads;
+                    if (i < al) ids[z] = colInd[ab + (OffT)i];
                 }
             }
             uint32_t h = 0;
@@ -1581,7 +1586,11 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
             struct Edge {
                 OffT j, hi;
                 uint32_t aux;
-                __device__ __forceinline__ OffT first(uint32_t l) const { return ((j + 1) & ~(OffT)3) + 4 * l; }
+                // the tail from the aligned position at or before it: its
+                // first position and what is from there to its end (positions
+                // by what is left: one past the tail may pass 2^32)
+                __device__ __forceinline__ OffT base() const { return (j + 1) & ~(OffT)3; }
+                __device__ __forceinline__ uint32_t span() const { return (uint32_t)(hi - base()); }
                 __device__ __forceinline__ bool hashed() const { return (aux >> 13) != 0 && (aux >> 13) != kSlabAuxLong; }
             };
             auto edge = [&](uint64_t x) -> Edge {
@@ -1594,9 +1603,8 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
                 return e;
             };
             auto head = [&](const Edge &e) -> u32x4 {
-                const OffT q = e.first(sl);
                 u32x4 r = {0u, 0u, 0u, 0u};
-                if (e.hashed() && q < e.hi) r = *reinterpret_cast<gptr<u32x4>>(colInd + q);
+                if (e.hashed() && 4 * sl < e.span()) r = *reinterpret_cast<gptr<u32x4>>(colInd + e.base() + 4 * sl);
                 return r;
             };
             uint64_t x0 = k + (uint64_t)wv * per + sub;
@@ -1643,17 +1651,17 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
                 const Edge e2 = edge(x0 + 2 * deal);
                 const u32x4 nids = head(en);
                 const uint32_t st = ed.aux & kSlabAuxLong, len = ed.aux >> 13;
-                const OffT lo = ed.j + 1;
-                OffT q = ed.first(sl);
-                if (ed.hashed() && q < ed.hi) {
-                    uint32_t left = (uint32_t)(ed.hi - q);
+                const bool some = 4 * sl < ed.span();  // this lane's share of the tail
+                uint32_t left = some ? ed.span() - 4 * sl : 0u;
+                const uint32_t skip = sl == 0 ? (uint32_t)(ed.j + 1 - ed.base()) : 0u;  // ids before the tail
+                gptr<uint32_t> p = colInd + ed.base() + 4 * sl;
+                if (ed.hashed() && some) {
                     u32x4 a = ids;
-                    if (q < lo) {  // ids before the tail: 0 is in no row
+                    if (skip) {  // 0 is in no row
                         a[0] = 0u;
-                        a[1] = lo - q > 1 ? 0u : a[1];
-                        a[2] = lo - q > 2 ? 0u : a[2];
+                        a[1] = skip > 1 ? 0u : a[1];
+                        a[2] = skip > 2 ? 0u : a[2];
                     }
-                    gptr<uint32_t> p = colInd + q;
                     for (;;) {
                         u32x4 b = a;
                         if (left > step) b = *reinterpret_cast<gptr<u32x4>>(p + step);
@@ -1668,8 +1676,8 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
                     const uint32_t w = colInd[ed.j];
                     OffT gb = rowPtr[w];
                     const OffT ge = rowPtr[(uint64_t)w + 1];
-                    for (; q < ed.hi; q += (OffT)step) {  // four ids' halvings side by side
-                        const u32x4 a = *reinterpret_cast<gptr<u32x4>>(colInd + q);
+                    for (uint32_t before = skip; left; before = 0) {  // four ids' halvings side by side
+                        const u32x4 a = *reinterpret_cast<gptr<u32x4>>(p);
                         OffT at[4] = {gb, gb, gb, gb};  // the last id <= a[z], or the range's first
                         for (OffT n_ = ge - gb; n_ > 1;) {
                             const OffT half = n_ >> 1;
@@ -1681,11 +1689,11 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
                             n_ -= half;
                         }
 #pragma unroll
-                        for (int z = 0; z < 4; z++) {
-                            const OffT t = q + (OffT)z;
-                            h += t >= lo && t < ed.hi && colInd[at[z]] == a[z] ? 1u : 0u;
-                        }
+                        for (uint32_t z = 0; z < 4; z++)
+                            h += z >= before && z < left && colInd[at[z]] == a[z] ? 1u : 0u;
                         gb = at[3];  // the lane's next id is larger
+                        left = left > step ? left - step : 0u;
+                        p += step;
                     }
                 }
                 ed = en;
