@@ -7,18 +7,28 @@
 // (tc.cu:203-287).  A block takes a tile of kRowsTile consecutive positions
 // of colInd (edges), hashes the rows of v that they lie in into LDS, streams
 // adj+(w) for each of its edges with 16-byte loads, and looks every id up in
-// v's set: one 16-byte LDS read an id.  It checks the arrow wedges v -> w -> u
-// (1.2 to 4 times as many as the wedges (w, u) of v, more on skewed graphs),
-// but needs no wedge prefix, no tile search per wedge, no bitmap and no chain
-// of dependent probes: three launches a count (descriptors and zeroes, the count,
-// the results), whatever the number of graphs.
+// v's set: one 16-byte LDS read an id.  These are the arrow wedges v -> w -> u
+// (counted on R-MAT, Erdos-Renyi and Barabasi-Albert graphs 1.2 to 4 times as
+// many as the wedges (w, u) of v), with no wedge prefix, no tile search per
+// wedge, no bitmap and no chain of dependent probes: three launches a count
+// (descriptors and zeroes, the count, the results), whatever the number of
+// graphs.
+//
+// Nothing bounds the arrow wedges by the wedges: where many vertices of few
+// neighbours hang on a dense core there are ten to sixty times as many.  So an
+// edge whose adj+(w) is long beside what is left of v's row (kRowsLong,
+// kRowsFew) is done the other way round: the rest of v's row is searched in
+// adj+(w).  What is streamed is then at most kRowsLong ids an edge and kRowsFew
+// a wedge.  1,000 vertices all joined with 10^7 of two neighbours among them:
+// 7.6 ms streamed, 0.77 so, 0.84 by the staged kernel; 400 with 2 * 10^6: 0.49,
+// 0.18 and 0.34; R-MAT-16 102 -> 96 us, R-MAT-18 0.52 -> 0.48 ms.
 //
 // Measured against the staged kernel on its tuned shape (whole call): R-MAT-12
-// 28 us instead of 146, R-MAT-16 101 instead of 329, R-MAT-18 0.55 ms instead
-// of 0.88, Erdos-Renyi n = 10^6 of degree 16 0.24 ms instead of 0.58, 256
+// 28 us instead of 146, R-MAT-16 96 instead of 329, R-MAT-18 0.48 ms instead
+// of 0.88, Erdos-Renyi n = 10^6 of degree 16 0.21 ms instead of 0.58, 256
 // Erdos-Renyi and Barabasi-Albert graphs 1.3 ms instead of 2.83.  From 2^27
 // wedges on skewed graphs the split count is faster (R-MAT-18: 0.36 against
-// 0.55 ms, R-MAT-19: 0.50 against 1.7).  Bound by a tile's chain of loads and barriers at the 24 waves a CU
+// 0.48 ms, R-MAT-19: 0.50 against 1.7).  Bound by a tile's chain of loads and barriers at the 24 waves a CU
 // that its registers leave, on skewed graphs by a lookup's vector instructions
 // as well.
 #include "wtc_dev.h"
@@ -36,13 +46,22 @@ typedef uint32_t u32x4_e __attribute__((ext_vector_type(4), aligned(4)));
 constexpr int kRowsThreads = 512;
 static_assert(kRowsThreads == (int)kRowsTile, "a position per thread");
 constexpr uint32_t kRowsWaves = kRowsThreads / kWave;
-// Longest row (from its first position in the tile) hashed; the ids of a
-// longer one are searched in memory.
-constexpr uint32_t kRowsRowMax = 512;
 // Buckets of four slots per position: one bucket in 6,000 is left by an id
 // that finds it full.
 constexpr uint32_t kRowsSpread = 2;
-constexpr uint32_t kRowsBuckets = kRowsSpread * (kRowsTile + kRowsRowMax);
+// The table has that many for the tile and a last row of as many positions; a
+// longer last row gets what is left.
+constexpr uint32_t kRowsBuckets = kRowsSpread * 2 * kRowsTile;
+// Longest row (from its first position in the tile) hashed, two ids a bucket
+// at most; what is longer is searched in memory.  (With 512, two graphs of
+// 1,000 vertices all joined took 1.91 ms, the staged kernel 1.65; so 0.30.)
+constexpr uint32_t kRowsRowMax = 2048;
+static_assert(4 * (kRowsBuckets - kRowsSpread * (kRowsTile - 1)) > kRowsRowMax, "the longest row hashed leaves slots free");
+// An edge's adj+(w) of kRowsLong ids or more is not streamed where it has
+// kRowsFew times the ids of the rest of v's row or more: those are searched in
+// it.  (kRowsFew 8: R-MAT-18 0.54 ms, 16 and 32 0.48 and 0.49, R-MAT-16 97 and
+// 99 us; kRowsLong 128 or 256: within 1%, R-MAT-17 3% more.)
+constexpr uint32_t kRowsLong = 64, kRowsFew = 16;
 
 }  // namespace
 
@@ -77,7 +96,8 @@ __global__ __launch_bounds__(kBlock) void k_rows_init(const uint64_t *__restrict
 //     step, so that a long one takes many steps and little of them is empty
 //     (with up to 32 lanes: R-MAT-16 117 against 112 us, the serving mix 2.77
 //     against 2.65 ms); the next step's ids load while this one's are looked
-//     up.
+//     up.  The edges to be searched go to the last waves first, which have the
+//     least to stream (R-MAT-12 27.8 us, dealt from the first wave on 28.7).
 // The next tile's rows, ids and bounds of adj+(w) load while a tile is
 // streamed.  Three barriers a tile (with a running maximum over marks, a clear
 // of the table by the rows' extent and lists packed by a prefix, seven:
@@ -91,7 +111,9 @@ __global__ __launch_bounds__(kRowsThreads, 6) void k_rows(const GraphDesc *__res
                                                        unsigned long long *__restrict__ counts,
                                                        uint64_t *__restrict__ lines) {
     constexpr uint32_t kT = kRowsTile;
-    constexpr uint32_t kLists = 4;  // adj+(w) of up to 8, of up to 32 ids, and more; edges of a row not hashed
+    // adj+(w) of up to 8, of up to 32 ids, and more; the rest of v's row to be
+    // searched in it; edges of a row not hashed
+    constexpr uint32_t kStreams = 3, kSearch = kStreams, kUnhashed = kStreams + 1, kLists = kStreams + 2;
     __shared__ __align__(16) uint32_t s_tab[kRowsBuckets * 4];
     __shared__ OffT s_ws[kT];        // start of adj+(w)
     __shared__ uint32_t s_wl[kT];    // its length
@@ -218,6 +240,11 @@ __global__ __launch_bounds__(kRowsThreads, 6) void k_rows(const GraphDesc *__res
             // without it if it is too long (only the last row can be: a row
             // that ends in the tile has at most kT positions there)
             static_assert(kRowsRowMax >= kT, "a row ending in the tile is hashed");
+            // a row's region of the table: its first bucket, its buckets above 16 bits
+            auto region = [&](uint32_t st, uint32_t end) -> uint32_t {
+                constexpr uint32_t kEnd = kRowsBuckets / kRowsSpread;
+                return kRowsSpread * (st | ((end < kEnd ? end : kEnd) - st) << 16);
+            };
             const uint32_t st_last = uni32(row_at(nt - 1)), end_last = uni32(s_end[st_last]);
             const bool long_last = end_last - st_last > kRowsRowMax;
             const uint32_t bl = long_last ? st_last : end_last;
@@ -225,23 +252,30 @@ __global__ __launch_bounds__(kRowsThreads, 6) void k_rows(const GraphDesc *__res
             if (me < nt) {
                 const uint32_t st = row_at(me), end = s_end[st];
                 s_mark[me] = (uint16_t)st;
-                const uint64_t len = (uint64_t)(we - ws);
+                const uint32_t len = (uint32_t)(we - ws);  // < n
                 if (len != 0 && me + 1 != end) {  // else nothing to stream, or nothing after w in v's row
                     s_ws[me] = ws;
-                    s_wl[me] = (uint32_t)len;  // < n
-                    const uint32_t c = long_last && st == st_last ? kLists - 1 : len <= 8 ? 0u : len <= 32 ? 1u : 2u;
+                    s_wl[me] = len;
+                    uint32_t c = len <= 8 ? 0u : len <= 32 ? 1u : 2u;
+                    if (len >= kRowsLong) c = len >= kRowsFew * (end - me - 1) ? kSearch : c;
+                    c = long_last && st == st_last ? kUnhashed : c;
                     s_list[c][atomicAdd(&s_n[buf][c], 1u)] = (uint16_t)me;
                 }
-                if (me < bl) set_insert(s_tab, kRowsSpread * st, kRowsSpread * (end - st), id);
+                if (me < bl) {
+                    const uint32_t r = region(st, end);
+                    set_insert(s_tab, r & 0xffffu, r >> 16, id);
+                }
             }
-            for (uint32_t i = nt + threadIdx.x; i < bl; i += kRowsThreads)
-                set_insert(s_tab, kRowsSpread * st_last, kRowsSpread * (end_last - st_last), colInd[p0 + i]);
+            for (uint32_t i = nt + threadIdx.x; i < bl; i += kRowsThreads) {
+                const uint32_t r = region(st_last, end_last);
+                set_insert(s_tab, r & 0xffffu, r >> 16, colInd[p0 + i]);
+            }
             __syncthreads();
             const uint64_t cp0 = p0;
             p0 += tile_edges;
             if (tile + 1 < t1 && tile + 1 < g_end) load(p0, vb);
             uint32_t h = 0;
-            for (uint32_t c = 0; c + 1 < kLists; c++) {  // list c: 2 << c lanes an edge, four ids each a step
+            for (uint32_t c = 0; c < kStreams; c++) {  // list c: 2 << c lanes an edge, four ids each a step
                 const uint32_t lanes = 2u << c, o = 4 * (lane & (lanes - 1)), end = uni32(s_n[buf][c]);
                 uint32_t x = threadIdx.x >> (c + 1);
                 // the step ahead: ids of row st at `at` of the wl from ws
@@ -253,7 +287,7 @@ __global__ __launch_bounds__(kRowsThreads, 6) void k_rows(const GraphDesc *__res
                     from = s_ws[i];
                     wl = s_wl[i];
                     const uint32_t st = s_mark[i];
-                    set = kRowsSpread * (st | (s_end[st] - st) << 16);
+                    set = region(st, s_end[st]);
                     at = o;
                 };
                 auto ids = [&]() { q = *reinterpret_cast<gptr<u32x4_e>>(colInd + from + (at < wl ? at : 0u)); };
@@ -276,23 +310,46 @@ __global__ __launch_bounds__(kRowsThreads, 6) void k_rows(const GraphDesc *__res
                     h += set_hits(s_tab, hi, left > 2 ? left - 2 : 0u, cfirst, clen);
                 }
             }
-            const uint32_t rest = uni32(s_n[buf][kLists - 1]);
+            // four lanes an edge, two ids each a step, their halvings side by side
+            if (uni32(s_n[buf][kSearch])) {
+                for (uint32_t x = (kRowsThreads - 1 - threadIdx.x) >> 2; x < uni32(s_n[buf][kSearch]); x += kRowsThreads >> 2) {
+                    const uint32_t i = s_list[kSearch][x], wl = s_wl[i], end = s_end[s_mark[i]];
+                    const OffT from = s_ws[i];
+                    for (uint32_t q = i + 1 + (lane & 3u); q < end; q += 8) {
+                        const uint32_t y0 = colInd[cp0 + q], y1 = q + 4 < end ? colInd[cp0 + q + 4] : y0;
+                        OffT at0 = from, at1 = from;  // the last id <= y, or the first id
+                        for (uint32_t k = wl; k > 1;) {
+                            const uint32_t half = k >> 1;
+                            const uint32_t v0 = colInd[at0 + half], v1 = colInd[at1 + half];
+                            at0 = v0 <= y0 ? at0 + half : at0;
+                            at1 = v1 <= y1 ? at1 + half : at1;
+                            k -= half;
+                        }
+                        h += colInd[at0] == y0 ? 1u : 0u;
+                        h += q + 4 < end && colInd[at1] == y1 ? 1u : 0u;
+                    }
+                }
+            }
+            const uint32_t rest = uni32(s_n[buf][kUnhashed]);
             uint64_t end = 0;
             if (rest) {  // block-uniform: the last row is not hashed
                 const uint32_t r = wave_rightmost_le(n - 1, cp0 + st_last, [&](uint32_t y) { return (uint64_t)rowPtr[y]; });
                 end = rowPtr[(uint64_t)r + 1];
             }
-            for (uint32_t x = wv; x < rest; x += kRowsWaves) {  // searched in v's row after w
-                const uint32_t i = s_list[kLists - 1][x], wl = s_wl[i];
-                for (uint32_t at = lane; at < wl; at += kWave) {
-                    const uint32_t y = colInd[s_ws[i] + at];
-                    uint64_t lo = cp0 + i + 1, hi = end;
+            for (uint32_t x = wv; x < rest; x += kRowsWaves) {  // adj+(w) and v's row after w: the shorter in the longer
+                const uint32_t i = s_list[kUnhashed][x];
+                const uint64_t w0 = s_ws[i], v0 = cp0 + i + 1, wl = s_wl[i], vl = end - v0;
+                const uint64_t from = wl < vl ? w0 : v0, in = wl < vl ? v0 : w0;
+                const uint64_t ids = wl < vl ? wl : vl, top = in + (wl < vl ? vl : wl);
+                for (uint64_t at = lane; at < ids; at += kWave) {
+                    const uint32_t y = colInd[from + at];
+                    uint64_t lo = in, hi = top;
                     while (lo < hi) {
                         const uint64_t mid = lo + ((hi - lo) >> 1);
                         if (colInd[mid] < y) lo = mid + 1;
                         else hi = mid;
                     }
-                    h += lo < end && colInd[lo] == y ? 1u : 0u;
+                    h += lo < top && colInd[lo] == y ? 1u : 0u;
                 }
             }
             hits += h;
