@@ -338,13 +338,13 @@ bool split_eligible(const Tuning &t, const GraphDesc &d, uint64_t m) {
 }
 
 // Without a bitmap (a = 0) the split count has no top rows: the row count
-// takes such a graph up to kNoTopRows edges, the row walk above.  Walk and row
-// count on R-MAT graphs with a = 0: scale 18 6.7 and 0.54 ms, scale 20 (1.57e7
-// edges) 9.4 and 5.1, scale 21 (3.2e7) 17.4 and 16.7, scale 22 42 and 44.
+// takes such a graph, as in the server.  Walk and row count on R-MAT graphs
+// with a = 0: scale 18 6.7 and 0.48 ms, scale 20 7.9 and 3.0, scale 22 42 and
+// 18, scale 23 108 and 48, scale 24 280 and 127, scale 25 729 and 353.
 // Wedge ranges of it go to the staged kernel up to kNoTopStaged edges: a
 // quarter of scale 18 (3.8e6 edges) takes 0.46 ms there; from scale 19 on the
 // walk is as fast or faster (scale 20 1.88 ms against 2.06).
-constexpr uint64_t kNoTopRows = 1ull << 24, kNoTopStaged = 1ull << 22;
+constexpr uint64_t kNoTopStaged = 1ull << 22;
 
 int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *plan, const uint64_t *m,
               const uint64_t *W, char *split_base) {
@@ -352,7 +352,7 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
     if (G == 0) return WTC_ERR_ARG;
     // The row count takes whole graphs (every wedge of each); it needs no
     // prefix and no bitmap.
-    const bool no_top = t.kernel == kKernelSplit && G == 1 && m && hd[0].a == 0 && m[0] <= kNoTopRows;
+    const bool no_top = t.kernel == kKernelSplit && G == 1 && m && hd[0].a == 0;
     const bool want_rows = t.kernel == kKernelRows || no_top || (t.rows_else && t.kernel == kKernelSplit);
     // Kernel choice per set: a set of two or more graphs that all fit the
     // small-graph limit is counted by the small-graph kernel (one block per
