@@ -274,10 +274,13 @@ int wtc_ctx_set_work_split(wtc_ctx *ctx, uint32_t tiles_per_grab, int deal_to_xc
  * two or more graphs (a batch, a serving batch) in which every graph has
  * 2(n+1) + m <= max_words is done by the small-graph kernel: one block per
  * graph holds the graph's CSR and wedge prefix in LDS.  Any other set is
- * done by the wedge-parallel kernel.  0 turns the small-graph kernel off.
+ * done by the context's counting kernel.  0 turns the small-graph kernel off.
  * max_words may not exceed the device's LDS per block in words
  * (device_max_words; 40960 on MI355X).  Default 20480 or
- * $WTC_SMALL_GRAPH_WORDS.  Counts do not depend on it. */
+ * $WTC_SMALL_GRAPH_WORDS.  Where the row count is the counting kernel
+ * (WTC_KERNEL_ROWS, which the autotuner takes for batches, and the server), it
+ * is the faster one for small sets too and takes them unless the limit has
+ * been set, by this call or by that variable.  Counts do not depend on it. */
 int wtc_ctx_set_small_graphs(wtc_ctx *ctx, uint32_t max_words);
 int wtc_ctx_get_small_graphs(const wtc_ctx *ctx, uint32_t *max_words, uint32_t *device_max_words);
 
@@ -403,11 +406,15 @@ typedef struct {
     uint32_t max_batch;        /* graphs per batch (default 256)                  */
     uint32_t slots;            /* batches in flight (default 2, at most 8)        */
     uint32_t queue_capacity;   /* queued requests before WTC_ERR_BUSY (65536)     */
-    int32_t probe_ways;        /* counting-kernel tuning, 0 = default             */
-    uint32_t lds_chunk;        /* counting-kernel tuning, 0 = default             */
-    int32_t waves_per_block;   /* counting block: 1, 2, 4 or 8 waves, 0 = 4       */
-    int32_t small_graph_words; /* small-graph kernel limit (wtc_ctx_set_small_graphs):
-                                  0 = default, -1 = off, else the limit in words */
+    /* Tuning of the row walk, which the server takes for what neither the split
+       count nor the row count does: graphs of more than 2^31 - 1 vertices. */
+    int32_t probe_ways;        /* 0 = default                                     */
+    uint32_t lds_chunk;        /* 0 = default                                     */
+    int32_t waves_per_block;   /* 1, 2, 4 or 8 waves, 0 = 4                       */
+    int32_t small_graph_words; /* sets of graphs up to this many words by the small-graph
+                                  kernel (wtc_ctx_set_small_graphs); 0 = as
+                                  $WTC_SMALL_GRAPH_WORDS says, without it by the row
+                                  count, as -1                                    */
 } wtc_server_config;
 typedef struct {
     double queue_ms;      /* submit -> batch start                                */

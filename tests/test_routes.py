@@ -41,3 +41,59 @@ for n, k in ((20000, 420), (60000, 420)):  # 8.3 and 25 million edges
     assert ran(ks, "k_walk") and not ran(ks, "k_rows"), (n, ks)
 srv.close()
 """)
+
+
+SMALL = BAND + """
+graphs = [band(60 + i, 7) for i in range(4)]
+
+
+def batches(ctx):
+    b = wtc.Batch(ctx, graphs)
+    yield launches(lambda: b.count([8] * 4, [0] * 4))
+    yield launches(lambda: wtc.batch_count_host(ctx, graphs, [8] * 4, [0] * 4))
+
+
+def serves(words, kernel):
+    "Whether a served set of two graphs or more is counted by the kernel: no request alone is a set."
+    srv = wtc.Server(hbm_budget_bytes=1 << 28, small_graph_words=words)
+    gids = [srv.register(g) for g in graphs]
+    seen = False
+    for _ in range(300):
+        def burst():
+            sets = [srv.wait(r)[1].batch_graphs for r in [srv.submit(g, 8, 0) for g in gids * 16]]
+            assert len(sets) == 64
+        seen = seen or ran(launches(burst), kernel)
+        if seen:
+            break
+    srv.close()
+    return seen
+"""
+
+
+def test_small_graph_limit_is_kept_where_it_is_set(tmp_path):
+    """Sets of small graphs go to the row count where it is the chosen kernel,
+    but to the small-graph kernel where the caller has set its limit."""
+    fake_gpu.run(tmp_path, SMALL + """
+ctx = wtc.Context(0)
+ctx.use_tuned(wtc.autotune_shape(graphs[0].n, graphs[0].m, graphs[0].wedges(), batch=True))
+for limit, small in ((None, False), (20480, True), (0, False), (500, False), (40960, True)):
+    if limit is not None:
+        ctx.set_small_graphs(limit)
+    for ks in batches(ctx):
+        assert ran(ks, "k_count_small") == small and ran(ks, "k_rows") != small, (limit, ks)
+# a batch kept by the program follows the setting, at the limit's own default, too
+ctx = wtc.Context(0)
+ctx.use_tuned(wtc.autotune_shape(graphs[0].n, graphs[0].m, graphs[0].wedges(), batch=True))
+b = wtc.Batch(ctx, graphs)
+assert ran(launches(lambda: b.count([8] * 4, [0] * 4)), "k_rows")
+ctx.set_small_graphs(ctx.small_graphs()[0])
+assert ran(launches(lambda: b.count([8] * 4, [0] * 4)), "k_count_small")
+assert serves(20480, "k_count_small")
+assert serves(0, "k_rows") and serves(-1, "k_rows")
+""")
+    fake_gpu.run(tmp_path, SMALL + """
+ctx = wtc.Context(0)
+ctx.use_tuned(wtc.autotune_shape(graphs[0].n, graphs[0].m, graphs[0].wedges(), batch=True))
+assert all(ran(ks, "k_count_small") for ks in batches(ctx))
+assert serves(0, "k_count_small")
+""", {"WTC_SMALL_GRAPH_WORDS": "20480"})

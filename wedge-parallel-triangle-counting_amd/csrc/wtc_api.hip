@@ -36,6 +36,7 @@ struct wtc_batch {
     int key_ways = 0, key_wpb = 0, key_kernel = 0;
     uint32_t key_work = 0;
     uint32_t key_chunk = 0, key_small = 0;
+    bool key_asked = false;
 };
 
 namespace wtc {
@@ -359,13 +360,14 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
     // graph, CSR in LDS, so no bitmap); any other set by the wedge-parallel
     // kernel.  Mixing the two in one set runs them back to back, and the
     // small kernel's per-graph tail then costs more than it saves.
-    // Where the row count is the choice it takes small sets as well: replays
+    // Where the row count is the choice it takes small sets as well, unless the
+    // caller has set the limit himself: replays
     // of 4,096 graphs of n <= 512 in 0.178 ms against 0.251, of n <= 1024 in
     // 0.273 against 0.401.
     uint32_t small_words = 0, small_n = 0;
     uint64_t small_parts = 0;
     const uint32_t small_cap = std::min(t.small_words, t.small_words_max);
-    bool all_small = m && W && G >= 2 && small_cap > 0 && !want_rows;
+    bool all_small = m && W && G >= 2 && small_cap > 0 && (!want_rows || t.small_asked);
     for (uint32_t g = 0; g < G && all_small; g++)
         all_small = hd[g].n > 0 && 2 * ((uint64_t)hd[g].n + 1) + m[g] <= small_cap;
     for (uint32_t g = 0; g < G; g++) {
@@ -608,6 +610,8 @@ uint32_t default_small_words() {
     const long v = std::atol(e);
     return v < 0 ? 0u : (uint32_t)std::min<long>(v, kSmallWordsMax);
 }
+
+bool small_words_asked() { return std::getenv("WTC_SMALL_GRAPH_WORDS") != nullptr; }
 
 int init_small_graphs(Tuning &t, const hipDeviceProp_t &prop, uint32_t want) {
     t.lds_bytes = prop.sharedMemPerBlock;
@@ -898,6 +902,7 @@ int wtc_ctx_create(int device, wtc_ctx **out) {
     c->tune.ways = default_probe_ways();
     c->tune.wpb = default_count_waves();
     c->tune.kernel = default_count_kernel();
+    c->tune.small_asked = small_words_asked();
     if ((rc = init_small_graphs(c->tune, prop, default_small_words()))) {
         delete c;
         return rc;
@@ -913,6 +918,7 @@ int wtc_ctx_create(int device, wtc_ctx **out) {
 int wtc_ctx_set_small_graphs(wtc_ctx *c, uint32_t max_words) {
     if (!c || max_words > c->tune.small_words_max) return WTC_ERR_ARG;
     c->tune.small_words = max_words;
+    c->tune.small_asked = true;
     return WTC_OK;
 }
 
@@ -1336,6 +1342,7 @@ int batch_capture(wtc_ctx *c, wtc_batch *b, const std::vector<uint32_t> &s, cons
     b->key_work = count_work(c->tune.grab_for(c->tune.kernel), c->tune.deal);
     b->key_chunk = c->tune.chunk;
     b->key_small = c->tune.small_words;
+    b->key_asked = c->tune.small_asked;
     return WTC_OK;
 }
 
@@ -1467,7 +1474,7 @@ int wtc_batch_count(wtc_ctx *c, wtc_batch *b, const uint32_t *spread, const uint
     if (rc) return rc;
     if (!b->exec || s != b->key_s || aa != b->key_a || c->tune.ways != b->key_ways || c->tune.wpb != b->key_wpb || c->tune.kernel != b->key_kernel ||
         count_work(c->tune.grab_for(c->tune.kernel), c->tune.deal) != b->key_work ||
-        c->tune.chunk != b->key_chunk || c->tune.small_words != b->key_small) {
+        c->tune.chunk != b->key_chunk || c->tune.small_words != b->key_small || c->tune.small_asked != b->key_asked) {
         if ((rc = batch_capture(c, b, s, aa))) return rc;
     }
     Slot &sl = b->slot;

@@ -125,6 +125,9 @@ struct Tuning {
     // kSmallWordsMax).
     uint32_t small_words = 0;
     uint32_t small_words_max = 0;
+    // the caller set small_words: such sets go to that kernel where the row
+    // count is the choice, too
+    bool small_asked = false;
     // LDS per block in bytes: the split count's row bitmap (a bits) must fit
     size_t lds_bytes = 0;
     uint32_t grid_cache[2][2][4][4][kChunkMax + 2] = {};  // by kernel, offset width, ways, waves, staged
@@ -140,6 +143,7 @@ struct Tuning {
 // (2(n+1) + m): $WTC_SMALL_GRAPH_WORDS, else kSmallWordsDefault.
 constexpr uint32_t kSmallWordsDefault = 20480;
 uint32_t default_small_words();
+bool small_words_asked();  // by $WTC_SMALL_GRAPH_WORDS
 // Sets the tuning's small-graph limits for a device (want clamped to its
 // LDS per block) and raises the kernel's dynamic-LDS limit to match.
 int init_small_graphs(Tuning &t, const hipDeviceProp_t &prop, uint32_t want);

@@ -387,12 +387,14 @@ int wtc_server_create(int device, const wtc_server_config *cfg, wtc_server **out
     s->tune.wpb = s->cfg.waves_per_block;
     // a request whose graph the autotuner counts by the split count runs
     // alone with its workspace from the pool, any other set by the row count
+    // (of small graphs by their kernel if the configuration says up to which size)
     s->tune.kernel = kKernelSplit;
     s->tune.split_needs_base = true;
     s->tune.rows_else = true;
     int rc = init_small_graphs(s->tune, prop, s->cfg.small_graph_words < 0    ? 0u
                                               : s->cfg.small_graph_words == 0 ? default_small_words()
                                                                               : (uint32_t)s->cfg.small_graph_words);
+    s->tune.small_asked = s->cfg.small_graph_words > 0 || (s->cfg.small_graph_words == 0 && small_words_asked());
     if (!rc && s->cfg.small_graph_words > 0 && (uint32_t)s->cfg.small_graph_words > s->tune.small_words_max)
         rc = WTC_ERR_ARG;
     if (rc) {
