@@ -210,7 +210,9 @@ __global__ __launch_bounds__(kRowsThreads, 6) void k_rows(const GraphDesc *__res
                 reinterpret_cast<uint4 *>(s_tab)[i] = make_uint4(kSetFree, kSetFree, kSetFree, kSetFree);
             if (threadIdx.x < kT / 64) s_first[buf ^ 1][threadIdx.x] = 0ull;
             if (threadIdx.x < kLists) s_n[buf ^ 1][threadIdx.x] = 0u;
-            for (;;) {  // windows of rows up to the one holding the tile's last position
+            // windows of rows up to the one holding the tile's last position, or
+            // kRowWindows of them and the rows of the positions left
+            for (uint32_t win = 1;; win++) {
                 const uint64_t a = ra, z = rz;
                 if (z > a && z > p0 && a < p0 + nt) {
                     const uint32_t at = a > p0 ? (uint32_t)(a - p0) : 0u;
@@ -218,13 +220,27 @@ __global__ __launch_bounds__(kRowsThreads, 6) void k_rows(const GraphDesc *__res
                     s_end[at] = z - p0 < 0xffffull ? (uint16_t)(z - p0) : (uint16_t)0xffffu;
                     if (a >= p0) wedges += binom2_d(z - a);
                 }
+                if (win > kRowWindows) break;
                 const uint64_t vn = vb + kRowsThreads;
-                if (vn >= n || (uint64_t)rowPtr[vn] >= p0 + nt) break;  // block-uniform
-                vb = vn;
+                if (vn >= n) break;  // block-uniform
+                const uint64_t next = rowPtr[vn];
+                if (next >= p0 + nt) break;  // block-uniform
                 ra = rz = 0;
-                if (vb + threadIdx.x < n) {
-                    ra = rowPtr[vb + threadIdx.x];
-                    rz = rowPtr[vb + threadIdx.x + 1];
+                if (win < kRowWindows) {
+                    vb = vn;
+                    if (vb + threadIdx.x < n) {
+                        ra = rowPtr[vb + threadIdx.x];
+                        rz = rowPtr[vb + threadIdx.x + 1];
+                    }
+                } else {  // block-uniform
+                    const uint64_t q = p0 + threadIdx.x;
+                    if (threadIdx.x < nt && q >= next) {
+                        const uint32_t r = rightmost_le(rowPtr, (uint32_t)vn, n - 1, q);
+                        ra = rowPtr[r];
+                        rz = (uint64_t)ra == q ? rowPtr[(uint64_t)r + 1] : ra;
+                    }
+                    vb = vn + wave_rightmost_le((uint32_t)(n - 1 - vn), p0 + nt - 1,
+                                                [&](uint32_t r) { return (uint64_t)rowPtr[vn + r]; });
                 }
             }
             __syncthreads();

@@ -499,7 +499,13 @@ __global__ __launch_bounds__(kSplitBlock, 8) void k_split_l1(const GraphDesc *__
         if (threadIdx.x < kSplitPartsMax) s_cnt[threadIdx.x] = 0u;
         if (threadIdx.x == 0) s_open = 0;
         __syncthreads();
-        for (;;) {  // windows of kSplitBlock vertices from vb, up to the one holding t1 - 1
+        auto owner = [&](uint32_t at, OffT rb, OffT re) {  // of in-edge slot `at` and on
+            s_mark[at] = (uint16_t)at;
+            s_x[at].v.rb = rb;
+            s_x[at].v.e = re;
+            s_x[at].v.near = 0;
+        };
+        for (uint32_t win = 1;; win++) {  // windows of kSplitBlock vertices from vb, up to the one holding t1 - 1
             const uint64_t v = vb + threadIdx.x, vn = vb + kSplitBlock;
             const uint64_t next = vn > v_hi ? t1 : uni64(iep[vn]);
             if (v <= v_hi) {
@@ -507,15 +513,22 @@ __global__ __launch_bounds__(kSplitBlock, 8) void k_split_l1(const GraphDesc *__
                 const OffT rb = rowPtr[v], re = rowPtr[v + 1];
                 if (z > a && z > t0 && a < t1) {
                     const uint32_t at = a > t0 ? (uint32_t)(a - t0) : 0u;
-                    s_mark[at] = (uint16_t)at;
-                    s_x[at].v.rb = rb;
-                    s_x[at].v.e = re;
-                    s_x[at].v.near = 0;
+                    owner(at, rb, re);
                     if (at == 0) s_front = t0 - a;
                 }
             }
             if (next >= t1) break;  // block-uniform
             vb = vn;
+            if (win == kRowWindows) {  // block-uniform: the owners of the slots left
+                const gptr<uint64_t> iepG = to_global(iep);
+#pragma unroll 1
+                for (uint32_t i = threadIdx.x; i < nt; i += kSplitBlock) {
+                    if (t0 + i < next) continue;
+                    const uint32_t r = rightmost_le(iepG, (uint32_t)vb, v_hi, t0 + i);
+                    if (iepG[r] == t0 + i) owner(i, rowPtr[r], rowPtr[(uint64_t)r + 1]);
+                }
+                break;
+            }
         }
         __syncthreads();
         // running maximum of the marks: kPer consecutive slots a thread
@@ -1182,7 +1195,7 @@ __device__ __forceinline__ u32x4 pack_chunk(gptr<uint32_t> colInd, uint64_t end,
 // the prefix, loads the ids by two 16-byte loads of any alignment and packs
 // them.  Chunks of ids up to thr only are left unwritten: no tail holds them.
 template <typename OffT>
-__global__ __launch_bounds__(kBlock) void k_split_pack(const GraphDesc *__restrict__ desc,
+__global__ __launch_bounds__(kBlock, 8) void k_split_pack(const GraphDesc *__restrict__ desc,
                                                        const SplitDesc *__restrict__ sd) {
     __shared__ OffT s_re[kBlock], s_at[kBlock];  // a row's end; slot of its chunk 0 less the prefix
     __shared__ uint32_t s_tail[kBlock], s_near[kBlock], s_pre[kBlock], s_skip[kBlock];
@@ -1197,7 +1210,8 @@ __global__ __launch_bounds__(kBlock) void k_split_pack(const GraphDesc *__restri
     const uint32_t near_end = n > kPackNear ? n - kPackNear : 0;  // ids from here on are near
     const int layout = pack_layout(S.rows);
     const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x >> 6;
-    const uint64_t c0 = pack_slot((uint64_t)rowPtr[v_lo]), c1 = pack_slot((uint64_t)rowPtr[(uint64_t)v_hi + 1]);
+    const uint64_t p1 = rowPtr[(uint64_t)v_hi + 1];
+    const uint64_t c0 = pack_slot((uint64_t)rowPtr[v_lo]), c1 = pack_slot(p1);
     // two tiles a block, of kPackTileMin to kPackTile slots (R-MAT-20 43 us; with
     // 8,192 slots each, for which there are fewer tiles than blocks, 79)
     uint64_t slots = (c1 - c0) / (2ull * gridDim.x);
@@ -1206,9 +1220,30 @@ __global__ __launch_bounds__(kBlock) void k_split_pack(const GraphDesc *__restri
     for (uint64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
         const uint64_t s0 = c0 + tile * slots, s1 = s0 + slots < c1 ? s0 + slots : c1;
         uint64_t vb = v_lo + wave_rightmost_le(v_hi - v_lo, s0, [&](uint32_t x) { return pack_slot((uint64_t)rowPtr[(uint64_t)v_lo + x]); });
+        uint32_t win = 0;
+        uint64_t pos = 0;  // the first position of a window by positions, or 0
         for (;;) {  // windows of kBlock vertices from vb
-            const uint64_t v = vb + threadIdx.x, vn = vb + kBlock;
-            const bool more = vn <= v_hi && pack_slot((uint64_t)rowPtr[vn]) < s1;
+            uint64_t v = vb + threadIdx.x, vn = vb + kBlock;
+            const bool by_pos = pos != 0;  // block-uniform
+            if (by_pos) {  // the rows that start at one of kBlock positions
+                const uint64_t q = pos + threadIdx.x;
+                v = (uint64_t)v_hi + 1;
+                if (q < p1) {
+                    const uint32_t r = rightmost_le(rowPtr, (uint32_t)vb, v_hi, q);
+                    if ((uint64_t)rowPtr[r] == q) v = r;
+                }
+                pos += kBlock;
+                // the row after those that start before pos
+                vn = pos >= p1 ? (uint64_t)v_hi + 1
+                               : vb + 1 + wave_rightmost_le((uint32_t)(v_hi - vb), pos - 1, [&](uint32_t r) { return (uint64_t)rowPtr[vb + r]; });
+                pos = 0;
+            }
+            const uint64_t next = rowPtr[vn <= v_hi ? vn : (uint64_t)v_hi + 1];
+            const bool more = vn <= v_hi && pack_slot(next) < s1;
+            if (more && (by_pos || ++win % kRowWindows == 0)) {  // as many windows more with few positions: by these
+                const uint64_t far = vn + kRowWindows * kBlock;
+                if (far <= v_hi && (uint64_t)rowPtr[far] - next < 2 * kBlock) pos = next;
+            }
             uint32_t cnt = 0, near = 0, tail = 0, skip = 0;
             OffT re = 0, c = 0;
             if (v <= v_hi) {
