@@ -1240,10 +1240,6 @@ __global__ __launch_bounds__(kBlock, 8) void k_split_pack(const GraphDesc *__res
             }
             const uint64_t next = rowPtr[vn <= v_hi ? vn : (uint64_t)v_hi + 1];
             const bool more = vn <= v_hi && pack_slot(next) < s1;
-            if (more && (by_pos || ++win % kRowWindows == 0)) {  // as many windows more with few positions: by these
-                const uint64_t far = vn + kRowWindows * kBlock;
-                if (far <= v_hi && (uint64_t)rowPtr[far] - next < 2 * kBlock) pos = next;
-            }
             uint32_t cnt = 0, near = 0, tail = 0, skip = 0;
             OffT re = 0, c = 0;
             if (v <= v_hi) {
@@ -1306,6 +1302,10 @@ __global__ __launch_bounds__(kBlock, 8) void k_split_pack(const GraphDesc *__res
             }
             if (!more) break;  // block-uniform
             vb = vn;
+            if (by_pos || ++win % kRowWindows == 0) {  // few positions in as many windows more: by these
+                const uint64_t far = vn + kRowWindows * kBlock;
+                if (far <= v_hi && uni64(rowPtr[far] - next) < 2 * kBlock) pos = uni64(next);
+            }
             __syncthreads();  // s_w is read
         }
         __syncthreads();
