@@ -329,11 +329,10 @@ int split_layout(SplitDesc *sd, DenseDesc *dd, SplitGrids *grids, char *base, ui
 }
 
 // A bitmap length whose row does not fit one block's LDS (or a graph whose
-// keys overflow the transposition's parts, or whose ids the slab kernel's hash
-// sets could not hold) is counted by the row walk
+// keys overflow the transposition's parts) is counted by the row walk
 // against the bitmap in HBM, as the reference does.
 bool split_eligible(const Tuning &t, const GraphDesc &d, uint64_t m) {
-    return t.kernel == kKernelSplit && d.mode == kModeTiles && d.a > 0 && d.bm_rows > 0 && d.n <= kSetIdsEnd &&
+    return t.kernel == kKernelSplit && d.mode == kModeTiles && d.a > 0 && d.bm_rows > 0 &&
            (uint64_t)d.bm_rows + split_slabs(m) <= (uint64_t)kSplitPartsMax << kSplitPartMax &&
            split_rows_lds(d.bm_rows) <= t.lds_bytes && (reinterpret_cast<uintptr_t>(d.colInd) & 15u) == 0;
 }
@@ -474,7 +473,7 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
             hd[0].rowPtr = rp32;
         }
         WTC_HIPC(split_rows_grid(split_ob, split_rows, t.split_wpb, t.num_cus, &s.rows_grid));
-        WTC_HIPC(split_slabs_grid(split_ob, t.num_cus, &s.slabs_grid));
+        WTC_HIPC(split_slabs_grid(split_ob, hd[0].n, t.num_cus, &s.slabs_grid));
     }
     std::memcpy(s.h_desc.p, hd.data(), (size_t)G * sizeof(GraphDesc));
     if (split) {
@@ -568,7 +567,7 @@ int launch_set(Slot &s, const SetPlan &p, bool timed, bool desc_ready) {
         if (timed) WTC_HIPC(hipEventRecord(s.ev[2], s.stream));
         WTC_HIPC(launch_split_rows(ddesc, sd, ob, p.split_rows, p.split_wpb, lines, s.rows_grid, s.stream));
         if (timed) WTC_HIPC(hipEventRecord(s.ev[4], s.stream));
-        WTC_HIPC(launch_split_slabs(ddesc, sd, ob, meta, lines, s.slabs_grid, s.stream));
+        WTC_HIPC(launch_split_slabs(ddesc, sd, ob, (uint32_t)(p.split_rp_n - 1), meta, lines, s.slabs_grid, s.stream));
         if (timed) WTC_HIPC(hipEventRecord(s.ev[3], s.stream));
         WTC_HIPC(launch_publish(meta, lines, s.h_out.as<uint64_t>(), kMetaSlots + p.G, s.stream));
         return WTC_OK;

@@ -113,7 +113,8 @@ __global__ __launch_bounds__(kBlock) void k_dense_class(const GraphDesc *__restr
     const uint32_t v_lo = S.v_lo, v_hi = S.v_hi;
     if (threadIdx.x < kDenseClasses) s_cnt[threadIdx.x] = 0u;
     __syncthreads();
-    const uint64_t v = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    const uint64_t blk = (uint64_t)blockIdx.y * gridDim.x + blockIdx.x;
+    const uint64_t v = blk * kBlock + threadIdx.x;
     uint32_t cls = kSentinel, num = 0, pos = 0;
     uint64_t left = 0, dense_top = 0, dense_topw = 0, dense_all = 0;
     if (v < n) {
@@ -212,7 +213,7 @@ __global__ __launch_bounds__(kBlock) void k_dense_class(const GraphDesc *__restr
     if (threadIdx.x < 4) {
         uint64_t t = 0;
         for (int w = 0; w < kWavesPerBlock; w++) t += s_w[w][threadIdx.x];
-        uint64_t *to = threadIdx.x == 0 ? &part_in[(uint64_t)blockIdx.x * kBlock / kScanChunk] : &N.sums[threadIdx.x - 1];
+        uint64_t *to = threadIdx.x == 0 ? &part_in[blk * kBlock / kScanChunk] : &N.sums[threadIdx.x - 1];
         if (t) atomicAdd(reinterpret_cast<unsigned long long *>(to), (unsigned long long)t);
     }
 }
@@ -510,7 +511,11 @@ hipError_t launch_dense_class(const GraphDesc *desc, const SplitDesc *sd, const 
     k_dense_init<<<dim3(ib < 64 ? ib : 64), dim3(kBlock), 0, st>>>(dd, part_in, nblocks, counts, lines);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return WTC_LAUNCH_OFF(ob, k_dense_class, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, desc, sd, dd, part_in);
+    // a grid's threads in one direction are below 2^32
+    const uint32_t blocks = (uint32_t)(((uint64_t)n + kBlock - 1) / kBlock);
+    constexpr uint32_t kX = 1u << 23;
+    const dim3 grid(blocks < kX ? blocks : kX, (blocks + kX - 1) / kX);
+    return WTC_LAUNCH_OFF(ob, k_dense_class, grid, dim3(kBlock), 0, st, desc, sd, dd, part_in);
 }
 
 hipError_t launch_dense_count(const GraphDesc *desc, const DenseDesc *dd, int ob, uint32_t core, int num_cus,

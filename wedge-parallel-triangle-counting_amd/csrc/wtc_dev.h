@@ -199,7 +199,7 @@ __device__ __forceinline__ uint32_t wave_rightmost_le(uint32_t hi, uint64_t t, F
     const uint32_t lane = threadIdx.x & (kWave - 1);
     uint32_t lo = 0;  // f(lo) <= t
     while (lo < hi) {
-        const uint32_t step = (hi - lo + kWave - 1) / kWave;
+        const uint32_t step = (hi - lo - 1) / kWave + 1;
         const uint64_t at = (uint64_t)lo + (uint64_t)(lane + 1) * step;
         const bool le = at <= hi && f((uint32_t)at) <= t;
         const uint32_t k = (uint32_t)__builtin_popcountll(__ballot(le));  // a prefix of the lanes

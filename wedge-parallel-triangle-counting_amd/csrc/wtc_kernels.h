@@ -154,7 +154,7 @@ constexpr uint32_t kKeyChunk = 4 * kSplitBlock;
 constexpr uint32_t kSlabSpan = 2048;
 constexpr uint32_t kSlabRowMax = 1024;
 constexpr uint32_t kSlabWin = kSlabSpan + kSlabRowMax;
-constexpr uint32_t kSetIdsEnd = 0x7fffffffu;  // the LDS sets of ids (wtc_set.h) hold ids below this
+constexpr uint32_t kSetIdsEnd = 0x7fffffffu;  // the LDS sets of ids (wtc_set.h) hold ids below this, but for the wide ones
 constexpr uint32_t kSlabLong = 72;  // list tails are streamed by eight lanes where they hold this many ids on average
 constexpr uint32_t kSlabFree = 0x7fffffffu;  // a free slot (ids are below it)
 constexpr uint32_t kSlabMore = 0x80000000u;  // on a bucket's last slot: ids of the bucket are in the next, too

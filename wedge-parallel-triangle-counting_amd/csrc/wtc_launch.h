@@ -107,9 +107,9 @@ uint32_t split_far_ids(uint32_t rows);
 hipError_t split_rows_grid(int ob, uint32_t rows, int wpb, int num_cus, uint32_t *grid);
 hipError_t launch_split_rows(const GraphDesc *desc, const SplitDesc *sd, int ob, uint32_t rows, int wpb,
                              uint64_t *lines, uint32_t grid, hipStream_t st);
-// Persistent grid of the slab kernel (the list rows).
-hipError_t split_slabs_grid(int ob, int num_cus, uint32_t *grid);
-hipError_t launch_split_slabs(const GraphDesc *desc, const SplitDesc *sd, int ob, const uint64_t *meta,
+// Persistent grid of the slab kernel (the list rows) for a graph of n vertices.
+hipError_t split_slabs_grid(int ob, uint32_t n, int num_cus, uint32_t *grid);
+hipError_t launch_split_slabs(const GraphDesc *desc, const SplitDesc *sd, int ob, uint32_t n, const uint64_t *meta,
                               uint64_t *lines, uint32_t grid, hipStream_t st);
 // Blocks of the transposition's first level: two per CU (its LDS), and no
 // more than a block per 8192 edges.

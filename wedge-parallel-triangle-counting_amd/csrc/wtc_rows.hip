@@ -207,7 +207,7 @@ __global__ __launch_bounds__(kRowsThreads, 6) void k_rows(const GraphDesc *__res
             __syncthreads();  // the previous tile's lookups are done
 #pragma unroll
             for (uint32_t i = threadIdx.x; i < kRowsBuckets; i += kRowsThreads)
-                reinterpret_cast<uint4 *>(s_tab)[i] = make_uint4(kSetFree, kSetFree, kSetFree, kSetFree);
+                reinterpret_cast<uint4 *>(s_tab)[i] = make_uint4(kSetFree<false>, kSetFree<false>, kSetFree<false>, kSetFree<false>);
             if (threadIdx.x < kT / 64) s_first[buf ^ 1][threadIdx.x] = 0ull;
             if (threadIdx.x < kLists) s_n[buf ^ 1][threadIdx.x] = 0u;
             // windows of rows up to the one holding the tile's last position, or

@@ -1564,7 +1564,7 @@ __global__ __launch_bounds__(kWave * kWaves, (sizeof(OffT) == 4 ? 8 : 7)) void k
 // searches' chains of loads are the time (R-MAT-26 at a = 65,536: four ids a
 // lane side by side 218 ms, one after the other 308).
 // Same alignment and slack needs as the row kernel.
-template <typename OffT, int kWaves>
+template <typename OffT, int kWaves, bool kWide>
 __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc *__restrict__ desc,
                                                                 const SplitDesc *__restrict__ sd,
                                                                 const uint64_t *__restrict__ meta,
@@ -1671,10 +1671,10 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
                     const uint32_t nu = lane < naux >> 13 ? colInd[wb + (naux & kSlabAuxLong) + lane] : 0u;
                     const uint32_t st = aux & kSlabAuxLong, len = aux >> 13;
                     for (uint32_t i = lane; i < len; i += kWave)
-                        reinterpret_cast<uint4 *>(s_tab)[st + i] = make_uint4(kSetFree, kSetFree, kSetFree, kSetFree);
+                        reinterpret_cast<uint4 *>(s_tab)[st + i] = make_uint4(kSetFree<kWide>, kSetFree<kWide>, kSetFree<kWide>, kSetFree<kWide>);
                     for (uint32_t i = lane; i < len; i += kWave) {
                         if (i >= kWave) u = colInd[wb + st + i];
-                        set_insert(s_tab, st, len, u);
+                        set_insert<kWide>(s_tab, st, len, u);
                     }
                     aux = naux;
                     u = nu;
@@ -1701,7 +1701,7 @@ __global__ __launch_bounds__(kWave * kWaves) void k_split_slabs(const GraphDesc 
                         u32x4 b = a;
                         if (left > step) b = *reinterpret_cast<gptr<u32x4>>(p + step);
                         const uint32_t u[4] = {a[0], a[1], a[2], a[3]};
-                        h += set_hits(s_tab, u, left, st, len);
+                        h += set_hits<kWide>(s_tab, u, left, st, len);
                         if (left <= step) break;
                         left -= step;
                         p += step;
@@ -1922,26 +1922,32 @@ hipError_t launch_split_rows(const GraphDesc *desc, const SplitDesc *sd, int ob,
 // The slab kernel's block (three to a CU by their LDS).
 constexpr int kSlabWaves = 8;
 
-static const void *split_slabs_kernel(int ob) {
-    return ob == 8 ? reinterpret_cast<const void *>(&k_split_slabs<uint64_t, kSlabWaves>)
-                   : reinterpret_cast<const void *>(&k_split_slabs<uint32_t, kSlabWaves>);
+template <bool kWide>
+static const void *split_slabs_fn(int ob) {
+    return ob == 8 ? reinterpret_cast<const void *>(&k_split_slabs<uint64_t, kSlabWaves, kWide>)
+                   : reinterpret_cast<const void *>(&k_split_slabs<uint32_t, kSlabWaves, kWide>);
 }
 
-hipError_t split_slabs_grid(int ob, int num_cus, uint32_t *grid) {
+// The slab kernel for a graph of n vertices (its sets of ids).
+static const void *split_slabs_kernel(int ob, uint32_t n) {
+    return n > kSetIdsEnd ? split_slabs_fn<true>(ob) : split_slabs_fn<false>(ob);
+}
+
+hipError_t split_slabs_grid(int ob, uint32_t n, int num_cus, uint32_t *grid) {
     int per_cu = 0;
     hipError_t e =
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, split_slabs_kernel(ob), kSlabWaves * kWave, 0);
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, split_slabs_kernel(ob, n), kSlabWaves * kWave, 0);
     if (e != hipSuccess) return e;
     if (per_cu < 1) return hipErrorInvalidConfiguration;
     *grid = (uint32_t)per_cu * (uint32_t)(num_cus > 0 ? num_cus : 1);
     return hipSuccess;
 }
 
-hipError_t launch_split_slabs(const GraphDesc *desc, const SplitDesc *sd, int ob, const uint64_t *meta,
+hipError_t launch_split_slabs(const GraphDesc *desc, const SplitDesc *sd, int ob, uint32_t n, const uint64_t *meta,
                               uint64_t *lines, uint32_t grid, hipStream_t st) {
     if (grid == 0) return hipErrorInvalidValue;
     void *args[] = {&desc, &sd, &meta, &lines};
-    return hipLaunchKernel(split_slabs_kernel(ob), dim3(grid), dim3(kSlabWaves * kWave), args, 0, st);
+    return hipLaunchKernel(split_slabs_kernel(ob, n), dim3(grid), dim3(kSlabWaves * kWave), args, 0, st);
 }
 
 }  // namespace wtc
