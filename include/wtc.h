@@ -346,7 +346,8 @@ int wtc_count_noalloc(const void *d_row_ptr, uint32_t offset_bytes, const uint32
 /* Diagnostics for parity tests: the device wedge prefix (n+1 entries, the
  * h_wedgeSum of tc.cu:348-361), the 4095-entry search tree (the
  * c_binary_search_cache of tc.cu:364-368, filled for single-graph counts) and
- * the bitmap words (tc.cu:329-346) left by the last count on `ctx`. */
+ * the bitmap words (tc.cu:329-346) left by the last count on `ctx`.
+ * WTC_ERR_ARG if that was a row or split count, which leave neither. */
 int wtc_ctx_debug_prefix(wtc_ctx *ctx, uint64_t n, uint64_t *wedge_sum, uint64_t *tree);
 int wtc_ctx_debug_bitmap(wtc_ctx *ctx, uint64_t words, uint32_t *out);
 /* What the dense part of the last split count on `ctx` took (the wedges among

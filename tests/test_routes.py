@@ -97,3 +97,32 @@ ctx.use_tuned(wtc.autotune_shape(graphs[0].n, graphs[0].m, graphs[0].wedges(), b
 assert all(ran(ks, "k_count_small") for ks in batches(ctx))
 assert serves(0, "k_count_small")
 """, {"WTC_SMALL_GRAPH_WORDS": "20480"})
+
+
+def test_prefix_and_bitmap_of_a_count_that_has_none(tmp_path):
+    """The debug copies of the wedge prefix and the bitmap are of the last count:
+    after a row or split count, which leave neither, they are refused instead
+    of showing an earlier count's."""
+    fake_gpu.run(tmp_path, BAND + """
+def refused(f):
+    try:
+        f()
+    except wtc.WtcError as e:
+        return e.code == -1
+    return False
+
+
+g = band(5000, 40)
+ctx = wtc.Context(0)
+dg = ctx.upload(g)
+ctx.set_count_kernel(wtc.KERNEL_WALK)
+dg.count(8, 64)
+ctx.debug_prefix(g.n), ctx.debug_bitmap(128)
+for kernel in (wtc.KERNEL_ROWS, wtc.KERNEL_SPLIT):
+    ctx.set_count_kernel(kernel)
+    dg.count(8, 64)
+    assert refused(lambda: ctx.debug_prefix(g.n)) and refused(lambda: ctx.debug_bitmap(128)), kernel
+    ctx.set_count_kernel(wtc.KERNEL_STAGED)
+    dg.count(8, 64)
+    ctx.debug_prefix(g.n), ctx.debug_bitmap(128)
+""")

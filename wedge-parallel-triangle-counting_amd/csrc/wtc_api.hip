@@ -1056,9 +1056,10 @@ int wtc_ctx_debug_split(wtc_ctx *c, uint64_t *dense_top_wedges, uint64_t *dense_
 }
 
 // Copies the wedge prefix and search tree left by the last single-graph count
-// on this context (diagnostics for the parity tests).
+// on this context (diagnostics for the parity tests).  A row count has neither,
+// a split count its own.
 int wtc_ctx_debug_prefix(wtc_ctx *c, uint64_t n, uint64_t *wedge_sum, uint64_t *tree) {
-    if (!c) return WTC_ERR_ARG;
+    if (!c || c->slot.rows || c->slot.split) return WTC_ERR_ARG;
     WTC_HIPC(hipSetDevice(c->device));
     if (wedge_sum) {
         if (c->slot.ws.cap < (n + 1) * sizeof(uint64_t)) return WTC_ERR_ARG;
@@ -1072,7 +1073,7 @@ int wtc_ctx_debug_prefix(wtc_ctx *c, uint64_t n, uint64_t *wedge_sum, uint64_t *
 }
 
 int wtc_ctx_debug_bitmap(wtc_ctx *c, uint64_t words, uint32_t *out) {
-    if (!c || !out) return WTC_ERR_ARG;
+    if (!c || !out || c->slot.rows || c->slot.split) return WTC_ERR_ARG;
     if (c->slot.bm.cap < words * sizeof(uint32_t)) return WTC_ERR_ARG;
     WTC_HIPC(hipSetDevice(c->device));
     WTC_HIPC(hipMemcpy(out, c->slot.bm.p, words * sizeof(uint32_t), hipMemcpyDeviceToHost));
