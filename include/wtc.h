@@ -243,15 +243,19 @@ int wtc_ctx_set_tuning(wtc_ctx *ctx, int probe_ways, uint32_t lds_chunk, int wav
  *                     probes, tc.cu:273-286) against hash sets of adj+(w)
  *                     in LDS.  No a*a/8-byte bitmap in HBM; about 27 or 43
  *                     bytes per edge of workspace (4- or 8-byte offsets)
- *                     instead.  Batches, a = 0, a row of a bits that does
- *                     not fit a block's LDS and colInd not 16-byte aligned:
- *                     the row walk.  Same count for every wedge range.
+ *                     instead.  a = 0: a whole graph by the row count
+ *                     (below), a range of it by the staged kernel up to 2^22
+ *                     edges, else the row walk.  Batches, a row of a bits that
+ *                     does not fit a block's LDS and colInd not 16-byte
+ *                     aligned: the row walk.  Same count for every wedge
+ *                     range.
  *   WTC_KERNEL_ROWS   whole graphs, alone or in sets: every edge v -> w
  *                     closes |adj+(v) and adj+(w)| triangles; the rows of v
  *                     of 512 edges at a time hashed into LDS, adj+(w)
- *                     streamed through them.  No prefix, no bitmap (the
- *                     spread and bitmap length have no effect), three
- *                     launches.  Wedge ranges: WTC_KERNEL_STAGED.
+ *                     streamed through them, or the rest of v's row searched
+ *                     in adj+(w) where that is far longer.  No prefix, no
+ *                     bitmap (the spread and bitmap length have no effect),
+ *                     three launches.  Wedge ranges: WTC_KERNEL_STAGED.
  * Default WTC_KERNEL_WALK or $WTC_COUNT_KERNEL. */
 #define WTC_KERNEL_WALK 0
 #define WTC_KERNEL_STAGED 1

@@ -156,8 +156,6 @@ constexpr uint32_t kSlabRowMax = 1024;
 constexpr uint32_t kSlabWin = kSlabSpan + kSlabRowMax;
 constexpr uint32_t kSetIdsEnd = 0x7fffffffu;  // the LDS sets of ids (wtc_set.h) hold ids below this, but for the wide ones
 constexpr uint32_t kSlabLong = 72;  // list tails are streamed by eight lanes where they hold this many ids on average
-constexpr uint32_t kSlabFree = 0x7fffffffu;  // a free slot (ids are below it)
-constexpr uint32_t kSlabMore = 0x80000000u;  // on a bucket's last slot: ids of the bucket are in the next, too
 constexpr uint32_t kSlabTile = 1024, kSlabTileMin = 128, kSlabCost = 48;  // a tile's work; a slab's share of it
 
 // Workspace and device-filled state of a split count.  The top rows are the
@@ -242,8 +240,8 @@ constexpr uint32_t kDenseSparsest = 32;
 // as much moves R-MAT-20 to R-MAT-26 by less than 1% (half: R-MAT-22 6%).
 constexpr float kDenseEdgeCost = 75000.0f, kDenseWedgeCost = 1050.0f;
 // sums[]: the dense in-edges whose middle vertex is a top row, their wedges,
-// all dense in-edges, and the product's work counter.
-enum : uint32_t { kDenseTopEdges = 0, kDenseTopWedges = 1, kDenseEdges = 2, kDenseNext = 3, kDenseSums = 4 };
+// and all dense in-edges.
+enum : uint32_t { kDenseTopEdges = 0, kDenseTopWedges = 1, kDenseEdges = 2, kDenseSums = 3 };
 
 struct DenseDesc {
     void *R;                             // core x core bits: the rows of the last `core` ranks

@@ -44,8 +44,9 @@ bool valid_count_waves(int wpb);
 // staged through LDS).  Both count the same wedges of the same tiles.
 // kKernelSplit: a single graph with a > 0 counted by the split count (its
 // in-edges grouped by middle vertex: the top-a rows against one LDS bitmap
-// row, the rest against LDS windows of colInd; wtc_split.hip); any other set
-// with it by k_walk.
+// row, the rest against hash sets of the rows; wtc_split.hip).  With it a whole
+// graph with a = 0 is counted by the row count, a range of one by k_count or
+// k_walk by its size, and any other set by k_walk.
 // kKernelRows: whole graphs, alone or in sets, counted edge by edge against
 // hashed rows (wtc_rows.hip); wedge ranges with it by k_count.
 enum : int { kKernelWalk = 0, kKernelStaged = 1, kKernelSplit = 2, kKernelRows = 3 };

@@ -151,7 +151,7 @@ char *pool_ptr(wtc_server *s, size_t off) { return s->pool_mem.as<char>() + off;
 size_t req_ws_bytes(const SrvGraph *g) { return ((size_t)g->n + 1) * sizeof(uint64_t); }
 size_t req_bm_bytes(uint32_t a) { return a ? bm_words_for(a) * sizeof(uint32_t) : 0; }
 // Graphs of fewer wedges than this are counted by the row count where the split
-// count's workspace does not fit the budget (R-MAT-18: 0.55 ms instead of 0.35).
+// count's workspace does not fit the budget (R-MAT-18: 0.48 ms instead of 0.34).
 constexpr uint64_t kSplitOrRows = 1ull << 28;
 // What a request needs besides its graph and prefix: the split count's
 // workspace, or a bitmap.

@@ -641,7 +641,7 @@ __global__ __launch_bounds__(kSplitBlock, 8) void k_split_l1(const GraphDesc *__
                 t[u].lo = pack_row<OffT>(s_x[p].v.rb, e);
                 t[u].hi = pack_count((near + kPackNearIds - 1) / kPackNearIds, pack_div(tail - near + far_ids - 1, far_ids));
             } else {
-                                t[u] = TailPair<OffT>{j, e};
+                t[u] = TailPair<OffT>{j, e};
             }
             rank[u] = atomicAdd(&s_cnt[key[u] >> shift], 1u);
         }
@@ -1043,8 +1043,9 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_keysum(const SplitDesc *_
 
 // Block b (key_part then holding the exclusive prefix of the key blocks):
 // rp_in of its keys; the block of key `rows` puts the top rows' in-edges
-// into meta, the last block rp_in[keys] and the rest of meta (tile counters
-// and wedge tallies zeroed, the counted wedges and all in-edges).
+// into meta, the last block rp_in[keys] and the rest of meta (the wedges of
+// the two kernels, what the dense part took, the counted wedges and all
+// in-edges).
 template <typename OffT>
 __global__ __launch_bounds__(kSplitBlock) void k_split_keyscan(const SplitDesc *__restrict__ sd,
                                                                const DenseDesc *__restrict__ dd,
@@ -1360,7 +1361,8 @@ __device__ __forceinline__ uint32_t rows_tail_hits(const uint32_t *s_bits, gptr<
     return h;
 }
 
-// Persistent blocks take tiles of the rows' work from one counter.  The work
+// Persistent blocks take tiles of the rows' work from one counter, or short
+// ones from sixteen.  The work
 // of a row is kSplitRowCost for its bitmap and one unit per in-edge, so a
 // tile is up to `tile` in-edges of few rows, or fewer in-edges where rows
 // have few each: tiles of in-edges alone left blocks with hundreds of such
@@ -1538,7 +1540,7 @@ __global__ __launch_bounds__(kWave * kWaves, (sizeof(OffT) == 4 ? 8 : 7)) void k
 
 // ---------------------------------------------------------------- list part
 
-// Persistent blocks take tiles of the slabs' work from one counter: a slab's
+// Persistent blocks take tiles of the slabs' work from sixteen counters: a slab's
 // work is kSlabCost for its rows and one unit per in-edge, in tiles of at most
 // kSlabTile, as in the row kernel (with tiles of in-edges alone, those over
 // the many slabs with few in-edges took 0.45 ms on R-MAT-20 however few the
@@ -1781,7 +1783,7 @@ hipError_t launch_split_range(const GraphDesc *desc, SplitDesc *sd, int ob, hipS
 
 namespace {
 
-template <typename OffT, typename KeyIn, bool kFinal, uint32_t kF>
+template <typename KeyIn, bool kFinal, uint32_t kF>
 hipError_t launch_level_count(const SplitDesc *sd, uint32_t grid, hipStream_t st) {
     k_split_level_count<KeyIn, kFinal, kF><<<dim3(grid), dim3(kSplitBlock), 0, st>>>(sd);
     return hipGetLastError();
@@ -1798,20 +1800,20 @@ template <typename OffT>
 hipError_t launch_final(bool scatter, bool from_b, uint32_t shift, const SplitDesc *sd, uint32_t grid, hipStream_t st) {
     if (from_b)
         return scatter ? launch_level_scatter<OffT, uint8_t, true, kSplitSub>(sd, grid, st)
-                       : launch_level_count<OffT, uint8_t, true, kSplitSub>(sd, grid, st);
+                       : launch_level_count<uint8_t, true, kSplitSub>(sd, grid, st);
     switch (shift) {
         case 8:
             return scatter ? launch_level_scatter<OffT, uint16_t, true, 256>(sd, grid, st)
-                           : launch_level_count<OffT, uint16_t, true, 256>(sd, grid, st);
+                           : launch_level_count<uint16_t, true, 256>(sd, grid, st);
         case 9:
             return scatter ? launch_level_scatter<OffT, uint16_t, true, 512>(sd, grid, st)
-                           : launch_level_count<OffT, uint16_t, true, 512>(sd, grid, st);
+                           : launch_level_count<uint16_t, true, 512>(sd, grid, st);
         case 10:
             return scatter ? launch_level_scatter<OffT, uint16_t, true, 1024>(sd, grid, st)
-                           : launch_level_count<OffT, uint16_t, true, 1024>(sd, grid, st);
+                           : launch_level_count<uint16_t, true, 1024>(sd, grid, st);
         case 11:
             return scatter ? launch_level_scatter<OffT, uint16_t, true, 2048>(sd, grid, st)
-                           : launch_level_count<OffT, uint16_t, true, 2048>(sd, grid, st);
+                           : launch_level_count<uint16_t, true, 2048>(sd, grid, st);
         default: return hipErrorInvalidValue;
     }
 }
@@ -1833,7 +1835,7 @@ hipError_t transpose(const GraphDesc *desc, const SplitDesc *sd, const DenseDesc
     k_split_bases<false><<<dim3(1), blk, 0, st>>>(sd);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (three) {
-        if ((e = launch_level_count<OffT, uint16_t, false, kSplitFan2>(sd, g2, st)) != hipSuccess) return e;
+        if ((e = launch_level_count<uint16_t, false, kSplitFan2>(sd, g2, st)) != hipSuccess) return e;
         k_split_levelcols2<<<dim3(g.parts), blk, 0, st>>>(sd);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         k_split_bases<true><<<dim3(1), blk, 0, st>>>(sd);
