@@ -1,6 +1,10 @@
 """The tc_GPU drop-ins on a CSR whose offsets do not fit its edge count: such a
 call is refused from its two end offsets, before colInd, which may be shorter
 than numEdges says, is read and before anything is allocated."""
+import os
+import shutil
+import subprocess
+
 import pytest
 
 import fake_gpu
@@ -74,3 +78,13 @@ def test_without_a_thread_to_check_on(tmp_path, threads):
     """Where no thread can be started the check runs on the calling thread: no
     exception leaves the C entry, and none ends the process."""
     fake_gpu.run(tmp_path, THREADS, {"WTC_HOST_THREADS": str(threads)})
+
+
+def test_the_check_lies_on_a_cache_line():
+    """The check's loop is not inlined where its alignment, and with it a tc_GPU
+    call's time, would change with other code."""
+    if shutil.which("nm") is None:
+        pytest.skip("needs nm")
+    out = subprocess.run(["nm", "-C", os.path.join(fake_gpu.PKG, "libwtc.so")], check=True, capture_output=True, text=True)
+    at = [int(x.split()[0], 16) for x in out.stdout.splitlines() if "int wtc::validate_oriented_rows_t<" in x]
+    assert len(at) >= 2 and all(a % 64 == 0 for a in at), at
