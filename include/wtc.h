@@ -283,8 +283,9 @@ int wtc_ctx_set_work_split(wtc_ctx *ctx, uint32_t tiles_per_grab, int deal_to_xc
  * (device_max_words; 40960 on MI355X).  Default 20480 or
  * $WTC_SMALL_GRAPH_WORDS.  Where the row count is the counting kernel
  * (WTC_KERNEL_ROWS, which the autotuner takes for batches, and the server), it
- * is the faster one for small sets too and takes them unless the limit has
- * been set, by this call or by that variable.  Counts do not depend on it. */
+ * takes the small sets that it is the faster one for by their sizes, unless the
+ * limit has been set, by this call or by that variable.  Counts do not depend
+ * on it. */
 int wtc_ctx_set_small_graphs(wtc_ctx *ctx, uint32_t max_words);
 int wtc_ctx_get_small_graphs(const wtc_ctx *ctx, uint32_t *max_words, uint32_t *device_max_words);
 
@@ -418,8 +419,8 @@ typedef struct {
     int32_t waves_per_block;   /* 1, 2, 4 or 8 waves, 0 = 4                       */
     int32_t small_graph_words; /* sets of graphs up to this many words by the small-graph
                                   kernel (wtc_ctx_set_small_graphs); 0 = as
-                                  $WTC_SMALL_GRAPH_WORDS says, without it by the row
-                                  count, as -1                                    */
+                                  $WTC_SMALL_GRAPH_WORDS says, without it where it is
+                                  faster than the row count; -1 = off             */
 } wtc_server_config;
 typedef struct {
     double queue_ms;      /* submit -> batch start                                */

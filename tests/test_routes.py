@@ -126,3 +126,28 @@ for kernel in (wtc.KERNEL_ROWS, wtc.KERNEL_SPLIT):
     dg.count(8, 64)
     ctx.debug_prefix(g.n), ctx.debug_bitmap(128)
 """)
+
+
+def test_small_sets_by_the_faster_kernel(tmp_path):
+    """Where the row count is the chosen kernel it takes the sets of small graphs
+    that it is the faster one for: small sets, graphs of few edges, or of many
+    wedges an edge; large sets of sparse graphs of a thousand vertices or more go
+    to the small-graph kernel."""
+    fake_gpu.run(tmp_path, BAND + """
+def sparse(n, m0):
+    return wtc.preprocess(wtc.gen_barabasi_albert(n, m0, seed=3))
+
+
+for g, k, small in ((sparse(64, 4), 2000, False), (sparse(250, 4), 2000, False), (sparse(1000, 4), 2000, True),
+                    (sparse(1000, 4), 40, False), (sparse(1000, 16), 2000, False), (sparse(2000, 2), 2000, True),
+                    (sparse(2000, 6), 2000, True), (sparse(2000, 6), 2, False), (sparse(4000, 2), 2000, True),
+                    (band(130, 129), 500, False),
+                    (sparse(4000, 8), 500, False)):  # the last has more words than the limit
+    ctx = wtc.Context(0)
+    ctx.use_tuned(wtc.autotune_shape(g.n, g.m, g.wedges(), batch=True))
+    graphs = [g] * k
+    b = wtc.Batch(ctx, graphs)
+    for call in (lambda: b.count([8] * k, [0] * k), lambda: wtc.batch_count_host(ctx, graphs, [8] * k, [0] * k)):
+        ks = launches(call)
+        assert ran(ks, "k_count_small") == small and ran(ks, "k_rows") != small, (g.n, g.m, g.wedges(), k, ks)
+""")

@@ -346,6 +346,31 @@ bool split_eligible(const Tuning &t, const GraphDesc &d, uint64_t m) {
 // walk is as fast or faster (scale 20 1.88 ms against 2.06).
 constexpr uint64_t kNoTopStaged = 1ull << 22;
 
+// Whether a set of small graphs is better counted by the small-graph kernel than
+// by the row count: what either takes in nanoseconds, fitted to 196 sets of 2 to
+// 20,000 graphs.  The small-graph kernel takes its launches and one block's time
+// (the more, the more words it stages), and then for a graph, for the words of
+// each of its slices and for its wedges; the row count its launches, and then for
+// its tiles of edges, however full (more where a block gets only a few of them),
+// and little for the wedges.  So small sets, graphs of a tile or two and graphs of
+// many wedges an edge go to the row count (20,000 Barabasi-Albert graphs of 64
+// vertices and 4 edges each 0.25 ms against 0.47, 7,155 complete graphs of 130
+// 2.7 against 9.0, two of 2,000 vertices 0.040 against 0.053), large ones of
+// sparse graphs of a thousand vertices or more to the small-graph kernel (7,515
+// of 2,000 vertices and 4 edges each 0.55 ms against 1.06).  The worst of the 196
+// choices costs 11%.
+bool small_kernel_faster(const std::vector<GraphDesc> &hd, const uint64_t *m, const uint64_t *W) {
+    double small = 0, wedges = 0, tiles = 0, most = 0;
+    for (size_t g = 0; g < hd.size(); g++) {
+        const double words = 2.0 * ((double)hd[g].n + 1) + (double)m[g], parts = small_parts_of(W[g]);
+        small += 19.7 + 0.33 * parts + (1.28e-3 * parts + 0.94e-3) * words + 2.61e-3 * (double)W[g];
+        tiles += (double)((m[g] + kRowsTile - 1) / kRowsTile);
+        wedges += (double)W[g];
+        most = std::max(most, words);
+    }
+    return 42000.0 + 1.5 * most + small < 36000.0 + 8.0 * tiles + std::min(4.0 * tiles, 12288.0) + 1.4e-3 * wedges;
+}
+
 int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *plan, const uint64_t *m,
               const uint64_t *W, char *split_base) {
     const uint32_t G = (uint32_t)hd.size();
@@ -359,16 +384,16 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
     // graph, CSR in LDS, so no bitmap); any other set by the wedge-parallel
     // kernel.  Mixing the two in one set runs them back to back, and the
     // small kernel's per-graph tail then costs more than it saves.
-    // Where the row count is the choice it takes small sets as well, unless the
-    // caller has set the limit himself: replays
-    // of 4,096 graphs of n <= 512 in 0.178 ms against 0.251, of n <= 1024 in
-    // 0.273 against 0.401.
+    // Where the row count is the choice it takes the small sets that it is the
+    // faster one for, unless the caller has set the limit: replays of 4,096 graphs
+    // of n <= 512 in 0.178 ms against 0.251, of n <= 1024 in 0.273 against 0.401.
     uint32_t small_words = 0, small_n = 0;
     uint64_t small_parts = 0;
     const uint32_t small_cap = std::min(t.small_words, t.small_words_max);
-    bool all_small = m && W && G >= 2 && small_cap > 0 && (!want_rows || t.small_asked);
+    bool all_small = m && W && G >= 2 && small_cap > 0;
     for (uint32_t g = 0; g < G && all_small; g++)
         all_small = hd[g].n > 0 && 2 * ((uint64_t)hd[g].n + 1) + m[g] <= small_cap;
+    if (all_small && want_rows && !t.small_asked) all_small = small_kernel_faster(hd, m, W);
     for (uint32_t g = 0; g < G; g++) {
         GraphDesc &d = hd[g];
         d.mode = kModeTiles;

@@ -126,7 +126,7 @@ struct Tuning {
     uint32_t small_words = 0;
     uint32_t small_words_max = 0;
     // the caller set small_words: such sets go to that kernel where the row
-    // count is the choice, too
+    // count is the choice, too, whichever is faster
     bool small_asked = false;
     // LDS per block in bytes: the split count's row bitmap (a bits) must fit
     size_t lds_bytes = 0;

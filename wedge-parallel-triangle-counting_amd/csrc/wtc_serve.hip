@@ -387,7 +387,8 @@ int wtc_server_create(int device, const wtc_server_config *cfg, wtc_server **out
     s->tune.wpb = s->cfg.waves_per_block;
     // a request whose graph the autotuner counts by the split count runs
     // alone with its workspace from the pool, any other set by the row count
-    // (of small graphs by their kernel if the configuration says up to which size)
+    // (of small graphs by their kernel where that is faster, or up to the size that
+    // the configuration says)
     s->tune.kernel = kKernelSplit;
     s->tune.split_needs_base = true;
     s->tune.rows_else = true;

@@ -503,7 +503,8 @@ class Context:
     def set_small_graphs(self, max_words: int):
         """In counts over two or more graphs, graphs with 2(n+1) + m <=
         max_words are counted from LDS by the small-graph kernel (0: off);
-        without a call, not where the row count is the counting kernel."""
+        without a call, not where the row count is the counting kernel and
+        the faster one."""
         _check(_lib.wtc_ctx_set_small_graphs(self._p, max_words), "set_small_graphs")
 
     def small_graphs(self):
