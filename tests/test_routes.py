@@ -151,3 +151,16 @@ for g, k, small in ((sparse(64, 4), 2000, False), (sparse(250, 4), 2000, False),
         ks = launches(call)
         assert ran(ks, "k_count_small") == small and ran(ks, "k_rows") != small, (g.n, g.m, g.wedges(), k, ks)
 """)
+
+
+def test_graphs_without_wedges_take_no_tiles(tmp_path):
+    """A set whose graphs have no wedges launches no counting kernel."""
+    fake_gpu.run(tmp_path, BAND + """
+ctx = wtc.Context(0)
+ctx.set_count_kernel(wtc.KERNEL_ROWS)
+star = wtc.preprocess(wtc.graph_from_pairs(np.stack([np.zeros(30000, int), 1 + np.arange(30000)], axis=1).astype(np.uint32)))
+for graphs, kernel in (([star] * 3, False), ([star, band(20000, 5), star], True)):
+    b = wtc.Batch(ctx, graphs)
+    ks = launches(lambda: b.count([8] * 3, [0] * 3))
+    assert ran(ks, "k_rows_init") and ran(ks, "k_rows") == kernel, ks
+""")

@@ -416,15 +416,18 @@ int stage_set(Slot &s, Tuning &t, int ob, std::vector<GraphDesc> &hd, SetPlan *p
     uint64_t rows_tiles = 0, rows_edges = 0;
     uint32_t &rg = t.rows_grid[ob == 8 ? 1 : 0];
     if (rows_ok && !rg) WTC_HIPC(rows_grid(ob, t.num_cus, &rg));
-    for (uint32_t g = 0; g < G && rows_ok; g++) rows_edges += m[g];
+    // a graph known to have no wedges has nothing to count (a set of 610 stars of
+    // 65,536 vertices 0.55 ms, without their tiles 0.05)
+    auto row_edges = [&](uint32_t g) -> uint64_t { return W && W[g] == 0 ? 0 : m[g]; };
+    for (uint32_t g = 0; g < G && rows_ok; g++) rows_edges += row_edges(g);
     const uint32_t tile_edges = rows_ok ? rows_tile_edges(rows_edges, rg) : kRowsTile;
     for (uint32_t g = 0; g < G && rows_ok; g++) {
         hd[g].bm_rows = 0;
         hd[g].bm_words = 0;
         hd[g].bitmap = nullptr;
-        hd[g].wcount = m[g];
+        hd[g].wcount = row_edges(g);
         hd[g].tile_base = rows_tiles;
-        rows_tiles += (m[g] + tile_edges - 1) / tile_edges;
+        rows_tiles += (hd[g].wcount + tile_edges - 1) / tile_edges;
     }
     // The split count takes a single graph with a bitmap length whose colInd
     // is 16-byte aligned (its slab kernel loads four ids at a time); its top
