@@ -122,13 +122,14 @@ __global__ __launch_bounds__(kRowsThreads, 6) void k_rows(const GraphDesc *__res
     __shared__ uint16_t s_list[kLists][kT];  // the edges to stream
     // rows' first positions as bits, and the lists' edges, of this tile and (zeroed) the next
     __shared__ unsigned long long s_first[2][kT / 64];
-    __shared__ uint32_t s_n[2][kLists];
+    constexpr uint32_t kCounts = 8, kRare = 4;  // list c's count at c, the rare lists' at kRare and on
+    __shared__ __align__(16) uint32_t s_n[2][kCounts];
     __shared__ uint64_t s_sum[kRowsWaves];
     const uint32_t lane = threadIdx.x & (kWave - 1), wv = uni32(threadIdx.x >> 6);
     uint32_t cur_g = kSentinel, buf = 0;
     uint64_t hits = 0, wedges = 0;
     if (threadIdx.x < kT / 64) s_first[1][threadIdx.x] = 0ull;
-    if (threadIdx.x < kLists) s_n[1][threadIdx.x] = 0u;
+    if (threadIdx.x < kCounts) s_n[1][threadIdx.x] = 0u;
     // x summed over the block (thread 0)
     auto block_sum = [&](uint64_t x) -> uint64_t {
         const uint64_t t = wave_sum(x);
@@ -209,7 +210,7 @@ __global__ __launch_bounds__(kRowsThreads, 6) void k_rows(const GraphDesc *__res
             for (uint32_t i = threadIdx.x; i < kRowsBuckets; i += kRowsThreads)
                 reinterpret_cast<uint4 *>(s_tab)[i] = make_uint4(kSetFree<false>, kSetFree<false>, kSetFree<false>, kSetFree<false>);
             if (threadIdx.x < kT / 64) s_first[buf ^ 1][threadIdx.x] = 0ull;
-            if (threadIdx.x < kLists) s_n[buf ^ 1][threadIdx.x] = 0u;
+            if (threadIdx.x < kCounts) s_n[buf ^ 1][threadIdx.x] = 0u;
             // windows of rows up to the one holding the tile's last position, or
             // kRowWindows of them and the rows of the positions left
             for (uint32_t win = 1;; win++) {
@@ -275,7 +276,7 @@ __global__ __launch_bounds__(kRowsThreads, 6) void k_rows(const GraphDesc *__res
                     uint32_t c = len <= 8 ? 0u : len <= 32 ? 1u : 2u;
                     if (len >= kRowsLong) c = len >= kRowsFew * (end - me - 1) ? kSearch : c;
                     c = long_last && st == st_last ? kUnhashed : c;
-                    s_list[c][atomicAdd(&s_n[buf][c], 1u)] = (uint16_t)me;
+                    s_list[c][atomicAdd(&s_n[buf][c + (c >= kStreams ? kRare - kStreams : 0u)], 1u)] = (uint16_t)me;
                 }
                 if (me < bl) {
                     const uint32_t r = region(st, end);
@@ -327,8 +328,10 @@ __global__ __launch_bounds__(kRowsThreads, 6) void k_rows(const GraphDesc *__res
                 }
             }
             // four lanes an edge, two ids each a step, their halvings side by side
-            if (uni32(s_n[buf][kSearch])) {
-                for (uint32_t x = (kRowsThreads - 1 - threadIdx.x) >> 2; x < uni32(s_n[buf][kSearch]); x += kRowsThreads >> 2) {
+            const uint2 rare = *reinterpret_cast<const uint2 *>(&s_n[buf][kRare]);
+            const uint32_t few = uni32(rare.x), rest = uni32(rare.y);
+            if (few) {
+                for (uint32_t x = (kRowsThreads - 1 - threadIdx.x) >> 2; x < few; x += kRowsThreads >> 2) {
                     const uint32_t i = s_list[kSearch][x], wl = s_wl[i], end = s_end[s_mark[i]];
                     const OffT from = s_ws[i];
                     for (uint32_t q = i + 1 + (lane & 3u); q < end; q += 8) {
@@ -346,7 +349,6 @@ __global__ __launch_bounds__(kRowsThreads, 6) void k_rows(const GraphDesc *__res
                     }
                 }
             }
-            const uint32_t rest = uni32(s_n[buf][kUnhashed]);
             uint64_t end = 0;
             if (rest) {  // block-uniform: the last row is not hashed
                 const uint32_t r = wave_rightmost_le(n - 1, cp0 + st_last, [&](uint32_t y) { return (uint64_t)rowPtr[y]; });
