@@ -24,13 +24,13 @@
 // 0.18 and 0.34; R-MAT-16 102 -> 96 us, R-MAT-18 0.52 -> 0.48 ms.
 //
 // Measured against the staged kernel on its tuned shape (whole call): R-MAT-12
-// 28 us instead of 146, R-MAT-16 96 instead of 329, R-MAT-18 0.48 ms instead
+// 28 us instead of 146, R-MAT-16 95 instead of 323, R-MAT-18 0.48 ms instead
 // of 0.88, Erdos-Renyi n = 10^6 of degree 16 0.21 ms instead of 0.58, 256
-// Erdos-Renyi and Barabasi-Albert graphs 1.3 ms instead of 2.83.  From 2^27
-// wedges on skewed graphs the split count is faster (R-MAT-18: 0.36 against
-// 0.48 ms, R-MAT-19: 0.50 against 1.7).  Bound by a tile's chain of loads and barriers at the 24 waves a CU
-// that its registers leave, on skewed graphs by a lookup's vector instructions
-// as well.
+// Erdos-Renyi and Barabasi-Albert graphs 1.23 ms instead of 2.69.  From 2^27
+// wedges on skewed graphs the split count is faster (R-MAT-18: 0.33 against
+// 0.48 ms, R-MAT-19: 0.47 against 1.7).  Bound by a tile's chain of loads and
+// barriers at the 24 waves a CU that its registers leave, on skewed graphs by
+// a lookup's vector instructions as well.
 #include "wtc_dev.h"
 #include "wtc_kernels.h"
 #include "wtc_launch.h"

@@ -1102,7 +1102,7 @@ __global__ __launch_bounds__(kSplitBlock) void k_split_keyscan(const SplitDesc *
 // chunk cut at fixed positions and the ends masked, a tail of R-MAT-24 touched
 // 3.3 lines and a lookup took 10.4 vector instructions; now 2.7 and 6.7.  Row
 // kernel 10.3 -> 8.4 ms there, 59.9 -> 48.2 on R-MAT-26; packing 0.39 -> 0.73
-// and 1.6 -> 2.6.
+// and 1.6 -> 2.6 (R-MAT-24 0.64 with eight waves a SIMD).
 // Layouts of the far chunks (PackLayout<L>):
 //   0: P = 6, B = 21, rows <= 2^19, field (x >> 5) << 7 | (x & 31): bits
 //      [5, 21) are the LDS byte address of x's bitmap word and bits [0, 5)
